@@ -29,14 +29,11 @@ __device__ __forceinline__ void gathered_dw_body(const GatherDwArgs& a, uint8_t*
 
   const int tiles_r = cdiv(g.R, BN);
   const int tiles_c = cdiv(g.Cc, BM);
-  const int per_grp = tiles_r * tiles_c * g.splits;
-  int L = xcd_tile_slot(2 * per_grp, bid);
+  const int L = xcd_tile_slot(2 * tiles_r * tiles_c * g.splits, bid);
   if (L < 0) return;
-  const int grp = L / per_grp;
-  L -= grp * per_grp;
-  const int split = L % g.splits;
-  const int tile = L / g.splits;
-  const int r0 = (tile % tiles_r) * BN, c0 = (tile / tiles_r) * BM;
+  const DwTileCoord tc = dw_tile_coord(L, tiles_r, tiles_c, g.splits);
+  const int grp = tc.grp, split = tc.split;
+  const int r0 = tc.tile_r * BN, c0 = tc.tile_c * BM;
 
   const int n_vis = a.counts[0];
   const int p_begin = grp == 0 ? 0 : n_vis;           // routed positions of the group: [p_begin, p_end)

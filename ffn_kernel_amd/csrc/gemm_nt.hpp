@@ -1531,14 +1531,10 @@ __device__ __forceinline__ void grouped_splitk_body(const SplitKArgs& g, uint8_t
   // row, which makes the fp32 partial stores 128-byte contiguous.
   const int tiles_r = cdiv(g.R, BN);
   const int tiles_c = cdiv(g.Cc, BM);
-  const int per_grp = tiles_r * tiles_c * g.splits;
-  int L = xcd_tile_slot(2 * per_grp, bid);
+  const int L = xcd_tile_slot(2 * tiles_r * tiles_c * g.splits, bid);
   if (L < 0) return;
-  const int grp = L / per_grp;
-  L -= grp * per_grp;
-  const int split = L % g.splits;
-  const int tile = L / g.splits;
-  const int tile_r = tile % tiles_r, tile_c = tile / tiles_r;
+  const DwTileCoord tc = dw_tile_coord(L, tiles_r, tiles_c, g.splits);
+  const int grp = tc.grp, split = tc.split, tile_r = tc.tile_r, tile_c = tc.tile_c;
 
   const int n_vis = g.counts[0];
   const int vpad = (n_vis + 63) & ~63;
