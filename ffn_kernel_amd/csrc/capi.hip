@@ -76,9 +76,12 @@ std::atomic<int> g_force_splits{-1};  // >= 1: that split-K factor where a GEMM 
 std::atomic<int> g_force_group_m{0};      // >= 1: M-tiles per super-group in the tile order of every routed GEMM
 std::atomic<int> g_force_bwd_gather{-1};  // MaskedLinear backward: 1 = weight gradients from g and x in place, 0 = from transposes, -1 = plan
 
+// Pseudo tile id of a measured weight-gradient plan: g and x read where they lie (gemm_dw_gather.hpp) on the 128x128 tile.
+constexpr int kTileGatherDw = 5;
+
 int forced_tile() {
   const int t = g_force_tile.load(std::memory_order_relaxed);
-  return (t >= 0 && t < TILE_COUNT) ? t : -1;
+  return (t >= 0 && t < TILE_COUNT && t != kTileGatherDw) ? t : -1;
 }
 bool use_tuned() { return g_force_tile.load(std::memory_order_relaxed) != -2; }
 // GemmArgs::group_m of a routed GEMM: the forced value, else the measured plan's, else 0 (the tile's own).
@@ -112,9 +115,6 @@ int resolve_routing(const ffnk_routing_t* rt, const RouteWs& r, const uint8_t* m
   out->counts = r.counts;
   return FFNK_OK;
 }
-
-// Pseudo tile id of a measured weight-gradient plan: g and x read where they lie (gemm_dw_gather.hpp) on the 128x128 tile.
-constexpr int kTileGatherDw = 5;
 
 struct BwdPlan {
   bool dw_k_contig;  // dW memory is [N, K] (k contiguous): R = N, Cc = K
@@ -299,15 +299,46 @@ RoutedPlan down_plan(int64_t M, int64_t d, int64_t h, int op = TUNED_DOWN) {
   RoutedPlan p;
   if (const int f = forced_tile(); f >= 0) {
     p.tile = f;
-    p.splits = pick_routed_splits(M, d, h, p.tile);
+    p.splits = p.splits_more = pick_routed_splits(M, d, h, p.tile);
   } else {
     p = pick_routed_plan(M, d, h, use_tuned(), op);
   }
   // a forced split-K factor: whole 64-element slabs, no empty range, what the reduce pass can address
   if (const int fs = forced_splits(); fs >= 1 && h % 64 == 0 && M < 65536 && cdiv64(h / 64, cdiv64(h / 64, fs)) == fs &&
       p.tile != TILE_256x256_W4)
-    p.splits = fs;
+    p.splits = p.splits_more = fs;
   return p;
+}
+int max_splits(const RoutedPlan& p) { return p.splits > p.splits_more ? p.splits : p.splits_more; }
+// fp32 tiles of the split tail of an unsplit 256x256 tile: only a launch of more than one round has one.
+size_t tail_bytes(const RoutedPlan& p, int64_t M, int64_t n_out, int64_t K) {
+  return is_big_tile(p.tile) && K % 64 == 0 && (cdiv64(M, 256) + 1) * cdiv64(n_out, 256) > kCus
+             ? ws_align((size_t)kTailSlots * 256 * 256 * 4) : 0;
+}
+// The MaskedFFN forward's down projection.  Where the scratch of the static entry point holds what the plan by tile count
+// alone (pick_routed_plan with TUNED_NONE) needs but not what the model's plan needs, the model's split factor is cut to what
+// fits, or the other plan runs: which shapes the static entry point takes does not depend on the model.
+RoutedPlan ffn_down_plan(int64_t M, int64_t d, int64_t h) {
+  RoutedPlan p = down_plan(M, d, h);
+  if (forced_tile() >= 0 || forced_splits() >= 1) return p;
+  const size_t fixed = route_ws_bytes(M) + ws_align((size_t)M * round_up64(h, 8) * 2), part = (size_t)M * d * 4;
+  auto fits = [&](const RoutedPlan& q) {
+    const int s = max_splits(q);
+    return fixed + (s > 1 ? ws_align(s * part) : tail_bytes(q, M, d, h)) <= (size_t)FFNK_STATIC_SCRATCH_BYTES;
+  };
+  if (fixed > (size_t)FFNK_STATIC_SCRATCH_BYTES || fits(p)) return p;
+  const RoutedPlan plain = pick_routed_plan(M, d, h, false, TUNED_NONE);
+  if (!fits(plain)) return p;
+  if (p.splits > 1) {
+    for (int s = max_splits(p) - 1; s >= 2; --s) {
+      if (!routed_split_ok(h, s)) continue;
+      RoutedPlan q = p;
+      if (q.splits > s) q.splits = s;
+      if (q.splits_more > s) q.splits_more = s;
+      if (fits(q)) return q;
+    }
+  }
+  return plain;
 }
 // dx GEMM of the MaskedFFN backward: few output tiles over a 2h-long contraction, so K is split like the forward's
 // down projection when the fp32 partials fit `room`; an unsplit big tile wants room for its split tail instead.
@@ -316,7 +347,7 @@ RoutedPlan ffn_bwd_dx_plan(int64_t M, int64_t d, int64_t h, bool dx_direct, size
   // projection reads K-contiguous weights through another loop).
   RoutedPlan dxp = down_plan(M, d, 2 * h, TUNED_NONE);
   if (!dx_direct || (size_t)dxp.splits * M * d * 4 > room) {
-    dxp.splits = 1;
+    dxp.splits = dxp.splits_more = 1;
     dxp.tile = routed_tile(M, d, false, 0, TUNED_NONE);
   }
   size_t n = 0;
@@ -367,29 +398,25 @@ int linear_stream_splits(int64_t M, int64_t K, int64_t N) {
 // MaskedLinear forward: the table's tile unless cutting K pays (few output tiles, long contraction).
 RoutedPlan linear_plan(int64_t M, int64_t K, int64_t N) {
   RoutedPlan p = down_plan(M, N, K, TUNED_PLAIN);
-  if (N % 4 != 0) p.splits = 1;  // the reduce pass moves four columns per thread
-  if (p.splits == 1) p.tile = routed_tile(M, N, false, K, TUNED_PLAIN);
+  if (N % 4 != 0) p.splits = p.splits_more = 1;  // the reduce pass moves four columns per thread
   return p;
 }
 // fp32 partials of the tiled MaskedLinear forward: split-K for the whole GEMM, or the split tail of
 // the 256x256 tile.
 size_t linear_partial_bytes(int64_t M, int64_t K, int64_t N) {
   const RoutedPlan p = linear_plan(M, K, N);
-  if (p.splits > 1) return ws_align((size_t)p.splits * M * N * 4);
-  if (is_big_tile(p.tile) && K % 64 == 0) return ws_align((size_t)kTailSlots * 256 * 256 * 4);
-  return 0;
+  if (p.splits > 1) return ws_align((size_t)max_splits(p) * M * N * 4);
+  return tail_bytes(p, M, N, K);
 }
-int down_tile(int64_t M, int64_t d, int64_t h) { return down_plan(M, d, h).tile; }
 int tiled_down_splits(int64_t M, int64_t d, int64_t h) {
-  return use_stream_path(M, d, h) ? 1 : down_plan(M, d, h).splits;
+  return use_stream_path(M, d, h) ? 1 : max_splits(ffn_down_plan(M, d, h));
 }
 // fp32 partials of the tiled down projection: all rows when K is split for the whole GEMM, or the
 // kTailSlots tiles of the split tail when the 256x256 tile runs unsplit.
 size_t tiled_down_partial_bytes(int64_t M, int64_t d, int64_t h) {
-  const RoutedPlan p = down_plan(M, d, h);
-  if (p.splits > 1) return ws_align((size_t)p.splits * M * d * 4);
-  if (is_big_tile(p.tile) && h % 64 == 0) return ws_align((size_t)kTailSlots * 256 * 256 * 4);
-  return 0;
+  const RoutedPlan p = ffn_down_plan(M, d, h);
+  if (p.splits > 1) return ws_align((size_t)max_splits(p) * M * d * 4);
+  return tail_bytes(p, M, d, h);
 }
 
 // Split-K factor of the weight-gradient GEMM when it shares a launch with the dx GEMM (both on 128x128
@@ -456,7 +483,7 @@ extern "C" {
 int ffnk_version(void) { return FFNK_VERSION; }
 
 int ffnk_debug_force_tile(int tile) {
-  return g_force_tile.exchange(((tile >= 0 && tile < TILE_COUNT) || tile == -2) ? tile : -1);
+  return g_force_tile.exchange(((tile >= 0 && tile < TILE_COUNT && tile != kTileGatherDw) || tile == -2) ? tile : -1);
 }
 
 int ffnk_debug_force_group_m(int group_m) { return g_force_group_m.exchange(group_m >= 1 && group_m <= 64 ? group_m : 0); }
@@ -526,10 +553,10 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
   int splits = 1;
   bool in_place = false;
   switch (op) {
-    case FFNK_OP_LINEAR_FWD: { const RoutedPlan lp = linear_plan(M, K, N); tile = lp.tile; splits = lp.splits; contraction = K; break; }
+    case FFNK_OP_LINEAR_FWD: { const RoutedPlan lp = linear_plan(M, K, N); tile = lp.tile; splits = max_splits(lp); contraction = K; break; }
     case FFNK_OP_FFN_FWD:
     case FFNK_OP_FFN_UP: tile = routed_tile(M, N, true, K); dual = true; contraction = K; break;
-    case FFNK_OP_FFN_DOWN: tile = down_plan(M, K, N).tile; contraction = N; break;  // out cols = d = K, contraction h = N
+    case FFNK_OP_FFN_DOWN: tile = ffn_down_plan(M, K, N).tile; contraction = N; break;  // out cols = d = K, contraction h = N
     case FFNK_OP_LINEAR_BWD:
     case FFNK_OP_BWD_DX: tile = routed_tile(M, K, false, 0, TUNED_NONE); contraction = N; break;
     case FFNK_OP_BWD_DW: {
@@ -569,7 +596,7 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
   out->direct_lds = (direct || in_place) ? 1 : 0;
   out->in_place = in_place ? 1 : 0;
   // 4: ring of four stages (128x128); 3: token panel in three stages, weight panel in two (single-weight 256x256 tiles)
-  out->lds_stages = !out->direct_lds ? 2 : tile == TILE_128x128_R4 ? 4 : (is_big_tile(tile) && !dual) ? 3 : 2;
+  out->lds_stages = !out->direct_lds ? 2 : tile == TILE_128x128_R4 ? 4 : (tile == TILE_128x256_R3 || tile == TILE_64x128_R3) ? 3 : (is_big_tile(tile) && !dual) ? 3 : 2;
   if (op == FFNK_OP_FFN_DOWN && !stream) out->split_k = tiled_down_splits(M, K, N);
   if (op == FFNK_OP_LINEAR_FWD && linear_stream_kind(M, K, N)) {
     out->path = FFNK_PATH_STREAM;
@@ -691,18 +718,20 @@ int ffnk_masked_linear_fwd_routed(const uint16_t* x, int64_t x_stride_m, const u
   const bool direct = direct_ok(K, M, x_stride_m, w_stride_n);
   RoutedPlan plan = linear_plan(M, K, N);
   if (!direct) {
-    plan.splits = 1;
+    plan.splits = plan.splits_more = 1;
     plan.tile = routed_tile(M, N, false, K);
   }
   if (plan.splits > 1) {
     g.splits = plan.splits;
+    g.splits_more = plan.splits_more;
     g.P = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + r.bytes);
   } else if (direct && is_big_tile(plan.tile)) {
     g.P_tail = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + r.bytes);
   }
   FFNK_HIP(launch_linear_gemm(plan.tile, direct, g, stream), "linear GEMM");
   if (plan.splits > 1)
-    FFNK_HIP(launch_routed_reduce(g.P, plan.splits, (int)M, (int)N, rt.perm, y, y_stride_m, stream), "linear reduce");
+    FFNK_HIP(launch_routed_reduce(g.P, plan.splits, plan.splits_more, tile_geom(plan.tile, false).block_m, (int)M, (int)N, rt.counts,
+                                  rt.perm, y, y_stride_m, stream), "linear reduce");
   return FFNK_OK;
 }
 
@@ -831,17 +860,20 @@ int ffn_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, cons
   dn.perm = rt.perm; dn.counts = rt.counts;
   dn.M = (int)M; dn.N = (int)d; dn.K = (int)h; dn.group_m = plan_group_m(TUNED_DOWN, M, h, d);
   const bool dn_direct = direct_ok(h, 0, ldh, down_stride_n);
-  const int dn_splits = dn_direct ? tiled_down_splits(M, d, h) : 1;
+  RoutedPlan dn_plan = ffn_down_plan(M, d, h);
+  if (!dn_direct) dn_plan.splits = dn_plan.splits_more = 1;
   float* partials = reinterpret_cast<float*>(wsb + r.bytes + ws_align((size_t)M * ldh * 2));
-  if (dn_splits > 1) {
-    dn.splits = dn_splits;
+  if (dn_plan.splits > 1) {
+    dn.splits = dn_plan.splits;
+    dn.splits_more = dn_plan.splits_more;
     dn.P = partials;
-  } else if (dn_direct && is_big_tile(down_tile(M, d, h))) {
+  } else if (dn_direct && is_big_tile(dn_plan.tile)) {
     dn.P_tail = partials;  // the last, partial round of 256x256 tiles runs cut into K ranges
   }
-  FFNK_HIP(launch_down_gemm(down_tile(M, d, h), dn_direct, dn, stream), "down-projection GEMM");
-  if (dn_splits > 1)
-    FFNK_HIP(launch_routed_reduce(dn.P, dn_splits, (int)M, (int)d, rt.perm, out, out_stride_m, stream), "down-projection reduce");
+  FFNK_HIP(launch_down_gemm(dn_plan.tile, dn_direct, dn, stream), "down-projection GEMM");
+  if (dn_plan.splits > 1)
+    FFNK_HIP(launch_routed_reduce(dn.P, dn_plan.splits, dn_plan.splits_more, tile_geom(dn_plan.tile, false).block_m, (int)M, (int)d,
+                                  rt.counts, rt.perm, out, out_stride_m, stream), "down-projection reduce");
   FFNK_HIP(mark(2), "event record");
   return FFNK_OK;
 }
@@ -1125,7 +1157,7 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
   const RoutedPlan dxp = ffn_bwd_dx_plan(M, d, h, dx_direct, 2 * ws_align((size_t)h * d * 2), &dx_need);
   if (dx_need > p.w2t_bytes) return fail(FFNK_E_WORKSPACE, "internal: dx partials %zu > %zu planned", dx_need, p.w2t_bytes);
   if (dxp.splits > 1) {
-    b.splits = dxp.splits;
+    b.splits = b.splits_more = dxp.splits;
     b.P = reinterpret_cast<float*>(wsb + p.off_w2t);
   } else if (dx_need > 0) {
     b.P_tail = reinterpret_cast<float*>(wsb + p.off_w2t);  // split tail of the last, partial round
@@ -1133,7 +1165,8 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
   if (w13_kmajor) FFNK_HIP(launch_down_gemm_kmajor(dxp.tile, b, stream), "dx GEMM");
   else FFNK_HIP(launch_down_gemm(dxp.tile, dx_direct, b, stream), "dx GEMM");
   if (dxp.splits > 1)
-    FFNK_HIP(launch_routed_reduce(b.P, dxp.splits, (int)M, (int)d, rt.perm, dx, dx_stride_m, stream), "dx reduce");
+    FFNK_HIP(launch_routed_reduce(b.P, dxp.splits, dxp.splits, tile_geom(dxp.tile, false).block_m, (int)M, (int)d, rt.counts, rt.perm,
+                                  dx, dx_stride_m, stream), "dx reduce");
 
   // ---- weight gradients: contraction over the rows of each group.  x and g are gathered into
   // 64-padded transposes; H, dt1 and dt3 (routed order already) are read in place by the K-major

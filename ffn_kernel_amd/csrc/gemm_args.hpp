@@ -38,8 +38,9 @@ struct GemmArgs {
   // Split-K (direct path, tail_mode 0, not the SwiGLU kernels): with splits > 1 the contraction is
   // cut into `splits` ranges of whole 64-element slabs, each workgroup handles one (tile, range) and
   // stores its fp32 partial sums to P[split][routed row][N]; a reduce pass adds them and scatters
-  // the rows.  For outputs too small to fill the chip with tiles over a long contraction.
-  int splits = 1;
+  // the rows.  For outputs too small to fill the chip with tiles over a long contraction.  splits is the factor for
+  // cdiv(M, tile rows) M-tiles, splits_more for one M-tile more (RoutedPlan): only the device knows which it is.
+  int splits = 1, splits_more = 1;
   float* P = nullptr;
   // Split tail (direct path, single weight per group): the launcher runs the whole rounds of 256 tiles
   // first and then the remaining tiles cut into tail_split_factor() K ranges each, so that the last,

@@ -14,6 +14,8 @@ hipError_t launch_splitk_gemm(int tile, const SplitKArgs& g, hipStream_t stream)
   switch (tile) {
     case TILE_256x256_W8: return launch_grouped_splitk<Tiles::T0>(g, stream);
     case TILE_256x256_W4: return launch_grouped_splitk<Tiles::T1>(g, stream);
+    case TILE_64x128_R3:
+    case TILE_128x256_R3:  // no such weight-gradient tile
     case TILE_128x128_W4: return launch_grouped_splitk<Tiles::T2>(g, stream);
     case TILE_SMALL_W4: return launch_grouped_splitk<Tiles::T3>(g, stream);
     case TILE_128x128_R4: return launch_grouped_splitk<Tiles::T4>(g, stream);

@@ -1337,14 +1337,15 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
   const int total = routed_tile_count(n_vis, g.M, g.N, SBM, SBN);
   int L, sub_m = 0, sub_n = 0, split = 0, splits = 1, tail_slot = 0;
   if (g.tail_mode == 0) {
-    splits = g.splits;
+    splits = routed_splits(n_vis, g.M, BM, g.splits, g.splits_more);
     L = xcd_tile_slot(total * splits, bid);
     if (splits > 1 && L >= 0) {  // range-major: neighbours in the order share panels, not a K range
       split = L / total;
       L -= split * total;
     }
   } else {
-    const int full = total / kCusPerChip * kCusPerChip;
+    // (tail_mode 1 with a split tail behind it leaves every remainder to the tail)
+    const int full = g.tail_mode == 3 || g.P_tail != nullptr ? total / kCusPerChip * kCusPerChip : whole_round_tiles(total);
     if (g.tail_mode == 1) {
       L = xcd_tile_slot(full, bid);
     } else if (g.tail_mode == 2) {
@@ -1617,22 +1618,24 @@ __global__ __launch_bounds__(CfgDx::NT) void fused_bwd_kernel(const GemmArgs gx,
 // Upper bound on the number of workgroups the kernel needs, rounded so that every XCD gets the
 // same number of slots.  The kernel derives the real tile count from counts[] on the device.
 template <class Cfg>
-inline int routed_gemm_grid(int M, int N) {
-  const int tiles_m = cdiv(M, Cfg::BM) + 1;  // the two groups can each end in a partial tile
+inline int routed_gemm_grid(int M, int N, int splits = 1, int splits_more = 1) {
+  const int64_t tiles_m = cdiv(M, Cfg::BM);  // or one more: the two groups can each end in a partial tile
   const int tiles_n = cdiv(N, Cfg::BN_OUT);
-  const int64_t total = (int64_t)tiles_m * tiles_n;
+  const int64_t less = tiles_m * splits, more = (tiles_m + 1) * splits_more;
+  const int64_t total = (less > more ? less : more) * tiles_n;
   return (int)(cdiv64(total, kXcds) * kXcds);
 }
 
 template <class Cfg>
 inline hipError_t launch_routed_gemm(const GemmArgs& g, hipStream_t stream) {
   if (g.M <= 0 || g.N <= 0) return hipSuccess;
-  if (g.splits > 1 && (Cfg::DUAL || !Cfg::DIRECT || g.tail_mode != 0 || g.P == nullptr)) return hipErrorInvalidValue;
+  if ((g.splits > 1 || g.splits_more > 1) && (Cfg::DUAL || !Cfg::DIRECT || g.tail_mode != 0 || g.P == nullptr)) return hipErrorInvalidValue;
+  if ((g.splits > 1) != (g.splits_more > 1)) return hipErrorInvalidValue;
   if (Cfg::B_KMAJOR && (g.N % 8 != 0 || g.K % kBK != 0 || g.k_switch % kBK != 0 || g.k_switch < 0 || g.k_switch >= g.K ||
                         g.ldb * (kBK * 2) + 2 * (int64_t)g.N >= ((int64_t)1 << 32)))
     return hipErrorInvalidValue;
   if (!Cfg::B_KMAJOR && g.k_switch != 0) return hipErrorInvalidValue;
-  const int grid = routed_gemm_grid<Cfg>(g.M, g.N) * (g.splits > 1 ? g.splits : 1);
+  const int grid = routed_gemm_grid<Cfg>(g.M, g.N, g.splits, g.splits_more);
   hipLaunchKernelGGL(routed_gemm_kernel<Cfg>, dim3(grid), dim3(Cfg::NT), 0, stream, g);
   return hipGetLastError();
 }

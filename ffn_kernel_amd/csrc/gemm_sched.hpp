@@ -23,6 +23,11 @@ __host__ __device__ inline int routed_tile_count(int n_vis, int M, int N, int bm
   return (cdiv(n_vis, bm) + cdiv(M - n_vis, bm)) * cdiv(N, bn);
 }
 
+// Split-K factor of a launch: `splits` where the two groups have cdiv(M, bm) M-tiles between them, else (one more) splits_more.
+__host__ __device__ inline int routed_splits(int n_vis, int M, int bm, int splits, int splits_more) {
+  return cdiv(n_vis, bm) + cdiv(M - n_vis, bm) > cdiv(M, bm) ? splits_more : splits;
+}
+
 // Position L of the order -> tile.  The order walks super-groups of M-tiles column by column, so that tiles sharing A rows /
 // B columns are neighbours.  Above kEvenGroups * group_m M-tiles: super-groups of group_m M-tiles from the first tile on.  Up to
 // there, where the edges of the super-groups weigh more: super-groups of one modality's M-tiles only (two modalities share
@@ -81,6 +86,14 @@ __host__ __device__ inline DwTileCoord dw_tile_coord(int L, int tiles_r, int til
   t.tile_r = first_r + (L % width) % gsz;
   t.tile_c = (L % width) / gsz;
   return t;
+}
+
+// Tiles of the whole rounds of a launch whose remainder runs as smaller tiles (GemmArgs::tail_mode 1 and 2).  Up to half a
+// round the remainder's 128-row tiles, two to a CU, are one round of their own at 0.6 of the big tile's time (SwiGLU GEMM,
+// K = 4096: 62 us against 103); past half a round they are two, and the big tile's round is the shorter one.
+__host__ __device__ inline int whole_round_tiles(int total) {
+  const int rest = total % kCusPerChip;
+  return rest > kCusPerChip / 2 ? total : total - rest;
 }
 
 // Split tail: the tiles past the last whole round of kCusPerChip are each cut into this many K

@@ -24,6 +24,8 @@ struct PlainTiles {
   using T3 = RoutedGemmCfg<128, 64, 2, 2, false, GATHER, SCATTER, DIRECT, kGroupMPlain>;
   // 128x128 behind a ring of four LDS stages (direct path; otherwise the two-stage tile)
   using T4 = RoutedGemmCfg<128, 128, 2, 2, false, GATHER, SCATTER, DIRECT, kGroupMPlain, false, DIRECT ? 4 : 2>;
+  using T6 = std::conditional_t<DIRECT, RoutedGemmCfg<128, 256, 2, 2, false, GATHER, SCATTER, true, kGroupMPlain, false, 3>, T2>;
+  using T7 = std::conditional_t<DIRECT, RoutedGemmCfg<64, 128, 2, 2, false, GATHER, SCATTER, true, kGroupMPlain, false, 3>, T3>;
 };
 
 // The same tiles over K-major weights ([K, N] rows, N contiguous; direct path only).
@@ -36,6 +38,8 @@ struct KMajorTiles {
   // 128x128 behind a ring of four LDS stages, for the routed GEMMs (the weight-gradient GEMMs, whose last slab is
   // ragged and cleared in LDS, stay on the two-stage tile)
   using T4 = RoutedGemmCfg<128, 128, 2, 2, false, GATHER, SCATTER, true, kGroupM, true, 4>;
+  using T6 = T2;
+  using T7 = T3;
 };
 
 // SwiGLU tiles: BN = gate rows + up rows held in LDS, i.e. BN / 2 output columns.
@@ -46,6 +50,8 @@ struct DualTiles {
   using T2 = RoutedGemmCfg<128, 128, 2, 2, true, true, false, DIRECT, kGroupM>;
   using T3 = RoutedGemmCfg<64, 128, 2, 2, true, true, false, DIRECT, kGroupM>;
   using T4 = RoutedGemmCfg<128, 128, 2, 2, true, true, false, DIRECT, kGroupM, false, DIRECT ? 4 : 2>;
+  using T6 = std::conditional_t<DIRECT, RoutedGemmCfg<128, 256, 2, 2, true, true, false, true, kGroupM, false, 3>, T2>;
+  using T7 = std::conditional_t<DIRECT, RoutedGemmCfg<64, 128, 2, 2, true, true, false, true, kGroupM, false, 3>, T3>;
 };
 
 template <class Tiles>
@@ -61,6 +67,8 @@ inline hipError_t dispatch_tile(int tile, const GemmArgs& g, hipStream_t stream)
     case TILE_128x128_W4: return launch_routed_gemm<typename Tiles::T2>(g, stream);
     case TILE_SMALL_W4: return launch_routed_gemm<typename Tiles::T3>(g, stream);
     case TILE_128x128_R4: return launch_routed_gemm<typename Tiles::T4>(g, stream);
+    case TILE_128x256_R3: return launch_routed_gemm<typename Tiles::T6>(g, stream);
+    case TILE_64x128_R3: return launch_routed_gemm<typename Tiles::T7>(g, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -95,7 +103,7 @@ inline hipError_t dispatch_big_tile_with_tail(const GemmArgs& g, hipStream_t str
   a.sched_bm = Big::BM;
   a.sched_bn = Big::BN_OUT;
   constexpr int q = (Big::BM / Small::BM) * (Big::BN_OUT / Small::BN_OUT);
-  hipLaunchKernelGGL(routed_gemm_kernel<Small>, dim3((kCusPerChip - 1) * q), dim3(Small::NT), 0, stream, a);
+  hipLaunchKernelGGL(routed_gemm_kernel<Small>, dim3(kCusPerChip / 2 * q), dim3(Small::NT), 0, stream, a);
   return hipGetLastError();
 }
 

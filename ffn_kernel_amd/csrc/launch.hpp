@@ -16,7 +16,10 @@ enum TileId : int {
   TILE_128x128_W4 = 2,  // 128x128 macro tile, 4 waves (2x2), wave tile 64x64
   TILE_SMALL_W4 = 3,    // 128x64 (plain) or 64x128 holding 64 gate + 64 up rows (SwiGLU), 4 waves
   TILE_128x128_R4 = 4,  // 128x128, 4 waves, ring of four LDS stages (one workgroup per CU; long contractions, few tiles)
-  TILE_COUNT = 5
+  // 5 names a form of the weight-gradient GEMM in its plans (kTileGatherDw), not a tile
+  TILE_128x256_R3 = 6,  // 128 rows x 256 weight rows (SwiGLU: 128 gate + 128 up), 4 waves, ring of three LDS stages
+  TILE_64x128_R3 = 7,   // 64 rows x 128 weight rows (SwiGLU: 64 gate + 64 up), 4 waves, ring of three LDS stages, two workgroups per CU
+  TILE_COUNT = 8
 };
 
 // The two 256x256 tiles: past one round of the chip they run whole rounds first and the remainder apart.
@@ -82,9 +85,9 @@ hipError_t launch_swiglu_bwd(const uint16_t* pre, int64_t ld_pre, uint16_t* T13,
 hipError_t launch_splitk_reduce(const float* P, int splits, int R, int Cc, uint16_t* out0, uint16_t* out1,
                                 int64_t sr, int64_t sc, hipStream_t stream);
 
-// out[perm[p], n] = bf16(sum_s P[s][p][n]): reduce pass of a split-K routed GEMM (N % 4 == 0, M < 65536).
-hipError_t launch_routed_reduce(const float* P, int splits, int M, int N, const int32_t* perm, uint16_t* out,
-                                int64_t ldo, hipStream_t stream);
+// out[perm[p], n] = bf16(sum_s P[s][p][n]): reduce pass of a split-K routed GEMM on tiles of bm rows (N % 4 == 0, M < 65536).
+hipError_t launch_routed_reduce(const float* P, int splits, int splits_more, int bm, int M, int N, const int32_t* counts,
+                                const int32_t* perm, uint16_t* out, int64_t ldo, hipStream_t stream);
 
 // Reduce pass of a split tail (GemmArgs::P_tail) of a GEMM on bm x bn tiles with scatter epilogue.
 hipError_t launch_routed_tail_reduce(const float* P_tail, int M, int N, int K, const int32_t* counts,

@@ -249,13 +249,15 @@ hipError_t launch_splitk_reduce(const float* P, int splits, int R, int Cc, uint1
 }
 
 // out[perm[p], n] = bf16(P[0][p][n] + P[1][p][n] + ...) in split order: the reduce pass of a split-K
-// routed GEMM.  One workgroup per (routed row, 1024 columns); N % 4 == 0.
-__global__ __launch_bounds__(256) void routed_reduce_kernel(const float* __restrict__ P, int splits, int M, int N,
+// routed GEMM on tiles of bm rows (GemmArgs::splits, splits_more).  One workgroup per (routed row, 1024 columns); N % 4 == 0.
+__global__ __launch_bounds__(256) void routed_reduce_kernel(const float* __restrict__ P, int splits, int splits_more, int bm,
+                                                            int M, int N, const int32_t* __restrict__ counts,
                                                             const int32_t* __restrict__ perm,
                                                             uint16_t* __restrict__ out, int64_t ldo) {
   const int p = blockIdx.y;
   const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (n >= N) return;
+  splits = routed_splits(counts[0], M, bm, splits, splits_more);
   float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
   for (int k = 0; k < splits; ++k) {
     const float4 v = *reinterpret_cast<const float4*>(P + ((int64_t)k * M + p) * N + n);
@@ -272,11 +274,11 @@ __global__ __launch_bounds__(256) void routed_reduce_kernel(const float* __restr
   }
 }
 
-hipError_t launch_routed_reduce(const float* P, int splits, int M, int N, const int32_t* perm, uint16_t* out,
-                                int64_t ldo, hipStream_t stream) {
+hipError_t launch_routed_reduce(const float* P, int splits, int splits_more, int bm, int M, int N, const int32_t* counts,
+                                const int32_t* perm, uint16_t* out, int64_t ldo, hipStream_t stream) {
   if (M <= 0 || N <= 0) return hipSuccess;
   dim3 grid((unsigned)cdiv(N, 1024), (unsigned)M);
-  hipLaunchKernelGGL(routed_reduce_kernel, grid, dim3(256), 0, stream, P, splits, M, N, perm, out, ldo);
+  hipLaunchKernelGGL(routed_reduce_kernel, grid, dim3(256), 0, stream, P, splits, splits_more, bm, M, N, counts, perm, out, ldo);
   return hipGetLastError();
 }
 

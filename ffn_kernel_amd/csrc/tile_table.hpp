@@ -59,6 +59,131 @@ inline int tuned_group_m(int op, int64_t M, int64_t k, int64_t n) {
   return t ? t->group_m : 0;
 }
 
+// Tile and split-K factor of a routed GEMM.  The visual and the text rows each end in a partial tile, so a call has
+// cdiv(M, block_m) M-tiles or one more, which only the device knows: `splits` is for the one count and `splits_more` for
+// the other (the kernel and the reduce pass pick by counts[]); either both are 1 or neither is.
+struct RoutedPlan {
+  int tile;
+  int splits;
+  int splits_more;
+};
+
+// Time of a direct-path GEMM in us, fitted to sweeps of every tile (and split factor) at M = 10 ... 4096 with one and with both
+// modalities present: SwiGLU GEMMs at six (d, h) from 1024 x 2048 to 7168 x 20480, single-weight GEMMs at
+// ten (K, N) from 1024 x 1024 to 20480 x 7168 (rms error 10 %).  A round of the chip takes base + slabs * per_slab, a partial last
+// round `partial` of that plus the rest by its share of the slots; the weights arrive at `tbs` TB/s (the smaller of the two
+// times is mostly hidden behind the larger).  What follows from it, against the tiles chosen by their number alone before:
+// SwiGLU GEMMs 2.5 % behind the best tile of each shape instead of 12 % (M = 300 / 512 / 1024 of one modality at d = 4096,
+// h = 14336: 128 -> 98, 150 -> 100, 274 -> 183 us), single-weight GEMMs 2.5 % instead of 12 % (M = 512 at K = 14336,
+// N = 4096: 105 -> 70 us; M = 1024 at 4096 x 4096: 49 -> 38 us).
+struct TileCost {
+  int tile;
+  double base, per_slab, partial, tbs;
+};
+constexpr TileCost kDualCosts[] = {{TILE_256x256_W4, 8.75, 1.25, 0.79, 6.5}, {TILE_128x128_W4, 0.0, 1.08, 0.50, 5.5},
+                                   {TILE_SMALL_W4, 0.0, 1.025, 0.41, 5.25},  {TILE_128x128_R4, 1.5, 0.56, 0.68, 6.1},
+                                   {TILE_128x256_R3, 2.2, 0.87, 0.66, 5.75}, {TILE_64x128_R3, 0.75, 0.61, 0.51, 5.15}};
+constexpr TileCost kPlainCosts[] = {{TILE_256x256_W8, 3.4, 1.56, 0.74, 12.0}, {TILE_256x256_W4, 11.1, 1.41, 0.65, 10.0},
+                                    {TILE_128x128_W4, 0.9, 1.00, 0.42, 5.8},  {TILE_SMALL_W4, 0.0, 0.87, 0.29, 5.2},
+                                    {TILE_128x128_R4, 2.5, 0.48, 0.475, 6.0}, {TILE_128x256_R3, 3.5, 0.86, 0.73, 7.2},
+                                    {TILE_64x128_R3, 0.2, 0.57, 0.24, 5.9}};
+
+inline double routed_tile_time(const TileCost& c, bool dual, int64_t tiles_m, int modalities, int64_t M, int64_t n_out, int64_t K,
+                               int splits) {
+  const TileGeom t = tile_geom(c.tile, dual);
+  const double slots = kCus * (c.tile == TILE_SMALL_W4 ? 3 : (c.tile == TILE_128x128_W4 || c.tile == TILE_64x128_R3) ? 2 : 1);
+  const double slabs = (double)(K / 64), tiles = (double)(tiles_m * cdiv64(n_out, t.block_n_out) * splits);
+  const double round = c.base + c.per_slab * (double)cdiv64(K / 64, splits);
+  const double full = (double)(int64_t)(tiles / slots), rest = tiles - full * slots;
+  double time = full * round;
+  if (rest > 0.0) {
+    const double share = round * (c.partial + (1.0 - c.partial) * rest / slots);
+    if (!is_big_tile(c.tile) || splits > 1 || full == 0.0) {
+      time += share;
+    } else if (dual) {  // past half a round another round, else 128x128 tiles (whole_round_tiles)
+      time += rest > slots / 2 ? round : 3.0 + 1.08 * slabs * (0.5 + 0.5 * rest * 4.0 / 512.0);
+    } else {            // split tail
+      const double cut = 8.0 + c.base + c.per_slab * slabs / (double)tail_split_factor((int)rest, (int)slabs);
+      time += cut < round ? cut : round;
+    }
+  }
+  const double weights = modalities * (dual ? 2.0 : 1.0) * (double)K * (double)n_out * 2.0e-6 / c.tbs;
+  const double hidden = dual ? 0.15 : 0.39;
+  time = (dual ? 4.9 : 6.9) + (time > weights ? time + hidden * weights : weights + hidden * time);
+  if (splits > 1) time += 2.0 + (double)splits * (double)M * (double)n_out * 8.0e-6 / 7.2;  // partials and the reduce pass
+  return time;
+}
+
+// Split factors the cost model considers: whole 64-element slabs, at least four to a range, no empty range.
+inline bool routed_split_ok(int64_t K, int s) {
+  const int64_t nk = K / 64;
+  return s == 1 || (nk / s >= 4 && cdiv64(nk, cdiv64(nk, s)) == s);
+}
+
+inline double best_split(const TileCost& c, int64_t tiles_m, int modalities, int64_t M, int64_t n_out, int64_t K, bool split,
+                         int first, int* best) {
+  constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16};
+  double best_time = -1.0;
+  for (const int s : kSplits) {
+    if (s < first || (s > 1 && (!split || c.tile == TILE_256x256_W4)) || !routed_split_ok(K, s)) continue;
+    const double t = routed_tile_time(c, false, tiles_m, modalities, M, n_out, K, s);
+    if (best_time < 0.0 || t < best_time) {
+      best_time = t;
+      *best = s;
+    }
+  }
+  return best_time;
+}
+
+// The plan with the smallest product of two times: both modalities present, about evenly (M-tiles: the likelier of the two
+// counts), and one modality alone.  `split`: the caller has a workspace for partials and N % 4 == 0.
+inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split) {
+  RoutedPlan p{TILE_SMALL_W4, 1, 1};
+  double best = -1.0;
+  const TileCost* costs = dual ? kDualCosts : kPlainCosts;
+  const int n_costs = dual ? (int)(sizeof(kDualCosts) / sizeof(TileCost)) : (int)(sizeof(kPlainCosts) / sizeof(TileCost));
+  const TileCost* pick = costs;
+  for (int i = 0; i < n_costs; ++i) {
+    const int64_t bm = tile_geom(costs[i].tile, dual).block_m;
+    const int64_t one = cdiv64(M, bm), both = M / bm + 1 + (M % bm > bm / 2 ? 1 : 0);
+    int s = 1;
+    const double t = dual ? routed_tile_time(costs[i], true, both, 2, M, n_out, K, 1) * routed_tile_time(costs[i], true, one, 1, M, n_out, K, 1)
+                          : best_split(costs[i], both, 2, M, n_out, K, split, 1, &s) * best_split(costs[i], one, 1, M, n_out, K, split, 1, &s);
+    if (best < 0.0 || t < best) {
+      best = t;
+      pick = costs + i;
+    }
+  }
+  p.tile = pick->tile;
+  if (!dual) {
+    const int64_t tiles_m = cdiv64(M, tile_geom(p.tile, false).block_m);
+    best_split(*pick, tiles_m, 2, M, n_out, K, split, 1, &p.splits);
+    best_split(*pick, tiles_m + 1, 2, M, n_out, K, split, 1, &p.splits_more);
+    if (p.splits == 1 || p.splits_more == 1) p.splits = p.splits_more = 1;
+  }
+  return p;
+}
+
+// The model is a pure function of the extents and takes a few microseconds of host time; every thread keeps the last plans.
+inline RoutedPlan model_routed_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split) {
+  struct Entry {
+    int64_t M = -1, n_out, K;
+    bool dual, split;
+    RoutedPlan plan;
+  };
+  static thread_local Entry memo[32];
+  Entry& e = memo[(uint64_t)(M * 31 + n_out * 7 + K * 3 + (dual ? 1 : 0)) % 32];
+  if (e.M != M || e.n_out != n_out || e.K != K || e.dual != dual || e.split != split)
+    e = Entry{M, n_out, K, dual, split, compute_model_plan(dual, M, n_out, K, split)};
+  return e.plan;
+}
+
+// Where the model applies: up to two rounds of 256x256 tiles; past them the rule below takes that tile.
+inline bool model_applies(bool dual, int64_t M, int64_t n_out, int64_t K) {
+  const TileGeom t = tile_geom(TILE_256x256_W8, dual);
+  return M > 0 && n_out > 0 && K > 0 && K % 64 == 0 && cdiv64(M, t.block_m) * cdiv64(n_out, t.block_n_out) < 2 * kCus;
+}
+
 // Routed GEMM over M rows and n_out output columns (K: the contraction, 0 = not known to the caller).
 // `op`: whose measured plans apply (TUNED_NONE: none; the tuner times each operation with its own gather /
 // scatter pattern and its own launches around the GEMM, so one operation's plan says nothing about another's).
@@ -68,6 +193,7 @@ inline int pick_routed_tile(int64_t M, int64_t n_out, bool dual, int64_t K = 0, 
     if (const TunedPlan* t = tuned_plan(dual ? TUNED_DUAL : op, M, K, n_out))
       if (dual || t->splits == 1) return t->tile;
   }
+  if (dual && model_applies(true, M, n_out, K)) return model_routed_plan(true, M, n_out, K, false).tile;
   auto tiles = [&](int tile) {
     const TileGeom t = tile_geom(tile, dual);
     return cdiv64(M, t.block_m) * cdiv64(n_out, t.block_n_out);
@@ -81,25 +207,13 @@ inline int pick_routed_tile(int64_t M, int64_t n_out, bool dual, int64_t K = 0, 
   return TILE_SMALL_W4;
 }
 
-// Tile and split-K factor of a routed GEMM with a single weight per group and a workspace for
-// partial sums (the FFN down projection).  When the output yields fewer tiles than the chip has
-// workgroup slots and the contraction is long, each workgroup would stream a long weight panel on
-// its own while most CUs idle; cutting K into `splits` ranges of whole 64-element slabs fills the
-// chip, at the price of fp32 partials (4 * splits * M * n_out bytes written, then read by the
-// reduce pass).  The choice minimises a cost model fitted to a sweep over M = 128 ... 4096 at
-// n_out = 4096, K = 14336 (it reproduces the measured best of every M there; the table's previous
-// choice was 1.1x to 1.7x slower):
+// The GEMMs the model above was not fitted for (the backward's dx GEMM over K-major weights): when the output yields fewer
+// tiles than the chip has workgroup slots and the contraction is long, cutting K into `splits` ranges of whole 64-element
+// slabs fills the chip, at the price of fp32 partials (4 * splits * M * n_out bytes written, then read by the reduce pass):
 //   time = rounds * (5 us + slabs_per_range * t_slab) + splits * M * n_out * 8 bytes / 4 TB/s
 //   rounds = ceil(tiles * splits / slots),  slots = 256 CUs * workgroups per CU by LDS use,
 //   t_slab = 1.2 us for the 256x256 tile, 0.8 us for the 128x128 and 128x64 tiles.
-// The unsplit 256x256 tile is priced with its split tail (see routed_plan_cost).
-// Limited to M <= 4096 (above it the tiles fill the chip, and the reduce pass launches one row per
-// blockIdx.y); larger M keeps pick_routed_tile and no split.
-struct RoutedPlan {
-  int tile;
-  int splits;
-};
-
+// The unsplit 256x256 tile is priced with its split tail.  Limited to M <= 4096 (above it the tiles fill the chip).
 inline double routed_plan_cost(int64_t M, int64_t n_out, int64_t K, int tile, int splits) {
   const TileGeom t = tile_geom(tile, false);
   const int64_t tiles = (cdiv64(M, t.block_m) + 1) * cdiv64(n_out, t.block_n_out);
@@ -140,11 +254,12 @@ inline RoutedPlan pick_routed_plan(int64_t M, int64_t n_out, int64_t K, bool use
   if (use_table && op != TUNED_NONE)
     if (const TunedPlan* t = tuned_plan(op, M, K, n_out)) {
       p.tile = t->tile;
-      p.splits = (K % 64 == 0 && M < 65536 && n_out % 4 == 0) ? t->splits : 1;
+      p.splits = p.splits_more = (K % 64 == 0 && M < 65536 && n_out % 4 == 0) ? t->splits : 1;
       return p;
     }
+  if (op != TUNED_NONE && model_applies(false, M, n_out, K)) return model_routed_plan(false, M, n_out, K, M < 65536 && n_out % 4 == 0);
   p.tile = pick_routed_tile(M, n_out, false, K, use_table, op);
-  p.splits = 1;
+  p.splits = p.splits_more = 1;
   if (M > 4096 || K % 64 != 0) return p;
   double best_cost = 0.0;
   const int cand[3] = {TILE_256x256_W8, TILE_128x128_W4, TILE_SMALL_W4};
@@ -154,7 +269,7 @@ inline RoutedPlan pick_routed_plan(int64_t M, int64_t n_out, int64_t K, bool use
     if (i == 0 || c < best_cost) {
       best_cost = c;
       p.tile = cand[i];
-      p.splits = s;
+      p.splits = p.splits_more = s;
     }
   }
   return p;

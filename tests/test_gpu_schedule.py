@@ -3,7 +3,7 @@ double precision computed with torch on the GPU."""
 import pytest
 import torch
 
-from ffn_kernel_amd import MaskedLinear, _lib
+from ffn_kernel_amd import MaskedFFN, MaskedLinear, _lib
 from ffn_kernel_amd.ops import masked_linear_backward
 from helpers import assert_close, note
 
@@ -61,3 +61,58 @@ def test_weight_gradient_super_groups(dev, forced, tile, splits, N):
     assert_close(dv.T, ((gd * mv).T @ xd).cpu(), "dWv")
     assert_close(dt.T, ((gd * (1 - mv)).T @ xd).cpu(), "dWt")
     assert_close(dx, torch.where(mask[:, None], gd @ Wv.double(), gd @ Wt.double()).cpu(), "dx")
+
+
+def select_ffn(x, W, mask):
+    """SwiGLU feed-forward, row-select form in double precision, the intermediate rounded to bf16 once as it is stored."""
+    out = torch.empty_like(x, dtype=torch.float64)
+    for sel, g, d, u in ((mask, 0, 1, 2), (~mask, 3, 4, 5)):
+        xs = x[sel].double()
+        t1 = xs @ W[g].double().T
+        mid = (t1 * torch.sigmoid(t1) * (xs @ W[u].double().T)).to(torch.bfloat16).double()
+        out[sel] = mid @ W[d].double().T
+    return out
+
+
+# The ring tiles of 128 x 256 and 64 x 128: contractions of fewer slabs than stages, exactly as many and more; single rows,
+# whole tiles, one row past them; columns below and past a tile; cut into K ranges with and without a remainder.
+@pytest.mark.parametrize("tile", [6, 7])
+@pytest.mark.parametrize("nv,nt,K,N,splits", [(1, 1, 64, 8, 1), (128, 64, 128, 256, 1), (129, 0, 192, 264, 1), (0, 257, 256, 136, 1),
+                                              (65, 63, 1024, 520, 3), (200, 130, 1536, 128, 5)])
+def test_ring_tiles(dev, forced, tile, nv, nt, K, N, splits):
+    note(f"ring tile {tile}: nv={nv} nt={nt} K={K} N={N} splits={splits}")
+    x, Wv, Wt, mask, _ = make_linear(dev, nv, nt, K, N, seed=K + N)
+    forced(tile, splits)
+    y = MaskedLinear.apply(x, Wv.T, Wt.T, mask)
+    h = 136  # M, d, h beyond the decode kernels' shapes: h is no multiple of 128
+    gen = torch.Generator(device=dev).manual_seed(3)
+    W = [(torch.randn(*s, generator=gen, device=dev) * 0.05).to(torch.bfloat16) for s in ((h, K), (K, h), (h, K)) * 2]
+    out = MaskedFFN.apply(x, *[w.T for w in W], mask)
+    forced()
+    assert_close(y, torch.where(mask[:, None], x.double() @ Wv.double().T, x.double() @ Wt.double().T).cpu(), "y")
+    assert_close(out, select_ffn(x, W, mask).cpu(), "ffn")
+
+
+# The split factor depends on the number of M-tiles, which only the device knows: as many as the rows need, or one more.
+@pytest.mark.parametrize("nv", [0, 128, 150, 199, 200])
+@pytest.mark.parametrize("K,N", [(4096, 512), (8192, 1024)])
+def test_split_factor_by_row_tiles(dev, nv, K, N):
+    note(f"split factor: nv={nv} of 200, K={K} N={N}")
+    assert _lib.tile_config(_lib.OP_LINEAR_FWD, 200, K, N)["split_k"] > 1
+    x, Wv, Wt, mask, _ = make_linear(dev, nv, 200 - nv, K, N, seed=nv)
+    y = MaskedLinear.apply(x, Wv.T, Wt.T, mask)
+    assert_close(y, torch.where(mask[:, None], x.double() @ Wv.double().T, x.double() @ Wt.double().T).cpu(), "y")
+
+
+# The remainder of a launch on 256-row SwiGLU tiles: exactly half a round, one tile past it (another whole round), and one
+# tile past a round.  d = 64, h = 128 * tiles_n columns: 256 columns of the output hold one M-tile's row of tiles.
+@pytest.mark.parametrize("tiles_m,h", [(6, 64 * 128), (43, 9 * 128), (257, 128)])
+def test_whole_rounds_and_remainder(dev, forced, tiles_m, h):
+    note(f"remainder of whole rounds: {tiles_m} M-tiles, h={h}")
+    x, _, _, mask, _ = make_linear(dev, 256 * 2, 256 * (tiles_m - 2) - 5, 64, 8, seed=tiles_m)
+    gen = torch.Generator(device=dev).manual_seed(5)
+    W = [(torch.randn(*s, generator=gen, device=dev) * 0.05).to(torch.bfloat16) for s in ((h, 64), (64, h), (h, 64)) * 2]
+    forced(1)
+    out = MaskedFFN.apply(x, *[w.T for w in W], mask)
+    forced()
+    assert_close(out, select_ffn(x, W, mask).cpu(), "ffn")
