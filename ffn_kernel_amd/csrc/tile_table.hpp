@@ -69,48 +69,51 @@ struct RoutedPlan {
 };
 
 // Time of a direct-path GEMM in us, fitted to sweeps of every tile (and split factor) at M = 10 ... 4096 with one and with both
-// modalities present: SwiGLU GEMMs at six (d, h) from 1024 x 2048 to 7168 x 20480, single-weight GEMMs at
-// ten (K, N) from 1024 x 1024 to 20480 x 7168 (rms error 10 %).  A round of the chip takes base + slabs * per_slab, a partial last
-// round `partial` of that plus the rest by its share of the slots; the weights arrive at `tbs` TB/s (the smaller of the two
-// times is mostly hidden behind the larger).  What follows from it, against the tiles chosen by their number alone before:
-// SwiGLU GEMMs 2.5 % behind the best tile of each shape instead of 12 % (M = 300 / 512 / 1024 of one modality at d = 4096,
-// h = 14336: 128 -> 98, 150 -> 100, 274 -> 183 us), single-weight GEMMs 2.5 % instead of 12 % (M = 512 at K = 14336,
-// N = 4096: 105 -> 70 us; M = 1024 at 4096 x 4096: 49 -> 38 us).
+// modalities present: SwiGLU GEMMs at seven (d, h) from 1024 x 2048 to 7168 x 20480, single-weight GEMMs at ten (K, N) from
+// 1024 x 1024 to 20480 x 7168 (rms error 9 %).  A round of the chip takes base + slabs * per_slab; a partial first round
+// takes `first` of that plus the rest by the workgroups on its fullest CU, a later one `again` plus the rest.  The weights
+// arrive at `tbs` TB/s; the smaller of the two times is mostly hidden behind the larger.  The plans that follow are 2-3 %
+// behind the best tile and split of each shape, the rules by tile count before were 12 % behind (SwiGLU GEMM at M = 300 / 512 /
+// 1024 of one modality, d = 4096, h = 14336: 128 -> 98, 150 -> 100, 274 -> 183 us; single-weight GEMM at M = 512, K = 14336,
+// N = 4096: 105 -> 70 us; at M = 1024, 4096 x 4096: 49 -> 38 us).
 struct TileCost {
-  int tile;
-  double base, per_slab, partial, tbs;
+  int tile, per_cu;
+  double base, per_slab, first, again, tbs;
 };
-constexpr TileCost kDualCosts[] = {{TILE_256x256_W4, 8.75, 1.25, 0.79, 6.5}, {TILE_128x128_W4, 0.0, 1.08, 0.50, 5.5},
-                                   {TILE_SMALL_W4, 0.0, 1.025, 0.41, 5.25},  {TILE_128x128_R4, 1.5, 0.56, 0.68, 6.1},
-                                   {TILE_128x256_R3, 2.2, 0.87, 0.66, 5.75}, {TILE_64x128_R3, 0.75, 0.61, 0.51, 5.15}};
-constexpr TileCost kPlainCosts[] = {{TILE_256x256_W8, 3.4, 1.56, 0.74, 12.0}, {TILE_256x256_W4, 11.1, 1.41, 0.65, 10.0},
-                                    {TILE_128x128_W4, 0.9, 1.00, 0.42, 5.8},  {TILE_SMALL_W4, 0.0, 0.87, 0.29, 5.2},
-                                    {TILE_128x128_R4, 2.5, 0.48, 0.475, 6.0}, {TILE_128x256_R3, 3.5, 0.86, 0.73, 7.2},
-                                    {TILE_64x128_R3, 0.2, 0.57, 0.24, 5.9}};
+constexpr TileCost kDualCosts[] = {
+    {TILE_256x256_W4, 1, 7.2, 1.313, 0.77, 0.71, 5.05}, {TILE_128x128_W4, 2, 0.0, 0.992, 0.70, 0.69, 5.8},
+    {TILE_SMALL_W4, 3, 0.0, 0.958, 0.59, 0.66, 5.6},    {TILE_128x128_R4, 1, 1.5, 0.504, 0.74, 0.88, 6.2},
+    {TILE_128x256_R3, 1, 2.0, 0.836, 0.77, 0.79, 5.75}, {TILE_64x128_R3, 2, 1.05, 0.716, 0.51, 0.57, 6.1}};
+constexpr TileCost kPlainCosts[] = {
+    {TILE_256x256_W8, 1, 3.2, 1.31, 0.77, 0.91, 6.0},  {TILE_256x256_W4, 1, 13.0, 1.33, 0.64, 0.60, 6.0},
+    {TILE_128x128_W4, 2, 0.6, 0.88, 0.60, 0.74, 6.5},  {TILE_SMALL_W4, 3, 0.0, 0.805, 0.42, 0.62, 6.2},
+    {TILE_128x128_R4, 1, 1.9, 0.46, 0.485, 0.88, 7.4}, {TILE_128x256_R3, 1, 3.7, 0.80, 0.70, 0.90, 6.9},
+    {TILE_64x128_R3, 2, 0.2, 0.56, 0.42, 0.60, 6.1}};
 
 inline double routed_tile_time(const TileCost& c, bool dual, int64_t tiles_m, int modalities, int64_t M, int64_t n_out, int64_t K,
                                int splits) {
   const TileGeom t = tile_geom(c.tile, dual);
-  const double slots = kCus * (c.tile == TILE_SMALL_W4 ? 3 : (c.tile == TILE_128x128_W4 || c.tile == TILE_64x128_R3) ? 2 : 1);
-  const double slabs = (double)(K / 64), tiles = (double)(tiles_m * cdiv64(n_out, t.block_n_out) * splits);
-  const double round = c.base + c.per_slab * (double)cdiv64(K / 64, splits);
-  const double full = (double)(int64_t)(tiles / slots), rest = tiles - full * slots;
-  double time = full * round;
-  if (rest > 0.0) {
-    const double share = round * (c.partial + (1.0 - c.partial) * rest / slots);
-    if (!is_big_tile(c.tile) || splits > 1 || full == 0.0) {
-      time += share;
+  const int64_t slabs = K / 64, slots = (int64_t)kCus * c.per_cu;
+  const int64_t tiles = tiles_m * cdiv64(n_out, t.block_n_out) * splits;
+  const int64_t full = tiles / slots, rest = tiles - full * slots;
+  const double round = c.base + c.per_slab * (double)cdiv64(slabs, splits);
+  double time = (double)full * round;
+  if (rest > 0) {
+    const double fill = c.per_cu == 1 ? (double)rest / (double)slots : (double)(cdiv64(rest, kCus) - 1) / (double)(c.per_cu - 1);
+    if (!is_big_tile(c.tile) || splits > 1 || full == 0) {
+      const double part = full > 0 ? c.again : c.first;
+      time += round * (part + (1.0 - part) * fill);
     } else if (dual) {  // past half a round another round, else 128x128 tiles (whole_round_tiles)
-      time += rest > slots / 2 ? round : 3.0 + 1.08 * slabs * (0.5 + 0.5 * rest * 4.0 / 512.0);
+      time += rest > slots / 2 ? round : 3.0 + 1.08 * (double)slabs * (0.5 + 0.5 * (double)rest * 4.0 / 512.0);
     } else {            // split tail
-      const double cut = 8.0 + c.base + c.per_slab * slabs / (double)tail_split_factor((int)rest, (int)slabs);
+      const double cut = 8.0 + c.base + c.per_slab * (double)slabs / (double)tail_split_factor((int)rest, (int)slabs);
       time += cut < round ? cut : round;
     }
   }
   const double weights = modalities * (dual ? 2.0 : 1.0) * (double)K * (double)n_out * 2.0e-6 / c.tbs;
   const double hidden = dual ? 0.15 : 0.39;
   time = (dual ? 4.9 : 6.9) + (time > weights ? time + hidden * weights : weights + hidden * time);
-  if (splits > 1) time += 2.0 + (double)splits * (double)M * (double)n_out * 8.0e-6 / 7.2;  // partials and the reduce pass
+  if (splits > 1) time += 3.0 + (double)splits * (double)M * (double)n_out * 8.0e-6 / 7.2;  // partials and the reduce pass
   return time;
 }
 
@@ -135,8 +138,8 @@ inline double best_split(const TileCost& c, int64_t tiles_m, int modalities, int
   return best_time;
 }
 
-// The plan with the smallest product of two times: both modalities present, about evenly (M-tiles: the likelier of the two
-// counts), and one modality alone.  `split`: the caller has a workspace for partials and N % 4 == 0.
+// The plan with the smallest weighted product of two times: both modalities present, about evenly (M-tiles: the likelier of
+// the two counts; weight 3), and one modality alone (weight 2).  `split`: the caller has a workspace for partials and N % 4 == 0.
 inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split) {
   RoutedPlan p{TILE_SMALL_W4, 1, 1};
   double best = -1.0;
@@ -147,8 +150,9 @@ inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_
     const int64_t bm = tile_geom(costs[i].tile, dual).block_m;
     const int64_t one = cdiv64(M, bm), both = M / bm + 1 + (M % bm > bm / 2 ? 1 : 0);
     int s = 1;
-    const double t = dual ? routed_tile_time(costs[i], true, both, 2, M, n_out, K, 1) * routed_tile_time(costs[i], true, one, 1, M, n_out, K, 1)
-                          : best_split(costs[i], both, 2, M, n_out, K, split, 1, &s) * best_split(costs[i], one, 1, M, n_out, K, split, 1, &s);
+    const double t2 = dual ? routed_tile_time(costs[i], true, both, 2, M, n_out, K, 1) : best_split(costs[i], both, 2, M, n_out, K, split, 1, &s);
+    const double t1 = dual ? routed_tile_time(costs[i], true, one, 1, M, n_out, K, 1) : best_split(costs[i], one, 1, M, n_out, K, split, 1, &s);
+    const double t = t2 * t2 * t2 * t1 * t1;
     if (best < 0.0 || t < best) {
       best = t;
       pick = costs + i;
