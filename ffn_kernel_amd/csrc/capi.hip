@@ -215,7 +215,7 @@ FfnBwdPlan plan_ffn_bwd(int64_t M, int64_t d, int64_t h, bool dup_k_contig, bool
 // when its rows are gathered, from the tile's first row otherwise (at most 256 rows away).
 bool direct_ok(int64_t K, int64_t gathered_rows, int64_t lda, int64_t ldb) {
   constexpr int64_t k4g = (int64_t)1 << 32;
-  if (K <= 0 || K % 64 != 0) return false;
+  if (!direct_contraction(K)) return false;
   if (gathered_rows > 0 && gathered_rows * lda * 2 >= k4g) return false;
   return 256 * lda * 2 < k4g && 256 * ldb * 2 < k4g;
 }
@@ -224,7 +224,7 @@ bool direct_ok(int64_t K, int64_t gathered_rows, int64_t lda, int64_t ldb) {
 // contiguous, row stride ldb.  Slabs are addressed with 32-bit byte offsets from their first row.
 bool kmajor_ok(int64_t K, int64_t N, int64_t ldb, const void* w0, const void* w1) {
   constexpr int64_t k4g = (int64_t)1 << 32;
-  return K > 0 && K % 64 == 0 && N >= 8 && N % 8 == 0 && ldb % 8 == 0 && ldb >= N && aligned16(w0) && aligned16(w1) &&
+  return direct_contraction(K) && N >= 8 && N % 8 == 0 && ldb % 8 == 0 && ldb >= N && aligned16(w0) && aligned16(w1) &&
          ldb * 128 + 2 * N < k4g;
 }
 
@@ -304,7 +304,7 @@ RoutedPlan down_plan(int64_t M, int64_t d, int64_t h, int op = TUNED_DOWN) {
     p = pick_routed_plan(M, d, h, use_tuned(), op);
   }
   // a forced split-K factor: whole 64-element slabs, no empty range, what the reduce pass can address
-  if (const int fs = forced_splits(); fs >= 1 && h % 64 == 0 && M < 65536 && cdiv64(h / 64, cdiv64(h / 64, fs)) == fs &&
+  if (const int fs = forced_splits(); fs >= 1 && direct_contraction(h) && M < 65536 && cdiv64(cdiv64(h, 64), cdiv64(cdiv64(h, 64), fs)) == fs &&
       p.tile != TILE_256x256_W4)
     p.splits = p.splits_more = fs;
   return p;
@@ -312,7 +312,7 @@ RoutedPlan down_plan(int64_t M, int64_t d, int64_t h, int op = TUNED_DOWN) {
 int max_splits(const RoutedPlan& p) { return p.splits > p.splits_more ? p.splits : p.splits_more; }
 // fp32 tiles of the split tail of an unsplit 256x256 tile: only a launch of more than one round has one.
 size_t tail_bytes(const RoutedPlan& p, int64_t M, int64_t n_out, int64_t K) {
-  return is_big_tile(p.tile) && K % 64 == 0 && (cdiv64(M, 256) + 1) * cdiv64(n_out, 256) > kCus
+  return is_big_tile(p.tile) && direct_contraction(K) && (cdiv64(M, 256) + 1) * cdiv64(n_out, 256) > kCus
              ? ws_align((size_t)kTailSlots * 256 * 256 * 4) : 0;
 }
 // The MaskedFFN forward's down projection.  Where the scratch of the static entry point holds what the plan by tile count
@@ -327,7 +327,8 @@ RoutedPlan ffn_down_plan(int64_t M, int64_t d, int64_t h) {
     return fixed + (s > 1 ? ws_align(s * part) : tail_bytes(q, M, d, h)) <= (size_t)FFNK_STATIC_SCRATCH_BYTES;
   };
   if (fixed > (size_t)FFNK_STATIC_SCRATCH_BYTES || fits(p)) return p;
-  const RoutedPlan plain = pick_routed_plan(M, d, h, false, TUNED_NONE);
+  RoutedPlan plain = pick_routed_plan(M, d, h, false, TUNED_NONE);
+  if (h % 64 != 0) plain = {TILE_128x128_W4, 1, 1};  // no partials and no tail
   if (!fits(plain)) return p;
   if (p.splits > 1) {
     for (int s = max_splits(p) - 1; s >= 2; --s) {
@@ -562,7 +563,7 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
     case FFNK_OP_BWD_DW: {
       // As launched for the reference's layout (nn.Linear.weight.T views, contiguous g): weights read in place.
       const BwdPlan bp = plan_bwd(M, K, N, true);
-      const bool w_kmajor = N > 0 && N % 64 == 0 && K >= 8 && K % 8 == 0 && direct_ok(N, M, N, 8);
+      const bool w_kmajor = K >= 8 && K % 8 == 0 && direct_ok(N, M, N, 8);
       in_place = bp.gather && gather_dw_ok(M, K, N, nullptr, N, nullptr, K);
       tile = in_place ? TILE_128x128_W4 : bp.tc.tile; contraction = M;
       splits = bwd_dw_launch_splits(M, K, N, bp, bwd_is_fused(M, K, bp, w_kmajor, in_place));
@@ -570,7 +571,7 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
     }
     default: return fail(FFNK_E_OP, "unknown op %d", op);
   }
-  const bool direct = contraction > 0 && contraction % 64 == 0;
+  const bool direct = direct_contraction(contraction);
   if (!direct && tile == TILE_256x256_W4) tile = TILE_256x256_W8;  // the four-wave tile runs on the direct path only
   const TileGeom gm = tile_geom(tile, dual);
   const bool stream = (op == FFNK_OP_FFN_FWD || op == FFNK_OP_FFN_UP || op == FFNK_OP_FFN_DOWN) && use_stream_path(M, K, N);
@@ -593,10 +594,10 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
   const bool kmajor_dx = op == FFNK_OP_LINEAR_BWD || op == FFNK_OP_BWD_DX;
   out->group_m = plan_gm > 0 ? plan_gm : (dual || kmajor_dx) ? 8 : 4;
   out->split_k = splits;
-  out->direct_lds = (direct || in_place) ? 1 : 0;
+  out->direct_lds = ((direct && contraction % 64 == 0) || in_place) ? 1 : 0;
   out->in_place = in_place ? 1 : 0;
   // 4: ring of four stages (128x128); 3: token panel in three stages, weight panel in two (single-weight 256x256 tiles)
-  out->lds_stages = !out->direct_lds ? 2 : tile == TILE_128x128_R4 ? 4 : (tile == TILE_128x256_R3 || tile == TILE_64x128_R3) ? 3 : (is_big_tile(tile) && !dual) ? 3 : 2;
+  out->lds_stages = !(direct || in_place) ? 2 : tile == TILE_128x128_R4 ? 4 : (tile == TILE_128x256_R3 || tile == TILE_64x128_R3) ? 3 : (is_big_tile(tile) && !dual) ? 3 : 2;
   if (op == FFNK_OP_FFN_DOWN && !stream) out->split_k = tiled_down_splits(M, K, N);
   if (op == FFNK_OP_LINEAR_FWD && linear_stream_kind(M, K, N)) {
     out->path = FFNK_PATH_STREAM;

@@ -6,8 +6,8 @@
 // on every mixed tile.
 //
 // Data path per workgroup: 64-column K slabs of the A and B panels go global -> LDS, two stages
-// deep (directly, bypassing registers, when K is a multiple of 64; staged through registers
-// otherwise); wavefronts read 16-byte MFMA fragments from an XOR-swizzled LDS layout and issue
+// deep (directly, bypassing registers; staged through registers where 32-bit offsets do not reach and
+// for short contractions that are no whole number of slabs); wavefronts read 16-byte MFMA fragments from an XOR-swizzled LDS layout and issue
 // v_mfma_f32_16x16x32_bf16 on the 256-row direct tiles (gemm_mainloop_fixed16) and v_mfma_f32_32x32x16_bf16
 // on the others (gemm_mainloop_slab_dma, gemm_mainloop_ring, gemm_mainloop_staged).
 //
@@ -102,7 +102,7 @@ struct RoutedGemmCfg {
   static constexpr bool DUAL = DUAL_;
   static constexpr bool GATHER_A = GATHER_A_;
   static constexpr bool SCATTER_C = SCATTER_C_;
-  static constexpr bool DIRECT = DIRECT_;   // global->LDS loads bypass registers (needs K % 64 == 0)
+  static constexpr bool DIRECT = DIRECT_;   // global->LDS loads bypass registers (needs K % 8 == 0)
   static constexpr int GROUP_M = GROUP_M_;
   // Weight panels are [K, N] rows with N contiguous (the backward's view of a forward weight) and
   // are transposed on the way from LDS to the MFMA operand, see KMajorB.
@@ -238,6 +238,28 @@ struct TileLanes {
   __device__ __forceinline__ int load_row(int j) const { return group_row(j) + (int)r_in; }
 };
 
+// ---------------------------------------------------------------------------------------------
+// Contractions that are no whole number of slabs (direct path, K % 8 == 0, K >= 64).  The slabs are counted from the END of
+// the contraction, so slab 0 would start `pad` = -K mod 64 elements ahead of it.  It is loaded from the contraction's start
+// instead - `pad` elements on, one scalar offset, no lane out of bounds - and its last `pad` elements, which are slab 1's
+// first, are cleared once they have landed, every lane clearing the LDS slots it filled itself.  The steady loops are those
+// of K % 64 == 0.  Against the register-staged loop with its guard on every load, which ran these before: MaskedLinear
+// M = 3001, K = 2056, N = 1544 48.1 -> 39.5 us; MaskedFFN d = 2104, h = 7176, M = 594 174 -> 91 us, d = 2040, h = 6528,
+// M = 27470 2136 -> 1778 us, and in decode, where K splits over workgroups, d = 5832, h = 11784, M = 13 298 -> 110 us.
+// ---------------------------------------------------------------------------------------------
+template <class Cfg>
+__device__ __forceinline__ void clear_head(const TileLanes<Cfg>& tl, int pad, uint8_t* a_panel, uint8_t* b_panel) {
+  const bool surplus = (int)tl.c_log * 8 >= kBK - pad;  // pad % 8 == 0: a 16-byte piece is all surplus or none of it
+  const uint4 zero = make_uint4(0, 0, 0, 0);
+#pragma unroll
+  for (int j = 0; j < TileLanes<Cfg>::NJA; ++j)
+    if (surplus) *reinterpret_cast<uint4*>(a_panel + (j * Cfg::NWAVES + tl.wave) * 1024 + tl.lane * 16) = zero;
+#pragma unroll
+  for (int j = 0; j < TileLanes<Cfg>::NJB; ++j)
+    if (Cfg::B_KMAJOR ? tl.kb_group_row(j) >= kBK - pad : surplus)
+      *reinterpret_cast<uint4*>(b_panel + (j * Cfg::NWAVES + tl.wave) * 1024 + tl.lane * 16) = zero;
+}
+
 // =============================================================================================
 // Register-staged path: 64-element K slabs, global -> registers -> LDS, double-buffered.  Handles
 // any K that is a multiple of 8 (chunks past the end are zero-filled).
@@ -332,14 +354,14 @@ __device__ __forceinline__ void gemm_mainloop_staged(const TileLanes<Cfg>& tl,
 // has been read (its stage can be refilled with the slab after next) and the next slab, issued
 // one iteration earlier, has landed (its first fragments are read during the last K step).
 // =============================================================================================
-template <class Cfg>
+template <class Cfg, class Late>
 __device__ __forceinline__ void gemm_mainloop_slab_dma(const TileLanes<Cfg>& tl,
                                                        const uint16_t* const (&baseA)[TileLanes<Cfg>::NJA],
                                                        const uint32_t (&offA)[TileLanes<Cfg>::NJA],
                                                        const uint16_t* const (&baseB)[TileLanes<Cfg>::NJB],
                                                        const uint32_t (&offB)[TileLanes<Cfg>::NJB], int k_len,
                                                        uint8_t* lds, typename Cfg::Acc (&acc)[Cfg::TM][Cfg::TN],
-                                                       const KMajorB& kb = KMajorB()) {
+                                                       const KMajorB& kb, const int pad, Late&& late_offsets) {
   static_assert(!Cfg::MFMA16, "16x16x32 tiles run gemm_mainloop_fixed16");
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int NWAVES = Cfg::NWAVES, TM = Cfg::TM, TN = Cfg::TN;
@@ -400,29 +422,31 @@ __device__ __forceinline__ void gemm_mainloop_slab_dma(const TileLanes<Cfg>& tl,
   zero_acc<Cfg>(acc);
   const int nk = k_len / kBK;
 
-  auto issue_a = [&](int stage, int kt) {
+  // head: elements from the slab's place to where it is loaded (slab 0 of a ragged contraction, see clear_head)
+  auto issue_a = [&](int stage, int kt, int head = 0) {
     uint8_t* st = lds + stage * STAGE;
-    const int ko = kt * kRowBytes;
+    const int ko = kt * kRowBytes + head * 2;
 #pragma unroll
     for (int j = 0; j < NJA; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA[j], FFNK_LDS_PTR(st + (j * NWAVES + wave) * 1024), 16, offA[j], ko, 0, 0);
   };
   // K-major: the slab's resource (weight and slab offset folded into the base, all scalar).
-  auto kmajor_rsrc = [&](int kt) {
+  auto kmajor_rsrc = [&](int kt, int head = 0) {
     const int ka = kb.kt_first + kt;
     const bool second = ka >= kb.kt_switch;
-    const uint64_t base = (second ? kw[1] : kw[0]) + (uint64_t)(uint32_t)(second ? ka - kb.kt_switch : ka) * kb.slab_bytes;
+    const uint64_t base = (second ? kw[1] : kw[0]) + (uint64_t)(uint32_t)(second ? ka - kb.kt_switch : ka) * kb.slab_bytes +
+                          (uint64_t)(uint32_t)head * (kb.slab_bytes / kBK);
     return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), 0, 0xffffffff, 0x00020000);
   };
-  auto issue_b = [&](int stage, int kt) {
+  auto issue_b = [&](int stage, int kt, int head = 0) {
     uint8_t* st = lds + stage * STAGE;
     if constexpr (Cfg::B_KMAJOR) {
-      const __amdgpu_buffer_rsrc_t rs = kmajor_rsrc(kt);
+      const __amdgpu_buffer_rsrc_t rs = kmajor_rsrc(kt, head);
 #pragma unroll
       for (int j = 0; j < NJB; ++j)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, FFNK_LDS_PTR(st + A_BYTES + (j * NWAVES + wave) * 1024), 16, offB[j], 0, 0, 0);
     } else {
-      const int ko = kt * kRowBytes;
+      const int ko = kt * kRowBytes + head * 2;
 #pragma unroll
       for (int j = 0; j < NJB; ++j)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB[j], FFNK_LDS_PTR(st + A_BYTES + (j * NWAVES + wave) * 1024), 16, offB[j], ko, 0, 0);
@@ -539,14 +563,20 @@ __device__ __forceinline__ void gemm_mainloop_slab_dma(const TileLanes<Cfg>& tl,
 
   // Head of the tile: the weight panels of the first two slabs go out first - their addresses do not
   // depend on the routing - so that they fly while the gathered token rows' indices are still loading.
-  issue_b(0, 0);
+  issue_b(0, 0, pad);
   if (nk > 1) issue_b(1, 1);
-  issue_a(0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  late_offsets();
+  issue_a(0, 0, pad);
   if (nk > 1) {
     issue_a(1, 1);
     dma_wait_barrier<NJA>();  // in issue order only the token panel of slab 1 may still be under way
   } else {
     dma_wait_barrier<0>();
+  }
+  if (pad > 0) {  // uniform over the launch's workgroups of this K range
+    clear_head<Cfg>(tl, pad, lds, lds + A_BYTES);
+    dma_wait_barrier<NJA>();
   }
   if constexpr (Cfg::B_KMAJOR) {
     if (nk == 1 && kb.last_rows < kBK) kmajor_clear_tail(0);
@@ -635,14 +665,14 @@ __device__ __forceinline__ void gemm_mainloop_slab_dma(const TileLanes<Cfg>& tl,
 //    them.  The range's last slab may be ragged: its surplus rows are cleared behind the data barrier that
 //    announces it (tail of the loop only).
 // =============================================================================================
-template <class Cfg>
+template <class Cfg, class Late>
 __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
                                                       const uint16_t* const (&baseA)[TileLanes<Cfg>::NJA],
                                                       const uint32_t (&offA)[TileLanes<Cfg>::NJA],
                                                       const uint16_t* const (&baseB)[TileLanes<Cfg>::NJB],
                                                       const uint32_t (&offB)[TileLanes<Cfg>::NJB], int k_len,
                                                       uint8_t* lds, typename Cfg::Acc (&acc)[Cfg::TM][Cfg::TN],
-                                                      const KMajorB& kb = KMajorB()) {
+                                                      const KMajorB& kb, const int pad, Late&& late_offsets) {
   static_assert(Cfg::MFMA16 && Cfg::DIRECT, "16x16x32 schedule of the direct 256-row tiles");
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int NWAVES = Cfg::NWAVES, TM = Cfg::TM, TN = Cfg::TN;
@@ -691,10 +721,11 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
       kw[i] = ((uint64_t)hi << 32) | lo;
     }
   }
-  auto kmajor_rsrc = [&](int kt) {
+  auto kmajor_rsrc = [&](int kt, int head = 0) {
     const int ka = kb.kt_first + kt;
     const bool second = ka >= kb.kt_switch;
-    const uint64_t base = (second ? kw[1] : kw[0]) + (uint64_t)(uint32_t)(second ? ka - kb.kt_switch : ka) * kb.slab_bytes;
+    const uint64_t base = (second ? kw[1] : kw[0]) + (uint64_t)(uint32_t)(second ? ka - kb.kt_switch : ka) * kb.slab_bytes +
+                          (uint64_t)(uint32_t)head * (kb.slab_bytes / kBK);
     return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), 0, 0xffffffff, 0x00020000);
   };
 
@@ -772,13 +803,14 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
       for (int j = 0; j < TN; ++j) fb[buf][j] = __builtin_shufflevector(fb_lo[buf][j], fb_hi[buf][j], 0, 1, 2, 3, 4, 5, 6, 7);
     }
   };
-  auto load_b = [&](int l, int b_off, int kt) {
+  // head: elements from the slab's place to where it is loaded (slab 0 of a ragged contraction, see clear_head)
+  auto load_b = [&](int l, int b_off, int kt, int head = 0) {
     if constexpr (KM)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(kmajor_rsrc(kt), FFNK_LDS_PTR(lds + b_off + (l * NWAVES + wave) * 1024), 16,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(kmajor_rsrc(kt, head), FFNK_LDS_PTR(lds + b_off + (l * NWAVES + wave) * 1024), 16,
                                                offB[l], 0, 0, 0);
     else
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB[l], FFNK_LDS_PTR(lds + b_off + (l * NWAVES + wave) * 1024), 16, offB[l],
-                                               kt * kRowBytes, 0, 0);
+                                               kt * kRowBytes + head * 2, 0, 0);
   };
   // K-major: clear rows [last_rows, 64) of the weight panel at b_off (the range's last slab, after it has landed and
   // before anyone reads it).  Rows are RB contiguous bytes each, whatever the swizzle inside them.
@@ -788,14 +820,14 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
     for (int o = (int)threadIdx.x * 16; o < bytes; o += Cfg::NT * 16) *reinterpret_cast<uint4*>(first + o) = make_uint4(0, 0, 0, 0);
     dma_wait_barrier<0>();
   };
-  auto load_a = [&](int l, int a_off, int kt) {
+  auto load_a = [&](int l, int a_off, int kt, int head = 0) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA[l], FFNK_LDS_PTR(lds + a_off + (l * NWAVES + wave) * 1024), 16, offA[l],
-                                             kt * kRowBytes, 0, Cfg::AUX_A);
+                                             kt * kRowBytes + head * 2, 0, Cfg::AUX_A);
   };
   // Two-stage form: load l of a slab - the weight panel's first, then the token panel's - into stage t.
-  auto load = [&](int l, int t, int kt) {
-    if (l < NJB) load_b(l, b_stage(t), kt);
-    else load_a(l - NJB, a_stage(t), kt);
+  auto load = [&](int l, int t, int kt, int head = 0) {
+    if (l < NJB) load_b(l, b_stage(t), kt, head);
+    else load_a(l - NJB, a_stage(t), kt, head);
   };
   // Four-wave tiles hold 256 accumulator registers per lane, which only fit the accumulation half of the
   // register file.  Left to the builtin, the compiler keeps part of them in ordinary registers and moves
@@ -887,7 +919,11 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
   // Head of the tile: slab 0 whole and, of slab 1, what the steady schedule would have issued by now: all of it in
   // the ring form, its first L1 loads in the two-stage form.
 #pragma unroll
-  for (int l = 0; l < L; ++l) load(l, 0, 0);
+  for (int l = 0; l < NJB; ++l) load(l, 0, 0, pad);
+  __builtin_amdgcn_sched_barrier(0);
+  late_offsets();
+#pragma unroll
+  for (int l = NJB; l < L; ++l) load(l, 0, 0, pad);
   if (nk > 1) {
     if constexpr (R3) {  // token panel first, as the steady schedule issues them
 #pragma unroll
@@ -902,6 +938,10 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
     }
   } else {
     dma_wait_barrier<0>();
+  }
+  if (pad > 0) {  // uniform over the launch's workgroups of this K range
+    clear_head<Cfg>(tl, pad, lds + a_stage(0), lds + b_stage(0));
+    dma_wait_barrier<R3 ? L : L1>();
   }
   if constexpr (KM) {
     if (nk == 1 && kb.last_rows < kBK) clear_tail(b_stage(0));
@@ -984,14 +1024,14 @@ __device__ __forceinline__ void static_for(F&& f) {
 // kt + 1 has landed (loads complete in order, so "at most (S - 2) slabs of loads outstanding").  Same
 // source-order schedule as the 256-row tiles.
 // =============================================================================================
-template <class Cfg>
+template <class Cfg, class Late>
 __device__ __forceinline__ void gemm_mainloop_ring(const TileLanes<Cfg>& tl,
                                                    const uint16_t* const (&baseA)[TileLanes<Cfg>::NJA],
                                                    const uint32_t (&offA)[TileLanes<Cfg>::NJA],
                                                    const uint16_t* const (&baseB)[TileLanes<Cfg>::NJB],
                                                    const uint32_t (&offB)[TileLanes<Cfg>::NJB], int k_len,
                                                    uint8_t* lds, typename Cfg::Acc (&acc)[Cfg::TM][Cfg::TN],
-                                                   const KMajorB& kb = KMajorB()) {
+                                                   const KMajorB& kb, const int pad, Late&& late_offsets) {
   static_assert(Cfg::RING && !Cfg::MFMA16, "ring schedule of the small direct tiles");
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int NWAVES = Cfg::NWAVES, TM = Cfg::TM, TN = Cfg::TN, S = Cfg::STAGES, D = S - 1;
@@ -1032,10 +1072,11 @@ __device__ __forceinline__ void gemm_mainloop_ring(const TileLanes<Cfg>& tl,
       kw[q] = ((uint64_t)hi << 32) | lo;
     }
   }
-  auto kmajor_rsrc = [&](int kt) {
+  auto kmajor_rsrc = [&](int kt, int head = 0) {
     const int ka = kb.kt_first + kt;
     const bool second = ka >= kb.kt_switch;
-    const uint64_t base = (second ? kw[1] : kw[0]) + (uint64_t)(uint32_t)(second ? ka - kb.kt_switch : ka) * kb.slab_bytes;
+    const uint64_t base = (second ? kw[1] : kw[0]) + (uint64_t)(uint32_t)(second ? ka - kb.kt_switch : ka) * kb.slab_bytes +
+                          (uint64_t)(uint32_t)head * (kb.slab_bytes / kBK);
     return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), 0, 0xffffffff, 0x00020000);
   };
   uint32_t koff[4];
@@ -1094,13 +1135,14 @@ __device__ __forceinline__ void gemm_mainloop_ring(const TileLanes<Cfg>& tl,
       for (int j = 0; j < TN; ++j) fb[buf][j] = __builtin_shufflevector(fb_lo[buf][j], fb_hi[buf][j], 0, 1, 2, 3, 4, 5, 6, 7);
     }
   };
-  auto load = [&](int l, int stage, int kt) {
+  // head: elements from the slab's place to where it is loaded (slab 0 of a ragged contraction, see clear_head)
+  auto load = [&](int l, int stage, int kt, int head = 0) {
     uint8_t* st = lds + stage * STAGE;
-    const int ko = kt * kRowBytes;
+    const int ko = kt * kRowBytes + head * 2;
     if (l < NJB) {
       if constexpr (KM)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(kmajor_rsrc(kt), FFNK_LDS_PTR(st + A_BYTES + (l * NWAVES + wave) * 1024), 16, offB[l],
-                                                 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(kmajor_rsrc(kt, head), FFNK_LDS_PTR(st + A_BYTES + (l * NWAVES + wave) * 1024), 16,
+                                                 offB[l], 0, 0, 0);
       else
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB[l], FFNK_LDS_PTR(st + A_BYTES + (l * NWAVES + wave) * 1024), 16, offB[l], ko, 0, 0);
     } else
@@ -1151,7 +1193,13 @@ __device__ __forceinline__ void gemm_mainloop_ring(const TileLanes<Cfg>& tl,
   for (int j = 0; j < D; ++j)
     if (j < nk) {
 #pragma unroll
-      for (int l = 0; l < L; ++l) load(l, j, j);
+      for (int l = 0; l < L; ++l) {
+        if (j == 0 && l == NJB) {
+          __builtin_amdgcn_sched_barrier(0);
+          late_offsets();
+        }
+        load(l, j, j, j == 0 ? pad : 0);
+      }
       issued += L;
     }
   if (D < nk) {
@@ -1160,6 +1208,10 @@ __device__ __forceinline__ void gemm_mainloop_ring(const TileLanes<Cfg>& tl,
     issued += LQ < L ? LQ : L;
   }
   dma_wait_barrier_n(issued - L);  // slab 0 has landed
+  if (pad > 0) {                   // uniform over the launch's workgroups of this K range
+    clear_head<Cfg>(tl, pad, lds, lds + A_BYTES);
+    dma_wait_barrier<63>();
+  }
 #pragma unroll
   for (int r = 0; r < ND; ++r) read_frag(0, 0, std::integral_constant<int, 0>{}, r);
 
@@ -1172,18 +1224,20 @@ __device__ __forceinline__ void gemm_mainloop_ring(const TileLanes<Cfg>& tl,
 #endif
 }
 
-// Main loop of a direct-path tile, by the tile's MFMA shape.
-template <class Cfg>
+// Main loop of a direct-path tile, by the tile's MFMA shape.  `pad`: see clear_head.  late_offsets() fills in offA where it
+// comes from loaded indices; it is called once slab 0's weight panel is on its way, and a scheduling barrier keeps the wait
+// for the indices behind those loads.
+template <class Cfg, class Late>
 __device__ __forceinline__ void gemm_mainloop_direct(const TileLanes<Cfg>& tl,
                                                      const uint16_t* const (&baseA)[TileLanes<Cfg>::NJA],
                                                      const uint32_t (&offA)[TileLanes<Cfg>::NJA],
                                                      const uint16_t* const (&baseB)[TileLanes<Cfg>::NJB],
                                                      const uint32_t (&offB)[TileLanes<Cfg>::NJB], int k_len,
                                                      uint8_t* lds, typename Cfg::Acc (&acc)[Cfg::TM][Cfg::TN],
-                                                     const KMajorB& kb = KMajorB()) {
-  if constexpr (Cfg::MFMA16) gemm_mainloop_fixed16<Cfg>(tl, baseA, offA, baseB, offB, k_len, lds, acc, kb);
-  else if constexpr (Cfg::RING) gemm_mainloop_ring<Cfg>(tl, baseA, offA, baseB, offB, k_len, lds, acc, kb);
-  else gemm_mainloop_slab_dma<Cfg>(tl, baseA, offA, baseB, offB, k_len, lds, acc, kb);
+                                                     const KMajorB& kb, const int pad, Late&& late_offsets) {
+  if constexpr (Cfg::MFMA16) gemm_mainloop_fixed16<Cfg>(tl, baseA, offA, baseB, offB, k_len, lds, acc, kb, pad, late_offsets);
+  else if constexpr (Cfg::RING) gemm_mainloop_ring<Cfg>(tl, baseA, offA, baseB, offB, k_len, lds, acc, kb, pad, late_offsets);
+  else gemm_mainloop_slab_dma<Cfg>(tl, baseA, offA, baseB, offB, k_len, lds, acc, kb, pad, late_offsets);
 }
 
 // Map a launch-order workgroup id to a position L in the tile order such that every XCD
@@ -1356,7 +1410,7 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
       sub_n = (bid % q) % qn;
     } else {
       const int n_tail = total - full;
-      splits = tail_split_factor(n_tail, g.K / kBK);
+      splits = tail_split_factor(n_tail, cdiv(g.K, kBK));
       tail_slot = bid;
       if (tail_slot >= n_tail * splits) return;
       split = tail_slot / n_tail;
@@ -1377,11 +1431,14 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
     TileLanes<Cfg> rl;
     rl.init();
     // This workgroup's part of the contraction (all of it unless the launch splits K).
-    const int nk = g.K / kBK;
+    // Slabs are counted from the end of the contraction: slab 0's place starts k_ahead elements ahead of it (clear_head).
+    const int nk = cdiv(g.K, kBK);
     const int per_split = cdiv(nk, splits);
     const int kt0 = min(split * per_split, nk);
     const int k_len = (min(kt0 + per_split, nk) - kt0) * kBK;
-    const int64_t k0 = (int64_t)kt0 * kBK;
+    const int k_ahead = nk * kBK - g.K;
+    const int64_t k0 = (int64_t)kt0 * kBK - k_ahead;
+    const int pad = kt0 == 0 ? k_ahead : 0;
     const uint16_t* baseA[NJA];
     uint32_t offA[NJA];
     const uint16_t* baseB[NJB];
@@ -1389,14 +1446,18 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
     // Gathered rows are addressed from the start of A (the host checks that 32 bits reach every
     // row); contiguous panels from their own first row.
     const uint16_t* a0 = (Cfg::GATHER_A ? g.A : g.A + (int64_t)row0 * g.lda) + k0;
+    int src[NJA];
 #pragma unroll
     for (int j = 0; j < NJA; ++j) {
       int p = row0 + rl.load_row(j);
       p = min(p, row_end - 1);  // rows past the group end repeat the last row; never stored
-      const int64_t src = Cfg::GATHER_A ? (int64_t)g.perm[p] : (int64_t)(p - row0);
+      src[j] = Cfg::GATHER_A ? g.perm[p] : p - row0;
       baseA[j] = a0;
-      offA[j] = (uint32_t)((src * g.lda + rl.c_log * 8) * 2);
     }
+    auto offsets_a = [&]() {
+#pragma unroll
+      for (int j = 0; j < NJA; ++j) offA[j] = (uint32_t)(((int64_t)src[j] * g.lda + rl.c_log * 8) * 2);
+    };
     KMajorB kb;
     if constexpr (Cfg::B_KMAJOR) {
       // Offsets inside a slab: row of the slab times the row stride, plus this lane's column chunk
@@ -1407,8 +1468,8 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
         baseB[j] = nullptr;
         offB[j] = (uint32_t)(((int64_t)rl.kb_group_row(j) * g.ldb + n) * 2);
       }
-      kb.w[0] = g.B0[grp];
-      kb.w[1] = g.k_switch > 0 ? g.B1[grp] : g.B0[grp];
+      kb.w[0] = g.B0[grp] - (int64_t)k_ahead * g.ldb;
+      kb.w[1] = g.k_switch > 0 ? g.B1[grp] : kb.w[0];  // (k_switch: whole slabs, k_ahead = 0)
       kb.kt_first = kt0;
       if (g.k_switch > 0) kb.kt_switch = g.k_switch / kBK;
       kb.slab_bytes = (uint32_t)(g.ldb * (kBK * 2));
@@ -1423,7 +1484,7 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
         offB[j] = (uint32_t)(((int64_t)(n - n_first) * g.ldb + rl.c_log * 8) * 2);
       }
     }
-    if (k_len > 0) gemm_mainloop_direct<Cfg>(rl, baseA, offA, baseB, offB, k_len, lds, acc, kb);
+    if (k_len > 0) gemm_mainloop_direct<Cfg>(rl, baseA, offA, baseB, offB, k_len, lds, acc, kb, pad, offsets_a);
     else zero_acc<Cfg>(acc);  // a range past the end of K contributes exact zeros
     if (!Cfg::DUAL && splits > 1) {
       if (g.tail_mode == 3)  // one compact fp32 tile per (tile, range) pair
@@ -1588,7 +1649,7 @@ __device__ __forceinline__ void grouped_splitk_body(const SplitKArgs& g, uint8_t
         offB[j] = (uint32_t)(((int64_t)(r - r_first) * g.lda + rl.c_log * 8) * 2);
       }
     }
-    gemm_mainloop_direct<Cfg>(rl, baseA, offA, baseB, offB, k_len, lds, acc, kb);
+    gemm_mainloop_direct<Cfg>(rl, baseA, offA, baseB, offB, k_len, lds, acc, kb, 0, [] {});
   } else {
     zero_acc<Cfg>(acc);  // a split without slabs (e.g. an empty modality) contributes exact zeros
   }
@@ -1631,8 +1692,9 @@ inline hipError_t launch_routed_gemm(const GemmArgs& g, hipStream_t stream) {
   if (g.M <= 0 || g.N <= 0) return hipSuccess;
   if ((g.splits > 1 || g.splits_more > 1) && (Cfg::DUAL || !Cfg::DIRECT || g.tail_mode != 0 || g.P == nullptr)) return hipErrorInvalidValue;
   if ((g.splits > 1) != (g.splits_more > 1)) return hipErrorInvalidValue;
-  if (Cfg::B_KMAJOR && (g.N % 8 != 0 || g.K % kBK != 0 || g.k_switch % kBK != 0 || g.k_switch < 0 || g.k_switch >= g.K ||
-                        g.ldb * (kBK * 2) + 2 * (int64_t)g.N >= ((int64_t)1 << 32)))
+  if (Cfg::DIRECT && (g.K <= 0 || g.K % 8 != 0)) return hipErrorInvalidValue;
+  if (Cfg::B_KMAJOR && (g.N % 8 != 0 || g.k_switch % kBK != 0 || g.k_switch < 0 || g.k_switch >= g.K ||
+                        (g.k_switch > 0 && g.K % kBK != 0) || g.ldb * (kBK * 2) + 2 * (int64_t)g.N >= ((int64_t)1 << 32)))
     return hipErrorInvalidValue;
   if (!Cfg::B_KMAJOR && g.k_switch != 0) return hipErrorInvalidValue;
   const int grid = routed_gemm_grid<Cfg>(g.M, g.N, g.splits, g.splits_more);

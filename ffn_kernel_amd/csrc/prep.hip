@@ -297,7 +297,7 @@ __global__ __launch_bounds__(256) void routed_tail_reduce_kernel(const float* __
   const int n_tail = total - full;
   const int tile_i = blockIdx.x;
   if (tile_i >= n_tail) return;
-  const int splits = tail_split_factor(n_tail, K / 64);
+  const int splits = tail_split_factor(n_tail, cdiv(K, 64));
   if (splits == 1) return;  // the GEMM stored this tile itself
   const TileCoord tc = routed_tile_coord(full + tile_i, n_vis, M, N, bm, bn, group_m);
   const int quads = bn / 4;                   // float4 columns per tile row

@@ -23,6 +23,12 @@ struct TileChoice {
   bool tuned;  // the pair is a measured plan (as timed by the tuner), not the rules' guess
 };
 
+// Contractions that the direct kernels run: whole 64-element slabs, or 16-byte pieces with the first slab partly ahead of
+// the contraction (clear_head in gemm_nt.hpp).  Under 128 elements the part ahead is a third of the work and more, and the
+// register-staged loop stays.
+constexpr int kRaggedMinK = 128;
+inline bool direct_contraction(int64_t K) { return K > 0 && (K % 64 == 0 || (K % 8 == 0 && K >= kRaggedMinK)); }
+
 // Measured plans.  `python -m ffn_kernel_amd.tune --emit` times every candidate (tile x split-K factor)
 // per operation, shape and M bucket on the GPU and writes tile_table_gen.hpp: one entry wherever the best
 // candidate beat the rules and the cost model below by a margin.  The pick_* functions consult these
@@ -76,27 +82,38 @@ struct RoutedPlan {
 // behind the best tile and split of each shape, the rules by tile count before were 12 % behind (SwiGLU GEMM at M = 300 / 512 /
 // 1024 of one modality, d = 4096, h = 14336: 128 -> 98, 150 -> 100, 274 -> 183 us; single-weight GEMM at M = 512, K = 14336,
 // N = 4096: 105 -> 70 us; at M = 1024, 4096 x 4096: 49 -> 38 us).
+// Where K % 64 != 0 the rows of a packed operand start anywhere in a 128-byte line and every 128-byte piece of a slab lies in
+// two lines: a slab takes `ragged` times as long, the more the fewer flops the tile has per byte it loads (all tiles at
+// M x K x N = 3001 x 2056 x 1544, 8192 x 4104 x 4096 and 1000 x 4104 x 4096 against K - 8: 256x256 1.03-1.09 times, 128x128
+// 1.2-1.3, the others 1.3-1.55; MaskedLinear at the first of them on the tile of K = 2048 (128x64) 43.9 us, on 128x256 36.7 us).
 struct TileCost {
   int tile, per_cu;
-  double base, per_slab, first, again, tbs;
+  double base, per_slab, first, again, tbs, ragged;
 };
 constexpr TileCost kDualCosts[] = {
-    {TILE_256x256_W4, 1, 7.2, 1.313, 0.77, 0.71, 5.05}, {TILE_128x128_W4, 2, 0.0, 0.992, 0.70, 0.69, 5.8},
-    {TILE_SMALL_W4, 3, 0.0, 0.958, 0.59, 0.66, 5.6},    {TILE_128x128_R4, 1, 1.5, 0.504, 0.74, 0.88, 6.2},
-    {TILE_128x256_R3, 1, 2.0, 0.836, 0.77, 0.79, 5.75}, {TILE_64x128_R3, 2, 1.05, 0.716, 0.51, 0.57, 6.1}};
+    {TILE_256x256_W4, 1, 7.2, 1.313, 0.77, 0.71, 5.05, 1.08},
+    {TILE_128x128_W4, 2, 0.0, 0.992, 0.70, 0.69, 5.8, 1.28},
+    {TILE_SMALL_W4, 3, 0.0, 0.958, 0.59, 0.66, 5.6, 1.45},
+    {TILE_128x128_R4, 1, 1.5, 0.504, 0.74, 0.88, 6.2, 1.45},
+    {TILE_128x256_R3, 1, 2.0, 0.836, 0.77, 0.79, 5.75, 1.4},
+    {TILE_64x128_R3, 2, 1.05, 0.716, 0.51, 0.57, 6.1, 1.5}};
 constexpr TileCost kPlainCosts[] = {
-    {TILE_256x256_W8, 1, 3.2, 1.31, 0.77, 0.91, 6.0},  {TILE_256x256_W4, 1, 13.0, 1.33, 0.64, 0.60, 6.0},
-    {TILE_128x128_W4, 2, 0.6, 0.88, 0.60, 0.74, 6.5},  {TILE_SMALL_W4, 3, 0.0, 0.805, 0.42, 0.62, 6.2},
-    {TILE_128x128_R4, 1, 1.9, 0.46, 0.485, 0.88, 7.4}, {TILE_128x256_R3, 1, 3.7, 0.80, 0.70, 0.90, 6.9},
-    {TILE_64x128_R3, 2, 0.2, 0.56, 0.42, 0.60, 6.1}};
+    {TILE_256x256_W8, 1, 3.2, 1.31, 0.77, 0.91, 6.0, 1.06},
+    {TILE_256x256_W4, 1, 13.0, 1.33, 0.64, 0.60, 6.0, 1.08},
+    {TILE_128x128_W4, 2, 0.6, 0.88, 0.60, 0.74, 6.5, 1.28},
+    {TILE_SMALL_W4, 3, 0.0, 0.805, 0.42, 0.62, 6.2, 1.45},
+    {TILE_128x128_R4, 1, 1.9, 0.46, 0.485, 0.88, 7.4, 1.45},
+    {TILE_128x256_R3, 1, 3.7, 0.80, 0.70, 0.90, 6.9, 1.4},
+    {TILE_64x128_R3, 2, 0.2, 0.56, 0.42, 0.60, 6.1, 1.5}};
 
 inline double routed_tile_time(const TileCost& c, bool dual, int64_t tiles_m, int modalities, int64_t M, int64_t n_out, int64_t K,
                                int splits) {
   const TileGeom t = tile_geom(c.tile, dual);
-  const int64_t slabs = K / 64, slots = (int64_t)kCus * c.per_cu;
+  const int64_t slabs = cdiv64(K, 64), slots = (int64_t)kCus * c.per_cu;
   const int64_t tiles = tiles_m * cdiv64(n_out, t.block_n_out) * splits;
   const int64_t full = tiles / slots, rest = tiles - full * slots;
-  const double round = c.base + c.per_slab * (double)cdiv64(slabs, splits);
+  const double per_slab = K % 64 == 0 ? c.per_slab : c.per_slab * c.ragged;
+  const double round = c.base + per_slab * (double)cdiv64(slabs, splits);
   double time = (double)full * round;
   if (rest > 0) {
     const double fill = c.per_cu == 1 ? (double)rest / (double)slots : (double)(cdiv64(rest, kCus) - 1) / (double)(c.per_cu - 1);
@@ -106,7 +123,7 @@ inline double routed_tile_time(const TileCost& c, bool dual, int64_t tiles_m, in
     } else if (dual) {  // past half a round another round, else 128x128 tiles (whole_round_tiles)
       time += rest > slots / 2 ? round : 3.0 + 1.08 * (double)slabs * (0.5 + 0.5 * (double)rest * 4.0 / 512.0);
     } else {            // split tail
-      const double cut = 8.0 + c.base + c.per_slab * (double)slabs / (double)tail_split_factor((int)rest, (int)slabs);
+      const double cut = 8.0 + c.base + per_slab * (double)slabs / (double)tail_split_factor((int)rest, (int)slabs);
       time += cut < round ? cut : round;
     }
   }
@@ -119,7 +136,7 @@ inline double routed_tile_time(const TileCost& c, bool dual, int64_t tiles_m, in
 
 // Split factors the cost model considers: whole 64-element slabs, at least four to a range, no empty range.
 inline bool routed_split_ok(int64_t K, int s) {
-  const int64_t nk = K / 64;
+  const int64_t nk = cdiv64(K, 64);
   return s == 1 || (nk / s >= 4 && cdiv64(nk, cdiv64(nk, s)) == s);
 }
 
@@ -185,7 +202,7 @@ inline RoutedPlan model_routed_plan(bool dual, int64_t M, int64_t n_out, int64_t
 // Where the model applies: up to two rounds of 256x256 tiles; past them the rule below takes that tile.
 inline bool model_applies(bool dual, int64_t M, int64_t n_out, int64_t K) {
   const TileGeom t = tile_geom(TILE_256x256_W8, dual);
-  return M > 0 && n_out > 0 && K > 0 && K % 64 == 0 && cdiv64(M, t.block_m) * cdiv64(n_out, t.block_n_out) < 2 * kCus;
+  return M > 0 && n_out > 0 && direct_contraction(K) && cdiv64(M, t.block_m) * cdiv64(n_out, t.block_n_out) < 2 * kCus;
 }
 
 // Routed GEMM over M rows and n_out output columns (K: the contraction, 0 = not known to the caller).
@@ -206,7 +223,7 @@ inline int pick_routed_tile(int64_t M, int64_t n_out, bool dual, int64_t K = 0, 
   // 128x128 (a third fewer LDS reads per flop; measured 4 % faster at M = 32768, d = 4096, h = 14336); so do the
   // single-weight kernels over a long contraction (1-2.5 % faster at K = 4096 and 14336, N = 4096, M >= 16384),
   // which otherwise keep eight wavefronts of 128x64 (less exposed when K is short).
-  if (tiles(TILE_256x256_W8) >= 2 * kCus) return dual || K >= 4096 ? TILE_256x256_W4 : TILE_256x256_W8;
+  if (tiles(TILE_256x256_W8) >= 2 * kCus) return dual || (K >= 4096 && K % 64 == 0) ? TILE_256x256_W4 : TILE_256x256_W8;
   if (tiles(TILE_128x128_W4) >= kCus) return TILE_128x128_W4;
   return TILE_SMALL_W4;
 }
@@ -225,7 +242,7 @@ inline double routed_plan_cost(int64_t M, int64_t n_out, int64_t K, int tile, in
   const double t_slab = (tile == TILE_256x256_W8 || tile == TILE_256x256_W4) ? 1.2 : tile == TILE_128x128_R4 ? 0.4 : 0.8;
   const int64_t slabs = cdiv64(cdiv64(K, 64), splits);
   const double reduce = splits > 1 ? (double)splits * (double)M * (double)n_out * 8.0 / 4.0e6 : 0.0;
-  if (tile == TILE_256x256_W8 && splits == 1 && K % 64 == 0 && tiles > slots) {
+  if (tile == TILE_256x256_W8 && splits == 1 && direct_contraction(K) && tiles > slots) {
     // Unsplit 256x256 tiles past one round: the launcher runs the whole rounds, then the remaining tiles
     // cut into K ranges (split tail) - a fraction of a round, a second launch and a small reduce pass.
     const int64_t tail = tiles % slots;
@@ -238,8 +255,8 @@ inline double routed_plan_cost(int64_t M, int64_t n_out, int64_t K, int tile, in
 
 // Best split for a given tile: ranges of at least 8 slabs, no empty range.
 inline int pick_routed_splits(int64_t M, int64_t n_out, int64_t K, int tile) {
-  if (M > 4096 || K % 64 != 0 || tile == TILE_256x256_W4) return 1;
-  const int64_t nk = K / 64;
+  if (M > 4096 || !direct_contraction(K) || tile == TILE_256x256_W4) return 1;
+  const int64_t nk = cdiv64(K, 64);
   int best = 1;
   double best_cost = routed_plan_cost(M, n_out, K, tile, 1);
   for (int s = 2; s <= 16 && nk / s >= 8; ++s) {
@@ -258,13 +275,13 @@ inline RoutedPlan pick_routed_plan(int64_t M, int64_t n_out, int64_t K, bool use
   if (use_table && op != TUNED_NONE)
     if (const TunedPlan* t = tuned_plan(op, M, K, n_out)) {
       p.tile = t->tile;
-      p.splits = p.splits_more = (K % 64 == 0 && M < 65536 && n_out % 4 == 0) ? t->splits : 1;
+      p.splits = p.splits_more = (direct_contraction(K) && M < 65536 && n_out % 4 == 0) ? t->splits : 1;
       return p;
     }
   if (op != TUNED_NONE && model_applies(false, M, n_out, K)) return model_routed_plan(false, M, n_out, K, M < 65536 && n_out % 4 == 0);
   p.tile = pick_routed_tile(M, n_out, false, K, use_table, op);
   p.splits = p.splits_more = 1;
-  if (M > 4096 || K % 64 != 0) return p;
+  if (M > 4096 || !direct_contraction(K)) return p;
   double best_cost = 0.0;
   const int cand[3] = {TILE_256x256_W8, TILE_128x128_W4, TILE_SMALL_W4};
   for (int i = 0; i < 3; ++i) {
