@@ -268,23 +268,54 @@ int routed_tile(int64_t M, int64_t n_out, bool dual, int64_t K = 0, int op = TUN
   return f >= 0 ? f : pick_routed_tile(M, n_out, dual, K, use_tuned(), op);
 }
 
+// Whole extents off the dot kernels' 512-element slices at M <= 8: the dot-product streams lead once there is a stream to speak
+// of (MaskedFFN d=3200 h=8960 M=1 44.3 -> 33.6 us, M=8 both modalities 68.5 -> 61.6; d=5760 h=11520 M=4 131 -> 124; linear
+// K=3200 N=6016 19.3 -> 16.6); at d=1152 h=1408 a call is its launches and both take 33.5 us.
+constexpr int64_t kDotMinWeight = (int64_t)1 << 21;
 bool use_stream_path(int64_t M, int64_t d, int64_t h) { return stream_shape_ok(M, d, h); }
 
-// M <= 8: both projections run as contiguous-row dot-product streams.
-bool use_dot_path(int64_t M, int64_t d, int64_t h) {
-  return use_stream_path(M, d, h) && stream_dot_ok((int)M, (int)d) && stream_dot_ok((int)M, (int)h);
+// Kernels of the two projections of a streamed forward: fragment-layout streams (extents under 1024), contiguous-row
+// dot-product streams (M <= 8), LDS-transposed MFMA streams.
+enum { STREAM_FRAG, STREAM_DOT, STREAM_TILE };
+struct StreamKinds { int up, down; };
+
+StreamKinds stream_kinds_any(int64_t M, int64_t d, int64_t h) {
+  return {stream_dot_any_ok((int)M, (int)d) ? STREAM_DOT : STREAM_TILE, stream_dot_any_ok((int)M, (int)h) ? STREAM_DOT : STREAM_TILE};
+}
+int any_down_splits(int64_t M, int64_t d, int64_t h) {
+  return stream_kinds_any(M, d, h).down == STREAM_DOT ? 1 : stream_tile_down_splits((int)M, (int)d, (int)h);
+}
+// Above 32 rows the tiled GEMMs are level or ahead once the weights are large and one modality is present (us, GEMM / streams):
+// d=5832 h=11784 M=64 133 / 139, d=4160 h=12480 M=64 77 / 86; below, d=3008 h=9024 M=40 84 / 72, d=2104 h=7176 M=64 51 / 39.
+bool ragged_stream_pays(int64_t M, int64_t K, int64_t N) { return M <= 32 || K * N <= ((int64_t)1 << 25); }
+
+// Extents that are multiples of 8 but not of 128 run on the streams too, except in the forward that keeps its
+// pre-activations (ffnk_masked_ffn_can_save) and where the static entry point's scratch does not hold the partials: which
+// shapes that entry point takes does not depend on this route.  Against the tiled GEMMs, which wait for a slab of weights
+// per barrier and have few workgroups at these sizes (us, GEMM -> streams): d=2104 h=7176 M=1 42.5 -> 29.6, d=5832
+// h=11784 M=3 194 -> 129, M=8 107 -> 80, M=13 200 -> 164; d=3008 h=9024 M=40 84 -> 72; linear K=2056 N=1544 M=1 22.0 -> 16.0.
+bool use_ragged_stream(int64_t M, int64_t d, int64_t h) {
+  if (M < 1 || M > kStreamMaxM || d > kMaxCols || h > kMaxCols || use_stream_path(M, d, h) || forced_tile() >= 0 ||
+      !stream_tile_any_ok((int)M, (int)d, (int)h) || !ragged_stream_pays(M, d, h))
+    return false;
+  const int s = any_down_splits(M, d, h);
+  return route_ws_bytes(M) + ws_align((size_t)M * round_up64(h, 8) * 2) + (s > 1 ? ws_align((size_t)s * M * d * 4) : 0) <=
+         (size_t)FFNK_STATIC_SCRATCH_BYTES;
 }
 
-// 9 <= M <= 64 (or smaller M whose extents the dot kernels do not take): LDS-transposed MFMA streams.
-bool use_tile_path(int64_t M, int64_t d, int64_t h) {
-  return use_stream_path(M, d, h) && !use_dot_path(M, d, h) && stream_tile_ok((int)M, (int)d, (int)h);
+StreamKinds stream_kinds(int64_t M, int64_t d, int64_t h) {
+  if (!use_stream_path(M, d, h)) return stream_kinds_any(M, d, h);
+  if (stream_dot_ok((int)M, (int)d) && stream_dot_ok((int)M, (int)h)) return {STREAM_DOT, STREAM_DOT};
+  if (!stream_tile_ok((int)M, (int)d, (int)h)) return {STREAM_FRAG, STREAM_FRAG};
+  return d * h >= kDotMinWeight ? stream_kinds_any(M, d, h) : StreamKinds{STREAM_TILE, STREAM_TILE};
 }
 
 int down_splits(int64_t M, int64_t d, int64_t h) {
-  if (use_dot_path(M, d, h)) return 1;
-  if (use_tile_path(M, d, h)) {
+  const int kind = stream_kinds(M, d, h).down;
+  if (kind == STREAM_DOT) return 1;
+  if (kind == STREAM_TILE) {
     // a forced factor (tuner) where every K range keeps the kernel's minimum of eight 128-element chunks
-    const int fs = forced_splits(), chunks = (int)(h / 128);
+    const int fs = forced_splits(), chunks = (int)cdiv64(h, 128);
     if (fs >= 1 && chunks - (int)cdiv64(chunks, fs) * (fs - 1) >= 8) return fs;
     return stream_tile_down_splits((int)M, (int)d, (int)h);
   }
@@ -389,8 +420,10 @@ FfnBwdPaths ffn_bwd_paths(int64_t M, int64_t d, int64_t h, int64_t g_stride_m, i
 int linear_stream_kind(int64_t M, int64_t K, int64_t N) {
   if (M < 1 || M > kStreamMaxM || K > kMaxCols || N > kMaxCols) return 0;
   if (stream_dot_ok((int)M, (int)K)) return 1;
-  if (stream_tile_down_ok((int)M, (int)N, (int)K)) return 2;
-  return 0;
+  const bool whole = stream_tile_down_ok((int)M, (int)N, (int)K);
+  if (stream_dot_any_ok((int)M, (int)K) && (whole ? K * N >= kDotMinWeight : forced_tile() < 0)) return 1;
+  if (whole) return 2;
+  return forced_tile() < 0 && stream_tile_down_any_ok((int)M, (int)N, (int)K) && ragged_stream_pays(M, K, N) ? 2 : 0;
 }
 int linear_stream_splits(int64_t M, int64_t K, int64_t N) {
   return linear_stream_kind(M, K, N) == 2 ? stream_tile_down_splits((int)M, (int)N, (int)K) : 1;
@@ -509,15 +542,25 @@ size_t ffnk_workspace_bytes(int op, int64_t M, int64_t K, int64_t N) {
       // perm + counts + the fp32 split-K partials where the GEMM (or the streamed projection) is split
       if (linear_stream_kind(M, K, N)) {
         const int splits = linear_stream_splits(M, K, N);
-        return route_ws_bytes(M) + (splits > 1 ? ws_align((size_t)splits * M * N * 4) : 0);
+        const size_t part = splits > 1 ? ws_align((size_t)splits * M * N * 4) : 0;
+        // (a row stride past the streams' 32-bit offsets sends a ragged shape to the tiled GEMM)
+        const size_t tiled = stream_tile_down_ok((int)M, (int)N, (int)K) ? 0 : linear_partial_bytes(M, K, N);
+        return route_ws_bytes(M) + (part > tiled ? part : tiled);
       }
       return route_ws_bytes(M) + linear_partial_bytes(M, K, N);
     }
-    case FFNK_OP_FFN_FWD:
+    case FFNK_OP_FFN_FWD: {
       // perm + counts + the [M, h] bf16 intermediate in routed order (N = h) + the fp32 split-K
       // partials of the down projection where it is split.
-      return route_ws_bytes(M) + ws_align((size_t)M * round_up64(N, 8) * 2) +
-             (use_stream_path(M, K, N) ? ws_align((size_t)down_splits(M, K, N) * M * K * 4) : tiled_down_partial_bytes(M, K, N));
+      size_t part = use_stream_path(M, K, N) ? ws_align((size_t)down_splits(M, K, N) * M * K * 4) : tiled_down_partial_bytes(M, K, N);
+      if (use_ragged_stream(M, K, N)) {
+        // (a forced factor may be larger than the rule's)
+        const int s = down_splits(M, K, N);
+        const size_t streamed = s > 1 ? ws_align((size_t)s * M * K * 4) : 0;
+        if (streamed > part) part = streamed;
+      }
+      return route_ws_bytes(M) + ws_align((size_t)M * round_up64(N, 8) * 2) + part;
+    }
     case FFNK_OP_LINEAR_BWD: {
       const BwdPlan a = plan_bwd(M, K, N, true), b = plan_bwd(M, K, N, false);
       return a.total > b.total ? a.total : b.total;
@@ -574,7 +617,7 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
   const bool direct = direct_contraction(contraction);
   if (!direct && tile == TILE_256x256_W4) tile = TILE_256x256_W8;  // the four-wave tile runs on the direct path only
   const TileGeom gm = tile_geom(tile, dual);
-  const bool stream = (op == FFNK_OP_FFN_FWD || op == FFNK_OP_FFN_UP || op == FFNK_OP_FFN_DOWN) && use_stream_path(M, K, N);
+  const bool stream = (op == FFNK_OP_FFN_FWD || op == FFNK_OP_FFN_UP || op == FFNK_OP_FFN_DOWN) && (use_stream_path(M, K, N) || use_ragged_stream(M, K, N));
   out->path = stream ? FFNK_PATH_STREAM : FFNK_PATH_MFMA_TILED;
   out->block_m = gm.block_m;
   out->block_n = gm.block_n_out;
@@ -607,7 +650,7 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
       out->block_m = (int)M;
       out->block_n = stream_dot_rows_per_block((int)N, false, (int)K);
       out->block_k = 512 * stream_dot_slices_per_wave((int)K);
-      out->split_k = (int)(K / out->block_k);
+      out->split_k = stream_dot_waves((int)K);
       out->lds_stages = 0;
       out->direct_lds = 0;
     } else {
@@ -633,7 +676,9 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
     out->group_m = 1;
     out->split_k = stream_waves_per_block((int)M, up) * (up ? 1 : down_splits(M, K, N));
     out->direct_lds = 0;
-    if (use_tile_path(M, K, N)) {
+    const StreamKinds kinds = stream_kinds(M, K, N);
+    const int kind = up ? kinds.up : kinds.down;
+    if (kind == STREAM_TILE) {
       // LDS-transposed streams: block_n weight rows (of each matrix) x 128-element chunks, three in flight
       out->block_n = stream_tile_rows_per_block((int)M, up);
       out->block_k = 128;
@@ -641,14 +686,14 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
       out->direct_lds = stream_tile_direct((int)M, up);
       out->split_k = up ? 1 : down_splits(M, K, N);
     }
-    if (use_dot_path(M, K, N)) {
+    if (kind == STREAM_DOT) {
       // dot-product streams: a workgroup is block_n weight rows x all of K, one wavefront per
       // block_k-element slice of K
       const int64_t contr = up ? K : N;
       out->block_m = (int)M;
       out->block_n = stream_dot_rows_per_block((int)(up ? N : K), up, (int)contr);
       out->block_k = 512 * stream_dot_slices_per_wave((int)contr);
-      out->split_k = (int)(contr / out->block_k);
+      out->split_k = stream_dot_waves((int)contr);
     }
   }
   return FFNK_OK;
@@ -690,10 +735,12 @@ int ffnk_masked_linear_fwd_routed(const uint16_t* x, int64_t x_stride_m, const u
   if (ws_bytes < need || !ws) return fail(FFNK_E_WORKSPACE, "workspace %zu < %zu bytes", ws_bytes, need);
   if (!aligned16(ws)) return fail(FFNK_E_ALIGN, "workspace not 16-byte aligned");
   const RouteWs r = carve_route(static_cast<uint8_t*>(ws), M);
-  if (const int kind = linear_stream_kind(M, K, N)) {
+  const bool far_rows = M * x_stride_m >= ((int64_t)1 << 30);  // past the LDS-transposed streams' 32-bit offsets
+  const int kind = linear_stream_kind(M, K, N);
+  if (kind && !(kind == 2 && far_rows && !stream_tile_down_ok((int)M, (int)N, (int)K))) {
     // Decode sizes: the weight-streaming kernels of the FFN's down projection, fed token rows in
     // token order; they route from the mask themselves.
-    if (kind == 2 && M * x_stride_m >= ((int64_t)1 << 30))
+    if (kind == 2 && far_rows)
       return fail(FFNK_E_STRIDE, "x_stride_m=%lld: the decode kernels address the token rows with 32-bit offsets",
                   (long long)x_stride_m);
     const int splits = linear_stream_splits(M, K, N);
@@ -813,7 +860,9 @@ int ffn_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, cons
     return FFNK_OK;
   }
 
-  if (use_stream_path(M, d, h)) {
+  const bool far_rows = M * x_stride_m >= ((int64_t)1 << 30);  // past the LDS-transposed streams' 32-bit offsets
+  if (use_stream_path(M, d, h) ||
+      (pre == nullptr && use_ragged_stream(M, d, h) && !(far_rows && stream_kinds(M, d, h).up == STREAM_TILE))) {
     float* P = reinterpret_cast<float*>(wsb + r.bytes + ws_align((size_t)M * ldh * 2));
     const int splits = down_splits(M, d, h);
     FFNK_HIP(mark(0), "event record");
@@ -821,12 +870,12 @@ int ffn_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, cons
     u.X = x; u.ldx = x_stride_m; u.gather_x = 1; u.mask = mask; u.M = (int)M;
     u.W0[0] = W1; u.W0[1] = U1; u.W1[0] = W3; u.W1[1] = U3; u.ldw = up_stride_n;
     u.Nrows = (int)h; u.K = (int)d; u.splits = 1; u.H = H; u.ldh = ldh; u.P = nullptr; u.out = nullptr; u.ldo = 0;
-    const bool dot = use_dot_path(M, d, h);
-    const bool tiled = use_tile_path(M, d, h);
-    if (tiled && M * x_stride_m >= ((int64_t)1 << 30))
+    const StreamKinds kinds = stream_kinds(M, d, h);
+    if (kinds.up == STREAM_TILE && far_rows)
       return fail(FFNK_E_STRIDE, "x_stride_m=%lld: the decode kernels address the token rows with 32-bit offsets",
                   (long long)x_stride_m);
-    FFNK_HIP(dot ? launch_stream_dot_up(u, stream) : tiled ? launch_stream_tile_up(u, stream) : launch_stream_up(u, stream),
+    FFNK_HIP(kinds.up == STREAM_DOT ? launch_stream_dot_up(u, stream)
+             : kinds.up == STREAM_TILE ? launch_stream_tile_up(u, stream) : launch_stream_up(u, stream),
              "streaming up-projection");
     FFNK_HIP(mark(1), "event record");
     StreamArgs dn;
@@ -834,7 +883,8 @@ int ffn_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, cons
     dn.W0[0] = W2; dn.W0[1] = U2; dn.W1[0] = dn.W1[1] = nullptr; dn.ldw = down_stride_n;
     dn.Nrows = (int)d; dn.K = (int)h; dn.splits = splits; dn.H = nullptr; dn.ldh = 0;
     dn.P = splits > 1 ? P : nullptr; dn.out = out; dn.ldo = out_stride_m;
-    FFNK_HIP(dot ? launch_stream_dot_down(dn, stream) : tiled ? launch_stream_tile_down(dn, stream) : launch_stream_down(dn, stream),
+    FFNK_HIP(kinds.down == STREAM_DOT ? launch_stream_dot_down(dn, stream)
+             : kinds.down == STREAM_TILE ? launch_stream_tile_down(dn, stream) : launch_stream_down(dn, stream),
              "streaming down-projection");
     if (splits > 1)
       FFNK_HIP(launch_stream_reduce(P, splits, (int)M, (int)d, mask, out, out_stride_m, stream), "streaming reduce");

@@ -102,7 +102,7 @@ struct StreamArgs {
   const uint16_t* W0[2];           // per group: weight rows [Nrows, K], K contiguous
   const uint16_t* W1[2];           // up-projection only: the second ("up") weight
   int64_t ldw;
-  int Nrows, K, splits;            // K % 256 == 0; splits > 1 only for the down projection
+  int Nrows, K, splits;            // K % 8 == 0; splits > 1 only for the down projection
   uint16_t* H; int64_t ldh;        // up-projection output, routed order [M, Nrows]
   float* P;                        // down-projection partials [splits][M][Nrows] (routed order), or NULL:
   uint16_t* out; int64_t ldo;      // ... splits == 1 and the result goes straight to out (token order)
@@ -115,6 +115,8 @@ hipError_t launch_stream_up(const StreamArgs& a, hipStream_t stream);
 hipError_t launch_stream_down(const StreamArgs& a, hipStream_t stream);
 // stream_dot.hip: M <= 8, contiguous-row dot-product kernels (splits == 1, P unused, no reduce pass).
 bool stream_dot_ok(int M, int K);
+bool stream_dot_any_ok(int M, int K);  // K any multiple of 8
+int stream_dot_waves(int K);           // wavefronts per workgroup = K slices
 int stream_dot_slices_per_wave(int K);
 int stream_dot_rows_per_block(int Nrows, bool dual, int K);
 hipError_t launch_stream_dot_up(const StreamArgs& a, hipStream_t stream);
@@ -122,6 +124,8 @@ hipError_t launch_stream_dot_down(const StreamArgs& a, hipStream_t stream);
 // stream_tile.hip: 9 <= M <= 64, contiguous loads + LDS transpose + shared token-row slab.
 bool stream_tile_ok(int M, int d, int h);
 bool stream_tile_down_ok(int M, int Nrows, int K);  // single-weight projection alone (MaskedLinear forward)
+bool stream_tile_any_ok(int M, int d, int h);           // extents any multiples of 8
+bool stream_tile_down_any_ok(int M, int Nrows, int K);
 int stream_tile_rows_per_block(int M, bool dual);
 int stream_tile_depth(int M, bool dual);
 int stream_tile_direct(int M, bool dual);  // 1: the token-row slab is filled by direct global->LDS loads

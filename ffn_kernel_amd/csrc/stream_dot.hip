@@ -73,7 +73,7 @@ struct DotTile {
 };
 
 // One wavefront: K slice `wave` of every weight row of the workgroup, T token rows.
-template <int T, bool DUAL, int C, int DEPTH>
+template <int T, bool DUAL, int C, int DEPTH, bool RAGGED>
 __device__ __forceinline__ void dot_rows(const StreamArgs& a, const DotTile& t, const int* s_perm, float* s_red) {
   static_assert(DEPTH % 4 == 0, "row slices are reduced four at a time");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -87,12 +87,16 @@ __device__ __forceinline__ void dot_rows(const StreamArgs& a, const DotTile& t, 
     const int p = t.p0 + min(i, t.mg - 1);  // surplus token slots repeat the last row; never stored
     const int64_t src = a.gather_x ? (int64_t)s_perm[p] : (int64_t)p;
 #pragma unroll
-    for (int c = 0; c < C; ++c)
-      xr[i][c] = *reinterpret_cast<const u32x4_t*>(a.X + src * a.ldx + k0 + c * kDotSlice);
+    for (int c = 0; c < C; ++c) {
+      if (RAGGED && k0 + c * kDotSlice >= a.K) xr[i][c] = u32x4_t{0u, 0u, 0u, 0u};
+      else xr[i][c] = *reinterpret_cast<const u32x4_t*>(a.X + src * a.ldx + k0 + c * kDotSlice);
+    }
   }
 
-  const uint16_t* w0 = a.W0[t.grp] + k0;
-  const uint16_t* w1 = DUAL ? a.W1[t.grp] + k0 : nullptr;
+  // RAGGED: the rows end inside the last wavefront's slice.  Its loads go through a buffer descriptor of one row each
+  // (2 K bytes from the row's start), whose range check returns zeros past the row: no branch and no select per load.
+  const uint16_t* w0 = a.W0[t.grp] + (RAGGED ? 0 : k0);
+  const uint16_t* w1 = DUAL ? a.W1[t.grp] + (RAGGED ? 0 : k0) : nullptr;
   auto rv_ptr = [&](int i) -> const uint16_t* {
     const int row = min(t.n_begin + (DUAL ? (i >> 1) : i), a.Nrows - 1);  // rows past the end: loaded, never stored
     return ((DUAL && (i & 1)) ? w1 : w0) + (int64_t)row * a.ldw;
@@ -100,6 +104,15 @@ __device__ __forceinline__ void dot_rows(const StreamArgs& a, const DotTile& t, 
   u32x4_t ring[DEPTH][C];
   auto fetch = [&](int s, int i) {
     const uint16_t* p = rv_ptr(i);
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (RAGGED) {
+      const __amdgpu_buffer_rsrc_t row = __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, a.K * 2, 0x00020000);
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+        ring[s][c] = __builtin_amdgcn_raw_buffer_load_b128(row, (int)(k0 + c * kDotSlice) * 2, 0, 2 /* non-temporal */);
+      return;
+    }
+#endif
 #pragma unroll
     for (int c = 0; c < C; ++c)
       ring[s][c] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p + c * kDotSlice));
@@ -186,7 +199,7 @@ __device__ __forceinline__ int route8(const uint8_t* mask, int M, int* s_perm, i
 
 // grid.x = 2 * row_blocks (visual workgroups first), blockDim.x = 64 * (K / (512 * C)); rpb weight
 // rows per workgroup.  Dynamic LDS: [waves][rpb * MATS][T_MAX] floats.
-template <int T_MAX, bool DUAL, int C, int DEPTH, int NWV_MAX>
+template <int T_MAX, bool DUAL, int C, int DEPTH, int NWV_MAX, bool RAGGED>
 __global__ __launch_bounds__(NWV_MAX * kWave) void stream_dot_kernel(const StreamArgs a, const int rpb) {
   extern __shared__ __attribute__((aligned(16))) float s_red[];
   __shared__ int s_perm[kDotMaxM];
@@ -202,19 +215,19 @@ __global__ __launch_bounds__(NWV_MAX * kWave) void stream_dot_kernel(const Strea
   t.n_rows = rpb;
   const int nwv = blockDim.x >> 6;
   if (T_MAX >= 8 && t.mg > 4) {
-    dot_rows<(T_MAX >= 8 ? 8 : 1), DUAL, C, DEPTH>(a, t, s_perm, s_red);
+    dot_rows<(T_MAX >= 8 ? 8 : 1), DUAL, C, DEPTH, RAGGED>(a, t, s_perm, s_red);
     __syncthreads();
     dot_finish<(T_MAX >= 8 ? 8 : 1), DUAL>(a, t, s_perm, s_red, nwv);
   } else if (T_MAX >= 4 && t.mg > 2) {
-    dot_rows<(T_MAX >= 4 ? 4 : 1), DUAL, C, DEPTH>(a, t, s_perm, s_red);
+    dot_rows<(T_MAX >= 4 ? 4 : 1), DUAL, C, DEPTH, RAGGED>(a, t, s_perm, s_red);
     __syncthreads();
     dot_finish<(T_MAX >= 4 ? 4 : 1), DUAL>(a, t, s_perm, s_red, nwv);
   } else if (T_MAX >= 2 && t.mg > 1) {
-    dot_rows<(T_MAX >= 2 ? 2 : 1), DUAL, C, DEPTH>(a, t, s_perm, s_red);
+    dot_rows<(T_MAX >= 2 ? 2 : 1), DUAL, C, DEPTH, RAGGED>(a, t, s_perm, s_red);
     __syncthreads();
     dot_finish<(T_MAX >= 2 ? 2 : 1), DUAL>(a, t, s_perm, s_red, nwv);
   } else {
-    dot_rows<1, DUAL, C, DEPTH>(a, t, s_perm, s_red);
+    dot_rows<1, DUAL, C, DEPTH, RAGGED>(a, t, s_perm, s_red);
     __syncthreads();
     dot_finish<1, DUAL>(a, t, s_perm, s_red, nwv);
   }
@@ -227,49 +240,63 @@ bool stream_dot_ok(int M, int K) {
   return slices <= 16 || (slices % 2 == 0 && slices <= 32);
 }
 
+// The RAGGED kernels hold the bandwidth of the others (d=5832 h=11784, M=3, both modalities: 6.4 TB/s) and lead the
+// LDS-transposed streams by 10-40 % over extents both take (d=5832 h=11784, one modality: M=3 126 -> 89 us, M=8 105 -> 80 us).
+// Any multiple of 8 that needs at most 16 wavefronts of two slices (the RAGGED kernels, unless stream_dot_ok).
+bool stream_dot_any_ok(int M, int K) {
+  return M >= 1 && M <= kDotMaxM && K % 8 == 0 && K >= kDotSlice && cdiv(K, kDotSlice) <= 32;
+}
+
 // 512-element slices per wavefront: two when that still leaves at least four wavefronts.
 int stream_dot_slices_per_wave(int K) {
-  const int slices = K / kDotSlice;
+  const int slices = cdiv(K, kDotSlice);
+  if (K % kDotSlice != 0 || slices > 16) return slices >= 8 ? 2 : 1;
   return (slices % 2 == 0 && slices >= 8) ? 2 : 1;
 }
+int stream_dot_waves(int K) { return cdiv(K, kDotSlice * stream_dot_slices_per_wave(K)); }
 
 // Weight rows per workgroup: about `per_cu` workgroups per CU and modality, in whole reduce batches.
 int stream_dot_rows_per_block(int Nrows, bool dual, int K) {
   const int c = stream_dot_slices_per_wave(K);
-  const int waves = K / (kDotSlice * c);
+  const int waves = cdiv(K, kDotSlice * c);
   const int per_cu = waves <= 4 ? 2 : 1;
   const int unit = dual ? 4 : 8;
   int rpb = cdiv(cdiv(Nrows, 256 * per_cu), unit) * unit;
   // LDS: waves * rpb * mats * 8 floats <= 48 KB
   const int cap = (48 * 1024 / (waves * (dual ? 2 : 1) * 8 * 4)) / unit * unit;
-  if (rpb > cap) rpb = cap;
+  // Past that, the rows of a CU in as many equal workgroups as it takes: workgroups of `cap` rows each would leave a last,
+  // nearly empty round (K = 8192, 28672 gate + up rows: 299 workgroups on 256 CUs).
+  if (rpb > cap) rpb = cdiv(cdiv(Nrows, 256 * per_cu * cdiv(rpb, cap)), unit) * unit;
   return rpb < unit ? unit : rpb;
 }
 
-template <int T_MAX, bool DUAL, int C>
+template <int T_MAX, bool DUAL, int C, bool RAGGED>
 static void launch_dot_c(const StreamArgs& a, hipStream_t stream) {
-  const int waves = a.K / (kDotSlice * C);
+  const int waves = stream_dot_waves(a.K);
   const int rpb = stream_dot_rows_per_block(a.Nrows, DUAL, a.K);
   const int row_blocks = cdiv(a.Nrows, rpb);
   const size_t lds = (size_t)waves * rpb * (DUAL ? 2 : 1) * T_MAX * sizeof(float);
   if (waves <= 4)
-    hipLaunchKernelGGL((stream_dot_kernel<T_MAX, DUAL, C, 8, 4>), dim3(2 * row_blocks), dim3(waves * kWave), lds, stream, a, rpb);
+    hipLaunchKernelGGL((stream_dot_kernel<T_MAX, DUAL, C, 8, 4, RAGGED>), dim3(2 * row_blocks), dim3(waves * kWave), lds, stream, a, rpb);
   else if (waves <= 8)
-    hipLaunchKernelGGL((stream_dot_kernel<T_MAX, DUAL, C, 8, 8>), dim3(2 * row_blocks), dim3(waves * kWave), lds, stream, a, rpb);
+    hipLaunchKernelGGL((stream_dot_kernel<T_MAX, DUAL, C, 8, 8, RAGGED>), dim3(2 * row_blocks), dim3(waves * kWave), lds, stream, a, rpb);
   else
-    hipLaunchKernelGGL((stream_dot_kernel<T_MAX, DUAL, C, 4, 16>), dim3(2 * row_blocks), dim3(waves * kWave), lds, stream, a, rpb);
+    hipLaunchKernelGGL((stream_dot_kernel<T_MAX, DUAL, C, 4, 16, RAGGED>), dim3(2 * row_blocks), dim3(waves * kWave), lds, stream, a, rpb);
 }
 
 template <bool DUAL>
 static hipError_t launch_dot(const StreamArgs& a, hipStream_t stream) {
-  if (!stream_dot_ok(a.M, a.K) || a.splits != 1 || a.ldw % 8 != 0 || a.ldx % 8 != 0) return hipErrorInvalidValue;
+  if (!stream_dot_any_ok(a.M, a.K) || a.splits != 1 || a.ldw % 8 != 0 || a.ldx % 8 != 0) return hipErrorInvalidValue;
   if (DUAL ? (a.H == nullptr) : (a.out == nullptr)) return hipErrorInvalidValue;
   const int c = stream_dot_slices_per_wave(a.K);
+  const bool ragged = a.K % (c * kDotSlice) != 0;
   const int tmax = a.M > 4 ? 8 : a.M > 2 ? 4 : a.M > 1 ? 2 : 1;
 #define FFNK_DOT_CASE(TM)                                        \
   case TM:                                                       \
-    if (c == 2) launch_dot_c<TM, DUAL, 2>(a, stream);            \
-    else launch_dot_c<TM, DUAL, 1>(a, stream);                   \
+    if (ragged && c == 2) launch_dot_c<TM, DUAL, 2, true>(a, stream);  \
+    else if (ragged) launch_dot_c<TM, DUAL, 1, true>(a, stream); \
+    else if (c == 2) launch_dot_c<TM, DUAL, 2, false>(a, stream); \
+    else launch_dot_c<TM, DUAL, 1, false>(a, stream);            \
     break;
   switch (tmax) {
     FFNK_DOT_CASE(1)

@@ -48,14 +48,24 @@ constexpr TileShapeEntry kTileShapesDown[4] = {{2, 4, 0}, {2, 3, 0}, {2, 3, 1}, 
 constexpr const TileShapeEntry& tile_shape(int ntm_max, bool dual) { return dual ? kTileShapesUp[ntm_max - 1] : kTileShapesDown[ntm_max - 1]; }
 constexpr int kTMaxM = 64;
 
+// FORM_WHOLE: K whole chunks, Nrows whole row blocks.  The other two (RAGGED) take any multiples of 8: the last chunk
+// overlaps the one before it; the last row block starts at Nrows - ROWS, streams rows of the block before it a second
+// time and stores its own only.  FORM_SPLIT_LINES: rows are no whole number of 128-byte lines, so neighbouring chunks of a
+// row share a line, and a non-temporal load gives that line up before its second half is wanted: plain loads take
+// 164 us instead of 179 (MaskedFFN d=5832 h=11784 M=13) and 32 instead of 34 (linear K=5000 N=6184 M=16).  Over whole
+// lines the non-temporal ones are the faster (d=4160 h=12480 M=48: 131 us against 140).
+enum { FORM_WHOLE, FORM_RAGGED, FORM_SPLIT_LINES };
+
 struct TileJob {
   int grp, split, p0, mg, n0, c0, nc;  // n0: first weight row of the workgroup; c0 / nc: chunk range
+  int n_store;                         // first weight row whose outputs the workgroup stores (n0 where Nrows is whole row blocks)
 };
 
 // xs: [2][NTM * 16 token rows][16 pieces] 16-byte slots; wst: this wavefront's [2 tiles][16 rows][16 pieces].
-template <int NTM, bool DUAL, int kTWaves, int kTD, bool XDMA>
+template <int NTM, bool DUAL, int kTWaves, int kTD, bool XDMA, int FORM>
 __device__ __forceinline__ void tile_rows(const StreamArgs& a, const TileJob& t, const int* s_perm, u32x4_t* xs,
                                           u32x4_t* wst) {
+  constexpr bool RAGGED = FORM != FORM_WHOLE;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 15, lq = lane >> 4;
   const int64_t kbase = (int64_t)t.c0 * kTK;
@@ -112,7 +122,18 @@ __device__ __forceinline__ void tile_rows(const StreamArgs& a, const TileJob& t,
   // pull from the same few HBM channels.
   const int nc = t.nc;
   const int rot = (int)((blockIdx.x * 11u) % (unsigned)nc);
-  auto phys = [&](int c) { const int pc = c + rot; return (pc >= nc ? pc - nc : pc) * kTK; };
+  // RAGGED: a last chunk that would pass the end of the rows starts earlier, overlapping the chunk before it; what the two
+  // share (overlap(c) pieces of 8 elements) is cleared in both operands' fragments, so that no product is counted twice
+  // and a non-finite value meets no zero it would not meet elsewhere.
+  const int k_last = RAGGED ? (int)(a.K - kbase) - kTK : 0;  // start of the last whole chunk
+  auto phys = [&](int c) {
+    const int pc = c + rot, ko = (pc >= nc ? pc - nc : pc) * kTK;
+    return RAGGED ? min(ko, k_last) : ko;
+  };
+  auto overlap = [&](int c) {
+    const int pc = c + rot, ko = (pc >= nc ? pc - nc : pc) * kTK;
+    return max(0, ko - k_last) / 8;
+  };
   u32x4_t wr[kTD][2][4];
   auto loadw = [&](int s, int c) {
     const int64_t ko = phys(c);
@@ -120,7 +141,8 @@ __device__ __forceinline__ void tile_rows(const StreamArgs& a, const TileJob& t,
     for (int w = 0; w < 2; ++w)
 #pragma unroll
       for (int u = 0; u < 4; ++u)
-        wr[s][w][u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(wp[w] + u * w_step + ko));
+        wr[s][w][u] = FORM == FORM_SPLIT_LINES ? *reinterpret_cast<const u32x4_t*>(wp[w] + u * w_step + ko)
+                                                : __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(wp[w] + u * w_step + ko));
   };
   u32x4_t xr[XDMA ? 1 : kTD][XP];
   auto loadx = [&](int s, int c) {
@@ -217,11 +239,11 @@ __device__ __forceinline__ void tile_rows(const StreamArgs& a, const TileJob& t,
       }
     }
     const u32x4_t* xb = xs + (c & 1) * (NTM * 256);
+    const int shared_pieces = RAGGED ? overlap(c) : 0;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const int piece = (s * 4 + lq) ^ lrow;
-      const bf16x8_t wf0 = __builtin_bit_cast(bf16x8_t, wst[lrow * 16 + piece]);
-      const bf16x8_t wf1 = __builtin_bit_cast(bf16x8_t, wst[256 + lrow * 16 + piece]);
+      u32x4_t wv0 = wst[lrow * 16 + piece], wv1 = wst[256 + lrow * 16 + piece];
       u32x4_t xv[NTM];
       if (XDMA) {
 #pragma unroll
@@ -237,6 +259,17 @@ __device__ __forceinline__ void tile_rows(const StreamArgs& a, const TileJob& t,
 #pragma unroll
         for (int m = 0; m < NTM; ++m) xv[m] = xb[(m * 16 + lrow) * 16 + piece];
       }
+      if (RAGGED && s * 4 < shared_pieces) {  // uniform over the workgroup
+        const bool keep = s * 4 + lq >= shared_pieces;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          wv0[e] = keep ? wv0[e] : 0u;
+          wv1[e] = keep ? wv1[e] : 0u;
+#pragma unroll
+          for (int m = 0; m < NTM; ++m) xv[m][e] = keep ? xv[m][e] : 0u;
+        }
+      }
+      const bf16x8_t wf0 = __builtin_bit_cast(bf16x8_t, wv0), wf1 = __builtin_bit_cast(bf16x8_t, wv1);
 #pragma unroll
       for (int m = 0; m < NTM; ++m) {
         const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, xv[m]);
@@ -290,6 +323,7 @@ __device__ __forceinline__ void tile_rows(const StreamArgs& a, const TileJob& t,
     const int row = m * 16 + lrow;
     if (row >= t.mg) continue;
     if (DUAL) {
+      if (RAGGED && rbase[0] + 4 * lq < t.n_store) continue;
       const f32x4_t g = acc[0][m], u = acc[1][m];
       uint2 v2;
       v2.x = pack2bf(swiglu(g[0], u[0]), swiglu(g[1], u[1]));
@@ -300,6 +334,7 @@ __device__ __forceinline__ void tile_rows(const StreamArgs& a, const TileJob& t,
       for (int w = 0; w < 2; ++w) {
         const f32x4_t o = acc[w][m];
         const int n_out = rbase[w] + 4 * lq;
+        if (RAGGED && n_out < t.n_store) continue;
         if (a.P != nullptr) {
           *reinterpret_cast<float4*>(a.P + ((int64_t)t.split * a.M + (t.p0 + row)) * a.Nrows + n_out) =
               make_float4(o[0], o[1], o[2], o[3]);
@@ -336,8 +371,9 @@ __device__ __forceinline__ int route64(const uint8_t* mask, int M, int* s_perm, 
 }
 
 // grid.x = 2 groups x splits x row blocks (visual workgroups first); 256 threads.
-template <int NTM_MAX, bool DUAL, int kTWaves, int kTD, bool XDMA>
+template <int NTM_MAX, bool DUAL, int kTWaves, int kTD, bool XDMA, int FORM>
 __global__ __launch_bounds__(kTWaves * kWave, 2) void stream_tile_kernel(const StreamArgs a) {
+  constexpr bool RAGGED = FORM != FORM_WHOLE;
   __shared__ u32x4_t xs[(XDMA ? kTD : 2) * NTM_MAX * 256];
   __shared__ u32x4_t wst_all[kTWaves * 512];
   // The routing table shares the staging tiles' memory (it is read before the first chunk is staged): with four
@@ -346,7 +382,7 @@ __global__ __launch_bounds__(kTWaves * kWave, 2) void stream_tile_kernel(const S
   int* s_nvis_p = s_perm + kTMaxM;
   const int n_vis = route64(a.mask, a.M, s_perm, s_nvis_p);
   constexpr int ROWS = DUAL ? 16 * kTWaves : 32 * kTWaves;
-  const int row_blocks = a.Nrows / ROWS;
+  const int row_blocks = RAGGED ? cdiv(a.Nrows, ROWS) : a.Nrows / ROWS;
   const int per_grp = row_blocks * a.splits;
   TileJob t;
   t.grp = blockIdx.x / per_grp;
@@ -355,17 +391,18 @@ __global__ __launch_bounds__(kTWaves * kWave, 2) void stream_tile_kernel(const S
   t.p0 = t.grp == 0 ? 0 : n_vis;
   t.mg = t.grp == 0 ? n_vis : a.M - n_vis;
   if (t.mg == 0) return;  // modality absent: its weights are never read (uniform over the workgroup)
-  t.n0 = (rem % row_blocks) * ROWS;
-  const int n_chunks = a.K / kTK;
+  t.n_store = (rem % row_blocks) * ROWS;
+  t.n0 = RAGGED ? min(t.n_store, a.Nrows - ROWS) : t.n_store;
+  const int n_chunks = RAGGED ? cdiv(a.K, kTK) : a.K / kTK;
   const int cps = cdiv(n_chunks, a.splits);
   t.c0 = min(t.split * cps, n_chunks);
   t.nc = min(t.c0 + cps, n_chunks) - t.c0;
   u32x4_t* wst = wst_all + (threadIdx.x >> 6) * 512;
   const int ntm = cdiv(t.mg, 16);
-  if (NTM_MAX >= 4 && ntm >= 4) tile_rows<(NTM_MAX >= 4 ? 4 : 1), DUAL, kTWaves, kTD, XDMA>(a, t, s_perm, xs, wst);
-  else if (NTM_MAX >= 3 && ntm == 3) tile_rows<(NTM_MAX >= 3 ? 3 : 1), DUAL, kTWaves, kTD, XDMA>(a, t, s_perm, xs, wst);
-  else if (NTM_MAX >= 2 && ntm == 2) tile_rows<(NTM_MAX >= 2 ? 2 : 1), DUAL, kTWaves, kTD, XDMA>(a, t, s_perm, xs, wst);
-  else tile_rows<1, DUAL, kTWaves, kTD, XDMA>(a, t, s_perm, xs, wst);
+  if (NTM_MAX >= 4 && ntm >= 4) tile_rows<(NTM_MAX >= 4 ? 4 : 1), DUAL, kTWaves, kTD, XDMA, FORM>(a, t, s_perm, xs, wst);
+  else if (NTM_MAX >= 3 && ntm == 3) tile_rows<(NTM_MAX >= 3 ? 3 : 1), DUAL, kTWaves, kTD, XDMA, FORM>(a, t, s_perm, xs, wst);
+  else if (NTM_MAX >= 2 && ntm == 2) tile_rows<(NTM_MAX >= 2 ? 2 : 1), DUAL, kTWaves, kTD, XDMA, FORM>(a, t, s_perm, xs, wst);
+  else tile_rows<1, DUAL, kTWaves, kTD, XDMA, FORM>(a, t, s_perm, xs, wst);
 }
 
 static const TileShapeEntry& shape_for(int M, bool dual) { return tile_shape(cdiv(M < 1 ? 1 : M > kTMaxM ? kTMaxM : M, 16), dual); }
@@ -387,11 +424,21 @@ bool stream_tile_down_ok(int M, int Nrows, int K) {
          Nrows % stream_tile_rows_per_block(M, false) == 0;
 }
 
+// The same for any multiples of 8 (the RAGGED kernels): at least kTMinChunks chunks, the last one cut short, and at least
+// one row block.
+bool stream_tile_any_ok(int M, int d, int h) {
+  return M >= 1 && M <= kTMaxM && d % 8 == 0 && h % 8 == 0 && cdiv(d, kTK) >= kTMinChunks && cdiv(h, kTK) >= kTMinChunks;
+}
+bool stream_tile_down_any_ok(int M, int Nrows, int K) {
+  return M >= 1 && M <= kTMaxM && K % 8 == 0 && cdiv(K, kTK) >= kTMinChunks && Nrows % 8 == 0 &&
+         Nrows >= stream_tile_rows_per_block(M, false);
+}
+
 // K split of the down projection: about one workgroup per CU and modality, at least eight chunks
 // per workgroup, every split non-empty.
 int stream_tile_down_splits(int M, int d, int h) {
-  const int row_blocks = d / stream_tile_rows_per_block(M, false);
-  const int n_chunks = h / kTK;
+  const int row_blocks = cdiv(d, stream_tile_rows_per_block(M, false));
+  const int n_chunks = cdiv(h, kTK);
   int s = cdiv(256, row_blocks);
   if (s > n_chunks / kTMinChunks) s = n_chunks / kTMinChunks;
   if (s < 1) s = 1;
@@ -404,16 +451,22 @@ template <int NTM_MAX, bool DUAL>
 static void launch_tile_n(const StreamArgs& a, hipStream_t stream) {
   constexpr int W = tile_shape(NTM_MAX, DUAL).waves, D = tile_shape(NTM_MAX, DUAL).depth;
   constexpr bool X = tile_shape(NTM_MAX, DUAL).dma != 0;
-  const int blocks = 2 * (a.Nrows / ((DUAL ? 16 : 32) * W)) * a.splits;
-  hipLaunchKernelGGL((stream_tile_kernel<NTM_MAX, DUAL, W, D, X>), dim3(blocks), dim3(W * kWave), 0, stream, a);
+  constexpr int ROWS = (DUAL ? 16 : 32) * W;
+  const int blocks = 2 * cdiv(a.Nrows, ROWS) * a.splits;
+  if (a.K % kTK == 0 && a.Nrows % ROWS == 0)
+    hipLaunchKernelGGL((stream_tile_kernel<NTM_MAX, DUAL, W, D, X, FORM_WHOLE>), dim3(blocks), dim3(W * kWave), 0, stream, a);
+  else if (a.ldw % 64 == 0)
+    hipLaunchKernelGGL((stream_tile_kernel<NTM_MAX, DUAL, W, D, X, FORM_RAGGED>), dim3(blocks), dim3(W * kWave), 0, stream, a);
+  else
+    hipLaunchKernelGGL((stream_tile_kernel<NTM_MAX, DUAL, W, D, X, FORM_SPLIT_LINES>), dim3(blocks), dim3(W * kWave), 0, stream, a);
 }
 
 template <bool DUAL>
 static hipError_t launch_tile(const StreamArgs& a, hipStream_t stream) {
-  if (a.M < 1 || a.M > kTMaxM || a.K % kTK != 0 || a.splits < 1 || a.Nrows % stream_tile_rows_per_block(a.M, DUAL) != 0 ||
-      a.ldw % 8 != 0 || a.ldx % 8 != 0)
+  if (a.M < 1 || a.M > kTMaxM || a.K % 8 != 0 || a.splits < 1 || a.Nrows % 8 != 0 ||
+      a.Nrows < stream_tile_rows_per_block(a.M, DUAL) || a.ldw % 8 != 0 || a.ldx % 8 != 0)
     return hipErrorInvalidValue;
-  const int n_chunks = a.K / kTK;
+  const int n_chunks = cdiv(a.K, kTK);
   if (n_chunks - cdiv(n_chunks, a.splits) * (a.splits - 1) < kTMinChunks) return hipErrorInvalidValue;  // a short split
   if ((int64_t)a.M * a.ldx >= (1ll << 30)) return hipErrorInvalidValue;  // 32-bit byte offsets into the token rows
   if (DUAL && (a.splits != 1 || a.H == nullptr)) return hipErrorInvalidValue;
