@@ -42,6 +42,30 @@ __device__ __forceinline__ float swiglu(float g, float u) {
   return g * s * u;
 }
 
+// p[0] + p[stride] + ... + p[(n - 1) * stride], in that order.  The loads of up to four terms are in flight together: one
+// after the other, a reduce pass over few workgroups is n memory round trips long (MaskedFFN d=4096 h=14336, with the mask's
+// load behind them in the decode reduce: M=27 118.9 -> 118.2 us, M=64 75.9 -> 75.6).
+__device__ __forceinline__ float4 sum_partials(const float* p, int64_t stride, int n) {
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto term = [&](int k) { return *reinterpret_cast<const float4*>(p + (int64_t)k * stride); };
+  auto add = [&](const float4 v) { s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w; };
+  int k = 0;
+  for (; k + 4 <= n; k += 4) {
+    const float4 a = term(k), b = term(k + 1), c = term(k + 2), d = term(k + 3);
+    add(a); add(b); add(c); add(d);
+  }
+  if (n - k == 3) {
+    const float4 a = term(k), b = term(k + 1), c = term(k + 2);
+    add(a); add(b); add(c);
+  } else if (n - k == 2) {
+    const float4 a = term(k), b = term(k + 1);
+    add(a); add(b);
+  } else if (n - k == 1) {
+    add(term(k));
+  }
+  return s;
+}
+
 // Workspace carving: every sub-buffer starts on a 256-byte boundary.
 constexpr size_t kWsAlign = 256;
 __host__ __device__ constexpr size_t ws_align(size_t n) { return (n + kWsAlign - 1) / kWsAlign * kWsAlign; }

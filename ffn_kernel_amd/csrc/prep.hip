@@ -216,11 +216,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   uint16_t* out = g == 0 ? out0 : out1;
   const int r = (int)(idx / Cc), c = (int)(idx % Cc);
   if constexpr (VEC) {
-    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int k = 0; k < splits; ++k) {
-      const float4 v = *reinterpret_cast<const float4*>(p + (int64_t)k * plane);
-      s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-    }
+    const float4 s = sum_partials(p, plane, splits);
     uint2 v2;
     v2.x = pack2bf(s.x, s.y);
     v2.y = pack2bf(s.z, s.w);
@@ -258,12 +254,9 @@ __global__ __launch_bounds__(256) void routed_reduce_kernel(const float* __restr
   const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (n >= N) return;
   splits = routed_splits(counts[0], M, bm, splits, splits_more);
-  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int k = 0; k < splits; ++k) {
-    const float4 v = *reinterpret_cast<const float4*>(P + ((int64_t)k * M + p) * N + n);
-    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-  }
-  uint16_t* o = out + (int64_t)perm[p] * ldo + n;
+  const int row = perm[p];
+  const float4 s = sum_partials(P + (int64_t)p * N + n, (int64_t)M * N, splits);
+  uint16_t* o = out + (int64_t)row * ldo + n;
   if ((reinterpret_cast<uintptr_t>(o) & 7) == 0) {
     uint2 v2;
     v2.x = pack2bf(s.x, s.y);
@@ -310,12 +303,9 @@ __global__ __launch_bounds__(256) void routed_tail_reduce_kernel(const float* __
   for (int r = blockIdx.y * band + threadIdx.x / quads; r < (blockIdx.y + 1) * band; r += rows_per_pass) {
     const int p = tc.row0 + r;
     if (p >= tc.row_end) break;
-    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int k = 0; k < splits; ++k) {
-      const float4 v = *reinterpret_cast<const float4*>(P_tail + ((int64_t)k * n_tail + tile_i) * tile_elems + (int64_t)r * bn + 4 * q);
-      s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-    }
-    uint16_t* o = C + (int64_t)perm[p] * ldc + n;
+    const int row = perm[p];
+    const float4 s = sum_partials(P_tail + (int64_t)tile_i * tile_elems + (int64_t)r * bn + 4 * q, (int64_t)n_tail * tile_elems, splits);
+    uint16_t* o = C + (int64_t)row * ldc + n;
     if (n + 3 < N && (reinterpret_cast<uintptr_t>(o) & 7) == 0) {
       uint2 v2;
       v2.x = pack2bf(s.x, s.y);

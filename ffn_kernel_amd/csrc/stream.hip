@@ -220,15 +220,12 @@ __global__ __launch_bounds__(256) void stream_reduce_kernel(const float* __restr
                                                             uint16_t* __restrict__ out, int64_t ldo) {
   __shared__ int s_perm[kSMaxM];
   __shared__ int s_nvis;
-  route_small(mask, M, s_perm, &s_nvis);
   const int p = blockIdx.y;
   const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
+  // the partials are under way before the mask is waited for
+  const float4 s = n < N ? sum_partials(P + (int64_t)p * N + n, (int64_t)M * N, splits) : make_float4(0.f, 0.f, 0.f, 0.f);
+  route_small(mask, M, s_perm, &s_nvis);
   if (n >= N) return;
-  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int k = 0; k < splits; ++k) {
-    const float4 v = *reinterpret_cast<const float4*>(P + ((int64_t)k * M + p) * N + n);
-    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-  }
   uint16_t* o = out + (int64_t)s_perm[p] * ldo + n;
   if ((reinterpret_cast<uintptr_t>(o) & 7) == 0) {
     uint2 v2;
