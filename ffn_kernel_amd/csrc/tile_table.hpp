@@ -82,6 +82,10 @@ struct RoutedPlan {
 // behind the best tile and split of each shape, the rules by tile count before were 12 % behind (SwiGLU GEMM at M = 300 / 512 /
 // 1024 of one modality, d = 4096, h = 14336: 128 -> 98, 150 -> 100, 274 -> 183 us; single-weight GEMM at M = 512, K = 14336,
 // N = 4096: 105 -> 70 us; at M = 1024, 4096 x 4096: 49 -> 38 us).
+// The single-weight 256x256 (eight waves) and ring tiles were fitted again to all tiles at 130 (M, K, N), M = 700 ... 20000, K and N
+// of 512 ... 8192: the former took 12-30 % longer than predicted past a round.  Over 1503 drawn shapes whose plan this changed the
+// down projection is 3.2 % faster at M < 700, 5.2 % at 700-4095 and 2.1 % from 4096 up in the geometric mean (single shapes:
+// M = 1415, K = 4456, N = 1600 81 -> 47 us; the worst 0.69 times as fast); MaskedFFN d = 4096, h = 14336, M = 300 208 -> 196 us.
 // Where K % 64 != 0 the rows of a packed operand start anywhere in a 128-byte line and every 128-byte piece of a slab lies in
 // two lines: a slab takes `ragged` times as long, the more the fewer flops the tile has per byte it loads (all tiles at
 // M x K x N = 3001 x 2056 x 1544, 8192 x 4104 x 4096 and 1000 x 4104 x 4096 against K - 8: 256x256 1.03-1.09 times, 128x128
@@ -98,13 +102,13 @@ constexpr TileCost kDualCosts[] = {
     {TILE_128x256_R3, 1, 2.0, 0.836, 0.77, 0.79, 5.75, 1.4},
     {TILE_64x128_R3, 2, 1.05, 0.716, 0.51, 0.57, 6.1, 1.5}};
 constexpr TileCost kPlainCosts[] = {
-    {TILE_256x256_W8, 1, 3.2, 1.31, 0.77, 0.91, 6.0, 1.06},
+    {TILE_256x256_W8, 1, 3.2, 1.467, 0.75, 0.91, 6.0, 1.06},
     {TILE_256x256_W4, 1, 13.0, 1.33, 0.64, 0.60, 6.0, 1.08},
     {TILE_128x128_W4, 2, 0.6, 0.88, 0.60, 0.74, 6.5, 1.28},
     {TILE_SMALL_W4, 3, 0.0, 0.805, 0.42, 0.62, 6.2, 1.45},
     {TILE_128x128_R4, 1, 1.9, 0.46, 0.485, 0.88, 7.4, 1.45},
-    {TILE_128x256_R3, 1, 3.7, 0.80, 0.70, 0.90, 6.9, 1.4},
-    {TILE_64x128_R3, 2, 0.2, 0.56, 0.42, 0.60, 6.1, 1.5}};
+    {TILE_128x256_R3, 1, 3.7, 0.714, 0.70, 0.97, 6.9, 1.4},
+    {TILE_64x128_R3, 2, 0.2, 0.54, 0.42, 0.47, 6.1, 1.5}};
 
 inline double routed_tile_time(const TileCost& c, bool dual, int64_t tiles_m, int modalities, int64_t M, int64_t n_out, int64_t K,
                                int splits) {
