@@ -211,15 +211,6 @@ FfnBwdPlan plan_ffn_bwd(int64_t M, int64_t d, int64_t h, bool dup_k_contig, bool
   return p;
 }
 
-// The direct global->LDS path addresses operands with 32-bit byte offsets: from the start of A
-// when its rows are gathered, from the tile's first row otherwise (at most 256 rows away).
-bool direct_ok(int64_t K, int64_t gathered_rows, int64_t lda, int64_t ldb) {
-  constexpr int64_t k4g = (int64_t)1 << 32;
-  if (!direct_contraction(K)) return false;
-  if (gathered_rows > 0 && gathered_rows * lda * 2 >= k4g) return false;
-  return 256 * lda * 2 < k4g && 256 * ldb * 2 < k4g;
-}
-
 // The K-major kernels read a weight where the backward finds it: [K, N] rows of the contraction, N
 // contiguous, row stride ldb.  Slabs are addressed with 32-bit byte offsets from their first row.
 bool kmajor_ok(int64_t K, int64_t N, int64_t ldb, const void* w0, const void* w1) {

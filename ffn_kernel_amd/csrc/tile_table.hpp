@@ -29,6 +29,17 @@ struct TileChoice {
 constexpr int kRaggedMinK = 128;
 inline bool direct_contraction(int64_t K) { return K > 0 && (K % 64 == 0 || (K % 8 == 0 && K >= kRaggedMinK)); }
 
+// The direct global->LDS path addresses operands with 32-bit byte offsets: from the start of A when its rows are gathered,
+// from the tile's first row otherwise (at most 256 rows away).  The base of a contraction that is no whole number of slabs
+// lies 2 * (-K mod 64) bytes ahead of the operand (clear_head), and the offsets past slab 0 are larger by as much.
+inline bool direct_ok(int64_t K, int64_t gathered_rows, int64_t lda, int64_t ldb) {
+  constexpr int64_t k4g = (int64_t)1 << 32;
+  if (!direct_contraction(K)) return false;
+  const int64_t ahead = 2 * (round_up64(K, 64) - K);
+  if (gathered_rows > 0 && gathered_rows * lda * 2 + ahead >= k4g) return false;
+  return 256 * lda * 2 + ahead < k4g && 256 * ldb * 2 + ahead < k4g;
+}
+
 // Measured plans.  `python -m ffn_kernel_amd.tune --emit` times every candidate (tile x split-K factor)
 // per operation, shape and M bucket on the GPU and writes tile_table_gen.hpp: one entry wherever the best
 // candidate beat the rules and the cost model below by a margin.  The pick_* functions consult these

@@ -1,0 +1,44 @@
+"""The rules that choose a kernel for a call, and the launchers' own checks, run on the host without a GPU."""
+import ctypes
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from ffn_kernel_amd import build
+
+HERE = Path(__file__).resolve().parent
+
+
+@pytest.fixture(scope="session")
+def rules(tmp_path_factory):
+    objs = sorted(build.OBJ_DIR.glob("*.o"))
+    if len(objs) != len(list(build.CSRC.glob("*.hip"))):
+        build.build_library(verbose=False)
+        objs = sorted(build.OBJ_DIR.glob("*.o"))
+    so = tmp_path_factory.mktemp("host") / "host_checks.so"
+    cmd = [shutil.which("hipcc") or "/opt/rocm/bin/hipcc", "--offload-host-only", "-x", "hip", "-std=c++17", "-O1", "-fPIC", "-c",
+           str(HERE / "host_checks.cpp"), "-o", str(so.with_suffix(".o"))]
+    subprocess.run(cmd, check=True, capture_output=True)
+    subprocess.run(["g++", "-shared", "-o", str(so), str(so.with_suffix(".o")), *map(str, objs), "-L/opt/rocm/lib", "-lamdhip64"],
+                   check=True, capture_output=True)
+    lib = ctypes.CDLL(str(so))
+    lib.hc_direct_ok.argtypes = [ctypes.c_int64] * 4
+    return lib
+
+
+def _last_byte(M, K, lda):
+    """End of the furthest 16-byte load of the gathered operand, from the base the direct kernels use (gemm_nt.hpp: the base
+    is -K mod 64 elements ahead; a lane's offset is its row and piece, a slab's the scalar offset)."""
+    slabs = -(-K // 64)
+    return (M - 1) * lda * 2 + 7 * 16 + (slabs - 1) * 128 + 16
+
+
+# K = 149640: 56 elements past the last whole slab but one; M * K = 2^31 - 8.  Rows as packed, and further apart.
+@pytest.mark.parametrize("M,K,lda", [(14351, 149640, 149640), (14351, 149632, 149632), (1 << 20, 2040, 2040), ((1 << 20) + 4096, 2040, 2040),
+                                     (131071, 4104, 16384), (65536, 32760, 32760), (65544, 32760, 32760)])
+def test_direct_offsets_fit_32_bits(rules, M, K, lda):
+    if rules.hc_direct_ok(K, M, lda, K):
+        assert _last_byte(M, K, lda) <= (1 << 32) - 1
+    assert rules.hc_direct_ok(K, M // 2, lda, K)  # well inside: the direct path
