@@ -21,7 +21,7 @@ int fused_bwd_dw_blocks(int R, int Cc, int splits) {
 hipError_t launch_fused_bwd(const GemmArgs& gx, const SplitKArgs& gw, bool ring, hipStream_t stream) {
   if (gx.M <= 0 || gx.N <= 0 || gw.R <= 0 || gw.Cc <= 0 || gw.splits <= 0) return hipErrorInvalidValue;
   if (gx.splits != 1 || gx.tail_mode != 0 || gx.k_switch != 0) return hipErrorInvalidValue;
-  if (gx.N % 8 != 0 || gx.K <= 0 || gx.K % 8 != 0 || gx.ldb * (kBK * 2) + 2 * (int64_t)gx.N >= ((int64_t)1 << 32)) return hipErrorInvalidValue;
+  if (gx.N % 8 != 0 || !direct_slabs_ok(gx.K) || gx.ldb * (kBK * 2) + 2 * (int64_t)gx.N >= ((int64_t)1 << 32)) return hipErrorInvalidValue;
   const int dw_blocks = fused_bwd_dw_blocks(gw.R, gw.Cc, gw.splits);
   const int dx_blocks = routed_gemm_grid<FusedDx>(gx.M, gx.N);
   if (ring)
@@ -66,7 +66,7 @@ hipError_t launch_gathered_dw(const GatherDwArgs& gw, hipStream_t stream) {
 hipError_t launch_fused_bwd_gather(const GemmArgs& gx, const GatherDwArgs& gw, hipStream_t stream) {
   if (gx.M <= 0 || gx.N <= 0 || !gather_dw_args_ok(gw)) return hipErrorInvalidValue;
   if (gx.splits != 1 || gx.tail_mode != 0 || gx.k_switch != 0) return hipErrorInvalidValue;
-  if (gx.N % 8 != 0 || gx.K <= 0 || gx.K % 8 != 0 || gx.ldb * (kBK * 2) + 2 * (int64_t)gx.N >= ((int64_t)1 << 32)) return hipErrorInvalidValue;
+  if (gx.N % 8 != 0 || !direct_slabs_ok(gx.K) || gx.ldb * (kBK * 2) + 2 * (int64_t)gx.N >= ((int64_t)1 << 32)) return hipErrorInvalidValue;
   const int dw_blocks = gathered_dw_blocks(gw.s.R, gw.s.Cc, gw.s.splits);
   const int dx_blocks = routed_gemm_grid<FusedDx>(gx.M, gx.N);
   hipLaunchKernelGGL((fused_bwd_gather_kernel<FusedDx>), dim3(dw_blocks + dx_blocks), dim3(FusedDx::NT), 0, stream, gx, gw, dw_blocks);

@@ -102,7 +102,7 @@ struct RoutedGemmCfg {
   static constexpr bool DUAL = DUAL_;
   static constexpr bool GATHER_A = GATHER_A_;
   static constexpr bool SCATTER_C = SCATTER_C_;
-  static constexpr bool DIRECT = DIRECT_;   // global->LDS loads bypass registers (needs K % 8 == 0)
+  static constexpr bool DIRECT = DIRECT_;   // global->LDS loads bypass registers (needs direct_slabs_ok(K))
   static constexpr int GROUP_M = GROUP_M_;
   // Weight panels are [K, N] rows with N contiguous (the backward's view of a forward weight) and
   // are transposed on the way from LDS to the MFMA operand, see KMajorB.
@@ -239,7 +239,7 @@ struct TileLanes {
 };
 
 // ---------------------------------------------------------------------------------------------
-// Contractions that are no whole number of slabs (direct path, K % 8 == 0, K >= 64).  The slabs are counted from the END of
+// Contractions that are no whole number of slabs (direct path, direct_slabs_ok).  The slabs are counted from the END of
 // the contraction, so slab 0 would start `pad` = -K mod 64 elements ahead of it.  It is loaded from the contraction's start
 // instead - `pad` elements on, one scalar offset, no lane out of bounds - and its last `pad` elements, which are slab 1's
 // first, are cleared once they have landed, every lane clearing the LDS slots it filled itself.  The steady loops are those
@@ -1692,7 +1692,7 @@ inline hipError_t launch_routed_gemm(const GemmArgs& g, hipStream_t stream) {
   if (g.M <= 0 || g.N <= 0) return hipSuccess;
   if ((g.splits > 1 || g.splits_more > 1) && (Cfg::DUAL || !Cfg::DIRECT || g.tail_mode != 0 || g.P == nullptr)) return hipErrorInvalidValue;
   if ((g.splits > 1) != (g.splits_more > 1)) return hipErrorInvalidValue;
-  if (Cfg::DIRECT && (g.K <= 0 || g.K % 8 != 0)) return hipErrorInvalidValue;
+  if (Cfg::DIRECT && !direct_slabs_ok(g.K)) return hipErrorInvalidValue;
   if (Cfg::B_KMAJOR && (g.N % 8 != 0 || g.k_switch % kBK != 0 || g.k_switch < 0 || g.k_switch >= g.K ||
                         (g.k_switch > 0 && g.K % kBK != 0) || g.ldb * (kBK * 2) + 2 * (int64_t)g.N >= ((int64_t)1 << 32)))
     return hipErrorInvalidValue;

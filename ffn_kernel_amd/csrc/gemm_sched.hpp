@@ -8,6 +8,10 @@ constexpr int kCusPerChip = 256;
 constexpr int kTailSlots = 256;      // (tile, K range) pairs of a split tail never exceed one per CU
 constexpr int kTailMaxSplits = 16;
 
+// Contractions that the direct kernels can load: whole 64-element slabs, or 16-byte pieces of at least one slab, whose first
+// slab is loaded whole from the contraction's start (clear_head): under 64 elements that load would run past the rows.
+__host__ __device__ inline bool direct_slabs_ok(int K) { return K > 0 && (K % 64 == 0 || (K % 8 == 0 && K >= 64)); }
+
 constexpr int kEvenGroups = 3;    // see routed_tile_coord
 constexpr int kEvenGroupMin = 6;  // 6 x 5 tiles on the 32 CUs of an XCD load the fewest panels
 

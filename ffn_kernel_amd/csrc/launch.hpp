@@ -40,7 +40,8 @@ hipError_t launch_down_gemm(int tile, bool direct, const GemmArgs& g, hipStream_
 // C(routed order) = route-gather(A) @ B_g^T (MaskedFFN backward: pre-activations, dH)
 hipError_t launch_gather_gemm(int tile, bool direct, const GemmArgs& g, hipStream_t stream);
 // The three single-weight GEMMs above over K-major weights: B0[g] (and B1[g] past GemmArgs::k_switch)
-// is [K, N] rows with N contiguous.  K % 8 == 0 and N % 8 == 0 are required, with k_switch K % 64 == 0.
+// is [K, N] rows with N contiguous.  direct_slabs_ok(K) and N % 8 == 0 are required, with k_switch K % 64 == 0.
+// These and the direct forms above return hipErrorInvalidValue for any other K.
 hipError_t launch_linear_gemm_kmajor(int tile, const GemmArgs& g, hipStream_t stream);
 hipError_t launch_down_gemm_kmajor(int tile, const GemmArgs& g, hipStream_t stream);
 hipError_t launch_gather_gemm_kmajor(int tile, const GemmArgs& g, hipStream_t stream);

@@ -9,4 +9,32 @@ extern "C" {
 
 int hc_direct_ok(int64_t K, int64_t gathered_rows, int64_t lda, int64_t ldb) { return direct_ok(K, gathered_rows, lda, ldb); }
 
+// hipError_t of a launcher for operands it refuses before it launches anything (the operands are never read).
+// form: 0 linear, 1 SwiGLU, 2 down, 3 gather, 4 ... 6 the K-major forms of 0, 2 and 3, 7 and 8 the fused backward (two
+// stages, ring), 9 the same with the weight gradients in place.
+int hc_launch(int form, int tile, int M, int N, int K, int split_tail) {
+  static uint16_t operand[8] __attribute__((aligned(16)));
+  static float partials[4];
+  GemmArgs g;
+  g.A = operand; g.lda = K; g.B0[0] = g.B0[1] = g.B1[0] = g.B1[1] = operand; g.ldb = form >= 4 ? N : K;
+  g.C = operand; g.ldc = N; g.perm = nullptr; g.counts = nullptr; g.M = M; g.N = N; g.K = K;
+  g.P_tail = split_tail ? partials : nullptr;
+  SplitKArgs w;
+  w.A = w.B = operand; w.lda = w.ldb = 128; w.P = partials; w.counts = nullptr; w.M = M; w.R = w.Cc = 64; w.splits = 1;
+  GatherDwArgs gw;
+  gw.G = gw.X = operand; gw.ldg = gw.ldx = 64; gw.perm = nullptr; gw.counts = nullptr; gw.s = w;
+  switch (form) {
+    case 0: return launch_linear_gemm(tile, true, g, nullptr);
+    case 1: return launch_up_gemm(tile, true, g, nullptr);
+    case 2: return launch_down_gemm(tile, true, g, nullptr);
+    case 3: return launch_gather_gemm(tile, true, g, nullptr);
+    case 4: return launch_linear_gemm_kmajor(tile, g, nullptr);
+    case 5: return launch_down_gemm_kmajor(tile, g, nullptr);
+    case 6: return launch_gather_gemm_kmajor(tile, g, nullptr);
+    case 7: return launch_fused_bwd(g, w, false, nullptr);
+    case 8: return launch_fused_bwd(g, w, true, nullptr);
+    default: return launch_fused_bwd_gather(g, gw, nullptr);
+  }
+}
+
 }  // extern "C"

@@ -42,3 +42,23 @@ def test_direct_offsets_fit_32_bits(rules, M, K, lda):
     if rules.hc_direct_ok(K, M, lda, K):
         assert _last_byte(M, K, lda) <= (1 << 32) - 1
     assert rules.hc_direct_ok(K, M // 2, lda, K)  # well inside: the direct path
+
+
+INVALID_VALUE = 1  # hipErrorInvalidValue
+
+
+@pytest.fixture
+def refused(rules):
+    """Launcher calls that must be refused; on a machine with a GPU they are not tried."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("a launcher that let the call through would launch it")
+    return lambda *a: rules.hc_launch(*a) == INVALID_VALUE
+
+
+# Under one slab the direct kernels' first load would pass the rows' ends: only whole slabs and 64 elements or more.
+@pytest.mark.parametrize("K", [-64, 0, 8, 48, 56, 68, 130])
+def test_direct_launchers_refuse_short_contractions(refused, K):
+    for form in range(10):
+        for tile in (0, 1, 2, 3, 4, 6, 7) if form < 7 else (2,):
+            assert refused(form, tile, 64, 64, K, 0), (form, tile)
