@@ -87,10 +87,13 @@ inline hipError_t dispatch_tile(int tile, const GemmArgs& g, hipStream_t stream)
 template <class Tiles, class Big>
 inline hipError_t dispatch_big_tile_with_tail(const GemmArgs& g, hipStream_t stream) {
   using Small = typename Tiles::T2;
+  // With P_tail the kernel leaves every remainder to the split tail, which only these tiles have.
+  constexpr bool kSplitTail = !Big::DUAL && Big::SCATTER_C && Big::DIRECT;
+  if (!kSplitTail && g.P_tail != nullptr) return hipErrorInvalidValue;
   GemmArgs a = g;
   a.tail_mode = 1;
   if (hipError_t e = launch_routed_gemm<Big>(a, stream)) return e;
-  if (!Big::DUAL && Big::SCATTER_C && g.P_tail != nullptr) {
+  if (kSplitTail && g.P_tail != nullptr) {
     // Split tail: the remaining tiles on the big tile, each cut into K ranges (at most kTailSlots
     // (tile, range) pairs), then the reduce pass.
     a.tail_mode = 3;

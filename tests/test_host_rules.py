@@ -56,6 +56,14 @@ def refused(rules):
     return lambda *a: rules.hc_launch(*a) == INVALID_VALUE
 
 
+# A split tail exists for single-weight tiles that scatter their rows: with its workspace set, the others would leave half of
+# the tiles past the last whole round to a launch that does not come.
+@pytest.mark.parametrize("form", [1, 3, 6])
+@pytest.mark.parametrize("tile", [0, 1])
+def test_split_tail_is_refused_where_there_is_none(refused, form, tile):
+    assert refused(form, tile, 20 * 256, 20 * 256, 64, 1)
+
+
 # Under one slab the direct kernels' first load would pass the rows' ends: only whole slabs and 64 elements or more.
 @pytest.mark.parametrize("K", [-64, 0, 8, 48, 56, 68, 130])
 def test_direct_launchers_refuse_short_contractions(refused, K):
