@@ -605,7 +605,14 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
     }
     default: return fail(FFNK_E_OP, "unknown op %d", op);
   }
-  const bool direct = direct_contraction(contraction);
+  // (the weight-gradient GEMM contracts over whole slabs, padded or cleared, whatever M is)
+  const bool direct = op == FFNK_OP_BWD_DW ? contraction > 0 : direct_contraction(contraction);
+  // Kernels without the two ring tiles of three stages run the two-stage tiles in their place.
+  const bool kmajor_dx = op == FFNK_OP_LINEAR_BWD || op == FFNK_OP_BWD_DX;
+  if (!direct || kmajor_dx || op == FFNK_OP_BWD_DW) {
+    if (tile == TILE_128x256_R3) tile = TILE_128x128_W4;
+    if (tile == TILE_64x128_R3) tile = op == FFNK_OP_BWD_DW ? TILE_128x128_W4 : TILE_SMALL_W4;
+  }
   if (!direct && tile == TILE_256x256_W4) tile = TILE_256x256_W8;  // the four-wave tile runs on the direct path only
   const TileGeom gm = tile_geom(tile, dual);
   const bool stream = (op == FFNK_OP_FFN_FWD || op == FFNK_OP_FFN_UP || op == FFNK_OP_FFN_DOWN) && (use_stream_path(M, K, N) || use_ragged_stream(M, K, N));
@@ -625,10 +632,9 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
     case FFNK_OP_FFN_DOWN: plan_gm = plan_group_m(TUNED_DOWN, M, N, K); break;
     default: plan_gm = plan_group_m(TUNED_NONE, M, K, N); break;
   }
-  const bool kmajor_dx = op == FFNK_OP_LINEAR_BWD || op == FFNK_OP_BWD_DX;
   out->group_m = plan_gm > 0 ? plan_gm : (dual || kmajor_dx) ? 8 : 4;
   out->split_k = splits;
-  out->direct_lds = ((direct && contraction % 64 == 0) || in_place) ? 1 : 0;
+  out->direct_lds = (direct || in_place) ? 1 : 0;
   out->in_place = in_place ? 1 : 0;
   // 4: ring of four stages (128x128); 3: token panel in three stages, weight panel in two (single-weight 256x256 tiles)
   out->lds_stages = !(direct || in_place) ? 2 : tile == TILE_128x128_R4 ? 4 : (tile == TILE_128x256_R3 || tile == TILE_64x128_R3) ? 3 : (is_big_tile(tile) && !dual) ? 3 : 2;

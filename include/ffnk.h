@@ -76,9 +76,7 @@ typedef struct ffnk_tile_config_t {
   int32_t lds_stages;  /* LDS buffers in flight                                    */
   int32_t group_m;     /* M-tiles per L2 super-group in the tile order             */
   int32_t split_k;     /* contraction splits reduced by a second kernel (1 = none) */
-  int32_t direct_lds;  /* 1 = global->LDS loads bypass registers, whole 128-byte
-                          lines of the contraction; 0 also for a contraction that
-                          is no multiple of 64                                     */
+  int32_t direct_lds;  /* 1 = global->LDS loads bypass registers                   */
   int32_t in_place;    /* FFNK_OP_BWD_DW: 1 = the weight-gradient GEMM reads g and x
                           where they lie, 0 = routed transposes written first      */
 } ffnk_tile_config_t;

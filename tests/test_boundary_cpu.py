@@ -38,21 +38,42 @@ def test_workspace_bytes():
         _lib.workspace_bytes(_lib.OP_LINEAR_FWD, -1, 1, 1)
 
 
+# Forced tiles are reported as they run: the K-major dx GEMM and the weight-gradient GEMM have no ring tiles of three stages,
+# a staged contraction no ring at all, and the four-wave 256x256 tile exists on the direct path only.
+@pytest.mark.parametrize("tile,linear,staged,dx,dw", [(1, (256, 256, 3), (256, 256, 2), (256, 256, 3), (256, 256, 3)),
+                                                      (4, (128, 128, 4), (128, 128, 2), (128, 128, 4), (128, 128, 4)),
+                                                      (6, (128, 256, 3), (128, 128, 2), (128, 128, 2), (128, 128, 2)),
+                                                      (7, (64, 128, 3), (128, 64, 2), (128, 64, 2), (128, 128, 2))])
+def test_tile_config_names_the_tile_that_runs(tile, linear, staged, dx, dw):
+    lib = _lib.load()
+    lib.ffnk_debug_force_tile(tile)
+    try:
+        got = [tuple(_lib.tile_config(op, 4000, K, 1024)[k] for k in ("block_m", "block_n", "lds_stages"))
+               for op, K in ((_lib.OP_LINEAR_FWD, 1032), (_lib.OP_LINEAR_FWD, 72), (_lib.OP_BWD_DX, 1032), (_lib.OP_BWD_DW, 1032))]
+    finally:
+        lib.ffnk_debug_force_tile(-1)
+    assert got == [linear, staged, dx, dw]
+
+
 def test_tile_table_entries():
     big = _lib.tile_config(_lib.OP_FFN_UP, 32768, 4096, 14336)
     assert big["path"] == _lib.PATH_MFMA_TILED and big["block_m"] == 256 and big["direct_lds"] == 1
     assert big["block_k"] == 64 and big["lds_stages"] == 2  # two 64-element slabs, loaded global->LDS
     assert big["waves_m"] * big["waves_n"] == 4  # four waves of 128x128
     half = _lib.tile_config(_lib.OP_LINEAR_FWD, 2048, 96, 1024)
-    assert half["direct_lds"] == 0  # the direct path moves whole 128-byte lines: K % 64 == 0
-    # the four-wave 256x256 tile exists on the direct path only; a staged shape that would pick it runs eight waves
+    assert half["direct_lds"] == 0  # short contractions off whole 64-element slabs are staged through registers
+    # single-weight GEMMs over a long contraction of whole slabs: the four-wave 256x256 tile
     long_k = _lib.tile_config(_lib.OP_LINEAR_FWD, 32768, 4096, 4096)
     assert long_k["direct_lds"] == 1 and long_k["block_m"] == 256 and long_k["waves_m"] * long_k["waves_n"] == 4
     # single-weight 256x256 tiles keep their token panel in a ring of three LDS stages (the weight panel in two)
     assert long_k["lds_stages"] == 3
     assert _lib.tile_config(_lib.OP_FFN_DOWN, 32768, 4096, 14336)["lds_stages"] == 3
-    staged = _lib.tile_config(_lib.OP_LINEAR_FWD, 32768, 4096 + 8, 4096)
-    assert staged["direct_lds"] == 0 and staged["block_m"] == 256 and staged["waves_m"] * staged["waves_n"] == 8
+    # ... off whole slabs: the eight-wave one, on the direct path as well (from 128 elements up)
+    ragged = _lib.tile_config(_lib.OP_LINEAR_FWD, 32768, 4096 + 8, 4096)
+    assert ragged["direct_lds"] == 1 and ragged["block_m"] == 256 and ragged["waves_m"] * ragged["waves_n"] == 8
+    assert ragged["lds_stages"] == 3
+    # the weight-gradient GEMM contracts over whole slabs whatever M is
+    assert all(_lib.tile_config(_lib.OP_BWD_DW, M, 4096, 4096)["direct_lds"] == 1 for M in (8191, 8184, 8192))
     # M <= 8: dot-product streams, one wavefront per 1024-element K slice, no cross-workgroup split
     dec = _lib.tile_config(_lib.OP_FFN_FWD, 8, 4096, 14336)
     assert dec["path"] == _lib.PATH_STREAM and dec["lds_stages"] == 0 and dec["block_m"] == 8
