@@ -71,7 +71,7 @@ RouteWs carve_route(uint8_t* ws, int64_t M) {
 }
 
 // Tuner overrides, see ffnk_debug_force_tile / ffnk_debug_force_splits.
-std::atomic<int> g_force_tile{-1};    // 0..3: that tile; -1: table, then rules; -2: rules only
+std::atomic<int> g_force_tile{-1};    // 0..4, 6, 7: that tile; -1: table, then rules; -2: rules only
 std::atomic<int> g_force_splits{-1};  // >= 1: that split-K factor where a GEMM can be split
 std::atomic<int> g_force_group_m{0};      // >= 1: M-tiles per super-group in the tile order of every routed GEMM
 std::atomic<int> g_force_bwd_gather{-1};  // MaskedLinear backward: 1 = weight gradients from g and x in place, 0 = from transposes, -1 = plan

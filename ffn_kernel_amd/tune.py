@@ -43,7 +43,7 @@ import torch
 from . import _lib
 from .ops import masked_linear_backward, masked_linear_forward
 
-TILES = {0: "256x256/8w", 1: "256x256/4w", 2: "128x128/4w", 3: "small/4w", 4: "128x128/ring4"}
+TILES = {0: "256x256/8w", 1: "256x256/4w", 2: "128x128/4w", 3: "small/4w", 4: "128x128/ring4", 6: "128x256/ring3", 7: "64x128/ring3"}
 GROUP_MS = (2, 4, 8, 16)   # M-tiles per super-group tried in the second stage
 GM_MIN_ROWS = 4096         # ... for buckets that reach this many rows
 TILE_IN_PLACE = 5  # weight-gradient plans only (kTileGatherDw in csrc/capi.hip): g and x read where they lie
@@ -145,11 +145,12 @@ def _cdiv(a, b):
 
 
 def _valid_splits(contraction, M):
-    """Split-K factors worth trying: ranges of whole 64-element slabs, at least 8 each, none empty; past
-    8192 rows the tiles fill the chip on their own and the fp32 partials would run into gigabytes."""
-    nk = contraction // 64
+    """Split-K factors worth trying: ranges of whole 64-element slabs (the first one partly ahead of a contraction that
+    is no multiple of 64; direct_contraction in csrc/tile_table.hpp), at least 8 each, none empty; past 8192 rows the
+    tiles fill the chip on their own and the fp32 partials would run into gigabytes."""
+    nk = _cdiv(contraction, 64)
     out = [1]
-    if contraction % 64 == 0 and M <= 8192:
+    if (contraction % 64 == 0 or (contraction % 8 == 0 and contraction >= 128)) and M <= 8192:
         for s in SPLITS[1:]:
             if nk // s >= 8 and _cdiv(nk, _cdiv(nk, s)) == s:
                 out.append(s)
@@ -190,12 +191,12 @@ def _geomean(xs):
 
 
 def _tile_id(cfg, dual):
-    """Tile id behind an answer of ffnk_tile_config for a routed GEMM."""
+    """Tile id behind an answer of ffnk_tile_config for a routed GEMM of a forward (block_n: output columns, half the
+    weight rows that a SwiGLU tile holds)."""
+    cols = cfg["block_n"] * (2 if dual else 1)
     if cfg["block_m"] == 256:
         return 0 if cfg["waves_m"] * cfg["waves_n"] == 8 else 1
-    if cfg["lds_stages"] == 4:
-        return 4
-    return 2 if cfg["block_m"] == 128 and (dual or cfg["block_n"] == 128) else 3
+    return {(128, 128, 4): 4, (128, 256, 3): 6, (64, 128, 3): 7, (128, 128, 2): 2}.get((cfg["block_m"], cols, cfg["lds_stages"]), 3)
 
 
 def _gm_stage(measure, ref, own, margin):

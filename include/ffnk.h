@@ -131,8 +131,10 @@ FFNK_API int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile
  * Tuner-only hooks (python -m ffn_kernel_amd.tune, the counterpart of the reference's find_spec scripts
  * sweeps, and the tests that run every compiled tile).  ffnk_debug_force_tile: every LDS-tiled GEMM
  * launched by this process uses tile id `tile` (0 = 256x256 / 8 waves, 1 = 256x256 / 4 waves,
- * 2 = 128x128 / 4 waves, 3 = small, 4 = 128x128 / 4 waves behind a ring of four LDS stages); -1 returns to the tile table (measured plans first, then the
- * rules); -2 uses the rules only, ignoring the measured plans (what the tuner compares against).
+ * 2 = 128x128 / 4 waves, 3 = small, 4 = 128x128 / 4 waves behind a ring of four LDS stages, 6 = 128x256 and
+ * 7 = 64x128 behind a ring of three; GEMMs without a ring run 2 or 3 in their place); -1 returns to the tile table
+ * (measured plans first, then the rules); -2 uses the rules only, ignoring the measured plans (what the tuner compares
+ * against).  Other values count as -1.
  * ffnk_debug_force_splits: every GEMM that can cut its contraction (single-weight routed GEMMs with
  * a workspace, weight-gradient GEMMs) uses `splits` ranges (1..16) where the shape allows it; -1
  * returns to the table.  Both are process-global atomics read at every call (ffnk_workspace_bytes

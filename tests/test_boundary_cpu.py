@@ -55,6 +55,23 @@ def test_tile_config_names_the_tile_that_runs(tile, linear, staged, dx, dw):
     assert got == [linear, staged, dx, dw]
 
 
+# The tuner pins the plan it reads back from ffnk_tile_config: every tile of both kinds of GEMM must come back as itself.
+@pytest.mark.parametrize("K", [4096, 4104])
+@pytest.mark.parametrize("op,dual", [(_lib.OP_LINEAR_FWD, False), (_lib.OP_FFN_DOWN, False), (_lib.OP_FFN_UP, True)])
+def test_tuner_reads_back_every_tile(op, dual, K):
+    from ffn_kernel_amd import tune
+    lib = _lib.load()
+    compiled = []
+    for tile in range(16):
+        lib.ffnk_debug_force_tile(tile)
+        read = tune._tile_id(_lib.tile_config(op, 5000, K, K), dual)
+        if lib.ffnk_debug_force_tile(-1) == tile:
+            compiled.append(tile)
+            assert read == tile
+    assert compiled == sorted(tune.TILES)
+    assert tune._valid_splits(K, 4096) == [s for s in tune.SPLITS if s <= 8]
+
+
 def test_tile_table_entries():
     big = _lib.tile_config(_lib.OP_FFN_UP, 32768, 4096, 14336)
     assert big["path"] == _lib.PATH_MFMA_TILED and big["block_m"] == 256 and big["direct_lds"] == 1
