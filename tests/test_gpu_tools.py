@@ -46,7 +46,8 @@ def test_tuner_emits_a_table_the_library_can_compile(dev, tmp_path, capsys):
     for op, lo, hi, k, n, tile, splits, group_m in entries[:-1]:
         assert int(group_m) in (0, 2, 4, 8, 16)
         # tile 5 is a form of the weight-gradient GEMM (operands read in place), not a tile of the routed GEMMs
-        assert int(op) in (0, 1, 2, 3) and int(lo) <= int(hi) and 0 <= int(tile) <= (5 if int(op) == 2 else 4) and 1 <= int(splits) <= 16
+        assert int(op) in (0, 1, 2, 3) and int(lo) <= int(hi) and 1 <= int(splits) <= 16
+        assert int(tile) in ((0, 1, 2, 3, 4, 5) if int(op) == 2 else tune.TILES)
     recs = json.loads((tmp_path / "t.json").read_text())
     assert {r["op"] for r in recs} == {"ffn_fwd", "linear_fwd", "linear_bwd"}
     lib = _lib.load()
