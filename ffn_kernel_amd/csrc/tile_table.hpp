@@ -85,44 +85,57 @@ struct RoutedPlan {
   int splits_more;
 };
 
-// Time of a direct-path GEMM in us, fitted to sweeps of every tile (and split factor) at M = 10 ... 4096 with one and with both
-// modalities present: SwiGLU GEMMs at seven (d, h) from 1024 x 2048 to 7168 x 20480, single-weight GEMMs at ten (K, N) from
-// 1024 x 1024 to 20480 x 7168 (rms error 9 %).  A round of the chip takes base + slabs * per_slab; a partial first round
-// takes `first` of that plus the rest by the workgroups on its fullest CU, a later one `again` plus the rest.  The weights
-// arrive at `tbs` TB/s; the smaller of the two times is mostly hidden behind the larger.  The plans that follow are 2-3 %
-// behind the best tile and split of each shape, the rules by tile count before were 12 % behind (SwiGLU GEMM at M = 300 / 512 /
-// 1024 of one modality, d = 4096, h = 14336: 128 -> 98, 150 -> 100, 274 -> 183 us; single-weight GEMM at M = 512, K = 14336,
-// N = 4096: 105 -> 70 us; at M = 1024, 4096 x 4096: 49 -> 38 us).
-// The single-weight 256x256 (eight waves) and ring tiles were fitted again to all tiles at 130 (M, K, N), M = 700 ... 20000, K and N
-// of 512 ... 8192: the former took 12-30 % longer than predicted past a round.  Over 1503 drawn shapes whose plan this changed the
-// down projection is 3.2 % faster at M < 700, 5.2 % at 700-4095 and 2.1 % from 4096 up in the geometric mean (single shapes:
-// M = 1415, K = 4456, N = 1600 81 -> 47 us; the worst 0.69 times as fast); MaskedFFN d = 4096, h = 14336, M = 300 208 -> 196 us.
-// Where K % 64 != 0 the rows of a packed operand start anywhere in a 128-byte line and every 128-byte piece of a slab lies in
-// two lines: a slab takes `ragged` times as long, the more the fewer flops the tile has per byte it loads (all tiles at
-// M x K x N = 3001 x 2056 x 1544, 8192 x 4104 x 4096 and 1000 x 4104 x 4096 against K - 8: 256x256 1.03-1.09 times, 128x128
-// 1.2-1.3, the others 1.3-1.55; MaskedLinear at the first of them on the tile of K = 2048 (128x64) 43.9 us, on 128x256 36.7 us).
+// Time of a direct-path GEMM in us, fitted to every tile and split factor at drawn shapes, weights and rows cold, one or both
+// modalities present: 8000 SwiGLU GEMMs (M = 33 ... 8192, d = 1024 ... 8192, h = 2 ... 3.5 d) and 8000 single-weight GEMMs
+// (M = 9 ... 12000, K = 128 ... 28672, N = 512 ... 8192), a quarter of them off multiples of 64; rms error 7 %.  A round of
+// the chip takes base + slabs * per_slab.  A partial round takes a part of it that depends on the workgroups of the fullest CU:
+// `first` (the launch is less than a round) and `again` (behind whole rounds) hold, per number of workgroups, the part just
+// past the number below it and the part when every CU has as many.  The weights arrive at `tbs` TB/s, token rows and results
+// at `io`; of the products' and the weights' times the smaller is partly hidden behind the larger.  Where K % 64 != 0 the rows
+// of a packed operand start anywhere in a 128-byte line and every 128-byte piece of a slab lies in two lines: a slab takes
+// `ragged` times as long, the more the fewer flops the tile has per byte it loads.
+// Without the steps by workgroups per CU (a partial round taken as linear in them) and with the likelier M-tile count alone,
+// the plans were 2.8 % (single weight) and 4.7 % (SwiGLU) behind the best of each shape in the geometric mean, and more than
+// 8 % behind the rules by tile count below in 2.9 % and 5.1 % of 3900 / 4500 shapes that no fit has seen (K = 11392, N = 4544,
+// M = 403: 127 us, rules 84); with both, 1.5 % and 3.8 % behind the best, 22 % and 14 % ahead of the rules, and more than 8 %
+// behind them in 0.8 % and 2.8 % (K = 11392, N = 4544, M = 403: 75 us).
+constexpr int kMaxPerCu = 3;
 struct TileCost {
   int tile, per_cu;
-  double base, per_slab, first, again, tbs, ragged;
+  double base, per_slab, tbs, ragged;
+  double first[2 * kMaxPerCu], again[2 * kMaxPerCu];
 };
+struct GemmCost {
+  double launch, hidden, io, tail;   // tail: the second launch of a big tile's remainder
+  double reduce, reduce_tbs;         // split plans: the reduce pass, and the partials' way out and back
+};
+constexpr GemmCost kDualCost = {4.073, 0.683, 3.0, 3.968, 0.0, 1.0}, kPlainCost = {5.448, 0.32, 11.972, 17.518, 2.151, 7.525};
 constexpr TileCost kDualCosts[] = {
-    {TILE_256x256_W4, 1, 7.2, 1.313, 0.77, 0.71, 5.05, 1.08},
-    {TILE_128x128_W4, 2, 0.0, 0.992, 0.70, 0.69, 5.8, 1.28},
-    {TILE_SMALL_W4, 3, 0.0, 0.958, 0.59, 0.66, 5.6, 1.45},
-    {TILE_128x128_R4, 1, 1.5, 0.504, 0.74, 0.88, 6.2, 1.45},
-    {TILE_128x256_R3, 1, 2.0, 0.836, 0.77, 0.79, 5.75, 1.4},
-    {TILE_64x128_R3, 2, 1.05, 0.716, 0.51, 0.57, 6.1, 1.5}};
+    {TILE_256x256_W4, 1, 8.145, 1.056, 9.0, 1.319, {0.956, 1.0}, {1.003, 1.0}},
+    {TILE_128x128_W4, 2, 0.64, 0.853, 8.894, 1.277, {0.825, 0.841, 1.012, 1.0}, {0.762, 0.857, 0.862, 1.0}},
+    {TILE_SMALL_W4, 3, 0.0, 0.899, 7.554, 1.341, {0.648, 0.74, 0.779, 0.77, 1.105, 1.0}, {0.434, 0.556, 0.638, 0.704, 0.962, 1.0}},
+    {TILE_128x128_R4, 1, 2.181, 0.436, 9.0, 1.464, {1.015, 1.0}, {0.899, 1.0}},
+    {TILE_128x256_R3, 1, 2.476, 0.724, 9.0, 1.486, {0.982, 1.0}, {0.907, 1.0}},
+    {TILE_64x128_R3, 2, 0.0, 0.612, 7.659, 1.469, {0.679, 0.65, 1.124, 1.0}, {0.531, 0.606, 0.99, 1.0}}};
 constexpr TileCost kPlainCosts[] = {
-    {TILE_256x256_W8, 1, 3.2, 1.467, 0.75, 0.91, 6.0, 1.06},
-    {TILE_256x256_W4, 1, 13.0, 1.33, 0.64, 0.60, 6.0, 1.08},
-    {TILE_128x128_W4, 2, 0.6, 0.88, 0.60, 0.74, 6.5, 1.28},
-    {TILE_SMALL_W4, 3, 0.0, 0.805, 0.42, 0.62, 6.2, 1.45},
-    {TILE_128x128_R4, 1, 1.9, 0.46, 0.485, 0.88, 7.4, 1.45},
-    {TILE_128x256_R3, 1, 3.7, 0.714, 0.70, 0.97, 6.9, 1.4},
-    {TILE_64x128_R3, 2, 0.2, 0.54, 0.42, 0.47, 6.1, 1.5}};
+    {TILE_256x256_W8, 1, 4.964, 1.261, 6.216, 1.106, {0.772, 1.0}, {0.886, 1.0}},
+    {TILE_256x256_W4, 1, 12.067, 1.188, 4.001, 1.117, {0.769, 1.0}, {0.207, 1.0}},
+    {TILE_128x128_W4, 2, 3.08, 0.874, 5.329, 1.234, {0.51, 0.714, 0.862, 1.0}, {0.565, 0.691, 0.867, 1.0}},
+    {TILE_SMALL_W4, 3, 1.882, 0.891, 5.278, 1.235, {0.327, 0.581, 0.598, 0.682, 0.939, 1.0}, {0.339, 0.404, 0.517, 0.642, 0.899, 1.0}},
+    {TILE_128x128_R4, 1, 3.892, 0.417, 6.008, 1.352, {0.642, 1.0}, {0.826, 1.0}},
+    {TILE_128x256_R3, 1, 6.127, 0.679, 5.596, 1.317, {0.694, 1.0}, {0.825, 1.0}},
+    {TILE_64x128_R3, 2, 2.924, 0.519, 5.577, 1.38, {0.404, 0.589, 0.868, 1.0}, {0.425, 0.499, 0.808, 1.0}}};
+
+// Part of a round that `rest` workgroups take on per_cu slots of every CU.
+inline double round_part(const double* knots, int64_t rest) {
+  const int n = (int)cdiv64(rest, kCus);
+  const double lo = knots[2 * (n - 1)], hi = knots[2 * n - 1];
+  return lo + (hi - lo) * ((double)rest / (double)kCus - (double)(n - 1));
+}
 
 inline double routed_tile_time(const TileCost& c, bool dual, int64_t tiles_m, int modalities, int64_t M, int64_t n_out, int64_t K,
                                int splits) {
+  const GemmCost& g = dual ? kDualCost : kPlainCost;
   const TileGeom t = tile_geom(c.tile, dual);
   const int64_t slabs = cdiv64(K, 64), slots = (int64_t)kCus * c.per_cu;
   const int64_t tiles = tiles_m * cdiv64(n_out, t.block_n_out) * splits;
@@ -131,21 +144,20 @@ inline double routed_tile_time(const TileCost& c, bool dual, int64_t tiles_m, in
   const double round = c.base + per_slab * (double)cdiv64(slabs, splits);
   double time = (double)full * round;
   if (rest > 0) {
-    const double fill = c.per_cu == 1 ? (double)rest / (double)slots : (double)(cdiv64(rest, kCus) - 1) / (double)(c.per_cu - 1);
-    if (!is_big_tile(c.tile) || splits > 1 || full == 0) {
-      const double part = full > 0 ? c.again : c.first;
-      time += round * (part + (1.0 - part) * fill);
-    } else if (dual) {  // past half a round another round, else 128x128 tiles (whole_round_tiles)
-      time += rest > slots / 2 ? round : 3.0 + 1.08 * (double)slabs * (0.5 + 0.5 * (double)rest * 4.0 / 512.0);
+    if (!is_big_tile(c.tile) || splits > 1 || full == 0 || (dual && rest > slots / 2)) {  // whole_round_tiles
+      time += round * round_part(full > 0 ? c.again : c.first, rest);
+    } else if (dual) {  // four 128-row tiles for each of the remainder
+      const TileCost& s = kDualCosts[1];
+      const double small = s.base + (K % 64 == 0 ? s.per_slab : s.per_slab * s.ragged) * (double)slabs;
+      time += g.tail + small * round_part(s.first, 4 * rest);
     } else {            // split tail
-      const double cut = 8.0 + c.base + per_slab * (double)slabs / (double)tail_split_factor((int)rest, (int)slabs);
-      time += cut < round ? cut : round;
+      time += g.tail + c.base + per_slab * (double)slabs / (double)tail_split_factor((int)rest, (int)slabs);
     }
   }
   const double weights = modalities * (dual ? 2.0 : 1.0) * (double)K * (double)n_out * 2.0e-6 / c.tbs;
-  const double hidden = dual ? 0.15 : 0.39;
-  time = (dual ? 4.9 : 6.9) + (time > weights ? time + hidden * weights : weights + hidden * time);
-  if (splits > 1) time += 3.0 + (double)splits * (double)M * (double)n_out * 8.0e-6 / 7.2;  // partials and the reduce pass
+  time = g.launch + (double)M * (double)(K + n_out) * 2.0e-6 / g.io +
+         (time > weights ? time + g.hidden * weights : weights + g.hidden * time);
+  if (splits > 1) time += g.reduce + (double)splits * (double)M * (double)n_out * 8.0e-6 / g.reduce_tbs;
   return time;
 }
 
@@ -155,49 +167,81 @@ inline bool routed_split_ok(int64_t K, int s) {
   return s == 1 || (nk / s >= 4 && cdiv64(nk, cdiv64(nk, s)) == s);
 }
 
-inline double best_split(const TileCost& c, int64_t tiles_m, int modalities, int64_t M, int64_t n_out, int64_t K, bool split,
-                         int first, int* best) {
-  constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16};
-  double best_time = -1.0;
-  for (const int s : kSplits) {
-    if (s < first || (s > 1 && (!split || c.tile == TILE_256x256_W4)) || !routed_split_ok(K, s)) continue;
-    const double t = routed_tile_time(c, false, tiles_m, modalities, M, n_out, K, s);
-    if (best_time < 0.0 || t < best_time) {
-      best_time = t;
-      *best = s;
-    }
-  }
-  return best_time;
+// What a plan is chosen by.  With both modalities present the rows of the two make cdiv(M, block_m) M-tiles or one more, and
+// where that starts another round the times differ by up to a half.  One more it is at (M / block_m rounded up) *
+// ((M - 1) mod block_m) of the M - 1 ways to split M; masks that set every row by itself split M about evenly.  The score is
+// the product of three times: over all splits (weight 1), at an even split (weight 2), of one modality alone (weight 2).
+inline double plan_score(const TileCost& c, bool dual, int64_t M, int64_t n_out, int64_t K, int splits, int splits_more) {
+  const int64_t bm = tile_geom(c.tile, dual).block_m, less = cdiv64(M, bm);
+  const double p = M > 1 ? (double)(less * ((M - 1) % bm)) / (double)(M - 1) : 0.0;
+  int64_t dev = 0;  // a third of sqrt(M): how far such a mask is off an even split
+  while ((dev + 1) * (dev + 1) * 9 <= M) ++dev;
+  const int64_t visual = (M + 1) / 2 + dev < M ? (M + 1) / 2 + dev : M;
+  const bool even_more = cdiv64(visual, bm) + cdiv64(M - visual, bm) > less;
+  const double t = routed_tile_time(c, dual, less, 2, M, n_out, K, splits);
+  const double more = routed_tile_time(c, dual, less + 1, 2, M, n_out, K, splits_more);
+  const double one = routed_tile_time(c, dual, less, 1, M, n_out, K, splits);
+  const double even = even_more ? more : t;
+  return ((1.0 - p) * t + p * more) * even * even * one * one;
 }
 
-// The plan with the smallest weighted product of two times: both modalities present, about evenly (M-tiles: the likelier of
-// the two counts; weight 3), and one modality alone (weight 2).  `split`: the caller has a workspace for partials and N % 4 == 0.
+// The rules by tile count: where the model does not apply, and what its plan has to beat.
+inline int rule_tile(int64_t M, int64_t n_out, bool dual, int64_t K) {
+  auto tiles = [&](int tile) {
+    const TileGeom t = tile_geom(tile, dual);
+    return cdiv64(M, t.block_m) * cdiv64(n_out, t.block_n_out);
+  };
+  // Past two rounds of the chip, four 128x128-per-wave wavefronts lead for the SwiGLU kernel at 128 rows x
+  // 128x128 (a third fewer LDS reads per flop; measured 4 % faster at M = 32768, d = 4096, h = 14336); so do the
+  // single-weight kernels over a long contraction (1-2.5 % faster at K = 4096 and 14336, N = 4096, M >= 16384),
+  // which otherwise keep eight wavefronts of 128x64 (less exposed when K is short).
+  if (tiles(TILE_256x256_W8) >= 2 * kCus) return dual || (K >= 4096 && K % 64 == 0) ? TILE_256x256_W4 : TILE_256x256_W8;
+  if (tiles(TILE_128x128_W4) >= kCus) return TILE_128x128_W4;
+  return TILE_SMALL_W4;
+}
+
+inline RoutedPlan rule_plan(int64_t M, int64_t n_out, int64_t K);
+
+// The plan with the smallest score among all tiles and split factors.  `split`: the caller has a workspace for partials and
+// N % 4 == 0.  The rules' plan stays unless the model sees a gain of kModelMargin, near which its choice is as often the slower
+// one (M = 8192, K = 2048, N = 1024, runs of both modalities: 256x256 tiles 58 us, the rules' 128x128 53): without it 6.0 % of
+// the SwiGLU and 2.1 % of the single-weight shapes ran more than 3 % slower than on the rules' plan, with it 5.1 % and 1.7 %.
+constexpr double kModelMargin = 1.03;
 inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split) {
-  RoutedPlan p{TILE_SMALL_W4, 1, 1};
-  double best = -1.0;
+  constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16};
   const TileCost* costs = dual ? kDualCosts : kPlainCosts;
   const int n_costs = dual ? (int)(sizeof(kDualCosts) / sizeof(TileCost)) : (int)(sizeof(kPlainCosts) / sizeof(TileCost));
-  const TileCost* pick = costs;
-  for (int i = 0; i < n_costs; ++i) {
-    const int64_t bm = tile_geom(costs[i].tile, dual).block_m;
-    const int64_t one = cdiv64(M, bm), both = M / bm + 1 + (M % bm > bm / 2 ? 1 : 0);
-    int s = 1;
-    const double t2 = dual ? routed_tile_time(costs[i], true, both, 2, M, n_out, K, 1) : best_split(costs[i], both, 2, M, n_out, K, split, 1, &s);
-    const double t1 = dual ? routed_tile_time(costs[i], true, one, 1, M, n_out, K, 1) : best_split(costs[i], one, 1, M, n_out, K, split, 1, &s);
-    const double t = t2 * t2 * t2 * t1 * t1;
+  const RoutedPlan rule = dual ? RoutedPlan{rule_tile(M, n_out, true, K), 1, 1} : rule_plan(M, n_out, K);
+  RoutedPlan p = rule;
+  double best = -1.0, keep = -1.0;
+  auto consider = [&](const TileCost& c, int s, int s_more) {
+    const double t = plan_score(c, dual, M, n_out, K, s, s_more);
     if (best < 0.0 || t < best) {
       best = t;
-      pick = costs + i;
+      p = {c.tile, s, s_more};
     }
+  };
+  for (int i = 0; i < n_costs; ++i) {
+    const TileCost& c = costs[i];
+    consider(c, 1, 1);
+    if (!dual && split && c.tile != TILE_256x256_W4) {
+      // the best factor for each M-tile count; either both are split or neither is
+      const int64_t less = cdiv64(M, tile_geom(c.tile, false).block_m);
+      int s = 0, s_more = 0;
+      double t_less = 0.0, t_more = 0.0;
+      for (const int k : kSplits) {
+        if (k == 1 || !routed_split_ok(K, k)) continue;
+        const double a = routed_tile_time(c, false, less, 2, M, n_out, K, k) * routed_tile_time(c, false, less, 1, M, n_out, K, k);
+        const double b = routed_tile_time(c, false, less + 1, 2, M, n_out, K, k);
+        if (s == 0 || a < t_less) { t_less = a; s = k; }
+        if (s_more == 0 || b < t_more) { t_more = b; s_more = k; }
+      }
+      if (s > 1) consider(c, s, s_more);
+    }
+    if (c.tile == rule.tile && (rule.splits == 1 || split)) keep = plan_score(c, dual, M, n_out, K, rule.splits, rule.splits_more);
   }
-  p.tile = pick->tile;
-  if (!dual) {
-    const int64_t tiles_m = cdiv64(M, tile_geom(p.tile, false).block_m);
-    best_split(*pick, tiles_m, 2, M, n_out, K, split, 1, &p.splits);
-    best_split(*pick, tiles_m + 1, 2, M, n_out, K, split, 1, &p.splits_more);
-    if (p.splits == 1 || p.splits_more == 1) p.splits = p.splits_more = 1;
-  }
-  return p;
+  constexpr double m = kModelMargin * kModelMargin * kModelMargin * kModelMargin * kModelMargin;  // a score is five times long
+  return keep > 0.0 && keep < best * m ? rule : p;
 }
 
 // The model is a pure function of the extents and takes a few microseconds of host time; every thread keeps the last plans.
@@ -230,17 +274,7 @@ inline int pick_routed_tile(int64_t M, int64_t n_out, bool dual, int64_t K = 0, 
       if (dual || t->splits == 1) return t->tile;
   }
   if (dual && model_applies(true, M, n_out, K)) return model_routed_plan(true, M, n_out, K, false).tile;
-  auto tiles = [&](int tile) {
-    const TileGeom t = tile_geom(tile, dual);
-    return cdiv64(M, t.block_m) * cdiv64(n_out, t.block_n_out);
-  };
-  // At least two full rounds of 256x256 tiles.  The SwiGLU kernel runs them with four wavefronts of
-  // 128x128 (a third fewer LDS reads per flop; measured 4 % faster at M = 32768, d = 4096, h = 14336); so do the
-  // single-weight kernels over a long contraction (1-2.5 % faster at K = 4096 and 14336, N = 4096, M >= 16384),
-  // which otherwise keep eight wavefronts of 128x64 (less exposed when K is short).
-  if (tiles(TILE_256x256_W8) >= 2 * kCus) return dual || (K >= 4096 && K % 64 == 0) ? TILE_256x256_W4 : TILE_256x256_W8;
-  if (tiles(TILE_128x128_W4) >= kCus) return TILE_128x128_W4;
-  return TILE_SMALL_W4;
+  return rule_tile(M, n_out, dual, K);
 }
 
 // The GEMMs the model above was not fitted for (the backward's dx GEMM over K-major weights): when the output yields fewer
@@ -285,16 +319,9 @@ inline int pick_routed_splits(int64_t M, int64_t n_out, int64_t K, int tile) {
   return best;
 }
 
-inline RoutedPlan pick_routed_plan(int64_t M, int64_t n_out, int64_t K, bool use_table = true, int op = TUNED_DOWN) {
+inline RoutedPlan rule_plan(int64_t M, int64_t n_out, int64_t K) {
   RoutedPlan p;
-  if (use_table && op != TUNED_NONE)
-    if (const TunedPlan* t = tuned_plan(op, M, K, n_out)) {
-      p.tile = t->tile;
-      p.splits = p.splits_more = (direct_contraction(K) && M < 65536 && n_out % 4 == 0) ? t->splits : 1;
-      return p;
-    }
-  if (op != TUNED_NONE && model_applies(false, M, n_out, K)) return model_routed_plan(false, M, n_out, K, M < 65536 && n_out % 4 == 0);
-  p.tile = pick_routed_tile(M, n_out, false, K, use_table, op);
+  p.tile = rule_tile(M, n_out, false, K);
   p.splits = p.splits_more = 1;
   if (M > 4096 || !direct_contraction(K)) return p;
   double best_cost = 0.0;
@@ -309,6 +336,18 @@ inline RoutedPlan pick_routed_plan(int64_t M, int64_t n_out, int64_t K, bool use
     }
   }
   return p;
+}
+
+inline RoutedPlan pick_routed_plan(int64_t M, int64_t n_out, int64_t K, bool use_table = true, int op = TUNED_DOWN) {
+  RoutedPlan p;
+  if (use_table && op != TUNED_NONE)
+    if (const TunedPlan* t = tuned_plan(op, M, K, n_out)) {
+      p.tile = t->tile;
+      p.splits = p.splits_more = (direct_contraction(K) && M < 65536 && n_out % 4 == 0) ? t->splits : 1;
+      return p;
+    }
+  if (op != TUNED_NONE && model_applies(false, M, n_out, K)) return model_routed_plan(false, M, n_out, K, M < 65536 && n_out % 4 == 0);
+  return rule_plan(M, n_out, K);
 }
 
 // Weight-gradient GEMM: two [R, Cc] outputs, contraction over about M / 2 rows each.

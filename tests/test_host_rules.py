@@ -70,3 +70,17 @@ def test_direct_launchers_refuse_short_contractions(refused, K):
     for form in range(10):
         for tile in (0, 1, 2, 3, 4, 6, 7) if form < 7 else (2,):
             assert refused(form, tile, 64, 64, K, 0), (form, tile)
+
+
+# Row counts at which the plan on the left took 1.2 ... 1.5 times as long as the rules' plan on the right (weights cold; us as
+# measured): unsplit 64x128 tiles of long contractions, 256-row tiles whose count passes a round for some masks.
+@pytest.mark.parametrize("dual,M,K,N,slow,us,rules_us", [
+    (False, 403, 11392, 4544, (7, 1), 127, 84), (False, 2127, 1216, 7104, (0, 1), 78, 52), (False, 466, 10112, 3968, (7, 1), 110, 75),
+    (False, 3448, 6208, 520, (3, 1), 57, 43), (False, 1571, 5376, 2472, (3, 1), 81, 62), (False, 333, 9344, 3456, (7, 1), 64, 49),
+    (False, 81, 3648, 4608, (7, 1), 30, 23), (False, 1247, 7040, 3264, (6, 1), 95, 76),
+    (True, 1059, 1248, 3256, (6, 1), 47, 31), (True, 791, 1088, 2240, (4, 1), 27, 19), (True, 88, 2552, 8232, (6, 1), 69, 48),
+    (True, 335, 4256, 9120, (1, 1), 109, 77), (True, 730, 1440, 4904, (1, 1), 52, 38)])
+def test_plans_measured_slow_are_not_chosen(dual, M, K, N, slow, us, rules_us):
+    from ffn_kernel_amd import _lib, tune
+    cfg = _lib.tile_config(_lib.OP_FFN_UP if dual else _lib.OP_LINEAR_FWD, M, K, N)
+    assert (tune._tile_id(cfg, dual), cfg["split_k"]) != slow
