@@ -1391,7 +1391,7 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
   const int total = routed_tile_count(n_vis, g.M, g.N, SBM, SBN);
   int L, sub_m = 0, sub_n = 0, split = 0, splits = 1, tail_slot = 0;
   if (g.tail_mode == 0) {
-    splits = routed_splits(n_vis, g.M, BM, g.splits, g.splits_more);
+    if (g.splits > 1) splits = routed_splits(n_vis, g.M, BM, g.splits, g.splits_more);
     L = xcd_tile_slot(total * splits, bid);
     if (splits > 1 && L >= 0) {  // range-major: neighbours in the order share panels, not a K range
       split = L / total;

@@ -48,13 +48,16 @@ __host__ __device__ inline TileCoord routed_tile_coord(int L, int n_vis, int M, 
     first_m = L / (group_m * tiles_n) * group_m;
     gsz = group_m < tiles_m - first_m ? group_m : tiles_m - first_m;
   } else {
-    const int row = L / tiles_n;
-    const int base = row < tiles_v ? 0 : tiles_v;                     // first M-tile of the modality
-    const int own = row < tiles_v ? tiles_v : tiles_m - tiles_v;      // ... and how many it has
-    const int groups = cdiv(own, group_m > kEvenGroupMin ? group_m : kEvenGroupMin);
-    const int s = ((row - base + 1) * groups - 1) / own;              // the super-group [s * own / groups, (s + 1) * own / groups) with this row
-    first_m = base + s * own / groups;
-    gsz = base + (s + 1) * own / groups - first_m;
+    const bool visual = L < tiles_v * tiles_n;
+    first_m = visual ? 0 : tiles_v;                         // first M-tile of the modality
+    gsz = visual ? tiles_v : tiles_m - tiles_v;             // ... and how many it has
+    const int cap = group_m > kEvenGroupMin ? group_m : kEvenGroupMin;
+    if (gsz > cap) {  // (divisions of a few hundred cycles each, ahead of a tile's first load)
+      const int own = gsz, base = first_m, groups = cdiv(own, cap);
+      const int s = ((L / tiles_n - base + 1) * groups - 1) / own;  // the super-group [s * own / groups, (s + 1) * own / groups) with this row
+      first_m = base + s * own / groups;
+      gsz = base + (s + 1) * own / groups - first_m;
+    }
   }
   L -= first_m * tiles_n;
   const int tile_m = first_m + L % gsz;
