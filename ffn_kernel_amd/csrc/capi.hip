@@ -259,10 +259,15 @@ int routed_tile(int64_t M, int64_t n_out, bool dual, int64_t K = 0, int op = TUN
   return f >= 0 ? f : pick_routed_tile(M, n_out, dual, K, use_tuned(), op);
 }
 
-// Whole extents off the dot kernels' 512-element slices at M <= 8: the dot-product streams lead once there is a stream to speak
-// of (MaskedFFN d=3200 h=8960 M=1 44.3 -> 33.6 us, M=8 both modalities 68.5 -> 61.6; d=5760 h=11520 M=4 131 -> 124; linear
-// K=3200 N=6016 19.3 -> 16.6); at d=1152 h=1408 a call is its launches and both take 33.5 us.
-constexpr int64_t kDotMinWeight = (int64_t)1 << 21;
+// Whole extents off the dot kernels' 512-element slices at M <= 8, against the LDS-transposed streams.  Up to four rows the
+// dot-product streams lead wherever there is a stream to speak of: 1410 drawn MaskedFFN calls of d * h >= 2^21 took 1.05 ... 1.7
+// times as long on the others, the worst of them 0.97.  Five rows and more are eight dot products per weight, and the cut
+// last slice weighs more: up to K * N = 2^23 and 4352 weight rows 1.1 ... 1.4 times (MaskedFFN and MaskedLinear, 200 calls);
+// past that 0.93 ... 1.1 (d=2176 h=7296 M=8 one modality: 29.0 us there, 39.3 here; K=1152 N=4864 M=8 8.9, 11.5).
+constexpr int64_t kDotMinWeight = (int64_t)1 << 21, kDotManyRowsWeight = (int64_t)1 << 23, kDotManyRowsN = 4352;
+bool whole_dot_pays(int64_t M, int64_t K, int64_t N) {
+  return K * N >= kDotMinWeight && (M <= 4 || stream_dot_ok((int)M, (int)K) || (K * N < kDotManyRowsWeight && N <= kDotManyRowsN));
+}
 bool use_stream_path(int64_t M, int64_t d, int64_t h) { return stream_shape_ok(M, d, h); }
 
 // Kernels of the two projections of a streamed forward: fragment-layout streams (extents under 1024), contiguous-row
@@ -298,7 +303,10 @@ StreamKinds stream_kinds(int64_t M, int64_t d, int64_t h) {
   if (!use_stream_path(M, d, h)) return stream_kinds_any(M, d, h);
   if (stream_dot_ok((int)M, (int)d) && stream_dot_ok((int)M, (int)h)) return {STREAM_DOT, STREAM_DOT};
   if (!stream_tile_ok((int)M, (int)d, (int)h)) return {STREAM_FRAG, STREAM_FRAG};
-  return d * h >= kDotMinWeight ? stream_kinds_any(M, d, h) : StreamKinds{STREAM_TILE, STREAM_TILE};
+  StreamKinds kinds = stream_kinds_any(M, d, h);
+  if (!whole_dot_pays(M, d, h)) kinds.up = STREAM_TILE;
+  if (!whole_dot_pays(M, h, d)) kinds.down = STREAM_TILE;
+  return kinds;
 }
 
 int down_splits(int64_t M, int64_t d, int64_t h) {
@@ -412,7 +420,7 @@ int linear_stream_kind(int64_t M, int64_t K, int64_t N) {
   if (M < 1 || M > kStreamMaxM || K > kMaxCols || N > kMaxCols) return 0;
   if (stream_dot_ok((int)M, (int)K)) return 1;
   const bool whole = stream_tile_down_ok((int)M, (int)N, (int)K);
-  if (stream_dot_any_ok((int)M, (int)K) && (whole ? K * N >= kDotMinWeight : forced_tile() < 0)) return 1;
+  if (stream_dot_any_ok((int)M, (int)K) && (whole ? whole_dot_pays(M, K, N) : forced_tile() < 0)) return 1;
   if (whole) return 2;
   return forced_tile() < 0 && stream_tile_down_any_ok((int)M, (int)N, (int)K) && ragged_stream_pays(M, K, N) ? 2 : 0;
 }
