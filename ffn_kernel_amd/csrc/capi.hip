@@ -281,9 +281,11 @@ StreamKinds stream_kinds_any(int64_t M, int64_t d, int64_t h) {
 int any_down_splits(int64_t M, int64_t d, int64_t h) {
   return stream_kinds_any(M, d, h).down == STREAM_DOT ? 1 : stream_tile_down_splits((int)M, (int)d, (int)h);
 }
-// Above 32 rows the tiled GEMMs are level or ahead once the weights are large and one modality is present (us, GEMM / streams):
-// d=5832 h=11784 M=64 133 / 139, d=4160 h=12480 M=64 77 / 86; below, d=3008 h=9024 M=40 84 / 72, d=2104 h=7176 M=64 51 / 39.
-bool ragged_stream_pays(int64_t M, int64_t K, int64_t N) { return M <= 32 || K * N <= ((int64_t)1 << 25); }
+// Above 32 rows, time on the tiled GEMMs over time on the streams, geometric means over 13000 drawn shapes (both modalities /
+// one).  33 - 48 rows: MaskedFFN 1.08 - 1.22 / 1.03 - 1.23 up to d * h = 2^25, past it 1.06 - 1.16 / 0.90 - 1.09; MaskedLinear
+// 1.11 - 1.20 / 1.00 - 1.09 and 1.09 / 0.97.  49 - 64 rows: MaskedFFN 1.04 - 1.20 / 0.98 - 1.17 and 1.01 / 0.95; MaskedLinear
+// 1.02 - 1.18 / 0.94 - 1.08 and 0.94 / 0.97.
+bool ragged_stream_pays(int64_t M, int64_t K, int64_t N) { return M <= 48 || K * N <= ((int64_t)1 << 25); }
 
 // Extents that are multiples of 8 but not of 128 run on the streams too, except in the forward that keeps its
 // pre-activations (ffnk_masked_ffn_can_save) and where the static entry point's scratch does not hold the partials: which

@@ -97,3 +97,12 @@ def test_dot_streams_where_they_lead(M, d, h, up_dot, down_dot):
         assert cfg["path"] == _lib.PATH_STREAM and (cfg["block_m"] == M) == dot
     lin = _lib.tile_config(_lib.OP_LINEAR_FWD, M, d, h)
     assert lin["path"] == _lib.PATH_STREAM and (lin["block_m"] == M) == up_dot
+
+
+# Ragged extents above 32 rows: streams up to 48 rows whatever the weights, up to 2^25 elements of them at 49 ... 64.
+@pytest.mark.parametrize("M,K,N,stream", [(33, 5832, 11784, True), (48, 5832, 11784, True), (49, 5832, 11784, False), (64, 5832, 11784, False),
+                                          (64, 4104, 8168, True), (48, 8168, 8168, True), (49, 8168, 8168, False)])
+def test_ragged_streams_where_they_lead(M, K, N, stream):
+    from ffn_kernel_amd import _lib
+    for op in (_lib.OP_LINEAR_FWD, _lib.OP_FFN_UP, _lib.OP_FFN_DOWN):
+        assert (_lib.tile_config(op, M, K, N)["path"] == _lib.PATH_STREAM) == stream
