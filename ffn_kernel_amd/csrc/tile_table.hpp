@@ -202,19 +202,31 @@ inline int rule_tile(int64_t M, int64_t n_out, bool dual, int64_t K) {
 
 inline RoutedPlan rule_plan(int64_t M, int64_t n_out, int64_t K);
 
-// The plan with the smallest score among all tiles and split factors.  `split`: the caller has a workspace for partials and
-// N % 4 == 0.  The rules' plan stays unless the model sees a gain of kModelMargin, near which its choice is as often the slower
+inline int max_splits(const RoutedPlan& p) { return p.splits > p.splits_more ? p.splits : p.splits_more; }
+// fp32 workspace of a plan: the partials of all rows where K is split for the whole GEMM, or the kTailSlots tiles of the split
+// tail of an unsplit 256x256 tile - only a launch of more than one round has one.
+inline size_t plan_partial_bytes(const RoutedPlan& p, int64_t M, int64_t n_out, int64_t K) {
+  if (p.splits > 1) return ws_align((size_t)max_splits(p) * M * n_out * 4);
+  return is_big_tile(p.tile) && direct_contraction(K) && (cdiv64(M, 256) + 1) * cdiv64(n_out, 256) > kCus
+             ? ws_align((size_t)kTailSlots * 256 * 256 * 4) : 0;
+}
+
+// The plan with the smallest score among all tiles and split factors.  `split`: N % 4 == 0 and the reduce pass takes M; `room`:
+// bytes that the caller has for partials.  The rules' plan stays unless the model sees a gain of kModelMargin, near which its choice is as often the slower
 // one (M = 8192, K = 2048, N = 1024, runs of both modalities: 256x256 tiles 58 us, the rules' 128x128 53): without it 6.0 % of
 // the SwiGLU and 2.1 % of the single-weight shapes ran more than 3 % slower than on the rules' plan, with it 5.1 % and 1.7 %.
 constexpr double kModelMargin = 1.03;
-inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split) {
+constexpr size_t kAnyRoom = ~(size_t)0;
+inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split, size_t room = kAnyRoom) {
   constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16};
   const TileCost* costs = dual ? kDualCosts : kPlainCosts;
   const int n_costs = dual ? (int)(sizeof(kDualCosts) / sizeof(TileCost)) : (int)(sizeof(kPlainCosts) / sizeof(TileCost));
   const RoutedPlan rule = dual ? RoutedPlan{rule_tile(M, n_out, true, K), 1, 1} : rule_plan(M, n_out, K);
-  RoutedPlan p = rule;
+  RoutedPlan p{TILE_SMALL_W4, 1, 1};
   double best = -1.0, keep = -1.0;
+  auto fits = [&](const RoutedPlan& q) { return dual || plan_partial_bytes(q, M, n_out, K) <= room; };
   auto consider = [&](const TileCost& c, int s, int s_more) {
+    if (!fits({c.tile, s, s_more})) return;
     const double t = plan_score(c, dual, M, n_out, K, s, s_more);
     if (best < 0.0 || t < best) {
       best = t;
@@ -230,7 +242,7 @@ inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_
       int s = 0, s_more = 0;
       double t_less = 0.0, t_more = 0.0;
       for (const int k : kSplits) {
-        if (k == 1 || !routed_split_ok(K, k)) continue;
+        if (k == 1 || !routed_split_ok(K, k) || !fits({c.tile, k, k})) continue;
         const double a = routed_tile_time(c, false, less, 2, M, n_out, K, k) * routed_tile_time(c, false, less, 1, M, n_out, K, k);
         const double b = routed_tile_time(c, false, less + 1, 2, M, n_out, K, k);
         if (s == 0 || a < t_less) { t_less = a; s = k; }
@@ -238,23 +250,24 @@ inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_
       }
       if (s > 1) consider(c, s, s_more);
     }
-    if (c.tile == rule.tile && (rule.splits == 1 || split)) keep = plan_score(c, dual, M, n_out, K, rule.splits, rule.splits_more);
+    if (c.tile == rule.tile && (rule.splits == 1 || split) && fits(rule)) keep = plan_score(c, dual, M, n_out, K, rule.splits, rule.splits_more);
   }
   constexpr double m = kModelMargin * kModelMargin * kModelMargin * kModelMargin * kModelMargin;  // a score is five times long
   return keep > 0.0 && keep < best * m ? rule : p;
 }
 
 // The model is a pure function of the extents and takes a few microseconds of host time; every thread keeps the last plans.
-inline RoutedPlan model_routed_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split) {
+inline RoutedPlan model_routed_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split, size_t room = kAnyRoom) {
   struct Entry {
     int64_t M = -1, n_out, K;
     bool dual, split;
+    size_t room;
     RoutedPlan plan;
   };
   static thread_local Entry memo[32];
   Entry& e = memo[(uint64_t)(M * 31 + n_out * 7 + K * 3 + (dual ? 1 : 0)) % 32];
-  if (e.M != M || e.n_out != n_out || e.K != K || e.dual != dual || e.split != split)
-    e = Entry{M, n_out, K, dual, split, compute_model_plan(dual, M, n_out, K, split)};
+  if (e.M != M || e.n_out != n_out || e.K != K || e.dual != dual || e.split != split || e.room != room)
+    e = Entry{M, n_out, K, dual, split, room, compute_model_plan(dual, M, n_out, K, split, room)};
   return e.plan;
 }
 

@@ -9,6 +9,21 @@ extern "C" {
 
 int hc_direct_ok(int64_t K, int64_t gathered_rows, int64_t lda, int64_t ldb) { return direct_ok(K, gathered_rows, lda, ldb); }
 
+// {tile, splits, splits_more} of a single-weight GEMM whose caller has `room` bytes for partials; what a plan needs; its score.
+void hc_plan(int64_t M, int64_t N, int64_t K, size_t room, int* out) {
+  const RoutedPlan p = compute_model_plan(false, M, N, K, true, room);
+  out[0] = p.tile; out[1] = p.splits; out[2] = p.splits_more;
+}
+size_t hc_plan_bytes(int64_t M, int64_t N, int64_t K, int tile, int splits, int splits_more) {
+  return plan_partial_bytes({tile, splits, splits_more}, M, N, K);
+}
+double hc_plan_score(int64_t M, int64_t N, int64_t K, int tile, int splits, int splits_more) {
+  for (const TileCost& c : kPlainCosts)
+    if (c.tile == tile && routed_split_ok(K, splits) && routed_split_ok(K, splits_more) && (tile != TILE_256x256_W4 || splits == 1))
+      return plan_score(c, false, M, N, K, splits, splits_more);
+  return -1.0;
+}
+
 // hipError_t of a launcher for operands it refuses before it launches anything (the operands are never read).
 // form: 0 linear, 1 SwiGLU, 2 down, 3 gather, 4 ... 6 the K-major forms of 0, 2 and 3, 7 and 8 the fused backward (two
 // stages, ring), 9 the same with the weight gradients in place.

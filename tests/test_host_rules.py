@@ -25,6 +25,9 @@ def rules(tmp_path_factory):
                    check=True, capture_output=True)
     lib = ctypes.CDLL(str(so))
     lib.hc_direct_ok.argtypes = [ctypes.c_int64] * 4
+    lib.hc_plan.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_size_t, ctypes.POINTER(ctypes.c_int)]
+    lib.hc_plan_bytes.argtypes = lib.hc_plan_score.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int] * 3
+    lib.hc_plan_bytes.restype, lib.hc_plan_score.restype = ctypes.c_size_t, ctypes.c_double
     return lib
 
 
@@ -106,3 +109,26 @@ def test_ragged_streams_where_they_lead(M, K, N, stream):
     from ffn_kernel_amd import _lib
     for op in (_lib.OP_LINEAR_FWD, _lib.OP_FFN_UP, _lib.OP_FFN_DOWN):
         assert (_lib.tile_config(op, M, K, N)["path"] == _lib.PATH_STREAM) == stream
+
+
+# The down projection of a MaskedFFN forward whose best plan does not fit the static scratch beside the intermediate (which
+# takes any extents off whole slabs there): the best of the plans that fit, with a smaller split factor or with none.
+@pytest.mark.parametrize("M,d,h", [(397, 6584, 22040), (1189, 3144, 10576), (1604, 2392, 6496), (763, 2824, 8224), (285, 5040, 14816), (1016, 1968, 6288)])
+def test_down_projection_plan_within_the_static_scratch(rules, M, d, h):
+    from ffn_kernel_amd import _lib, tune
+    fixed = _lib.workspace_bytes(_lib.OP_LINEAR_FWD, M, 72, 4) + -(-M * h * 2 // 256) * 256  # partition (a GEMM without partials) and intermediate
+    room = _lib.STATIC_SCRATCH_BYTES - fixed
+    plan = (ctypes.c_int * 3)()
+    rules.hc_plan(M, d, h, ctypes.c_size_t(-1).value, plan)
+    assert rules.hc_plan_bytes(M, d, h, *plan) > room  # the plan without a bound
+    cfg = _lib.tile_config(_lib.OP_FFN_DOWN, M, d, h)
+    rules.hc_plan(M, d, h, room, plan)
+    assert tuple(plan)[0] == tune._tile_id(cfg, False) and max(plan[1:]) == cfg["split_k"]
+    assert _lib.workspace_bytes(_lib.OP_FFN_FWD, M, d, h) <= _lib.STATIC_SCRATCH_BYTES
+    score = rules.hc_plan_score(M, d, h, *plan)
+    for tile in tune.TILES:
+        for s in range(1, 17):
+            for more in ({1} if s == 1 else range(2, 17)):
+                other = rules.hc_plan_score(M, d, h, tile, s, more)
+                if other > 0 and rules.hc_plan_bytes(M, d, h, tile, s, more) <= room:
+                    assert score <= other * 1.03 ** 5
