@@ -278,9 +278,6 @@ struct StreamKinds { int up, down; };
 StreamKinds stream_kinds_any(int64_t M, int64_t d, int64_t h) {
   return {stream_dot_any_ok((int)M, (int)d) ? STREAM_DOT : STREAM_TILE, stream_dot_any_ok((int)M, (int)h) ? STREAM_DOT : STREAM_TILE};
 }
-int any_down_splits(int64_t M, int64_t d, int64_t h) {
-  return stream_kinds_any(M, d, h).down == STREAM_DOT ? 1 : stream_tile_down_splits((int)M, (int)d, (int)h);
-}
 // Above 32 rows, time on the tiled GEMMs over time on the streams, geometric means over 13000 drawn shapes (both modalities /
 // one).  33 - 48 rows: MaskedFFN 1.08 - 1.22 / 1.03 - 1.23 up to d * h = 2^25, past it 1.06 - 1.16 / 0.90 - 1.09; MaskedLinear
 // 1.11 - 1.20 / 1.00 - 1.09 and 1.09 / 0.97.  49 - 64 rows: MaskedFFN 1.04 - 1.20 / 0.98 - 1.17 and 1.01 / 0.95; MaskedLinear
@@ -288,17 +285,12 @@ int any_down_splits(int64_t M, int64_t d, int64_t h) {
 bool ragged_stream_pays(int64_t M, int64_t K, int64_t N) { return M <= 48 || K * N <= ((int64_t)1 << 25); }
 
 // Extents that are multiples of 8 but not of 128 run on the streams too, except in the forward that keeps its
-// pre-activations (ffnk_masked_ffn_can_save) and where the static entry point's scratch does not hold the partials: which
-// shapes that entry point takes does not depend on this route.  Against the tiled GEMMs, which wait for a slab of weights
-// per barrier and have few workgroups at these sizes (us, GEMM -> streams): d=2104 h=7176 M=1 42.5 -> 29.6, d=5832
-// h=11784 M=3 194 -> 129, M=8 107 -> 80, M=13 200 -> 164; d=3008 h=9024 M=40 84 -> 72; linear K=2056 N=1544 M=1 22.0 -> 16.0.
+// pre-activations (ffnk_masked_ffn_can_save).  Against the tiled GEMMs, which wait for a slab of weights per barrier and have
+// few workgroups at these sizes (us, GEMM -> streams): d=2104 h=7176 M=1 42.5 -> 29.6, d=5832 h=11784 M=3 194 -> 129, M=8
+// 107 -> 80, M=13 200 -> 164; d=3008 h=9024 M=40 84 -> 72; linear K=2056 N=1544 M=1 22.0 -> 16.0.
 bool use_ragged_stream(int64_t M, int64_t d, int64_t h) {
-  if (M < 1 || M > kStreamMaxM || d > kMaxCols || h > kMaxCols || use_stream_path(M, d, h) || forced_tile() >= 0 ||
-      !stream_tile_any_ok((int)M, (int)d, (int)h) || !ragged_stream_pays(M, d, h))
-    return false;
-  const int s = any_down_splits(M, d, h);
-  return route_ws_bytes(M) + ws_align((size_t)M * round_up64(h, 8) * 2) + (s > 1 ? ws_align((size_t)s * M * d * 4) : 0) <=
-         (size_t)FFNK_STATIC_SCRATCH_BYTES;
+  return M >= 1 && M <= kStreamMaxM && d <= kMaxCols && h <= kMaxCols && !use_stream_path(M, d, h) && forced_tile() < 0 &&
+         stream_tile_any_ok((int)M, (int)d, (int)h) && ragged_stream_pays(M, d, h);
 }
 
 StreamKinds stream_kinds(int64_t M, int64_t d, int64_t h) {
@@ -341,18 +333,15 @@ RoutedPlan down_plan(int64_t M, int64_t d, int64_t h, int op = TUNED_DOWN) {
     p.splits = p.splits_more = fs;
   return p;
 }
-// The MaskedFFN forward's down projection.  The static entry point takes a fixed set of shapes, those whose plan by tile count
-// fits its scratch (rule_plan; off whole slabs any unsplit tile), and gives the bits of the others, so they all share one
-// plan: where the model's does not fit, the best of those that do (over 3104 drawn calls near the limit 5 % faster than the
-// model's plan with its factors cut, or else 128x128 tiles; single ones 0.7 ... 1.4 times).
-RoutedPlan ffn_down_plan(int64_t M, int64_t d, int64_t h) {
+// Workspace of the MaskedFFN forward without partials: the row partition and the [M, h] bf16 intermediate in routed order.
+size_t ffn_fixed_bytes(int64_t M, int64_t h) { return route_ws_bytes(M) + ws_align((size_t)M * round_up64(h, 8) * 2); }
+// The MaskedFFN forward's down projection: the model's plan where the caller's workspace is sized for it, the best of the plans
+// that fit where it is not (the static entry point).
+RoutedPlan ffn_down_plan(int64_t M, int64_t d, int64_t h, size_t ws_limit = kAnyRoom) {
   const RoutedPlan p = down_plan(M, d, h);
-  if (forced_tile() >= 0 || forced_splits() >= 1) return p;
-  const size_t fixed = route_ws_bytes(M) + ws_align((size_t)M * round_up64(h, 8) * 2);
-  if (fixed > (size_t)FFNK_STATIC_SCRATCH_BYTES) return p;
-  const size_t room = (size_t)FFNK_STATIC_SCRATCH_BYTES - fixed;
-  if (plan_partial_bytes(p, M, d, h) <= room || (h % 64 == 0 && plan_partial_bytes(rule_plan(M, d, h), M, d, h) > room)) return p;
-  return model_routed_plan(false, M, d, h, M < 65536 && d % 4 == 0, room);
+  const size_t fixed = ffn_fixed_bytes(M, h);
+  if (forced_tile() >= 0 || forced_splits() >= 1 || fixed >= ws_limit || plan_partial_bytes(p, M, d, h) <= ws_limit - fixed) return p;
+  return model_routed_plan(false, M, d, h, M < 65536 && d % 4 == 0, ws_limit - fixed);
 }
 // dx GEMM of the MaskedFFN backward: few output tiles over a 2h-long contraction, so K is split like the forward's
 // down projection when the fp32 partials fit `room`; an unsplit big tile wants room for its split tail instead.
@@ -422,13 +411,18 @@ RoutedPlan linear_plan(int64_t M, int64_t K, int64_t N) {
 size_t linear_partial_bytes(int64_t M, int64_t K, int64_t N) {
   return plan_partial_bytes(linear_plan(M, K, N), M, N, K);
 }
-int tiled_down_splits(int64_t M, int64_t d, int64_t h) {
-  return use_stream_path(M, d, h) ? 1 : max_splits(ffn_down_plan(M, d, h));
-}
-// fp32 partials of the tiled down projection: all rows when K is split for the whole GEMM, or the
-// kTailSlots tiles of the split tail when the 256x256 tile runs unsplit.
-size_t tiled_down_partial_bytes(int64_t M, int64_t d, int64_t h) {
-  return plan_partial_bytes(ffn_down_plan(M, d, h), M, d, h);
+// Workspace of the MaskedFFN forward with at most `ws_limit` bytes for it: partition, intermediate, and the fp32 partials of the
+// down projection where it is split (the larger need where strides or saved pre-activations send a ragged shape to the GEMMs).
+size_t ffn_fwd_bytes(int64_t M, int64_t d, int64_t h, size_t ws_limit = kAnyRoom) {
+  const size_t fixed = ffn_fixed_bytes(M, h);
+  if (use_stream_path(M, d, h)) return fixed + ws_align((size_t)down_splits(M, d, h) * M * d * 4);
+  size_t part = plan_partial_bytes(ffn_down_plan(M, d, h, ws_limit), M, d, h);
+  if (use_ragged_stream(M, d, h)) {
+    const int s = down_splits(M, d, h);  // (a forced factor may be larger than the rule's)
+    const size_t streamed = s > 1 ? ws_align((size_t)s * M * d * 4) : 0;
+    if (streamed > part) part = streamed;
+  }
+  return fixed + part;
 }
 
 // Split-K factor of the weight-gradient GEMM when it shares a launch with the dx GEMM (both on 128x128
@@ -527,18 +521,7 @@ size_t ffnk_workspace_bytes(int op, int64_t M, int64_t K, int64_t N) {
       }
       return route_ws_bytes(M) + linear_partial_bytes(M, K, N);
     }
-    case FFNK_OP_FFN_FWD: {
-      // perm + counts + the [M, h] bf16 intermediate in routed order (N = h) + the fp32 split-K
-      // partials of the down projection where it is split.
-      size_t part = use_stream_path(M, K, N) ? ws_align((size_t)down_splits(M, K, N) * M * K * 4) : tiled_down_partial_bytes(M, K, N);
-      if (use_ragged_stream(M, K, N)) {
-        // (a forced factor may be larger than the rule's)
-        const int s = down_splits(M, K, N);
-        const size_t streamed = s > 1 ? ws_align((size_t)s * M * K * 4) : 0;
-        if (streamed > part) part = streamed;
-      }
-      return route_ws_bytes(M) + ws_align((size_t)M * round_up64(N, 8) * 2) + part;
-    }
+    case FFNK_OP_FFN_FWD: return ffn_fwd_bytes(M, K, N);
     case FFNK_OP_LINEAR_BWD: {
       const BwdPlan a = plan_bwd(M, K, N, true), b = plan_bwd(M, K, N, false);
       return a.total > b.total ? a.total : b.total;
@@ -625,7 +608,7 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
   out->in_place = in_place ? 1 : 0;
   // 4: ring of four stages (128x128); 3: token panel in three stages, weight panel in two (single-weight 256x256 tiles)
   out->lds_stages = !(direct || in_place) ? 2 : tile == TILE_128x128_R4 ? 4 : (tile == TILE_128x256_R3 || tile == TILE_64x128_R3) ? 3 : (is_big_tile(tile) && !dual) ? 3 : 2;
-  if (op == FFNK_OP_FFN_DOWN && !stream) out->split_k = tiled_down_splits(M, K, N);
+  if (op == FFNK_OP_FFN_DOWN && !stream) out->split_k = max_splits(ffn_down_plan(M, K, N));
   if (op == FFNK_OP_LINEAR_FWD && linear_stream_kind(M, K, N)) {
     out->path = FFNK_PATH_STREAM;
     out->waves_m = out->waves_n = 1;
@@ -786,7 +769,7 @@ int ffn_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, cons
                  const uint16_t* U3, int64_t up_stride_k, int64_t up_stride_n, const uint16_t* W2, const uint16_t* U2,
                  int64_t down_stride_k, int64_t down_stride_n, const uint8_t* mask, uint16_t* out, int64_t out_stride_m,
                  uint16_t* pre, int64_t pre_stride_m, int64_t M, int64_t d, int64_t h, void* ws, size_t ws_bytes,
-                 void* stream_, void* const* events, const ffnk_routing_t* routing = nullptr) {
+                 void* stream_, void* const* events, const ffnk_routing_t* routing = nullptr, size_t ws_limit = kAnyRoom) {
   hipStream_t stream = (hipStream_t)stream_;
   auto mark = [&](int i) -> hipError_t {
     if (events && events[i]) return hipEventRecord((hipEvent_t)events[i], stream);
@@ -808,7 +791,7 @@ int ffn_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, cons
       return fail(FFNK_E_STRIDE, "pre_stride_m=%lld: need >= 2h, a multiple of 8, and 16-byte aligned rows",
                   (long long)pre_stride_m);
   }
-  const size_t need = ffnk_workspace_bytes(FFNK_OP_FFN_FWD, M, d, h);
+  const size_t need = ffn_fwd_bytes(M, d, h, ws_limit);
   if (ws_bytes < need || !ws) return fail(FFNK_E_WORKSPACE, "workspace %zu < %zu bytes", ws_bytes, need);
   if (!aligned16(ws)) return fail(FFNK_E_ALIGN, "workspace not 16-byte aligned");
 
@@ -895,7 +878,7 @@ int ffn_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, cons
   dn.perm = rt.perm; dn.counts = rt.counts;
   dn.M = (int)M; dn.N = (int)d; dn.K = (int)h; dn.group_m = plan_group_m(TUNED_DOWN, M, h, d);
   const bool dn_direct = direct_ok(h, 0, ldh, down_stride_n);
-  RoutedPlan dn_plan = ffn_down_plan(M, d, h);
+  RoutedPlan dn_plan = ffn_down_plan(M, d, h, ws_limit);
   if (!dn_direct) dn_plan.splits = dn_plan.splits_more = 1;
   float* partials = reinterpret_cast<float*>(wsb + r.bytes + ws_align((size_t)M * ldh * 2));
   if (dn_plan.splits > 1) {
@@ -932,7 +915,7 @@ int ffnk_masked_ffn_fwd_static(const uint16_t* x, int64_t x_stride_m, const uint
                                const uint8_t* mask, uint16_t* out, int64_t out_stride_m, int64_t M, int64_t d,
                                int64_t h, void* stream_) {
   if (int e = check_extents(M, d, h)) return e;
-  const size_t need = ffnk_workspace_bytes(FFNK_OP_FFN_FWD, M, d, h);
+  const size_t need = ffn_fwd_bytes(M, d, h, FFNK_STATIC_SCRATCH_BYTES);
   if (need > (size_t)FFNK_STATIC_SCRATCH_BYTES)
     return fail(FFNK_E_WORKSPACE, "ffnk_masked_ffn_fwd_static: M=%lld d=%lld h=%lld needs %zu bytes of scratch, the static "
                                   "buffer holds %zu; use ffnk_masked_ffn_fwd with a workspace",
@@ -944,7 +927,7 @@ int ffnk_masked_ffn_fwd_static(const uint16_t* x, int64_t x_stride_m, const uint
   // Nothing in the scratch has to start at zero: every region the forward reads (perm, counts, the
   // intermediate, the fp32 partials) is written by an earlier kernel of the same call.
   return ffn_fwd_impl(x, x_stride_m, W1, W3, U1, U3, up_stride_k, up_stride_n, W2, U2, down_stride_k, down_stride_n, mask,
-                      out, out_stride_m, nullptr, 0, M, d, h, ws, (size_t)FFNK_STATIC_SCRATCH_BYTES, stream_, nullptr);
+                      out, out_stride_m, nullptr, 0, M, d, h, ws, (size_t)FFNK_STATIC_SCRATCH_BYTES, stream_, nullptr, nullptr, FFNK_STATIC_SCRATCH_BYTES);
 }
 
 int ffnk_masked_ffn_fwd_routed(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, const uint16_t* W3,

@@ -224,9 +224,11 @@ FFNK_API int ffnk_masked_ffn_fwd_ev(const uint16_t* x, int64_t x_stride_m,
  * cannot allocate device memory around the call (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  It has no counterpart in the reference.  Scratch is a static
  * device array of FFNK_STATIC_SCRATCH_BYTES inside the library (each GPU the library runs on holds
- * its own copy until the process ends); shapes whose ffnk_workspace_bytes(FFNK_OP_FFN_FWD, M, d, h)
- * exceeds that return FFNK_E_WORKSPACE (at d = 4096, h = 14336 every M up to 256 fits).  Same
- * kernels and results as ffnk_masked_ffn_fwd.  All calls on one GPU share that GPU's array:
+ * its own copy until the process ends).  Where ffnk_workspace_bytes(FFNK_OP_FFN_FWD, M, d, h) is no more than that, the
+ * same kernels run as in ffnk_masked_ffn_fwd and give the same bits (at d = 4096, h = 14336 every M up to 256 fits);
+ * where only the down projection's partial sums do not fit beside the row partition and the [M, h] intermediate, the
+ * contraction is cut into fewer ranges or none, and results agree to fp32 summation order; shapes whose partition and
+ * intermediate exceed the array return FFNK_E_WORKSPACE.  All calls on one GPU share that GPU's array:
  * calls that overlap on one GPU (different streams or threads) race; calls on one stream are
  * ordered and safe.  The first call on each GPU looks the array's address up (no allocation); make
  * that call outside stream capture.

@@ -111,20 +111,20 @@ def test_ragged_streams_where_they_lead(M, K, N, stream):
         assert (_lib.tile_config(op, M, K, N)["path"] == _lib.PATH_STREAM) == stream
 
 
-# The down projection of a MaskedFFN forward whose best plan does not fit the static scratch beside the intermediate (which
-# takes any extents off whole slabs there): the best of the plans that fit, with a smaller split factor or with none.
-@pytest.mark.parametrize("M,d,h", [(397, 6584, 22040), (1189, 3144, 10576), (1604, 2392, 6496), (763, 2824, 8224), (285, 5040, 14816), (1016, 1968, 6288)])
+# The down projection of a MaskedFFN forward whose best plan does not fit the static scratch beside the intermediate, over whole
+# slabs and off them: that plan on a caller's workspace, the best of those that fit on the scratch.  (M=724: taken before.)
+@pytest.mark.parametrize("M,d,h", [(397, 6584, 22040), (1189, 3144, 10576), (1016, 1968, 6288), (724, 3584, 7488), (800, 4096, 14336), (301, 8192, 28672)])
 def test_down_projection_plan_within_the_static_scratch(rules, M, d, h):
     from ffn_kernel_amd import _lib, tune
     fixed = _lib.workspace_bytes(_lib.OP_LINEAR_FWD, M, 72, 4) + -(-M * h * 2 // 256) * 256  # partition (a GEMM without partials) and intermediate
     room = _lib.STATIC_SCRATCH_BYTES - fixed
     plan = (ctypes.c_int * 3)()
     rules.hc_plan(M, d, h, ctypes.c_size_t(-1).value, plan)
-    assert rules.hc_plan_bytes(M, d, h, *plan) > room  # the plan without a bound
     cfg = _lib.tile_config(_lib.OP_FFN_DOWN, M, d, h)
+    assert (tune._tile_id(cfg, False), cfg["split_k"]) == (plan[0], max(plan[1:]))
+    assert _lib.workspace_bytes(_lib.OP_FFN_FWD, M, d, h) == fixed + rules.hc_plan_bytes(M, d, h, *plan) > _lib.STATIC_SCRATCH_BYTES
     rules.hc_plan(M, d, h, room, plan)
-    assert tuple(plan)[0] == tune._tile_id(cfg, False) and max(plan[1:]) == cfg["split_k"]
-    assert _lib.workspace_bytes(_lib.OP_FFN_FWD, M, d, h) <= _lib.STATIC_SCRATCH_BYTES
+    assert rules.hc_plan_bytes(M, d, h, *plan) <= room
     score = rules.hc_plan_score(M, d, h, *plan)
     for tile in tune.TILES:
         for s in range(1, 17):
@@ -132,3 +132,14 @@ def test_down_projection_plan_within_the_static_scratch(rules, M, d, h):
                 other = rules.hc_plan_score(M, d, h, tile, s, more)
                 if other > 0 and rules.hc_plan_bytes(M, d, h, tile, s, more) <= room:
                     assert score <= other * 1.03 ** 5
+
+
+@pytest.mark.parametrize("M,d,h,taken", [(397, 6584, 22040, True), (724, 3584, 7488, True), (414, 4480, 13824, True), (256, 4096, 14336, True),
+                                         (1170, 4096, 14336, True), (1171, 4096, 14336, False), (32768, 4096, 14336, False)])
+def test_static_entry_point_takes_what_leaves_room_for_the_intermediate(M, d, h, taken):
+    """The size check comes before any pointer is looked at: FFNK_E_WORKSPACE, or FFNK_E_NULL for the missing output."""
+    from ffn_kernel_amd import _lib
+    rc = _lib.load().ffnk_masked_ffn_fwd_static(0, d, 0, 0, 0, 0, 1, d, 0, 0, 1, h, 0, 0, d, M, d, h, 0)
+    assert rc == (-1 if taken else -5)
+
+
