@@ -256,7 +256,14 @@ inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_
   return keep > 0.0 && keep < best * m ? rule : p;
 }
 
-// The model is a pure function of the extents and takes a few microseconds of host time; every thread keeps the last plans.
+// The model is a pure function of the extents and takes 5 us of host time (single-weight GEMMs); every thread keeps the last
+// plans.  Extents are mostly multiples of 32 and more: the slot comes from the top of a product, where all their bits arrive.
+inline unsigned model_plan_slot(bool dual, int64_t M, int64_t n_out, int64_t K, bool split, size_t room) {
+  constexpr uint64_t kMul = 0x9E3779B97F4A7C15ull;
+  uint64_t x = (uint64_t)M;
+  for (const uint64_t v : {(uint64_t)n_out, (uint64_t)K, (uint64_t)room * 4 + (dual ? 2 : 0) + (split ? 1 : 0)}) x = (x ^ (x >> 29)) * kMul + v;
+  return (unsigned)((x ^ (x >> 32)) * kMul >> 59);
+}
 inline RoutedPlan model_routed_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split, size_t room = kAnyRoom) {
   struct Entry {
     int64_t M = -1, n_out, K;
@@ -265,7 +272,7 @@ inline RoutedPlan model_routed_plan(bool dual, int64_t M, int64_t n_out, int64_t
     RoutedPlan plan;
   };
   static thread_local Entry memo[32];
-  Entry& e = memo[(uint64_t)(M * 31 + n_out * 7 + K * 3 + (dual ? 1 : 0)) % 32];
+  Entry& e = memo[model_plan_slot(dual, M, n_out, K, split, room)];
   if (e.M != M || e.n_out != n_out || e.K != K || e.dual != dual || e.split != split || e.room != room)
     e = Entry{M, n_out, K, dual, split, room, compute_model_plan(dual, M, n_out, K, split, room)};
   return e.plan;

@@ -24,6 +24,8 @@ double hc_plan_score(int64_t M, int64_t N, int64_t K, int tile, int splits, int 
   return -1.0;
 }
 
+unsigned hc_plan_slot(int dual, int64_t M, int64_t N, int64_t K) { return model_plan_slot(dual != 0, M, N, K, !dual, kAnyRoom); }
+
 // hipError_t of a launcher for operands it refuses before it launches anything (the operands are never read).
 // form: 0 linear, 1 SwiGLU, 2 down, 3 gather, 4 ... 6 the K-major forms of 0, 2 and 3, 7 and 8 the fused backward (two
 // stages, ring), 9 the same with the weight gradients in place.

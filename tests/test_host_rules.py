@@ -1,5 +1,6 @@
 """The rules that choose a kernel for a call, and the launchers' own checks, run on the host without a GPU."""
 import ctypes
+import random
 import shutil
 import subprocess
 from pathlib import Path
@@ -25,6 +26,7 @@ def rules(tmp_path_factory):
                    check=True, capture_output=True)
     lib = ctypes.CDLL(str(so))
     lib.hc_direct_ok.argtypes = [ctypes.c_int64] * 4
+    lib.hc_plan_slot.argtypes = [ctypes.c_int] + [ctypes.c_int64] * 3
     lib.hc_plan.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_size_t, ctypes.POINTER(ctypes.c_int)]
     lib.hc_plan_bytes.argtypes = lib.hc_plan_score.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int] * 3
     lib.hc_plan_bytes.restype, lib.hc_plan_score.restype = ctypes.c_size_t, ctypes.c_double
@@ -143,3 +145,12 @@ def test_static_entry_point_takes_what_leaves_room_for_the_intermediate(M, d, h,
     assert rc == (-1 if taken else -5)
 
 
+def test_plans_of_a_model_keep_their_own_slots(rules):
+    """The projections of a layer at one row count: eight keys thrown into 32 slots meet seven of them on average."""
+    gen = random.Random(7)
+    distinct = []
+    for _ in range(500):
+        M, widths = gen.randrange(65, 8192), [64 * gen.randrange(8, 256) for _ in range(4)]
+        keys = {(gen.random() < 0.25, gen.choice(widths), gen.choice(widths)) for _ in range(8)}
+        distinct.append(len({rules.hc_plan_slot(int(d), M, n, k) for d, n, k in keys}) / len(keys))
+    assert sum(distinct) / len(distinct) > 0.85
