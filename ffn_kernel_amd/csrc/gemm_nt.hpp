@@ -243,9 +243,10 @@ struct TileLanes {
 // the contraction, so slab 0 would start `pad` = -K mod 64 elements ahead of it.  It is loaded from the contraction's start
 // instead - `pad` elements on, one scalar offset, no lane out of bounds - and its last `pad` elements, which are slab 1's
 // first, are cleared once they have landed, every lane clearing the LDS slots it filled itself.  The steady loops are those
-// of K % 64 == 0.  Against the register-staged loop with its guard on every load, which ran these before: MaskedLinear
-// M = 3001, K = 2056, N = 1544 48.1 -> 39.5 us; MaskedFFN d = 2104, h = 7176, M = 594 174 -> 91 us, d = 2040, h = 6528,
-// M = 27470 2136 -> 1778 us, and in decode, where K splits over workgroups, d = 5832, h = 11784, M = 13 298 -> 110 us.
+// of K % 64 == 0.  Against the register-staged loop with its guard on every load, which ran these before (runs of both
+// modalities / one): MaskedLinear M = 3001, K = 2056, N = 1544 50.4 -> 41.2 / 49.4 -> 41.6 us; MaskedFFN d = 2104, h = 7176,
+// M = 594 206 -> 120 / 202 -> 109 us, d = 2040, h = 6528, M = 27470 2234 -> 1905 us, and at few rows, where K splits over
+// workgroups, d = 5832, h = 11784, M = 13 329 -> 208 / 306 -> 119 us (which runs on the weight streams).
 // ---------------------------------------------------------------------------------------------
 template <class Cfg>
 __device__ __forceinline__ void clear_head(const TileLanes<Cfg>& tl, int pad, uint8_t* a_panel, uint8_t* b_panel) {

@@ -52,8 +52,9 @@ constexpr int kTMaxM = 64;
 // overlaps the one before it; the last row block starts at Nrows - ROWS, streams rows of the block before it a second
 // time and stores its own only.  FORM_SPLIT_LINES: rows are no whole number of 128-byte lines, so neighbouring chunks of a
 // row share a line, and a non-temporal load gives that line up before its second half is wanted: plain loads take
-// 164 us instead of 179 (MaskedFFN d=5832 h=11784 M=13) and 32 instead of 34 (linear K=5000 N=6184 M=16).  Over whole
-// lines the non-temporal ones are the faster (d=4160 h=12480 M=48: 131 us against 140).
+// 171 us instead of 189 (MaskedFFN d=5832 h=11784 M=13, both modalities) and 34.7 instead of 37.8 (linear K=5000 N=6184 M=16,
+// both), 1.2 % and 1.6 % less over 2000 drawn calls each, none slower.  Over whole lines the non-temporal ones are the
+// faster (d=4160 h=12480 M=48, both: 131 us against 140).
 enum { FORM_WHOLE, FORM_RAGGED, FORM_SPLIT_LINES };
 
 struct TileJob {
