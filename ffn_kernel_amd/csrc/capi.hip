@@ -262,11 +262,12 @@ int routed_tile(int64_t M, int64_t n_out, bool dual, int64_t K = 0, int op = TUN
 // Whole extents off the dot kernels' 512-element slices at M <= 8, against the LDS-transposed streams.  Up to four rows the
 // dot-product streams lead wherever there is a stream to speak of: 1410 drawn MaskedFFN calls of d * h >= 2^21 took 1.05 ... 1.7
 // times as long on the others, the worst of them 0.97.  Five rows and more are eight dot products per weight, and the cut
-// last slice weighs more: up to K * N = 2^23 and 4352 weight rows 1.1 ... 1.4 times (MaskedFFN and MaskedLinear, 200 calls);
-// past that 0.93 ... 1.1 (d=2176 h=7296 M=8 one modality: 29.0 us there, 39.3 here; K=1152 N=4864 M=8 8.9, 11.5).
-constexpr int64_t kDotMinWeight = (int64_t)1 << 21, kDotManyRowsWeight = (int64_t)1 << 23, kDotManyRowsN = 4352;
+// last slice of a short contraction weighs more.  10317 drawn MaskedLinear calls, caches flushed, time on the others over time
+// here: up to 4096 weight rows 1.26 - 1.45 for K <= 4096, 0.98 - 1.24 above; more rows 0.82 - 1.03 up to K = 5120 (worst 0.60)
+// and 0.99 - 1.13 above it.
+constexpr int64_t kDotMinWeight = (int64_t)1 << 21, kDotManyRowsN = 4352, kDotManyRowsK = 5120;
 bool whole_dot_pays(int64_t M, int64_t K, int64_t N) {
-  return K * N >= kDotMinWeight && (M <= 4 || stream_dot_ok((int)M, (int)K) || (K * N < kDotManyRowsWeight && N <= kDotManyRowsN));
+  return K * N >= kDotMinWeight && (M <= 4 || stream_dot_ok((int)M, (int)K) || N <= kDotManyRowsN || K > kDotManyRowsK);
 }
 bool use_stream_path(int64_t M, int64_t d, int64_t h) { return stream_shape_ok(M, d, h); }
 
@@ -278,16 +279,18 @@ struct StreamKinds { int up, down; };
 StreamKinds stream_kinds_any(int64_t M, int64_t d, int64_t h) {
   return {stream_dot_any_ok((int)M, (int)d) ? STREAM_DOT : STREAM_TILE, stream_dot_any_ok((int)M, (int)h) ? STREAM_DOT : STREAM_TILE};
 }
-// Above 32 rows, time on the tiled GEMMs over time on the streams, geometric means over 13000 drawn shapes (both modalities /
-// one).  33 - 48 rows: MaskedFFN 1.08 - 1.22 / 1.03 - 1.23 up to d * h = 2^25, past it 1.06 - 1.16 / 0.90 - 1.09; MaskedLinear
-// 1.11 - 1.20 / 1.00 - 1.09 and 1.09 / 0.97.  49 - 64 rows: MaskedFFN 1.04 - 1.20 / 0.98 - 1.17 and 1.01 / 0.95; MaskedLinear
-// 1.02 - 1.18 / 0.94 - 1.08 and 0.94 / 0.97.
+// Above 32 rows, time on the tiled GEMMs over time on the streams, geometric means over 7000 drawn shapes, caches flushed (both
+// modalities / one), by K * N.  33 - 48 rows: MaskedFFN 1.06 - 1.24 / 1.15 - 1.31 up to 2^25, 1.07 - 1.13 / 0.95 - 1.08 past it;
+// MaskedLinear 1.10 - 1.24 / 1.01 - 1.14 and 1.06 - 1.11 / 0.95 - 0.97.  49 - 64 rows up to 2^25: MaskedFFN 1.04 - 1.20 /
+// 1.10 - 1.26, MaskedLinear 1.01 - 1.20 / 0.99 - 1.12; past it the GEMMs lead with one modality (d=5832 h=11784 M=64 133
+// against 139 us, d=4160 h=12480 77 against 86).
 bool ragged_stream_pays(int64_t M, int64_t K, int64_t N) { return M <= 48 || K * N <= ((int64_t)1 << 25); }
 
 // Extents that are multiples of 8 but not of 128 run on the streams too, except in the forward that keeps its
 // pre-activations (ffnk_masked_ffn_can_save).  Against the tiled GEMMs, which wait for a slab of weights per barrier and have
-// few workgroups at these sizes (us, GEMM -> streams): d=2104 h=7176 M=1 42.5 -> 29.6, d=5832 h=11784 M=3 194 -> 129, M=8
-// 107 -> 80, M=13 200 -> 164; d=3008 h=9024 M=40 84 -> 72; linear K=2056 N=1544 M=1 22.0 -> 16.0.
+// few workgroups at these sizes (us, GEMM -> streams, caches flushed): one modality d=2104 h=7176 M=1 46.6 -> 25.7, d=5832
+// h=11784 M=3 115 -> 81, M=8 116 -> 92, M=13 119 -> 115, linear K=2056 N=1544 M=1 14.0 -> 6.1; both modalities d=5832 h=11784
+// M=3 124 -> 84, M=8 206 -> 151, M=13 208 -> 171, d=3008 h=9024 M=40 94 -> 82.
 bool use_ragged_stream(int64_t M, int64_t d, int64_t h) {
   return M >= 1 && M <= kStreamMaxM && d <= kMaxCols && h <= kMaxCols && !use_stream_path(M, d, h) && forced_tile() < 0 &&
          stream_tile_any_ok((int)M, (int)d, (int)h) && ragged_stream_pays(M, d, h);

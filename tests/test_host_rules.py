@@ -91,10 +91,11 @@ def test_plans_measured_slow_are_not_chosen(dual, M, K, N, slow, us, rules_us):
     assert (tune._tile_id(cfg, dual), cfg["split_k"]) != slow
 
 
-# Whole extents off the dot kernels' 512-element slices: up to four rows the dot-product streams, above that only small weights
-# (the larger ones took up to 1.35 times as long on them: 29.0 us on the LDS-transposed streams at M = 8, d = 2176, h = 7296).
-@pytest.mark.parametrize("M,d,h,up_dot,down_dot", [(4, 2176, 7296, True, True), (5, 2176, 7296, False, False), (8, 2304, 7552, False, False),
-                                                   (8, 1152, 2176, True, True), (8, 1152, 4864, False, True), (8, 1024, 22528, True, False)])
+# Whole extents off the dot kernels' 512-element slices: up to four rows the dot-product streams, above that where the weight
+# rows are few or the contraction is long (others took up to 1.6 times as long on them).
+@pytest.mark.parametrize("M,d,h,up_dot,down_dot", [(4, 2176, 7296, True, True), (5, 2176, 7296, False, True), (8, 5120 - 128, 8320, False, True),
+                                                   (8, 5120 + 128, 8320, True, True), (8, 1152, 2176, True, True), (8, 1152, 4864, False, True),
+                                                   (8, 1024, 22528, True, False)])
 def test_dot_streams_where_they_lead(M, d, h, up_dot, down_dot):
     from ffn_kernel_amd import _lib
     for op, dot in ((_lib.OP_FFN_UP, up_dot), (_lib.OP_FFN_DOWN, down_dot)):
