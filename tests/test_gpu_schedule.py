@@ -104,9 +104,9 @@ def test_split_factor_by_row_tiles(dev, nv, K, N):
     assert_close(y, torch.where(mask[:, None], x.double() @ Wv.double().T, x.double() @ Wt.double().T).cpu(), "y")
 
 
-# The remainder of a launch on 256-row SwiGLU tiles: exactly half a round, one tile past it (another whole round), and one
-# tile past a round.  d = 64, h = 128 * tiles_n columns: 256 columns of the output hold one M-tile's row of tiles.
-@pytest.mark.parametrize("tiles_m,h", [(6, 64 * 128), (43, 9 * 128), (257, 128)])
+# The remainder of a launch on 256-row SwiGLU tiles: exactly half a round (256 + 128 tiles), one tile past it (256 + 129: another
+# whole round), and one tile past a round.  d = 64, h = 128 * tiles_n columns.
+@pytest.mark.parametrize("tiles_m,h", [(6, 64 * 128), (55, 7 * 128), (257, 128)])
 def test_whole_rounds_and_remainder(dev, forced, tiles_m, h):
     note(f"remainder of whole rounds: {tiles_m} M-tiles, h={h}")
     x, _, _, mask, _ = make_linear(dev, 256 * 2, 256 * (tiles_m - 2) - 5, 64, 8, seed=tiles_m)
