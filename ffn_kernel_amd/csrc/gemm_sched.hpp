@@ -37,7 +37,7 @@ __host__ __device__ inline int routed_splits(int n_vis, int M, int bm, int split
 // there, where the edges of the super-groups weigh more: super-groups of one modality's M-tiles only (two modalities share
 // no weight panel), at most group_m each (or kEvenGroupMin), the modality's M-tiles dealt evenly to them.  MaskedFFN at
 // d = 4096, h = 14336: forward at M = 1411 (three M-tiles of each modality) 507.5 -> 501.7 us, the backward's dx GEMM at
-// M = 4096 (eight of each; before, all sixteen were one super-group and 41 % of its L2 requests missed) 775 -> 706 us;
+// M = 4096 (eight of each; before, all sixteen were one super-group and 41 % of its L2 requests missed, now 33 %) 775 -> 706 us;
 // forward at M = 902, d = 7296 and at M = 4381, d = 1728: 1.0-1.5 % faster.  Dealt evenly at any size, M = 32768 lost 1.5 %.
 __host__ __device__ inline TileCoord routed_tile_coord(int L, int n_vis, int M, int N, int bm, int bn, int group_m) {
   const int tiles_v = cdiv(n_vis, bm);
@@ -74,8 +74,8 @@ __host__ __device__ inline TileCoord routed_tile_coord(int L, int n_vis, int M, 
 // (tiles of different ranges share nothing), and inside a range the order walks super-groups of kDwGroup row tiles column by
 // column, so the 32 tiles that an XCD runs at a time are 8 x 4 of them and load 12 panels per slab.  With the row tiles of
 // the whole output walked first, 32 of a long column ran at a time and loaded 33: the MaskedFFN's weight gradients at
-// M = 4096, d = 4096, h = 14336 missed L2 with 47 % of their requests and moved 4.5 TB/s; 500 -> 475 us per launch with
-// the super-groups, and MaskedLinear's backward at K = N = 2048 ... 6000 gains 1.5-3 %.
+// M = 4096, d = 4096, h = 14336 missed L2 with 47 % of their requests and moved 4.5 TB/s; with the super-groups 20 % miss,
+// 500 -> 475 us per launch, and MaskedLinear's backward at K = N = 2048 ... 6000 gains 1.5-3 %.
 constexpr int kDwGroup = 8;
 struct DwTileCoord {
   int grp, split, tile_r, tile_c;
