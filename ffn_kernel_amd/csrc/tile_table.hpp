@@ -85,15 +85,16 @@ struct RoutedPlan {
   int splits_more;
 };
 
-// Time of a direct-path GEMM in us, fitted to every tile and split factor at drawn shapes, weights and rows cold, one or both
-// modalities present: 8000 SwiGLU GEMMs (M = 33 ... 8192, d = 1024 ... 8192, h = 2 ... 3.5 d) and 8000 single-weight GEMMs
-// (M = 9 ... 12000, K = 128 ... 28672, N = 512 ... 8192), a quarter of them off multiples of 64; rms error 7 %.  A round of
-// the chip takes base + slabs * per_slab.  A partial round takes a part of it that depends on the workgroups of the fullest CU:
-// `first` (the launch is less than a round) and `again` (behind whole rounds) hold, per number of workgroups, the part just
-// past the number below it and the part when every CU has as many.  The weights arrive at `tbs` TB/s, token rows and results
-// at `io`; of the products' and the weights' times the smaller is partly hidden behind the larger.  Where K % 64 != 0 the rows
-// of a packed operand start anywhere in a 128-byte line and every 128-byte piece of a slab lies in two lines: a slab takes
-// `ragged` times as long, the more the fewer flops the tile has per byte it loads.
+// Time of a direct-path GEMM in us, fitted to every tile and split factor at drawn shapes, up to four sets of weights in turn
+// (600 MB of them, where the layer is that large), one or both modalities present: 8000 SwiGLU GEMMs (M = 33 ... 8192,
+// d = 1024 ... 8192, h = 2 ... 3.5 d) and 8000 single-weight GEMMs (M = 9 ... 12000, K = 128 ... 28672, N = 512 ... 8192), a
+// quarter of them off multiples of 64; rms error 7 %.  A round of the chip takes base + slabs * per_slab.  A partial round
+// takes a part of it that depends on the workgroups of the fullest CU: `first` (the launch is less than a round) and `again`
+// (behind whole rounds) hold, per number of workgroups, the part just past the number below it and the part when every CU
+// has as many.  The weights arrive at `tbs` TB/s, token rows and results at `io`; of the products' and the weights' times the
+// smaller is partly hidden behind the larger.  Where K % 64 != 0 the rows of a packed operand start anywhere in a 128-byte
+// line and every 128-byte piece of a slab lies in two lines: a slab takes `ragged` times as long, the more the fewer flops the
+// tile has per byte it loads.
 // Without the steps by workgroups per CU (a partial round taken as linear in them) and with the likelier M-tile count alone,
 // the plans were 2.8 % (single weight) and 4.7 % (SwiGLU) behind the best of each shape in the geometric mean, and more than
 // 8 % behind the rules by tile count below in 2.9 % and 5.1 % of 3900 / 4500 shapes that no fit has seen (K = 11392, N = 4544,
@@ -212,9 +213,10 @@ inline size_t plan_partial_bytes(const RoutedPlan& p, int64_t M, int64_t n_out, 
 }
 
 // The plan with the smallest score among all tiles and split factors.  `split`: N % 4 == 0 and the reduce pass takes M; `room`:
-// bytes that the caller has for partials.  The rules' plan stays unless the model sees a gain of kModelMargin, near which its choice is as often the slower
-// one (M = 8192, K = 2048, N = 1024, runs of both modalities: 256x256 tiles 58 us, the rules' 128x128 53): without it 6.0 % of
-// the SwiGLU and 2.1 % of the single-weight shapes ran more than 3 % slower than on the rules' plan, with it 5.1 % and 1.7 %.
+// bytes that the caller has for partials.  The rules' plan stays unless the model sees a gain of kModelMargin, near which its
+// choice is as often the slower one (MaskedFFN d = 1024, h = 2048, M = 8192, runs of both modalities: 133 us with the model's
+// 256x256 tiles under the down projection, 129 with the rules' 128x128): without it 6.0 % of the SwiGLU and 2.1 % of the
+// single-weight shapes ran more than 3 % slower than on the rules' plan, with it 5.1 % and 1.7 %.
 constexpr double kModelMargin = 1.03;
 constexpr size_t kAnyRoom = ~(size_t)0;
 inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split, size_t room = kAnyRoom) {
