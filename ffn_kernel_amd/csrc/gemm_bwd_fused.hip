@@ -14,8 +14,7 @@ static_assert(FusedDx::BM == RingDx::BM && FusedDx::BN_OUT == RingDx::BN_OUT && 
               "both forms of the fused launch cut the same tiles");
 
 int fused_bwd_dw_blocks(int R, int Cc, int splits) {
-  const int64_t total = 2LL * cdiv(R, FusedDw::BN) * cdiv(Cc, FusedDw::BM) * splits;
-  return (int)(cdiv64(total, kXcds) * kXcds);  // a multiple of the XCD count: the dx tiles keep their XCD mapping
+  return dw_blocks(cdiv(R, FusedDw::BN), cdiv(Cc, FusedDw::BM), splits);  // a multiple of the XCD count: the dx tiles keep their XCD mapping
 }
 
 hipError_t launch_fused_bwd(const GemmArgs& gx, const SplitKArgs& gw, bool ring, hipStream_t stream) {

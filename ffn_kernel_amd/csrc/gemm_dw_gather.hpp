@@ -29,13 +29,12 @@ __device__ __forceinline__ void gathered_dw_body(const GatherDwArgs& a, uint8_t*
 
   const int tiles_r = cdiv(g.R, BN);
   const int tiles_c = cdiv(g.Cc, BM);
-  const int L = xcd_tile_slot(2 * tiles_r * tiles_c * g.splits, bid);
-  if (L < 0) return;
-  const DwTileCoord tc = dw_tile_coord(L, tiles_r, tiles_c, g.splits);
+  const int n_vis = a.counts[0];
+  const DwTileCoord tc = dw_tile_coord(bid, tiles_r, tiles_c, g.splits, n_vis, g.M);
+  if (tc.grp < 0) return;
   const int grp = tc.grp, split = tc.split;
   const int r0 = tc.tile_r * BN, c0 = tc.tile_c * BM;
 
-  const int n_vis = a.counts[0];
   const int p_begin = grp == 0 ? 0 : n_vis;           // routed positions of the group: [p_begin, p_end)
   const int p_end = grp == 0 ? n_vis : g.M;
   const int nk_g = cdiv(p_end - p_begin, kBK);
@@ -190,8 +189,7 @@ __device__ __forceinline__ void gathered_dw_body(const GatherDwArgs& a, uint8_t*
 
 // Workgroups of a launch that runs the gathered weight-gradient GEMM: a multiple of the XCD count.
 inline int gathered_dw_blocks(int R, int Cc, int splits) {
-  const int64_t total = 2LL * cdiv(R, GatherDwCfg::BN) * cdiv(Cc, GatherDwCfg::BM) * splits;
-  return (int)(cdiv64(total, kXcds) * kXcds);
+  return dw_blocks(cdiv(R, GatherDwCfg::BN), cdiv(Cc, GatherDwCfg::BM), splits);
 }
 
 }  // namespace ffnk

@@ -25,7 +25,6 @@ namespace ffnk {
 
 constexpr int kBK = 64;          // K elements per LDS stage
 constexpr int kRowBytes = 128;   // kBK * sizeof(bf16)
-constexpr int kXcds = 8;         // MI355X: 8 XCDs, workgroups are dealt to them round-robin
 
 // ---------------------------------------------------------------------------------------------
 // LDS layout: a slab holds 128-byte rows (64 K elements).  The swizzle keeps every ds_read_b128 of
@@ -1594,12 +1593,11 @@ __device__ __forceinline__ void grouped_splitk_body(const SplitKArgs& g, uint8_t
   // row, which makes the fp32 partial stores 128-byte contiguous.
   const int tiles_r = cdiv(g.R, BN);
   const int tiles_c = cdiv(g.Cc, BM);
-  const int L = xcd_tile_slot(2 * tiles_r * tiles_c * g.splits, bid);
-  if (L < 0) return;
-  const DwTileCoord tc = dw_tile_coord(L, tiles_r, tiles_c, g.splits);
+  const int n_vis = g.counts[0];
+  const DwTileCoord tc = dw_tile_coord(bid, tiles_r, tiles_c, g.splits, n_vis, g.M);
+  if (tc.grp < 0) return;
   const int grp = tc.grp, split = tc.split, tile_r = tc.tile_r, tile_c = tc.tile_c;
 
-  const int n_vis = g.counts[0];
   const int vpad = (n_vis + 63) & ~63;
   const int k_begin_g = grp == 0 ? 0 : vpad;
   const int k_len_g = grp == 0 ? vpad : ((g.M - n_vis + 63) & ~63);
@@ -1707,8 +1705,7 @@ template <class Cfg>
 inline hipError_t launch_grouped_splitk(const SplitKArgs& g, hipStream_t stream) {
   if (g.R <= 0 || g.Cc <= 0 || g.splits <= 0) return hipSuccess;
   if (Cfg::B_KMAJOR && (g.R % 8 != 0 || g.lda * (kBK * 2) + 2 * (int64_t)g.R >= ((int64_t)1 << 32))) return hipErrorInvalidValue;
-  const int64_t total = 2LL * cdiv(g.R, Cfg::BN) * cdiv(g.Cc, Cfg::BM) * g.splits;
-  const int grid = (int)(cdiv64(total, kXcds) * kXcds);
+  const int grid = dw_blocks(cdiv(g.R, Cfg::BN), cdiv(g.Cc, Cfg::BM), g.splits);
   hipLaunchKernelGGL(grouped_splitk_kernel<Cfg>, dim3(grid), dim3(Cfg::NT), 0, stream, g);
   return hipGetLastError();
 }

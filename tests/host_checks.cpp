@@ -24,6 +24,13 @@ double hc_plan_score(int64_t M, int64_t N, int64_t K, int tile, int splits, int 
   return -1.0;
 }
 
+// Workgroups of a weight-gradient launch; the tile of workgroup `bid`: {group, range, row tile, column tile}, group -1: none.
+int hc_dw_blocks(int tiles_r, int tiles_c, int splits) { return dw_blocks(tiles_r, tiles_c, splits); }
+void hc_dw_tile(int bid, int tiles_r, int tiles_c, int splits, int n_vis, int M, int* out) {
+  const DwTileCoord t = dw_tile_coord(bid, tiles_r, tiles_c, splits, n_vis, M);
+  out[0] = t.grp; out[1] = t.split; out[2] = t.tile_r; out[3] = t.tile_c;
+}
+
 unsigned hc_plan_slot(int dual, int64_t M, int64_t N, int64_t K) { return model_plan_slot(dual != 0, M, N, K, !dual, kAnyRoom); }
 
 // hipError_t of a launcher for operands it refuses before it launches anything (the operands are never read).

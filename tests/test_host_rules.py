@@ -155,3 +155,23 @@ def test_plans_of_a_model_keep_their_own_slots(rules):
         keys = {(gen.random() < 0.25, gen.choice(widths), gen.choice(widths)) for _ in range(8)}
         distinct.append(len({rules.hc_plan_slot(int(d), M, n, k) for d, n, k in keys}) / len(keys))
     assert sum(distinct) / len(distinct) > 0.85
+
+
+# Weight-gradient launches: fewer tiles than XCDs, ragged super-groups, several K ranges; either group the larger one.
+@pytest.mark.parametrize("tiles_r,tiles_c,splits", [(1, 1, 1), (3, 2, 1), (9, 5, 1), (8, 8, 3), (17, 6, 2)])
+@pytest.mark.parametrize("n_vis,M", [(0, 70), (70, 70), (30, 70), (35, 70)])
+def test_weight_gradient_order(rules, tiles_r, tiles_c, splits, n_vis, M):
+    """Every tile of both groups once; every XCD an equal share of each group, the larger group first."""
+    t = (ctypes.c_int * 4)()
+    seen, per_xcd = [], {}
+    for b in range(rules.hc_dw_blocks(tiles_r, tiles_c, splits)):
+        rules.hc_dw_tile(b, tiles_r, tiles_c, splits, n_vis, M, t)
+        if t[0] >= 0:
+            seen.append(tuple(t))
+            per_xcd.setdefault(b % 8, []).append(t[0])
+    assert sorted(seen) == sorted((g, s, r, c) for g in (0, 1) for s in range(splits) for r in range(tiles_r) for c in range(tiles_c))
+    larger = 0 if 2 * n_vis >= M else 1
+    share = -(-tiles_r * tiles_c * splits // 8)
+    for groups in per_xcd.values():
+        assert groups.count(0) == groups.count(1) <= share
+        assert groups == sorted(groups, key=lambda g: g != larger)
