@@ -7,9 +7,9 @@
 namespace ffnk {
 
 using FusedDx = KMajorTiles<true, true>::T2;
-using FusedDw = PlainTiles<false, false, true>::T2;
+using FusedDw = DwTiles::T2;
 using RingDx = KMajorTiles<true, true>::T4;
-using RingDw = PlainTiles<false, false, true>::T4;
+using RingDw = DwTiles::T4;
 static_assert(FusedDx::BM == RingDx::BM && FusedDx::BN_OUT == RingDx::BN_OUT && FusedDw::BM == RingDw::BM && FusedDw::BN == RingDw::BN,
               "both forms of the fused launch cut the same tiles");
 

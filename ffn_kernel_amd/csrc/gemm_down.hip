@@ -10,7 +10,7 @@ hipError_t launch_down_gemm(int tile, bool direct, const GemmArgs& g, hipStream_
 }
 
 hipError_t launch_splitk_gemm(int tile, const SplitKArgs& g, hipStream_t stream) {
-  using Tiles = PlainTiles<false, false, true>;
+  using Tiles = DwTiles;
   switch (tile) {
     case TILE_256x256_W8: return launch_grouped_splitk<Tiles::T0>(g, stream);
     case TILE_256x256_W4: return launch_grouped_splitk<Tiles::T1>(g, stream);

@@ -15,7 +15,7 @@
 
 namespace ffnk {
 
-using GatherDwCfg = RoutedGemmCfg<128, 128, 2, 2, false, false, false, true, 8, true, 2>;
+using GatherDwCfg = RoutedGemmCfg<128, 128, 2, 2, false, false, false, true, 8, true, 2, true>;
 
 __device__ __forceinline__ void gathered_dw_body(const GatherDwArgs& a, uint8_t* lds, const int bid) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -133,7 +133,7 @@ __device__ __forceinline__ void gathered_dw_body(const GatherDwArgs& a, uint8_t*
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        acc[q / 2][q % 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fg[q % 2], fx[q / 2], acc[q / 2][q % 2], 0, 0, 0);
+        acc[q / 2][q % 2] = mfma32<Cfg>(fg[q % 2], fx[q / 2], acc[q / 2][q % 2]);
         __builtin_amdgcn_sched_barrier(0);
         if (q < 2) {
           if (rd) reads(cur ^ 1, stage_next, ks_next, q * 4, q * 4 + 4);
@@ -183,7 +183,7 @@ __device__ __forceinline__ void gathered_dw_body(const GatherDwArgs& a, uint8_t*
       if (kt + 1 < nk) body(1, kt + 1);
     }
   }
-  splitk_store<Cfg>(g, acc, grp, split, r0, c0, rl);
+  splitk_store<Cfg>(g, acc, grp, split, r0, c0, rl, lds);
 #endif
 }
 

@@ -92,7 +92,7 @@ struct KMajorB {
 };
 
 template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, bool DUAL_, bool GATHER_A_, bool SCATTER_C_,
-          bool DIRECT_, int GROUP_M_, bool B_KMAJOR_ = false, int STAGES_ = 2>
+          bool DIRECT_, int GROUP_M_, bool B_KMAJOR_ = false, int STAGES_ = 2, bool SWAP_ = false>
 struct RoutedGemmCfg {
   static constexpr int BM = BM_;            // token rows per tile
   static constexpr int BN = BN_;            // B rows held in LDS per tile (DUAL: half gate, half up)
@@ -106,6 +106,9 @@ struct RoutedGemmCfg {
   // Weight panels are [K, N] rows with N contiguous (the backward's view of a forward weight) and
   // are transposed on the way from LDS to the MFMA operand, see KMajorB.
   static constexpr bool B_KMAJOR = B_KMAJOR_;
+  // MFMA operands exchanged: a lane's runs of four consecutive results lie along the token panel's rows instead of the
+  // weight panel's (acc_col).  Same products in the same order.  Weight-gradient kernels, see splitk_store.
+  static constexpr bool SWAP = SWAP_;
   static constexpr int NWAVES = WAVES_M * WAVES_N;
   static constexpr int NT = NWAVES * kWave;
   static constexpr int BN_OUT = DUAL ? BN / 2 : BN;        // output columns per tile
@@ -167,12 +170,24 @@ __device__ __forceinline__ void zero_acc(typename Cfg::Acc (&acc)[Cfg::TM][Cfg::
 }
 
 // Where element v of an accumulator tile lies: the lane holds token row `lr` of the tile (the MFMA's
-// second operand) and, of the tile's weight rows (= output columns), those at acc_col(v, lh):
+// second operand) and, of the tile's weight rows (= output columns), those at acc_col(v, lh) - with Cfg::SWAP weight row `lr`
+// and the token rows at acc_col(v, lh):
 //   32x32x16: lr = lane & 31, lh = lane >> 5, columns 8 * (v / 4) + 4 * lh + v % 4
 //   16x16x32: lr = lane & 15, lh = lane >> 4, columns 4 * lh + v
 template <class Cfg>
 __device__ __forceinline__ constexpr int acc_col(int v, int lh) {
   return Cfg::MT == 32 ? 8 * (v / 4) + 4 * lh + (v % 4) : 4 * lh + v;
+}
+
+// acc += (weight fragment) x (token fragment), 32x32x16.
+template <class Cfg>
+__device__ __forceinline__ f32x16_t mfma32(bf16x8_t w, bf16x8_t t, f32x16_t acc) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (Cfg::SWAP) return __builtin_amdgcn_mfma_f32_32x32x16_bf16(t, w, acc, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, t, acc, 0, 0, 0);
+#else
+  return acc;
+#endif
 }
 
 constexpr int waitcnt_imm(int vm, int lgkm) {  // gfx9 s_waitcnt encoding, expcnt untouched
@@ -322,7 +337,7 @@ __device__ __forceinline__ void gemm_mainloop_staged(const TileLanes<Cfg>& tl,
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[j], af[i], acc[i][j], 0, 0, 0);
+          acc[i][j] = mfma32<Cfg>(bfr[j], af[i], acc[i][j]);
     }
   };
 
@@ -471,7 +486,7 @@ __device__ __forceinline__ void gemm_mainloop_slab_dma(const TileLanes<Cfg>& tl,
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[buf][j], fa[buf][i], acc[i][j], 0, 0, 0);
+        acc[i][j] = mfma32<Cfg>(fb[buf][j], fa[buf][i], acc[i][j]);
   };
 
   // ---- K-major weights: the same pipeline written out in source order.  The transposing reads are
@@ -521,7 +536,7 @@ __device__ __forceinline__ void gemm_mainloop_slab_dma(const TileLanes<Cfg>& tl,
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = 0; q < NM; ++q) {
-      acc[q / TN][q % TN] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[cur][q % TN], fa[cur][q / TN], acc[q / TN][q % TN], 0, 0, 0);
+      acc[q / TN][q % TN] = mfma32<Cfg>(fb[cur][q % TN], fa[cur][q / TN], acc[q / TN][q % TN]);
       __builtin_amdgcn_sched_barrier(0);
       if (q < RUSED) {
         if (reads) kmajor_reads(cur ^ 1, stage_next, step_next, q * RPS, (q + 1) * RPS);
@@ -836,10 +851,11 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
   constexpr bool kAccPinned = NWAVES == 4;
   auto mfma = [&](int buf, int m) {
     const int i = m / TN, j = m % TN;
+    const bf16x8_t p = Cfg::SWAP ? fa[i] : fb[buf][j], q = Cfg::SWAP ? fb[buf][j] : fa[i];
     if constexpr (kAccPinned)
-      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fb[buf][j]), "v"(fa[i]));
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(p), "v"(q));
     else
-      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[buf][j], fa[i], acc[i][j], 0, 0, 0);
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p, q, acc[i][j], 0, 0, 0);
   };
   // First K step of slab kt (weight stage u, token stage at a_cur): behind its MFMAs the fragments of the second
   // step, and loads: the last ones of slab kt + 1 (two-stage form), or the token panel of slab kt + 2 into the ring
@@ -1156,7 +1172,7 @@ __device__ __forceinline__ void gemm_mainloop_ring(const TileLanes<Cfg>& tl,
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = 0; q < NM; ++q) {
-      acc[q / TN][q % TN] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[cur][q % TN], fa[cur][q / TN], acc[q / TN][q % TN], 0, 0, 0);
+      acc[q / TN][q % TN] = mfma32<Cfg>(fb[cur][q % TN], fa[cur][q / TN], acc[q / TN][q % TN]);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int r = q * RPM; r < (q + 1) * RPM && r < ND; ++r)
@@ -1252,41 +1268,104 @@ __device__ __forceinline__ int xcd_tile_slot(int total, int bid) {
   return L < total ? L : -1;
 }
 
-// Epilogue shared by the routed kernels.  Per accumulator tile a lane holds token row lr and the output
-// columns acc_col(v, lh), i.e. runs of four consecutive columns (one 8-byte store each).
+// Results of a wave's tile on their way out, through the wave's own part of the K loop's LDS: written as the accumulators hold
+// them (runs of four results, 8 bytes, 16 or 32 rows per instruction), read and stored as 16 bytes per lane with every row of
+// the wave's tile - 64 to 256 bytes - in one instruction.  Stored from the accumulators, an instruction is 16 pieces of 32
+// bytes, and 256 CUs that store a tile at the same moment are bound by the pieces: a launch that only stores 256x256 tiles of a
+// [11008, 3584] matrix writes 2.75 TB/s in pieces of 32 bytes (8 a lane), 4.1 in 64, 5.0 in 128 and 5.2 in 512 (16 a lane).
+// Against stores from the accumulators: MaskedLinear M = 28536, K = 1536, N = 2624 237 -> 214 us, M = 16798, K = 960, N = 1536
+// 79.7 -> 74.1; forward + backward M = 1560, K = 4928, N = 7168 468 -> 434; MaskedFFN forward + backward d = 4096, h = 14336,
+// M = 4096 3725 -> 3582, d = 3456, h = 11072, M = 90 506 -> 418 (its weight gradients are nothing but stores: 67 -> 43 us each);
+// MaskedFFN forward d = 1024, h = 2048, M = 8192 137.3 -> 134.6, d = 4096, h = 14336, M = 32768 7883 -> 7826.
+// Rows are COLS results; 16-byte chunks are XORed with the row so that the 16 rows of a write and the rows of a read each
+// cover all banks.
 template <class Cfg>
-__device__ __forceinline__ void routed_epilogue(const GemmArgs& g, typename Cfg::Acc (&acc)[Cfg::TM][Cfg::TN], int row0,
-                                                int row_end, int n0, int wm, int wn, uint32_t lr, uint32_t lh) {
-  constexpr int TM = Cfg::TM, TN_OUT = Cfg::TN_OUT, MT = Cfg::MT, RUNS = Cfg::ACC_N / 4;
-  // A tile inside the matrix on every side, with 8-byte aligned runs: no guards, one row pointer per row group and
-  // the column of every store an immediate offset.  (The guarded form below costs a compare and two branches per
-  // run of four outputs - as many cycles as the SwiGLU itself.)
-  const bool inside = row0 + Cfg::BM <= row_end && n0 + Cfg::BN_OUT <= g.N && (reinterpret_cast<uintptr_t>(g.C) & 7) == 0 &&
-                      (g.ldc & 3) == 0 && !(Cfg::DUAL && g.C_pre != nullptr);
-  if (inside) {
-    int64_t dst[TM];
+struct WaveRows {
+  static constexpr int COLS = Cfg::SWAP ? Cfg::WTM : Cfg::WTN_OUT;  // contiguous results of an output row
+  static constexpr int ROWS = Cfg::SWAP ? Cfg::WTN_OUT : Cfg::WTM;
+  static constexpr int CH = COLS / 8;                               // 16-byte chunks per row
+  static constexpr int PER = kWave / CH;                            // rows per load and store
+  static constexpr int N = ROWS / PER;                              // loads and stores per lane
+  static constexpr int RP = 16 / CH;                                // rows that cover the banks once
+  static constexpr int BYTES = ROWS * COLS * 2;                     // of LDS per wave
+  static_assert(CH == 4 || CH == 8 || CH == 16, "rows of 32, 64 or 128 results");
+  static_assert(Cfg::NWAVES * BYTES <= Cfg::LDS_BYTES, "the K loop's stages hold the tile's results");
+
+  // value(i, j, q4): the run of four, packed, of accumulator tile acc[i][j].  The caller has put a barrier between the K loop's
+  // last LDS read and this; a wave reads what it wrote itself.
+  template <class Value>
+  static __device__ __forceinline__ void put(uint8_t* lds, int wave, uint32_t lr, uint32_t lh, Value&& value) {
+    constexpr int MT = Cfg::MT, RUNS = Cfg::ACC_N / 4;
+    uint8_t* row = lds + wave * BYTES + lr * (COLS * 2);
+    const uint32_t key = (lr / RP) & (CH - 1);
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int p = row0 + wm * Cfg::WTM + i * MT + (int)lr;
-      dst[i] = Cfg::SCATTER_C ? (int64_t)g.perm[p] : (int64_t)p;
-    }
+    for (int i = 0; i < Cfg::TM; ++i)
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      uint16_t* crow = g.C + dst[i] * g.ldc + (n0 + wn * Cfg::WTN_OUT + acc_col<Cfg>(0, (int)lh));
-#pragma unroll
-      for (int j = 0; j < TN_OUT; ++j) {
+      for (int j = 0; j < Cfg::TN_OUT; ++j)
 #pragma unroll
         for (int q4 = 0; q4 < RUNS; ++q4) {
-          float o[4];
+          const int rt = Cfg::SWAP ? j : i, ct = Cfg::SWAP ? i : j;
+          const uint32_t col = ct * MT + acc_col<Cfg>(4 * q4, (int)lh);
+          *reinterpret_cast<uint2*>(row + rt * MT * (COLS * 2) + (((col >> 3) ^ key) << 4) + (col & 4) * 2) = value(i, j, q4);
+        }
+  }
+  static __device__ __forceinline__ int row(int n, int lane) { return n * PER + lane / CH; }
+  static __device__ __forceinline__ int col(int lane) { return (lane % CH) * 8; }
+  static __device__ __forceinline__ uint4 get(const uint8_t* lds, int wave, int lane, int n) {
+    const uint32_t r = (uint32_t)row(n, lane);
+    return *reinterpret_cast<const uint4*>(lds + wave * BYTES + r * (COLS * 2) + ((((uint32_t)lane % CH) ^ ((r / RP) & (CH - 1))) << 4));
+  }
+};
+
+// Epilogue shared by the routed kernels.  Per accumulator tile a lane holds token row lr and the output
+// columns acc_col(v, lh), i.e. runs of four consecutive columns.
+template <class Cfg>
+__device__ __forceinline__ void routed_epilogue(const GemmArgs& g, typename Cfg::Acc (&acc)[Cfg::TM][Cfg::TN], int row0,
+                                                int row_end, int n0, const TileLanes<Cfg>& tl, uint8_t* lds) {
+  constexpr int TM = Cfg::TM, TN_OUT = Cfg::TN_OUT, MT = Cfg::MT, RUNS = Cfg::ACC_N / 4;
+  const int wm = tl.wm, wn = tl.wn;
+  const uint32_t lr = tl.lr, lh = tl.lh;
+  const bool save = Cfg::DUAL && g.C_pre != nullptr;  // uniform over the launch, like all of these
+  // Whole 16-byte chunks of the output's rows: through LDS, any edge a lane's own guard.
+  if (g.N % 8 == 0 && g.ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(g.C) & 15) == 0 &&
+      (!save || (g.ldc_pre % 8 == 0 && (reinterpret_cast<uintptr_t>(g.C_pre) & 15) == 0))) {
+    using W = WaveRows<Cfg>;
+    const int n = n0 + wn * Cfg::WTN_OUT + W::col(tl.lane), p0 = row0 + wm * Cfg::WTM;
+    // Output rows of the wave's tile, one per lane; a store's lanes fetch theirs from the lane that holds it.
+    int rows[cdiv(W::ROWS, kWave)];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if (Cfg::DUAL) o[e] = swiglu(acc[i][j][4 * q4 + e], acc[i][j + TN_OUT][4 * q4 + e]);
-            else o[e] = acc[i][j][4 * q4 + e];
-          }
-          uint2 v2;
-          v2.x = pack2bf(o[0], o[1]);
-          v2.y = pack2bf(o[2], o[3]);
-          *reinterpret_cast<uint2*>(crow + j * MT + (acc_col<Cfg>(4 * q4, 0) - acc_col<Cfg>(0, 0))) = v2;
+    for (int q = 0; q < cdiv(W::ROWS, kWave); ++q) {
+      const int p = p0 + q * kWave + tl.lane;
+      rows[q] = p < row_end && q * kWave + tl.lane < W::ROWS ? (Cfg::SCATTER_C ? g.perm[p] : p) : -1;
+    }
+    dma_wait_barrier<0>();  // every wave has read its last fragments
+    auto out = [&](uint16_t* base, int64_t ld) {
+#pragma unroll
+      for (int k = 0; k < W::N; ++k) {
+        const uint4 v = W::get(lds, tl.wave, tl.lane, k);
+        const int row = __shfl(rows[k * W::PER / kWave], k * W::PER % kWave + tl.lane / W::CH);
+        if (row >= 0 && n < g.N) *reinterpret_cast<uint4*>(base + row * ld + n) = v;
+      }
+    };
+    W::put(lds, tl.wave, lr, lh, [&](int i, int j, int q4) {
+      float o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (Cfg::DUAL) o[e] = swiglu(acc[i][j][4 * q4 + e], acc[i][j + TN_OUT][4 * q4 + e]);
+        else o[e] = acc[i][j][4 * q4 + e];
+      }
+      return make_uint2(pack2bf(o[0], o[1]), pack2bf(o[2], o[3]));
+    });
+    out(g.C, g.ldc);
+    if constexpr (Cfg::DUAL) {
+      if (save) {
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          W::put(lds, tl.wave, lr, lh, [&](int i, int j, int q4) {
+            const typename Cfg::Acc& t = acc[i][j + half * TN_OUT];
+            return make_uint2(pack2bf(t[4 * q4], t[4 * q4 + 1]), pack2bf(t[4 * q4 + 2], t[4 * q4 + 3]));
+          });
+          out(g.C_pre + (int64_t)half * g.N, g.ldc_pre);
         }
       }
     }
@@ -1493,7 +1572,7 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
       else
         routed_partial_store<Cfg>(g.P + (int64_t)split * g.M * g.N, g.N, g, acc, row0, row_end, n0, rl.wm, rl.wn, rl.lr, rl.lh);
     } else {
-      routed_epilogue<Cfg>(g, acc, row0, row_end, n0, rl.wm, rl.wn, rl.lr, rl.lh);
+      routed_epilogue<Cfg>(g, acc, row0, row_end, n0, rl, lds);
     }
   } else {
     constexpr int NJA = TileLanes<Cfg>::NJA, NJB = TileLanes<Cfg>::NJB;
@@ -1516,7 +1595,7 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
       pb[j] = (up ? g.B1[grp] : g.B0[grp]) + (int64_t)n * g.ldb + tl.c_log * 8;
     }
     gemm_mainloop_staged<Cfg>(tl, pa, pb, g.K, lds, acc);
-    routed_epilogue<Cfg>(g, acc, row0, row_end, n0, tl.wm, tl.wn, tl.lr, tl.lh);
+    routed_epilogue<Cfg>(g, acc, row0, row_end, n0, tl, lds);
   }
 }
 
@@ -1527,27 +1606,52 @@ __global__ __launch_bounds__(Cfg::NT) void routed_gemm_kernel(const GemmArgs g) 
 }
 
 // Store a weight-gradient tile: bf16 with the caller's strides when the contraction was not split, fp32 partials
-// otherwise.  acc[i][j][v]: BM-panel row (= output column c) c0 + wm*WTM + i*MT + lr;
-//                           BN-panel row (= output row r) r0 + wn*WTN + j*MT + acc_col(v, lh).
+// otherwise.  The BM-row panel's rows are the output's columns c, the BN-row panel's its rows r; a lane's runs of four
+// consecutive results lie along c with Cfg::SWAP and along r without, so that where the output is contiguous along that axis the
+// runs make up its rows (WaveRows) and a run of partials is one 16-byte store.
 template <class Cfg>
 __device__ __forceinline__ void splitk_store(const SplitKArgs& g, typename Cfg::Acc (&acc)[Cfg::TM][Cfg::TN], int grp, int split,
-                                             int r0, int c0, const TileLanes<Cfg>& rl) {
+                                             int r0, int c0, const TileLanes<Cfg>& rl, uint8_t* lds) {
   constexpr int TM = Cfg::TM, TN = Cfg::TN;
   constexpr int MT = Cfg::MT, RUNS = Cfg::ACC_N / 4;
-  if (g.out[0] != nullptr) {
-    // single split: the sums are complete, store bf16 with the caller's strides
-    uint16_t* out = g.out[grp];
+  const bool direct = g.out[0] != nullptr;  // single split: the sums are complete
+  uint16_t* out = g.out[grp];
+  const int64_t run_ld = Cfg::SWAP ? g.out_sr : g.out_sc;  // from one output row (of contiguous runs) to the next
+  if (direct && (Cfg::SWAP ? g.out_sc : g.out_sr) == 1 && run_ld % 8 == 0 && (Cfg::SWAP ? g.Cc : g.R) % 8 == 0 &&
+      (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
+    using W = WaveRows<Cfg>;
+    const int rows = Cfg::SWAP ? g.R : g.Cc, cols = Cfg::SWAP ? g.Cc : g.R;
+    const int row_w = (Cfg::SWAP ? r0 + rl.wn * Cfg::WTN_OUT : c0 + rl.wm * Cfg::WTM);
+    const int col = (Cfg::SWAP ? c0 + rl.wm * Cfg::WTM : r0 + rl.wn * Cfg::WTN_OUT) + W::col(rl.lane);
+    dma_wait_barrier<0>();  // every wave has read its last fragments
+    W::put(lds, rl.wave, rl.lr, rl.lh, [&](int i, int j, int q4) {
+      const typename Cfg::Acc& t = acc[i][j];
+      return make_uint2(pack2bf(t[4 * q4], t[4 * q4 + 1]), pack2bf(t[4 * q4 + 2], t[4 * q4 + 3]));
+    });
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int c = c0 + rl.wm * Cfg::WTM + i * MT + (int)rl.lr;
-      if (c >= g.Cc) continue;
+    for (int k = 0; k < W::N; ++k) {
+      const int row = row_w + W::row(k, rl.lane);
+      const uint4 v = W::get(lds, rl.wave, rl.lane, k);
+      if (row < rows && col < cols) *reinterpret_cast<uint4*>(out + row * run_ld + col) = v;
+    }
+    return;
+  }
+  float* P = g.P + ((int64_t)(grp * g.splits + split)) * g.R * g.Cc;
+  const int64_t run_stride = Cfg::SWAP ? g.out_sc : g.out_sr;
+  const int lr = (int)rl.lr, lh = (int)rl.lh;
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
+  for (int i = 0; i < TM; ++i) {
 #pragma unroll
-        for (int q4 = 0; q4 < RUNS; ++q4) {
-          const int r = r0 + rl.wn * Cfg::WTN_OUT + j * MT + acc_col<Cfg>(4 * q4, (int)rl.lh);
+    for (int j = 0; j < TN; ++j) {
+#pragma unroll
+      for (int q4 = 0; q4 < RUNS; ++q4) {
+        const int run = acc_col<Cfg>(4 * q4, lh);
+        const int c = c0 + rl.wm * Cfg::WTM + i * MT + (Cfg::SWAP ? run : lr);
+        const int r = r0 + rl.wn * Cfg::WTN_OUT + j * MT + (Cfg::SWAP ? lr : run);
+        const int left = Cfg::SWAP ? (r < g.R ? g.Cc - c : 0) : (c < g.Cc ? g.R - r : 0);  // results of the run inside the output
+        if (direct) {
           uint16_t* dst = out + (int64_t)r * g.out_sr + (int64_t)c * g.out_sc;
-          if (g.out_sr == 1 && r + 3 < g.R && (reinterpret_cast<uintptr_t>(dst) & 7) == 0) {
+          if (run_stride == 1 && left > 3 && (reinterpret_cast<uintptr_t>(dst) & 7) == 0) {
             uint2 v2;
             v2.x = pack2bf(acc[i][j][4 * q4], acc[i][j][4 * q4 + 1]);
             v2.y = pack2bf(acc[i][j][4 * q4 + 2], acc[i][j][4 * q4 + 3]);
@@ -1555,24 +1659,18 @@ __device__ __forceinline__ void splitk_store(const SplitKArgs& g, typename Cfg::
           } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-              if (r + e < g.R) dst[(int64_t)e * g.out_sr] = f2bf(acc[i][j][4 * q4 + e]);  // out_sc == 1: MT lanes -> 2 MT contiguous bytes
+              if (e < left) dst[(int64_t)e * run_stride] = f2bf(acc[i][j][4 * q4 + e]);  // the other axis contiguous: MT lanes -> 2 MT bytes
+          }
+        } else {
+          float* dst = P + (int64_t)r * g.Cc + c;
+          if (Cfg::SWAP && left > 3 && (g.Cc & 3) == 0) {
+            *reinterpret_cast<float4*>(dst) = make_float4(acc[i][j][4 * q4], acc[i][j][4 * q4 + 1], acc[i][j][4 * q4 + 2], acc[i][j][4 * q4 + 3]);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (e < left) dst[(int64_t)e * (Cfg::SWAP ? 1 : g.Cc)] = acc[i][j][4 * q4 + e];
           }
         }
-      }
-    }
-    return;
-  }
-  float* P = g.P + ((int64_t)(grp * g.splits + split)) * g.R * g.Cc;
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int c = c0 + rl.wm * Cfg::WTM + i * MT + (int)rl.lr;
-    if (c >= g.Cc) continue;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-#pragma unroll
-      for (int v = 0; v < Cfg::ACC_N; ++v) {
-        const int r = r0 + rl.wn * Cfg::WTN_OUT + j * MT + acc_col<Cfg>(v, (int)rl.lh);
-        if (r < g.R) P[(int64_t)r * g.Cc + c] = acc[i][j][v];  // MT lanes -> MT consecutive floats
       }
     }
   }
@@ -1653,7 +1751,7 @@ __device__ __forceinline__ void grouped_splitk_body(const SplitKArgs& g, uint8_t
     zero_acc<Cfg>(acc);  // a split without slabs (e.g. an empty modality) contributes exact zeros
   }
 
-  splitk_store<Cfg>(g, acc, grp, split, r0, c0, rl);
+  splitk_store<Cfg>(g, acc, grp, split, r0, c0, rl, lds);
 }
 
 template <class Cfg>

@@ -28,6 +28,23 @@ struct PlainTiles {
   using T7 = std::conditional_t<DIRECT, RoutedGemmCfg<64, 128, 2, 2, false, GATHER, SCATTER, true, kGroupMPlain, false, 3>, T3>;
 };
 
+// Weight-gradient tiles on transposed operands: an output that is contiguous along its columns (see splitk_store).
+struct DwTiles {
+  using T0 = RoutedGemmCfg<256, 256, 2, 4, false, false, false, true, kGroupMPlain, false, kBigStagesPlain, true>;
+  using T1 = RoutedGemmCfg<256, 256, 2, 2, false, false, false, true, kGroupMPlain, false, kBigStagesPlain, true>;
+  using T2 = RoutedGemmCfg<128, 128, 2, 2, false, false, false, true, kGroupMPlain, false, 2, true>;
+  using T3 = RoutedGemmCfg<128, 64, 2, 2, false, false, false, true, kGroupMPlain, false, 2, true>;
+  using T4 = RoutedGemmCfg<128, 128, 2, 2, false, false, false, true, kGroupMPlain, false, 4, true>;
+};
+// ... with one operand read in place.
+template <bool SWAP>
+struct KMajorDwTiles {
+  using T0 = RoutedGemmCfg<256, 256, 2, 4, false, false, false, true, kGroupM, true, kBigStagesPlain, SWAP>;
+  using T1 = RoutedGemmCfg<256, 256, 2, 2, false, false, false, true, kGroupM, true, kBigStagesPlain, SWAP>;
+  using T2 = RoutedGemmCfg<128, 128, 2, 2, false, false, false, true, kGroupM, true, 2, SWAP>;
+  using T3 = RoutedGemmCfg<128, 64, 2, 2, false, false, false, true, kGroupM, true, 2, SWAP>;
+};
+
 // The same tiles over K-major weights ([K, N] rows, N contiguous; direct path only).
 template <bool GATHER, bool SCATTER>
 struct KMajorTiles {
