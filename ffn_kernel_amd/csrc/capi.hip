@@ -346,18 +346,28 @@ RoutedPlan ffn_down_plan(int64_t M, int64_t d, int64_t h, size_t ws_limit = kAny
   if (forced_tile() >= 0 || forced_splits() >= 1 || fixed >= ws_limit || plan_partial_bytes(p, M, d, h) <= ws_limit - fixed) return p;
   return model_routed_plan(false, M, d, h, M < 65536 && d % 4 == 0, ws_limit - fixed);
 }
+// Tile of an unsplit GEMM of the backward: the time model's, although it was fitted to row-major weights - over 2320 drawn GEMMs
+// on K-major weights (M = 65 ... 16384, up to two rounds of 256x256 tiles and past them) its plans are 1.8 % (MaskedLinear's
+// dx), 2.9 % (dh) and 3.0 % (the feed-forward dx, K split) behind the best of all tiles and split factors in the geometric mean,
+// the rules by tile count, which these GEMMs ran on before, 32, 23 and 17 %.
+int bwd_tile(int64_t M, int64_t n_out, int64_t K, bool direct) {
+  if (forced_tile() < 0 && direct && model_applies(false, M, n_out, K)) return model_routed_plan(false, M, n_out, K, false).tile;
+  return routed_tile(M, n_out, false, 0, TUNED_NONE);
+}
 // dx GEMM of the MaskedFFN backward: few output tiles over a 2h-long contraction, so K is split like the forward's
 // down projection when the fp32 partials fit `room`; an unsplit big tile wants room for its split tail instead.
 RoutedPlan ffn_bwd_dx_plan(int64_t M, int64_t d, int64_t h, bool dx_direct, size_t room, size_t* need) {
-  // Rules and cost model only: the measured plans are timings of other kernels (the forward's down
-  // projection reads K-contiguous weights through another loop).
+  // No measured plans: they are timings of other kernels (the forward's down projection reads K-contiguous weights through
+  // another loop).
   RoutedPlan dxp = down_plan(M, d, 2 * h, TUNED_NONE);
-  if (!dx_direct || (size_t)dxp.splits * M * d * 4 > room) {
+  if (forced_tile() < 0 && forced_splits() < 1 && dx_direct && model_applies(false, M, d, 2 * h))
+    dxp = model_routed_plan(false, M, d, 2 * h, M < 65536, room);
+  if (!dx_direct || (size_t)max_splits(dxp) * M * d * 4 > room) {
     dxp.splits = dxp.splits_more = 1;
     dxp.tile = routed_tile(M, d, false, 0, TUNED_NONE);
   }
   size_t n = 0;
-  if (dxp.splits > 1) n = (size_t)dxp.splits * M * d * 4;
+  if (dxp.splits > 1) n = (size_t)max_splits(dxp) * M * d * 4;
   else if (dx_direct && is_big_tile(dxp.tile) && (size_t)kTailSlots * 256 * 256 * 4 <= room) n = (size_t)kTailSlots * 256 * 256 * 4;
   if (need) *need = n;
   return dxp;
@@ -475,6 +485,12 @@ bool gather_dw_ok(int64_t M, int64_t K, int64_t N, const void* g, int64_t g_stri
          M * g_stride_m * 2 + 2 * N < k4g && M * x_stride_m * 2 + 2 * K < k4g &&
          ((reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(x)) & 15) == 0;
 }
+// Tile of the dx GEMM in a launch of its own.
+int linear_dx_tile(int64_t M, int64_t K, int64_t N, bool direct) {
+  const int f = forced_tile();  // a forced ring tile of three stages stands for the two-stage tile here, as in the weight-gradient GEMM
+  if (f >= 0) return f == TILE_128x256_R3 ? TILE_128x128_W4 : f == TILE_64x128_R3 ? TILE_SMALL_W4 : f;
+  return bwd_tile(M, K, N, direct);
+}
 // One launch for both GEMMs: the dx GEMM on a 128x128 tile over weights read in place, and the weight gradients on the
 // same tile (the in-place form has no other).
 bool bwd_is_fused(int64_t M, int64_t K, const BwdPlan& p, bool w_kmajor, bool in_place) {
@@ -566,14 +582,20 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
     case FFNK_OP_FFN_UP: tile = routed_tile(M, N, true, K); dual = true; contraction = K; break;
     case FFNK_OP_FFN_DOWN: tile = ffn_down_plan(M, K, N).tile; contraction = N; break;  // out cols = d = K, contraction h = N
     case FFNK_OP_LINEAR_BWD:
-    case FFNK_OP_BWD_DX: tile = routed_tile(M, K, false, 0, TUNED_NONE); contraction = N; break;
+    case FFNK_OP_BWD_DX:
     case FFNK_OP_BWD_DW: {
       // As launched for the reference's layout (nn.Linear.weight.T views, contiguous g): weights read in place.
       const BwdPlan bp = plan_bwd(M, K, N, true);
       const bool w_kmajor = K >= 8 && K % 8 == 0 && direct_ok(N, M, N, 8);
       in_place = bp.gather && gather_dw_ok(M, K, N, nullptr, N, nullptr, K);
-      tile = in_place ? TILE_128x128_W4 : bp.tc.tile; contraction = M;
-      splits = bwd_dw_launch_splits(M, K, N, bp, bwd_is_fused(M, K, bp, w_kmajor, in_place));
+      const bool fused = bwd_is_fused(M, K, bp, w_kmajor, in_place);
+      if (op == FFNK_OP_BWD_DW) {
+        tile = in_place ? TILE_128x128_W4 : bp.tc.tile; contraction = M;
+        splits = bwd_dw_launch_splits(M, K, N, bp, fused);
+      } else {
+        tile = fused ? routed_tile(M, K, false, 0, TUNED_NONE) : linear_dx_tile(M, K, N, w_kmajor); contraction = N;
+        in_place = false;
+      }
       break;
     }
     default: return fail(FFNK_E_OP, "unknown op %d", op);
@@ -582,7 +604,7 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
   const bool direct = op == FFNK_OP_BWD_DW ? contraction > 0 : direct_contraction(contraction);
   // Kernels without the two ring tiles of three stages run the two-stage tiles in their place.
   const bool kmajor_dx = op == FFNK_OP_LINEAR_BWD || op == FFNK_OP_BWD_DX;
-  if (!direct || kmajor_dx || op == FFNK_OP_BWD_DW) {
+  if (!direct || op == FFNK_OP_BWD_DW) {
     if (tile == TILE_128x256_R3) tile = TILE_128x128_W4;
     if (tile == TILE_64x128_R3) tile = op == FFNK_OP_BWD_DW ? TILE_128x128_W4 : TILE_SMALL_W4;
   }
@@ -1025,14 +1047,15 @@ int ffnk_masked_linear_bwd_routed(const uint16_t* g, int64_t g_stride_m, const u
   a.C = dx; a.ldc = dx_stride_m;
   a.perm = rt.perm; a.counts = rt.counts;
   a.M = (int)M; a.N = (int)K; a.K = (int)N; a.group_m = plan_group_m(TUNED_NONE, M, N, K);
-  const int dx_tile = routed_tile(M, K, false, 0, TUNED_NONE);
+  const bool dx_direct = w_kmajor || direct_ok(N, M, g_stride_m, ldw);
   // Both GEMMs on the 128x128 tile and the weights readable in place: one launch runs the two side by
   // side (after the transposes it depends on), see below.
   const bool gather = p.gather && gather_dw_ok(M, K, N, g, g_stride_m, x, x_stride_m);
   const bool fused = bwd_is_fused(M, K, p, w_kmajor, gather);
   if (!fused) {
+    const int dx_tile = linear_dx_tile(M, K, N, dx_direct);
     if (w_kmajor) FFNK_HIP(launch_linear_gemm_kmajor(dx_tile, a, stream), "dx GEMM");
-    else FFNK_HIP(launch_linear_gemm(dx_tile, direct_ok(N, M, g_stride_m, ldw), a, stream), "dx GEMM");
+    else FFNK_HIP(launch_linear_gemm(dx_tile, dx_direct, a, stream), "dx GEMM");
   }
 
   // ---- dW_g = x_g^T g_g, contraction over the rows of group g ----
@@ -1146,8 +1169,10 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
   }
   a.A = g; a.lda = g_stride_m; a.B0[0] = w2t[0]; a.B0[1] = w2t[1]; a.ldb = ld2;
   a.C = DH; a.ldc = h;
-  if (w2_kmajor) FFNK_HIP(launch_gather_gemm_kmajor(routed_tile(M, h, false), a, stream), "dh GEMM");
-  else FFNK_HIP(launch_gather_gemm(routed_tile(M, h, false), direct_ok(d, M, g_stride_m, ld2), a, stream), "dh GEMM");
+  const bool dh_direct = w2_kmajor || direct_ok(d, M, g_stride_m, ld2);
+  const int dh_tile = bwd_tile(M, h, d, dh_direct);
+  if (w2_kmajor) FFNK_HIP(launch_gather_gemm_kmajor(dh_tile, a, stream), "dh GEMM");
+  else FFNK_HIP(launch_gather_gemm(dh_tile, dh_direct, a, stream), "dh GEMM");
 
   // ---- elementwise: T13 <- (dt1 | dt3), DH <- the SwiGLU intermediate ----
   FFNK_HIP(launch_swiglu_bwd(pre ? pre : T13, pre ? pre_stride_m : ld13, T13, ld13, DH, h, (int)M, (int)h, stream),
@@ -1178,7 +1203,8 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
   const RoutedPlan dxp = ffn_bwd_dx_plan(M, d, h, dx_direct, 2 * ws_align((size_t)h * d * 2), &dx_need);
   if (dx_need > p.w2t_bytes) return fail(FFNK_E_WORKSPACE, "internal: dx partials %zu > %zu planned", dx_need, p.w2t_bytes);
   if (dxp.splits > 1) {
-    b.splits = b.splits_more = dxp.splits;
+    b.splits = dxp.splits;
+    b.splits_more = dxp.splits_more;
     b.P = reinterpret_cast<float*>(wsb + p.off_w2t);
   } else if (dx_need > 0) {
     b.P_tail = reinterpret_cast<float*>(wsb + p.off_w2t);  // split tail of the last, partial round
@@ -1186,7 +1212,7 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
   if (w13_kmajor) FFNK_HIP(launch_down_gemm_kmajor(dxp.tile, b, stream), "dx GEMM");
   else FFNK_HIP(launch_down_gemm(dxp.tile, dx_direct, b, stream), "dx GEMM");
   if (dxp.splits > 1)
-    FFNK_HIP(launch_routed_reduce(b.P, dxp.splits, dxp.splits, tile_geom(dxp.tile, false).block_m, (int)M, (int)d, rt.counts, rt.perm,
+    FFNK_HIP(launch_routed_reduce(b.P, dxp.splits, dxp.splits_more, tile_geom(dxp.tile, false).block_m, (int)M, (int)d, rt.counts, rt.perm,
                                   dx, dx_stride_m, stream), "dx reduce");
 
   // ---- weight gradients: contraction over the rows of each group.  x and g are gathered into

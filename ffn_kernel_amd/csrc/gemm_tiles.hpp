@@ -55,8 +55,8 @@ struct KMajorTiles {
   // 128x128 behind a ring of four LDS stages, for the routed GEMMs (the weight-gradient GEMMs, whose last slab is
   // ragged and cleared in LDS, stay on the two-stage tile)
   using T4 = RoutedGemmCfg<128, 128, 2, 2, false, GATHER, SCATTER, true, kGroupM, true, 4>;
-  using T6 = T2;
-  using T7 = T3;
+  using T6 = RoutedGemmCfg<128, 256, 2, 2, false, GATHER, SCATTER, true, kGroupM, true, 3>;
+  using T7 = RoutedGemmCfg<64, 128, 2, 2, false, GATHER, SCATTER, true, kGroupM, true, 3>;
 };
 
 // SwiGLU tiles: BN = gate rows + up rows held in LDS, i.e. BN / 2 output columns.

@@ -51,7 +51,7 @@ enum TunedOp : int {
   TUNED_DUAL = 1,    // SwiGLU GEMM: k = contraction (d), n = output columns (h)
   TUNED_SPLITK = 2,  // weight-gradient GEMM: k = R (rows of the in-place operand), n = Cc
   TUNED_DOWN = 3,    // MaskedFFN down projection (routed-order rows in, scattered out; stage timing): k = contraction (h), n = output columns (d)
-  TUNED_NONE = -1,   // a GEMM the tuner does not measure (the backward's dx GEMMs): rules only
+  TUNED_NONE = -1,   // a GEMM the tuner does not measure (the backward's dx GEMMs): no measured plans
 };
 struct TunedPlan {
   int op;            // TunedOp, -1 ends the table
@@ -299,7 +299,7 @@ inline int pick_routed_tile(int64_t M, int64_t n_out, bool dual, int64_t K = 0, 
   return rule_tile(M, n_out, dual, K);
 }
 
-// The GEMMs the model above was not fitted for (the backward's dx GEMM over K-major weights): when the output yields fewer
+// What the model's plan has to beat, and where the model does not apply: when the output yields fewer
 // tiles than the chip has workgroup slots and the contraction is long, cutting K into `splits` ranges of whole 64-element
 // slabs fills the chip, at the price of fp32 partials (4 * splits * M * n_out bytes written, then read by the reduce pass):
 //   time = rounds * (5 us + slabs_per_range * t_slab) + splits * M * n_out * 8 bytes / 4 TB/s

@@ -4,8 +4,9 @@ import pytest
 import torch
 
 from ffn_kernel_amd import MaskedFFN, MaskedLinear, _lib
-from ffn_kernel_amd.ops import masked_linear_backward
-from helpers import assert_close, note
+from ffn_kernel_amd.ops import masked_ffn_backward, masked_ffn_forward, masked_linear_backward
+from helpers import assert_close, assert_close_pipeline, note
+from oracle import modules as om
 
 pytestmark = pytest.mark.gpu
 
@@ -116,3 +117,42 @@ def test_whole_rounds_and_remainder(dev, forced, tiles_m, h):
     out = MaskedFFN.apply(x, *[w.T for w in W], mask)
     forced()
     assert_close(out, select_ffn(x, W, mask).cpu(), "ffn")
+
+
+def ffn_case(dev, nv, nt, d, h, seed):
+    x, _, _, mask, _ = make_linear(dev, nv, nt, d, 8, seed)
+    gen = torch.Generator(device=dev).manual_seed(seed + 1)
+    W = [(torch.randn(*s, generator=gen, device=dev) * 0.05).to(torch.bfloat16) for s in ((h, d), (d, h), (h, d)) * 2]
+    return x, W, mask, torch.randn(nv + nt, d, generator=gen, device=dev).to(torch.bfloat16)
+
+
+def assert_ffn_backward(x, W, mask, g, what):
+    """Gradients of the feed-forward layer against the chain rule in double precision with the same bf16 storage points."""
+    views = [w.T for w in W]
+    out, pre = masked_ffn_forward(x, *views, mask, save_pre=True)
+    got = masked_ffn_backward(g, x, *views, mask, pre=pre)
+    dx, dW = om.ffn_backward_select(g.cpu(), x.cpu(), dict(zip(("w1", "w2", "w3", "u1", "u2", "u3"), (w.cpu() for w in W))), mask.cpu(),
+                                    torch.float64, round_intermediates=True)
+    assert_close_pipeline(got[0], dx, f"{what}: dx")
+    for i, k in enumerate(("w1", "w2", "w3", "u1", "u2", "u3")):
+        assert_close_pipeline(got[1 + i].T, dW[k], f"{what}: d{k}")
+
+
+# The ring tiles of three stages over K-major weights (dh and dx): contractions of fewer slabs than stages and more, through
+# both up-projection weights (h a multiple of 64) or over copies of them, ragged rows and columns, single rows, cut into ranges.
+@pytest.mark.parametrize("tile", [6, 7])
+@pytest.mark.parametrize("nv,nt,d,h,splits", [(1, 69, 64, 64, 1), (128, 64, 128, 320, 1), (129, 0, 264, 192, 1), (65, 130, 520, 136, 1),
+                                              (200, 130, 136, 1024, 3)])
+def test_backward_ring_tiles(dev, forced, tile, nv, nt, d, h, splits):
+    note(f"backward ring tile {tile}: nv={nv} nt={nt} d={d} h={h} splits={splits}")
+    case = ffn_case(dev, nv, nt, d, h, seed=d + h)
+    forced(tile, splits)
+    assert_ffn_backward(*case, f"tile {tile}")
+
+
+# dx of the feed-forward layer on its own plan, a contraction of 2h cut by the number of row tiles: as many as the rows need, or
+# one more.
+@pytest.mark.parametrize("nv", [0, 64, 100, 199, 200])
+def test_backward_split_factor_by_row_tiles(dev, nv):
+    note(f"backward split factor: nv={nv} of 200")
+    assert_ffn_backward(*ffn_case(dev, nv, 200 - nv, 512, 2048, seed=nv), f"nv {nv}")
