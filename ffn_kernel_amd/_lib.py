@@ -6,10 +6,12 @@ PyTorch/CPU fallback behind these calls).
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 from ctypes import c_char_p, c_int, c_int32, c_int64, c_size_t, c_void_p
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libffnk.so"
+CALL_PATH = LIB_PATH.with_name("_call.so")
 
 OP_LINEAR_FWD, OP_FFN_FWD, OP_LINEAR_BWD, OP_FFN_UP, OP_FFN_DOWN, OP_BWD_DX, OP_BWD_DW, OP_FFN_BWD = range(8)
 PATH_MFMA_TILED, PATH_STREAM, PATH_GENERIC = range(3)
@@ -126,6 +128,16 @@ def load() -> ctypes.CDLL:
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+def load_call():
+    """Load _call.so, the extension module that makes the usual calls.  Raises if it was not built."""
+    if not CALL_PATH.exists():
+        raise ImportError(f"{CALL_PATH} is missing: build it with `python -m ffn_kernel_amd.build`. There is no fallback path.")
+    spec = importlib.util.spec_from_file_location("ffn_kernel_amd._call", CALL_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
 
 
 def check(code: int, what: str) -> None:

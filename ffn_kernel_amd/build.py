@@ -1,6 +1,6 @@
-"""Build libffnk.so (the HIP kernels + C ABI) for gfx950 with hipcc.
+"""Build libffnk.so (the HIP kernels + C ABI) for gfx950 with hipcc, and _call.so, Python's way into it, with g++.
 
-    python -m ffn_kernel_amd.build            # compile every csrc/*.hip and link
+    python -m ffn_kernel_amd.build            # compile every csrc/*.hip and link; compile csrc/call.cpp
 
 hipcc cross-compiles without a GPU.  The library is written next to this file so that it
 travels with the source tree; nothing is installed outside the tree.
@@ -11,6 +11,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -18,6 +19,7 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 OBJ_DIR = CSRC / "build"
 LIB_PATH = PKG_DIR / "libffnk.so"
+CALL_PATH = PKG_DIR / "_call.so"
 
 ARCH = "gfx950"
 HIPCC_FLAGS = [
@@ -53,8 +55,27 @@ def _compile(src: Path) -> Path:
     return obj
 
 
+def _compile_call() -> Path:
+    """csrc/call.cpp -> _call.so, a CPython extension on torch's headers (host code only)."""
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    tmp = CALL_PATH.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{sysconfig.get_paths()['include']}"]
+    cmd += [flag for p in include_paths("cuda") for flag in ("-isystem", p)] + [str(CSRC / "call.cpp"), "-o", str(tmp)]
+    cmd += [f"-L{p}" for p in library_paths()] + ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed on call.cpp:\n{proc.stderr}")
+    if proc.stderr.strip():
+        sys.stderr.write(proc.stderr + "\n")
+    os.replace(tmp, CALL_PATH)
+    return CALL_PATH
+
+
 def build_library(jobs: int | None = None, verbose: bool = True) -> Path:
-    """Compile csrc/*.hip and link libffnk.so.  Always recompiles."""
+    """Compile csrc/*.hip and link libffnk.so; compile _call.so beside them.  Always recompiles."""
     OBJ_DIR.mkdir(parents=True, exist_ok=True)
     sources = sorted(CSRC.glob("*.hip"))
     if not sources:
@@ -63,7 +84,9 @@ def build_library(jobs: int | None = None, verbose: bool = True) -> Path:
     if verbose:
         print(f"[ffn_kernel_amd.build] hipcc {ARCH}: {len(sources)} files, {jobs} jobs", flush=True)
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        call = pool.submit(_compile_call)
         objs = list(pool.map(_compile, sources))
+        call.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     proc = subprocess.run(cmd, capture_output=True, text=True)

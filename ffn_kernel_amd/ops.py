@@ -114,11 +114,12 @@ class Routing:
     counts int32[2], as ffnk_route writes them.  One partition serves every operation that runs with the
     same mask - the projections of a layer, a forward and its backward - where the reference re-tests the
     mask inside every tile of every launch (linear.py:120-149, ffn.py:61-105)."""
-    __slots__ = ("perm", "counts", "M", "_struct")
+    __slots__ = ("perm", "counts", "M", "_struct", "address")
 
     def __init__(self, perm: torch.Tensor, counts: torch.Tensor):
         self.perm, self.counts, self.M = perm, counts, perm.shape[0]
         self._struct = _lib.RoutingStruct(perm.data_ptr(), counts.data_ptr())
+        self.address = ctypes.addressof(self._struct)
 
     def ref(self):
         return ctypes.byref(self._struct)
@@ -195,10 +196,52 @@ def _routing_arg(routing, mask: torch.Tensor, M: int, stream: int):
     return routing, (routing.ref() if routing is not None else None)
 
 
+def _routing_address(routing, mask: torch.Tensor, M: int, stream: int) -> int:
+    """_routing_arg for _call.so: the partition is kept by _route_cache.last while the call runs."""
+    routing, _ = _routing_arg(routing, mask, M, stream)
+    return 0 if routing is None else routing.address
+
+
+def _ffn_bwd_workspace_lean(M: int, d: int, h: int, dev: torch.device, g_ld: int, usn: int, dsk: int, dsn: int, gusk: int,
+                            gdsk: int) -> torch.Tensor:
+    """Workspace of the MaskedFFN backward for one layout of 16-byte aligned weights: the usual views skip the room for weight
+    copies and transposed intermediates."""
+    ws_bytes = _lib.load().ffnk_workspace_bytes_ffn_bwd(M, d, h, g_ld, usn, dsk, dsn, gusk, gdsk)
+    if ws_bytes == (1 << 64) - 1:
+        raise ValueError(f"ffnk_workspace_bytes_ffn_bwd: invalid extents M={M} d={d} h={h}")
+    return _workspace(ws_bytes, dev)
+
+
+def _ffn_bwd_workspace(a: torch.Tensor, d: int, h: int, g_ld: int) -> torch.Tensor:
+    """The workspace of _call.so's ffn_bwd: nn.Linear.weight.T views, gradients laid out like them."""
+    return _ffn_bwd_workspace_lean(a.shape[0], d, h, a.device, g_ld, d, 1, h, 1, 1)
+
+
+_native_call = None
+
+
+def _native():
+    """_call.so (csrc/call.cpp), bound to the library.  Its functions take the usual call - exact torch tensors on the
+    current GPU, nn.Linear.weight.T views, aligned rows - and return NotImplemented for any other, which the code below takes
+    or refuses."""
+    global _native_call
+    if _native_call is None:
+        module, lib = _lib.load_call(), _lib.load()
+        names = ("ffnk_workspace_bytes", "ffnk_masked_ffn_can_save", "ffnk_masked_linear_fwd_routed",
+                 "ffnk_masked_linear_bwd_routed", "ffnk_masked_ffn_fwd_routed", "ffnk_masked_ffn_bwd_routed")
+        module.bind(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names), _routing_address,
+                    _ffn_bwd_workspace, _lib.check, _ROUTED_MIN_ROWS)
+        _native_call = module
+    return _native_call
+
+
 def masked_linear_forward(a: torch.Tensor, b1: torch.Tensor, b2: torch.Tensor, mask: torch.Tensor,
                           routing: Routing | None = None) -> torch.Tensor:
     """c[m] = a[m] @ (b1 if mask[m] else b2).  Replaces _bf16_linear_forward (linear.py:418-452).
     routing: a partition of `mask` made by route(); None: the shared one (shared_routing)."""
+    c = _native().linear_fwd(a, b1, b2, mask, routing)
+    if c is not NotImplemented:
+        return c
     _require_cuda_bf16("a", a, 2)
     _require_cuda_bf16("b1", b1, 2)
     _require_cuda_bf16("b2", b2, 2)
@@ -238,6 +281,9 @@ def masked_linear_backward(grad: torch.Tensor, a: torch.Tensor, b1: torch.Tensor
                            mask: torch.Tensor, routing: Routing | None = None):
     """(da, db1, db2) of MaskedLinear.  Replaces _bf16_linear_backward (linear.py:455-496);
     db1/db2 keep b1's strides as the reference's empty_like(b1) does (linear.py:475)."""
+    grads = _native().linear_bwd(grad, a, b1, b2, mask, routing)
+    if grads is not NotImplemented:
+        return grads
     _require_cuda_bf16("grad", grad, 2)
     _require_cuda_bf16("a", a, 2)
     M, K = a.shape
@@ -280,6 +326,9 @@ def masked_ffn_forward(a, w1, w2, w3, u1, u2, u3, mask, save_pre: bool = False, 
     save_pre: also return the pre-activations [M, 2h] (routed order, gate | up) for
     masked_ffn_backward(..., pre=...), or None where the shape runs on a path that cannot keep them
     (decode sizes, d or h not a multiple of 8); the return value is then the pair (out, pre)."""
+    result = _native().ffn_fwd(a, w1, w2, w3, u1, u2, u3, mask, bool(save_pre), routing)
+    if result is not NotImplemented:
+        return result
     _require_cuda_bf16("a", a, 2)
     for name, w in (("w1", w1), ("w2", w2), ("w3", w3), ("u1", u1), ("u2", u2), ("u3", u3)):
         _require_cuda_bf16(name, w, 2)
@@ -338,6 +387,9 @@ def masked_ffn_backward(grad, a, w1, w2, w3, u1, u2, u3, mask, pre=None, routing
     weight views they belong to, as the linear backward's do.  pre: the pre-activations that
     masked_ffn_forward(..., save_pre=True) returned for the same inputs (read-only); None: they are
     recomputed."""
+    grads = _native().ffn_bwd(grad, a, w1, w2, w3, u1, u2, u3, mask, pre, routing)
+    if grads is not NotImplemented:
+        return grads
     _require_cuda_bf16("grad", grad, 2)
     _require_cuda_bf16("a", a, 2)
     for name, w in (("w1", w1), ("w2", w2), ("w3", w3), ("u1", u1), ("u2", u2), ("u3", u3)):
@@ -374,14 +426,11 @@ def masked_ffn_backward(grad, a, w1, w2, w3, u1, u2, u3, mask, pre=None, routing
     lib = _lib.load()
     with _on_device(dev):
         # Sized for this layout when every weight is 16-byte aligned (what the lean query assumes), for any
-        # layout otherwise: the usual views then skip the room for weight copies and transposed intermediates.
+        # layout otherwise.
         if all(w.data_ptr() % 16 == 0 for w in (*ups, *downs)):
-            ws_bytes = lib.ffnk_workspace_bytes_ffn_bwd(M, d, h, grad.stride(0) if M > 1 else d, usn, dsk, dsn, gusk, gdsk)
-            if ws_bytes == (1 << 64) - 1:
-                raise ValueError(f"ffnk_workspace_bytes_ffn_bwd: invalid extents M={M} d={d} h={h}")
+            ws = _ffn_bwd_workspace_lean(M, d, h, dev, grad.stride(0) if M > 1 else d, usn, dsk, dsn, gusk, gdsk)
         else:
-            ws_bytes = _lib.workspace_bytes(_lib.OP_FFN_BWD, M, d, h)
-        ws = _workspace(ws_bytes, dev)
+            ws = _workspace(_lib.workspace_bytes(_lib.OP_FFN_BWD, M, d, h), dev)
         stream = _stream_ptr(dev)
         routing, rt = _routing_arg(routing, mask, M, stream)
         head = (grad.data_ptr(), grad.stride(0) if M > 1 else d, a.data_ptr(), a.stride(0) if M > 1 else d,
@@ -410,10 +459,10 @@ _grad_mode = _GradMode()
 
 
 class MaskedLinear(Function):
-    """c = a @ (b1 where mask else b2), forward and backward (reference: ops.py:9-24)."""
+    """c = a @ (b1 where mask else b2), forward and backward (reference: ops.py:9-24).  Without the reference's custom_fwd /
+    custom_bwd: nothing in here reads the autocast state, and entering it costs 7 us of a forward + backward."""
 
     @staticmethod
-    @torch.amp.custom_fwd(device_type="cuda")
     def forward(ctx, a, b1, b2, mask):
         ctx.save_for_backward(a, mask)
         ctx.b1, ctx.b2 = b1, b2
@@ -426,7 +475,6 @@ class MaskedLinear(Function):
 
     @staticmethod
     @once_differentiable
-    @torch.amp.custom_bwd(device_type="cuda")
     def backward(ctx, grad):
         a, mask = ctx.saved_tensors
         da, db1, db2 = masked_linear_backward(grad, a, ctx.b1, ctx.b2, mask, routing=ctx.routing)
@@ -448,7 +496,6 @@ class MaskedFFN(Function):
         return super().apply(*args, **kwargs)
 
     @staticmethod
-    @torch.amp.custom_fwd(device_type="cuda")
     def forward(ctx, a, w1, w2, w3, u1, u2, u3, mask):
         ctx.weights = (w1, w2, w3, u1, u2, u3)
         _route_cache.last = None
@@ -466,7 +513,6 @@ class MaskedFFN(Function):
 
     @staticmethod
     @once_differentiable
-    @torch.amp.custom_bwd(device_type="cuda")
     def backward(ctx, grad):
         a, mask = ctx.saved_tensors[:2]
         pre = ctx.saved_tensors[2] if ctx.has_pre else None
