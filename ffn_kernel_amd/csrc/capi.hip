@@ -158,7 +158,7 @@ BwdPlan plan_bwd(int64_t M, int64_t K, int64_t N, bool dw_k_contig) {
 // clear what lies past a group's end before using it).
 constexpr int kBwdPadRows = 64;
 
-// MaskedFFN backward workspace: route | T13 [M + 64, 2h] | DH [M + 64, h] | W2^T, U2^T [h, d] | [W1^T|W3^T],
+// MaskedFFN backward workspace: route | T13 [M + 64, 2 * half], half = h or h rounded up to 64 | DH [M + 64, h] | W2^T, U2^T [h, d] | [W1^T|W3^T],
 // [U1^T|U3^T] [d, 2h] | g^T, x^T [d, ldt] | H^T, dt1^T, dt3^T [h, ldt] | fp32 split-K partials.
 struct FfnBwdPlan {
   BwdPlan up, dn;  // weight-gradient GEMM shapes: up = dW1/dW3 (K = d, N = h), dn = dW2 (K = h, N = d)
@@ -171,6 +171,7 @@ struct FfnBwdPlan {
 // read in place, and transposes of H, dt1, dt3 when their rows do not fit 32-bit slab offsets.
 struct FfnBwdPaths {
   bool w2_copy = true, w13_copy = true, acts_in_place = false, dx_direct = false;
+  int64_t half = 0;  // columns from dt1 to dt3 in T13: h, or the next multiple of 64 where the up weights are read in place
 };
 constexpr FfnBwdPaths kFfnBwdWorstCase{};
 // Weight-gradient split of the in-place path (H, dt1, dt3 read where they lie).
@@ -181,7 +182,7 @@ TileChoice ffn_bwd_in_place_choice(int64_t M, int64_t d, int64_t h) {
   return tc;
 }
 // Tile and split of the dx GEMM (2h-long contraction) and the bytes of partials or split tail it wants.
-RoutedPlan ffn_bwd_dx_plan(int64_t M, int64_t d, int64_t h, bool dx_direct, size_t room, size_t* need);
+RoutedPlan ffn_bwd_dx_plan(int64_t M, int64_t d, int64_t contraction, bool dx_direct, size_t room, size_t* need);
 FfnBwdPlan plan_ffn_bwd(int64_t M, int64_t d, int64_t h, bool dup_k_contig, bool ddn_k_contig,
                         const FfnBwdPaths& paths = kFfnBwdWorstCase) {
   FfnBwdPlan p;
@@ -194,10 +195,10 @@ FfnBwdPlan plan_ffn_bwd(int64_t M, int64_t d, int64_t h, bool dup_k_contig, bool
   // The dx GEMM's partials (or split tail) live where the copies would, as far as they fit there - the same bound
   // whether or not the copies are made, so that the dx GEMM's plan does not depend on the layout.
   size_t dx_need = 0;
-  ffn_bwd_dx_plan(M, d, h, paths.dx_direct, w2_copies, &dx_need);
+  ffn_bwd_dx_plan(M, d, 2 * (paths.half > 0 ? paths.half : h), paths.dx_direct, w2_copies, &dx_need);
   p.w2t_bytes = paths.w2_copy ? w2_copies : ws_align(dx_need);
   size_t o = route_ws_bytes(M);
-  p.off_t13 = o;  o += ws_align((size_t)(M + kBwdPadRows) * 2 * h * 2);
+  p.off_t13 = o;  o += ws_align((size_t)(M + kBwdPadRows) * 2 * round_up64(h, 64) * 2);
   p.off_dh = o;   o += ws_align((size_t)(M + kBwdPadRows) * h * 2);
   p.off_w2t = o;  o += p.w2t_bytes;
   p.off_w13t = o; o += paths.w13_copy ? 2 * ws_align((size_t)d * 2 * h * 2) : 0;
@@ -354,14 +355,14 @@ int bwd_tile(int64_t M, int64_t n_out, int64_t K, bool direct) {
   if (forced_tile() < 0 && direct && model_applies(false, M, n_out, K)) return model_routed_plan(false, M, n_out, K, false).tile;
   return routed_tile(M, n_out, false, 0, TUNED_NONE);
 }
-// dx GEMM of the MaskedFFN backward: few output tiles over a 2h-long contraction, so K is split like the forward's
+// dx GEMM of the MaskedFFN backward: few output tiles over a contraction of 2h (or 2 * half), so K is split like the forward's
 // down projection when the fp32 partials fit `room`; an unsplit big tile wants room for its split tail instead.
-RoutedPlan ffn_bwd_dx_plan(int64_t M, int64_t d, int64_t h, bool dx_direct, size_t room, size_t* need) {
+RoutedPlan ffn_bwd_dx_plan(int64_t M, int64_t d, int64_t contraction, bool dx_direct, size_t room, size_t* need) {
   // No measured plans: they are timings of other kernels (the forward's down projection reads K-contiguous weights through
   // another loop).
-  RoutedPlan dxp = down_plan(M, d, 2 * h, TUNED_NONE);
-  if (forced_tile() < 0 && forced_splits() < 1 && dx_direct && model_applies(false, M, d, 2 * h))
-    dxp = model_routed_plan(false, M, d, 2 * h, M < 65536, room);
+  RoutedPlan dxp = down_plan(M, d, contraction, TUNED_NONE);
+  if (forced_tile() < 0 && forced_splits() < 1 && dx_direct && model_applies(false, M, d, contraction))
+    dxp = model_routed_plan(false, M, d, contraction, M < 65536, room);
   if (!dx_direct || (size_t)max_splits(dxp) * M * d * 4 > room) {
     dxp.splits = dxp.splits_more = 1;
     dxp.tile = routed_tile(M, d, false, 0, TUNED_NONE);
@@ -379,18 +380,22 @@ FfnBwdPaths ffn_bwd_paths(int64_t M, int64_t d, int64_t h, int64_t g_stride_m, i
                           int64_t down_stride_n, const uint16_t* W1, const uint16_t* W3, const uint16_t* U1,
                           const uint16_t* U3, const uint16_t* W2, const uint16_t* U2, bool* w2_direct_out = nullptr,
                           bool* w2_kmajor_out = nullptr, bool* w13_kmajor_out = nullptr) {
-  const int64_t ld13 = 2 * h;
+  const int64_t half = round_up64(h, 64);
   const bool w2_direct = down_stride_n == 1 && down_stride_k % 8 == 0 && down_stride_k >= d && aligned16(W2) && aligned16(U2);
   // The forward's layout ([d, h] rows, h contiguous) is K-major for the dh GEMM: read in place.
   const bool w2_kmajor = !w2_direct && down_stride_k == 1 && kmajor_ok(d, h, down_stride_n, W2, U2) &&
                          direct_ok(d, M, g_stride_m, 8);
   // The up-projection weights ([h, d] rows, d contiguous) are K-major for the dx GEMM: the contraction
-  // runs through the gate weight's rows and on into the up weight's.
-  const bool w13_kmajor = h % 64 == 0 && kmajor_ok(2 * h, d, up_stride_n, W1, W3) && aligned16(U1) && aligned16(U3) &&
-                          direct_ok(2 * h, 0, ld13, 8);
+  // runs through the gate weight's rows and on into the up weight's, each padded to whole slabs (GemmArgs::k_rows; T13's rows
+  // are padded alike).  With copies of the four weights for h off multiples of 64, forward + backward took (us, copies -> in
+  // place): d = 6744, h = 16008, M = 389 1914 -> 1226 (one modality), d = 4824, h = 10736, M = 159 909 -> 654, d = 4408, h = 13192,
+  // M = 3021 3763 -> 3172, d = 1880, h = 5144, M = 1883 589 -> 511.
+  const bool w13_kmajor = kmajor_ok(2 * half, d, up_stride_n, W1, W3) && aligned16(U1) && aligned16(U3) && direct_ok(2 * half, 0, 2 * half, 8);
   FfnBwdPaths paths;
   paths.w2_copy = !(w2_direct || w2_kmajor);
   paths.w13_copy = !w13_kmajor;
+  paths.half = w13_kmajor ? half : h;
+  const int64_t ld13 = 2 * paths.half;
   paths.acts_in_place = ld13 * 128 + 2 * h < ((int64_t)1 << 32);
   paths.dx_direct = w13_kmajor || direct_ok(2 * h, 0, ld13, ld13);
   if (w2_direct_out) *w2_direct_out = w2_direct;
@@ -1125,10 +1130,10 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
     return fail(FFNK_E_STRIDE, "MaskedFFN backward: d, h and the row strides must be multiples of 8, rows 16-byte "
                                "aligned and the up-projection weights K-contiguous (up_stride_k == 1)");
   // Which optional regions this layout needs (ffnk_workspace_bytes_ffn_bwd asks the same function).
-  const int64_t ld13 = 2 * h;
   bool w2_direct = false, w2_kmajor = false, w13_kmajor = false;
   const FfnBwdPaths paths = ffn_bwd_paths(M, d, h, g_stride_m, up_stride_n, down_stride_k, down_stride_n, W1, W3, U1, U3, W2,
                                           U2, &w2_direct, &w2_kmajor, &w13_kmajor);
+  const int64_t half = paths.half, ld13 = 2 * half;
   const FfnBwdPlan p = plan_ffn_bwd(M, d, h, dup_stride_k == 1, ddown_stride_k == 1, paths);
   if (ws_bytes < p.total || !ws)
     return fail(FFNK_E_WORKSPACE, "workspace %zu < %zu bytes (ffnk_workspace_bytes_ffn_bwd sizes it for aligned pointers; "
@@ -1141,7 +1146,7 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
   Routing rt;
   if (int e = resolve_routing(routing, r, mask, M, stream, &rt)) return e;
 
-  // ---- pre-activations, routed order: T13[:, 0:h] = x A1, T13[:, h:2h] = x A3 ----
+  // ---- pre-activations, routed order: T13[:, 0:h] = x A1, T13[:, half:half + h] = x A3 ----
   GemmArgs a;
   a.A = x; a.lda = x_stride_m;
   a.B1[0] = a.B1[1] = nullptr; a.ldb = up_stride_n;
@@ -1151,7 +1156,7 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
   if (pre == nullptr) {
     a.B0[0] = W1; a.B0[1] = U1; a.C = T13;
     FFNK_HIP(launch_gather_gemm(routed_tile(M, h, false), up_direct, a, stream), "t1 GEMM");
-    a.B0[0] = W3; a.B0[1] = U3; a.C = T13 + h;
+    a.B0[0] = W3; a.B0[1] = U3; a.C = T13 + half;
     FFNK_HIP(launch_gather_gemm(routed_tile(M, h, false), up_direct, a, stream), "t3 GEMM");
   }
 
@@ -1175,16 +1180,18 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
   else FFNK_HIP(launch_gather_gemm(dh_tile, dh_direct, a, stream), "dh GEMM");
 
   // ---- elementwise: T13 <- (dt1 | dt3), DH <- the SwiGLU intermediate ----
-  FFNK_HIP(launch_swiglu_bwd(pre ? pre : T13, pre ? pre_stride_m : ld13, T13, ld13, DH, h, (int)M, (int)h, stream),
+  FFNK_HIP(launch_swiglu_bwd(pre ? pre : T13, pre ? pre_stride_m : ld13, (int)(pre ? h : half), T13, ld13, (int)half, DH, h, (int)M, (int)h,
+                             stream),
            "SwiGLU backward pass");
 
-  // ---- dx = (dt1 | dt3) @ (A1^T | A3^T)^T: one GEMM over the concatenated contraction of length 2h ----
+  // ---- dx = (dt1 | dt3) @ (A1^T | A3^T)^T: one GEMM over the concatenated contraction ----
   // In place over the K-major up-projection weights, or over one [d, 2h] copy per modality.
   GemmArgs b;
   b.A = T13; b.lda = ld13;
   if (w13_kmajor) {
     b.B0[0] = W1; b.B0[1] = U1; b.B1[0] = W3; b.B1[1] = U3; b.ldb = up_stride_n;
-    b.k_switch = (int)h;
+    b.k_switch = (int)half;
+    b.k_rows = (int)h;
   } else {
     uint16_t* w13[2] = {reinterpret_cast<uint16_t*>(wsb + p.off_w13t),
                         reinterpret_cast<uint16_t*>(wsb + p.off_w13t + ws_align((size_t)d * 2 * h * 2))};
@@ -1195,12 +1202,12 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
     b.B0[0] = w13[0]; b.B0[1] = w13[1]; b.B1[0] = b.B1[1] = nullptr; b.ldb = ld13;
   }
   b.C = dx; b.ldc = dx_stride_m; b.perm = rt.perm; b.counts = rt.counts;
-  b.M = (int)M; b.N = (int)d; b.K = (int)(2 * h); b.group_m = plan_group_m(TUNED_NONE, M, 2 * h, d);
+  b.M = (int)M; b.N = (int)d; b.K = (int)ld13; b.group_m = plan_group_m(TUNED_NONE, M, ld13, d);
   // Few output tiles over a 2h-long contraction: split K like the forward's down projection.  The
   // fp32 partials live where the W2^T copies were (dead since the dh GEMM), if they fit there.
   const bool dx_direct = paths.dx_direct;
   size_t dx_need = 0;
-  const RoutedPlan dxp = ffn_bwd_dx_plan(M, d, h, dx_direct, 2 * ws_align((size_t)h * d * 2), &dx_need);
+  const RoutedPlan dxp = ffn_bwd_dx_plan(M, d, ld13, dx_direct, 2 * ws_align((size_t)h * d * 2), &dx_need);
   if (dx_need > p.w2t_bytes) return fail(FFNK_E_WORKSPACE, "internal: dx partials %zu > %zu planned", dx_need, p.w2t_bytes);
   if (dxp.splits > 1) {
     b.splits = dxp.splits;
@@ -1243,7 +1250,7 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
     };
     if (int e = weight_grad_in_place(DH, h, GT, dW2, dU2, ddown_stride_k, ddown_stride_n)) return e;
     if (int e = weight_grad_in_place(T13, ld13, XT, dW1, dU1, dup_stride_n, dup_stride_k)) return e;
-    if (int e = weight_grad_in_place(T13 + h, ld13, XT, dW3, dU3, dup_stride_n, dup_stride_k)) return e;
+    if (int e = weight_grad_in_place(T13 + half, ld13, XT, dW3, dU3, dup_stride_n, dup_stride_k)) return e;
     return FFNK_OK;
   }
   uint16_t* HT = reinterpret_cast<uint16_t*>(wsb + p.off_ht);    // [h, ldt]
@@ -1253,7 +1260,7 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
                                     stream, false, true), "g / intermediate transpose");
   FFNK_HIP(launch_gather_transpose2(x, x_stride_m, (int)d, XT, T13, ld13, (int)h, D1T, p.ldt, rt.perm, rt.counts,
                                     (int)M, stream, false, true), "x / dt1 transpose");
-  FFNK_HIP(launch_gather_transpose2(T13 + h, ld13, (int)h, D3T, nullptr, 0, 0, nullptr, p.ldt, rt.perm, rt.counts,
+  FFNK_HIP(launch_gather_transpose2(T13 + half, ld13, (int)h, D3T, nullptr, 0, 0, nullptr, p.ldt, rt.perm, rt.counts,
                                     (int)M, stream, true, false), "dt3 transpose");
   auto weight_grad = [&](const BwdPlan& q, const uint16_t* gT, const uint16_t* xT, uint16_t* o0, uint16_t* o1,
                          int64_t sk, int64_t sn) -> int {

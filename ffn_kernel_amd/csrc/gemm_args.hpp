@@ -15,6 +15,9 @@ struct GemmArgs {
   // operand is B0[g] row k for k < k_switch and B1[g] row k - k_switch after it (two weights that
   // share the output axis, contracted in one pass).  0: B0 all the way.
   int k_switch = 0;
+  // Rows that each of the two weights has, where that is no multiple of 64: k_switch is the next one, K = 2 * k_switch, and A's
+  // columns [k_rows, k_switch) of both halves are zeros.  0: k_switch rows.
+  int k_rows = 0;
   uint16_t* C;           // [*, N] rows
   int64_t ldc;
   // SwiGLU kernels only, optional: the two pre-activations, bf16, rows like C (routed order):

@@ -89,6 +89,10 @@ struct KMajorB {
   // Rows of the range's last slab that belong to the contraction (1..64).  The rest of that slab is
   // cleared in LDS before it is read, so whatever lies behind the operand's last row never counts.
   int last_rows = 64;
+  // A weight whose last slab is ragged ahead of a second weight (GemmArgs::k_rows): that slab of each weight ends behind this many
+  // bytes, and what the loads address past them arrives in LDS as zeros (the descriptor's range check).
+  int kt_ragged = -1;
+  uint32_t ragged_bytes = 0;
 };
 
 template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, bool DUAL_, bool GATHER_A_, bool SCATTER_C_,
@@ -449,9 +453,11 @@ __device__ __forceinline__ void gemm_mainloop_slab_dma(const TileLanes<Cfg>& tl,
   auto kmajor_rsrc = [&](int kt, int head = 0) {
     const int ka = kb.kt_first + kt;
     const bool second = ka >= kb.kt_switch;
-    const uint64_t base = (second ? kw[1] : kw[0]) + (uint64_t)(uint32_t)(second ? ka - kb.kt_switch : ka) * kb.slab_bytes +
+    const int kw_slab = second ? ka - kb.kt_switch : ka;
+    const uint64_t base = (second ? kw[1] : kw[0]) + (uint64_t)(uint32_t)kw_slab * kb.slab_bytes +
                           (uint64_t)(uint32_t)head * (kb.slab_bytes / kBK);
-    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), 0, 0xffffffff, 0x00020000);
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), 0, kw_slab == kb.kt_ragged ? kb.ragged_bytes : 0xffffffffu,
+                                             0x00020000);
   };
   auto issue_b = [&](int stage, int kt, int head = 0) {
     uint8_t* st = lds + stage * STAGE;
@@ -739,9 +745,11 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
   auto kmajor_rsrc = [&](int kt, int head = 0) {
     const int ka = kb.kt_first + kt;
     const bool second = ka >= kb.kt_switch;
-    const uint64_t base = (second ? kw[1] : kw[0]) + (uint64_t)(uint32_t)(second ? ka - kb.kt_switch : ka) * kb.slab_bytes +
+    const int kw_slab = second ? ka - kb.kt_switch : ka;
+    const uint64_t base = (second ? kw[1] : kw[0]) + (uint64_t)(uint32_t)kw_slab * kb.slab_bytes +
                           (uint64_t)(uint32_t)head * (kb.slab_bytes / kBK);
-    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), 0, 0xffffffff, 0x00020000);
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), 0, kw_slab == kb.kt_ragged ? kb.ragged_bytes : 0xffffffffu,
+                                             0x00020000);
   };
 
   // LDS layout.  Two stages: stage s holds a slab's token panel, then its weight panel.  Ring: three token panels,
@@ -1091,9 +1099,11 @@ __device__ __forceinline__ void gemm_mainloop_ring(const TileLanes<Cfg>& tl,
   auto kmajor_rsrc = [&](int kt, int head = 0) {
     const int ka = kb.kt_first + kt;
     const bool second = ka >= kb.kt_switch;
-    const uint64_t base = (second ? kw[1] : kw[0]) + (uint64_t)(uint32_t)(second ? ka - kb.kt_switch : ka) * kb.slab_bytes +
+    const int kw_slab = second ? ka - kb.kt_switch : ka;
+    const uint64_t base = (second ? kw[1] : kw[0]) + (uint64_t)(uint32_t)kw_slab * kb.slab_bytes +
                           (uint64_t)(uint32_t)head * (kb.slab_bytes / kBK);
-    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), 0, 0xffffffff, 0x00020000);
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), 0, kw_slab == kb.kt_ragged ? kb.ragged_bytes : 0xffffffffu,
+                                             0x00020000);
   };
   uint32_t koff[4];
 #pragma unroll
@@ -1551,6 +1561,10 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
       kb.w[1] = g.k_switch > 0 ? g.B1[grp] : kb.w[0];  // (k_switch: whole slabs, k_ahead = 0)
       kb.kt_first = kt0;
       if (g.k_switch > 0) kb.kt_switch = g.k_switch / kBK;
+      if (g.k_rows > 0 && g.k_rows < g.k_switch) {
+        kb.kt_ragged = g.k_rows / kBK;
+        kb.ragged_bytes = (uint32_t)((g.k_rows % kBK) * g.ldb * 2);
+      }
       kb.slab_bytes = (uint32_t)(g.ldb * (kBK * 2));
     } else {
 #pragma unroll
@@ -1794,6 +1808,7 @@ inline hipError_t launch_routed_gemm(const GemmArgs& g, hipStream_t stream) {
                         (g.k_switch > 0 && g.K % kBK != 0) || g.ldb * (kBK * 2) + 2 * (int64_t)g.N >= ((int64_t)1 << 32)))
     return hipErrorInvalidValue;
   if (!Cfg::B_KMAJOR && g.k_switch != 0) return hipErrorInvalidValue;
+  if (g.k_rows != 0 && (g.k_rows < 0 || g.k_switch != round_up64(g.k_rows, kBK) || g.K != 2 * g.k_switch)) return hipErrorInvalidValue;
   const int grid = routed_gemm_grid<Cfg>(g.M, g.N, g.splits, g.splits_more);
   hipLaunchKernelGGL(routed_gemm_kernel<Cfg>, dim3(grid), dim3(Cfg::NT), 0, stream, g);
   return hipGetLastError();

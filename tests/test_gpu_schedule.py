@@ -156,3 +156,18 @@ def test_backward_ring_tiles(dev, forced, tile, nv, nt, d, h, splits):
 def test_backward_split_factor_by_row_tiles(dev, nv):
     note(f"backward split factor: nv={nv} of 200")
     assert_ffn_backward(*ffn_case(dev, nv, 200 - nv, 512, 2048, seed=nv), f"nv {nv}")
+
+
+# dx over up-projection weights whose rows end inside a slab: less than a slab, one row group short of whole slabs, one past, on
+# every tile and cut into ranges (whose ends may be either weight's ragged slab).  What lies behind the weights is NaN.
+@pytest.mark.parametrize("tile,splits", [(-1, -1), (0, 1), (1, 1), (2, 1), (3, 1), (4, 1), (6, 1), (7, 1), (2, 3), (7, 5)])
+@pytest.mark.parametrize("h", [8, 72, 200, 312, 1016])
+def test_backward_ragged_intermediate(dev, forced, tile, splits, h):
+    note(f"backward ragged intermediate: h={h} tile={tile} splits={splits}")
+    x, W, mask, g = ffn_case(dev, 90, 75, 136, h, seed=h)
+    for i in (0, 2, 3, 5):
+        behind = torch.full((h + 64, 136), float("nan"), dtype=torch.bfloat16, device=dev)
+        behind[:h] = W[i]
+        W[i] = behind[:h]
+    forced(tile, splits)
+    assert_ffn_backward(x, W, mask, g, f"h {h} tile {tile}")
