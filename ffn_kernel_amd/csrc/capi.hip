@@ -174,10 +174,10 @@ struct FfnBwdPaths {
   int64_t half = 0;  // columns from dt1 to dt3 in T13: h, or the next multiple of 64 where the up weights are read in place
 };
 constexpr FfnBwdPaths kFfnBwdWorstCase{};
-// Weight-gradient split of the in-place path (H, dt1, dt3 read where they lie).
+// Tile and split of the in-place path (H, dt1, dt3 read where they lie): the three GEMMs fill the chip together, unsplit in one
+// launch.  The measured plans are MaskedLinear's, of single launches.
 TileChoice ffn_bwd_in_place_choice(int64_t M, int64_t d, int64_t h) {
-  TileChoice tc = pick_splitk_tile(M, h, d, use_tuned());
-  if (tc.tile == kTileGatherDw) tc.tile = TILE_128x128_W4;  // a MaskedLinear plan of the same extents: the form does not exist here
+  TileChoice tc = pick_splitk_tile(M, h, d, false, kDwBatch);
   if (forced_splits() >= 1) tc.splits = forced_splits();
   return tc;
 }
@@ -1235,22 +1235,28 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
     const TileChoice tc = ffn_bwd_in_place_choice(M, d, h);
     const int tile = forced_tile() >= 0 ? forced_tile() : tc.tile;
     // out[r * sr + c * sc]: r runs over h (the in-place operand's columns), c over d
-    auto weight_grad_in_place = [&](const uint16_t* rows, int64_t ld_rows, const uint16_t* cT, uint16_t* o0, uint16_t* o1,
-                                    int64_t sr, int64_t sc) -> int {
+    auto weight_grad = [&](const uint16_t* rows, int64_t ld_rows, const uint16_t* cT, uint16_t* o0, uint16_t* o1, int64_t sr, int64_t sc) {
       SplitKArgs s;
       s.A = rows; s.lda = ld_rows;
       s.B = cT; s.ldb = p.ldt;
       s.P = P; s.counts = rt.counts; s.M = (int)M;
       s.R = (int)h; s.Cc = (int)d; s.splits = tc.splits;
-      if (tc.splits == 1) { s.out[0] = o0; s.out[1] = o1; s.out_sr = sr; s.out_sc = sc; }
-      FFNK_HIP(launch_splitk_gemm_kmajor(tile, s, stream), "dW split-K GEMM");
-      if (tc.splits > 1)
-        FFNK_HIP(launch_splitk_reduce(P, tc.splits, (int)h, (int)d, o0, o1, sr, sc, stream), "dW reduce");
-      return FFNK_OK;
+      s.out[0] = o0; s.out[1] = o1; s.out_sr = sr; s.out_sc = sc;
+      return s;
     };
-    if (int e = weight_grad_in_place(DH, h, GT, dW2, dU2, ddown_stride_k, ddown_stride_n)) return e;
-    if (int e = weight_grad_in_place(T13, ld13, XT, dW1, dU1, dup_stride_n, dup_stride_k)) return e;
-    if (int e = weight_grad_in_place(T13 + half, ld13, XT, dW3, dU3, dup_stride_n, dup_stride_k)) return e;
+    const SplitKArgs dw[kDwBatch] = {weight_grad(DH, h, GT, dW2, dU2, ddown_stride_k, ddown_stride_n),
+                                     weight_grad(T13, ld13, XT, dW1, dU1, dup_stride_n, dup_stride_k),
+                                     weight_grad(T13 + half, ld13, XT, dW3, dU3, dup_stride_n, dup_stride_k)};
+    if (tc.splits == 1) {
+      FFNK_HIP(launch_dw_batch_kmajor(tile, dw, stream), "dW GEMMs");
+      return FFNK_OK;
+    }
+    for (SplitKArgs s : dw) {
+      uint16_t *o0 = s.out[0], *o1 = s.out[1];
+      s.out[0] = s.out[1] = nullptr;
+      FFNK_HIP(launch_splitk_gemm_kmajor(tile, s, stream), "dW split-K GEMM");
+      FFNK_HIP(launch_splitk_reduce(P, tc.splits, (int)h, (int)d, o0, o1, s.out_sr, s.out_sc, stream), "dW reduce");
+    }
     return FFNK_OK;
   }
   uint16_t* HT = reinterpret_cast<uint16_t*>(wsb + p.off_ht);    // [h, ldt]

@@ -1629,7 +1629,7 @@ __device__ __forceinline__ void splitk_store(const SplitKArgs& g, typename Cfg::
   constexpr int TM = Cfg::TM, TN = Cfg::TN;
   constexpr int MT = Cfg::MT, RUNS = Cfg::ACC_N / 4;
   const bool direct = g.out[0] != nullptr;  // single split: the sums are complete
-  uint16_t* out = g.out[grp];
+  uint16_t* out = grp == 0 ? g.out[0] : g.out[1];  // (no index: g may be a local copy, which an index would put in scratch memory)
   const int64_t run_ld = Cfg::SWAP ? g.out_sr : g.out_sc;  // from one output row (of contiguous runs) to the next
   if (direct && (Cfg::SWAP ? g.out_sc : g.out_sr) == 1 && run_ld % 8 == 0 && (Cfg::SWAP ? g.Cc : g.R) % 8 == 0 &&
       (reinterpret_cast<uintptr_t>(out) & 15) == 0) {

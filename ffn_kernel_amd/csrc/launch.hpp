@@ -49,6 +49,9 @@ hipError_t launch_gather_gemm_kmajor(int tile, const GemmArgs& g, hipStream_t st
 hipError_t launch_splitk_gemm(int tile, const SplitKArgs& g, hipStream_t stream);
 // The same with A read in place: [rows, R] in routed order instead of a padded transpose (SplitKArgs).
 hipError_t launch_splitk_gemm_kmajor(int tile, const SplitKArgs& g, hipStream_t stream);
+// Three of them, unsplit (results to `out`), of the same extents, in one launch.
+constexpr int kDwBatch = 3;
+hipError_t launch_dw_batch_kmajor(int tile, const SplitKArgs (&g)[kDwBatch], hipStream_t stream);
 
 // The MaskedLinear backward's dx GEMM (K-major weights, as launch_linear_gemm_kmajor on the 128x128 tile)
 // and its weight-gradient GEMM (as launch_splitk_gemm on the 128x128 tile) in ONE launch: weight-gradient

@@ -372,8 +372,8 @@ inline RoutedPlan pick_routed_plan(int64_t M, int64_t n_out, int64_t K, bool use
   return rule_plan(M, n_out, K);
 }
 
-// Weight-gradient GEMM: two [R, Cc] outputs, contraction over about M / 2 rows each.
-inline TileChoice pick_splitk_tile(int64_t M, int64_t R, int64_t Cc, bool use_table = true) {
+// Weight-gradient GEMM: two [R, Cc] outputs, contraction over about M / 2 rows each; `batch` of them in one launch.
+inline TileChoice pick_splitk_tile(int64_t M, int64_t R, int64_t Cc, bool use_table = true, int batch = 1) {
   TileChoice c;
   c.tuned = false;
   if (use_table)
@@ -385,13 +385,13 @@ inline TileChoice pick_splitk_tile(int64_t M, int64_t R, int64_t Cc, bool use_ta
     }
   // Large outputs: the 256x256 tile fills the chip on its own, no split needed (and the GEMM then
   // stores bf16 directly, without partials or a reduce pass).
-  if (2 * cdiv64(R, 256) * cdiv64(Cc, 256) >= 2 * kCus) {
+  if (batch * 2 * cdiv64(R, 256) * cdiv64(Cc, 256) >= 2 * kCus) {
     c.tile = TILE_256x256_W8;
     c.splits = 1;
     return c;
   }
   c.tile = TILE_128x128_W4;
-  const int64_t tiles = 2 * cdiv64(R, 128) * cdiv64(Cc, 128);
+  const int64_t tiles = batch * 2 * cdiv64(R, 128) * cdiv64(Cc, 128);
   int64_t s = cdiv64(2 * kCus, tiles);            // aim at two workgroups per CU ...
   const int64_t slabs = cdiv64(cdiv64(M, 2), 64);  // 64-row slabs per group at an even split
   // ... with at least 16 slabs to each range: below that the partials and the reduce pass cost more than the idle CUs
