@@ -899,7 +899,14 @@ int ffn_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, cons
   up.perm = rt.perm; up.counts = rt.counts;
   up.M = (int)M; up.N = (int)h; up.K = (int)d; up.group_m = plan_group_m(TUNED_DUAL, M, d, h);
   up.C_pre = pre; up.ldc_pre = pre_stride_m;
-  FFNK_HIP(launch_up_gemm(routed_tile(M, h, true, d), direct_ok(d, M, x_stride_m, up_stride_n), up, stream), "up-projection GEMM");
+  const bool up_direct = direct_ok(d, M, x_stride_m, up_stride_n);
+  int up_tile = routed_tile(M, h, true, d);
+  // Where the plan is the four-wave 256x256 tile, up to eight rounds of the chip: beside 160-row ones in one launch (mixed_rows).
+  // Past that the two launches of whole rounds and remainder are the faster (M = 32768, d = 4096, h = 14336, 56 rounds: 7834 us
+  // against 8002; M = 23225, d = 2624, h = 8512, one modality, 24 rounds: 2241 against 2281).  A forced tile is run as it is.
+  if (up_tile == TILE_256x256_W4 && up_direct && forced_tile() < 0 && cdiv64(M, kTallRows) * cdiv64(h, 128) <= 8 * kCus)
+    up_tile = TILE_MIXED_W4;
+  FFNK_HIP(launch_up_gemm(up_tile, up_direct, up, stream), "up-projection GEMM");
   FFNK_HIP(mark(1), "event record");
   GemmArgs dn;
   dn.A = H; dn.lda = ldh;

@@ -8,7 +8,7 @@
 // Data path per workgroup: 64-column K slabs of the A and B panels go global -> LDS, two stages
 // deep (directly, bypassing registers; staged through registers where 32-bit offsets do not reach and
 // for short contractions that are no whole number of slabs); wavefronts read 16-byte MFMA fragments from an XOR-swizzled LDS layout and issue
-// v_mfma_f32_16x16x32_bf16 on the 256-row direct tiles (gemm_mainloop_fixed16) and v_mfma_f32_32x32x16_bf16
+// v_mfma_f32_16x16x32_bf16 on the 256- and 160-row direct tiles (gemm_mainloop_fixed16) and v_mfma_f32_32x32x16_bf16
 // on the others (gemm_mainloop_slab_dma, gemm_mainloop_ring, gemm_mainloop_staged).
 //
 // The backward GEMMs find one operand with the contraction running over its rows ([K, N], N
@@ -118,12 +118,12 @@ struct RoutedGemmCfg {
   static constexpr int BN_OUT = DUAL ? BN / 2 : BN;        // output columns per tile
   static constexpr int WTM = BM / WAVES_M;                 // rows per wave
   static constexpr int WTN_OUT = BN_OUT / WAVES_N;         // output columns per wave
-  // The 256-row direct tiles accumulate with v_mfma_f32_16x16x32_bf16 (four accumulator registers read
+  // The 256-row direct tiles (and the 160-row one beside them) accumulate with v_mfma_f32_16x16x32_bf16 (four accumulator registers read
   // and written per 16 K-products of a lane instead of sixteen per 16: the kernel runs at the board's
   // power limit and the narrower accumulator traffic is worth 5 % there); the others with 32x32x16.  K-major
   // weight panels included: MaskedFFN forward + backward at d = 4096, h = 14336 runs 4.5 % (M = 4096) to 7 %
   // (M = 32768) faster than with the backward's 256-row GEMMs on the two-stage 32x32x16 loop.
-  static constexpr bool MFMA16 = DIRECT_ && BM_ == 256;
+  static constexpr bool MFMA16 = DIRECT_ && (BM_ == 256 || BM_ == 160);
   // Cache policy of the token panel's global->LDS loads.  The down projection's token rows (the routed intermediate,
   // read in place) pass each XCD once: a round of tiles reads a line and no later round does.  Loaded with the
   // non-temporal hint they do not push the weight panels out of L2 (cfg4 down projection 2.91 -> 2.85 ms, M = 16384
@@ -144,14 +144,17 @@ struct RoutedGemmCfg {
   static constexpr int STAGES = STAGES_;
   // The 256-row direct tiles take STAGES == 3 to mean: token panel in a ring of three stages, weight panel in two
   // (gemm_mainloop_fixed16) - exactly the 160 KB of LDS a CU has.
-  static constexpr bool A_RING3 = MFMA16 && STAGES_ == 3;
+  static constexpr bool A_RING3 = MFMA16 && STAGES_ == 3 && BM_ == 256;
   static constexpr bool RING = STAGES_ > 2 && !MFMA16;
+  // The 160-row tile fits whole stages three times (gemm_mainloop_fixed16).
+  static constexpr bool RING3 = MFMA16 && BM_ == 160;
   static constexpr int LDS_BYTES = A_RING3 ? 3 * A_BYTES + 2 * BN * kRowBytes : STAGES * STAGE_BYTES;
   static_assert(STAGES_ >= 2 && STAGES_ <= 6 && LDS_BYTES <= 160 * 1024, "LDS stages");
-  static_assert(STAGES_ == 2 || A_RING3 || (DIRECT_ && BM_ <= 128), "ring: direct path of the small tiles");
-  static_assert(WTM % 32 == 0 && WTN_OUT % 32 == 0, "wave tile must be a multiple of 32x32");
+  static_assert(STAGES_ == 2 || A_RING3 || RING3 || (DIRECT_ && BM_ <= 128), "ring: direct path of the small tiles");
+  static_assert(!RING3 || STAGES_ == 3, "160-row tile: three stages");
+  static_assert(WTM % MT == 0 && WTN_OUT % 32 == 0, "wave tile must be a multiple of accumulator tiles");
   static_assert(NWAVES % 2 == 0, "lane mapping of the slab layout needs an even wave count");
-  static_assert((BM / 16) % NWAVES == 0 && (BN / 16) % NWAVES == 0, "panel rows must split evenly over waves");
+  static_assert((BM / 8) % NWAVES == 0 && (BN / 8) % NWAVES == 0, "panel rows must split evenly over waves");
   static_assert(!DUAL || (BN / 2) % 16 == 0, "gate/up split must fall on a 16-row load group");
   static_assert(!B_KMAJOR || (DIRECT && !DUAL && BN >= 64 && BN <= 512), "K-major weights: direct path, one weight");
 };
@@ -655,7 +658,7 @@ __device__ __forceinline__ void gemm_mainloop_slab_dma(const TileLanes<Cfg>& tl,
 }
 
 // =============================================================================================
-// Direct path of the 256-row tiles: 64-element slabs accumulated with v_mfma_f32_16x16x32_bf16 in a schedule
+// Direct path of the 256- and 160-row tiles: 64-element slabs accumulated with v_mfma_f32_16x16x32_bf16 in a schedule
 // written out in source order (every MFMA fenced by scheduling barriers), because with one or two wavefronts
 // per SIMD nothing else hides a wait, and an instruction that cannot issue - a load while the address unit's
 // queue is full - holds back the MFMAs behind it.
@@ -680,6 +683,9 @@ __device__ __forceinline__ void gemm_mainloop_slab_dma(const TileLanes<Cfg>& tl,
 //    (s_memtime, one lane per workgroup) put the data barrier of the two-stage form at 120 cycles per slab on
 //    the SwiGLU GEMM (K = 4096) and at 270 of 2 700 on the down projection (K = 14336), whose panels miss L2
 //    more often; the ring takes the down projection from 2.66 to 2.55 ms and leaves the SwiGLU GEMM where it was.
+//  * Cfg::RING3 (160 rows, 156 KB): both panels in a ring of three stages.  A stage is free a whole slab before it is loaded again,
+//    so there is no release barrier; the loads of slab kt + 2 go out from slab kt's first MFMA on, one behind every fifth, and the
+//    data barrier leaves them in flight.
 //  * K-major weight panels (Cfg::B_KMAJOR, see KMajorB): the same schedule; a weight fragment is two transposing
 //    reads, issued as asm statements in the slot where the row-major form issues its one read, and every K step
 //    starts with an s_waitcnt lgkmcnt(n) that leaves outstanding only the token reads issued behind the last of
@@ -705,6 +711,8 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
   constexpr int RPOS = 4;                // ... ahead of the release barrier
   // Token panel in a ring of three stages: slab kt's token rows sit in stage kt % 3, its weight rows in stage kt % 2.
   constexpr bool R3 = Cfg::A_RING3;
+  // Both panels in a ring of three stages (token stage and weight stage of slab kt: kt % 3).
+  constexpr bool RF = Cfg::RING3;
   constexpr bool KM = Cfg::B_KMAJOR;     // weight panel stored K-major: fragments come from transposing reads (see KMajorB)
   constexpr int RB = Cfg::BN * 2;        // ... bytes of one of its 64 rows
   // One load per wave behind every LEV-th MFMA.  One per four MFMAs is the address unit's own rate (16 cycles per
@@ -713,9 +721,14 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
   constexpr int LEV = NWAVES == 4 ? 5 : 4;
   // Two-stage form: loads of the slab after next that go out in the second step (the rest follow in the next slab's first).
   constexpr int L1 = R3 ? NJB : ((NM - RPOS) / LEV < L ? (NM - RPOS) / LEV : L);
+  // Ring of whole stages: loads of slab kt + 2 that go out in slab kt's first step, and of the others those ahead of the data barrier.
+  constexpr int LF0 = NM / LEV < L ? NM / LEV : L, LF1 = BAR / LEV < L - LF0 ? BAR / LEV : L - LF0;
+  static_assert(!RF || (L - LF0) * LEV <= NM, "ring schedule does not fit this wave tile");
   constexpr int NPRE = (BAR - RPOS) / LEV;  // ... of them ahead of the data barrier (a load follows the last MFMA of its group of LEV)
   static_assert(RPOS >= 0 && RPOS < BAR && NPRE <= L1, "release barrier ahead of the data barrier");
-  static_assert(TM >= 3 && TM >= TN && L1 >= 1 && L1 <= L && (L - L1) * LEV <= NM, "schedule does not fit this wave tile");
+  static_assert(TM >= 3 && (RF || TM >= TN) && L1 >= 1 && L1 <= L && (L - L1) * LEV <= NM, "schedule does not fit this wave tile");
+  static_assert(!RF || !KM, "ring of whole stages: row-major weights");
+  constexpr int BSTEP0 = TM >= TN ? TN : TM;  // first step: MFMAs from one weight-fragment read to the next
   static_assert(!R3 || (NJA * LEV <= NM && RPOS + NJB * LEV <= NM), "ring schedule does not fit this wave tile");
   const int wave = tl.wave_s;
 
@@ -852,6 +865,11 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
     if (l < NJB) load_b(l, b_stage(t), kt, head);
     else load_a(l - NJB, a_stage(t), kt, head);
   };
+  // Ring of whole stages: the same into the stage at byte offset st.
+  auto load_at = [&](int l, int st, int kt) {
+    if (l < NJB) load_b(l, st + A_BYTES, kt);
+    else load_a(l - NJB, st, kt);
+  };
   // Four-wave tiles hold 256 accumulator registers per lane, which only fit the accumulation half of the
   // register file.  Left to the builtin, the compiler keeps part of them in ordinary registers and moves
   // them back and forth inside the loop (v_accvgpr_read/write around every other MFMA); the asm form
@@ -882,17 +900,19 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
   constexpr int kYoungerStep0 = TM - TN + 1;          // first step: the token reads of row groups TN - 1 ... TM - 1
   constexpr int kLastB1 = BAR + 2 * G0 + (TN - 1) * BSTEP;
   constexpr int kYoungerStep1 = TM - (kLastB1 + 1) / TN;  // second step: row groups whose last MFMA lies behind slot kLastB1
-  static_assert(kYoungerStep0 >= 0 && kYoungerStep1 >= 0 && kYoungerStep0 < 16 && kYoungerStep1 < 16, "lgkmcnt is four bits");
-  auto step0 = [&](int u, int a_cur, int a_ld, int kt, bool next, bool next2) {
+  static_assert(!KM || (kYoungerStep0 >= 0 && kYoungerStep1 >= 0 && kYoungerStep0 < 16 && kYoungerStep1 < 16), "lgkmcnt is four bits");
+  auto step0 = [&](int u, int b_cur, int a_cur, int a_ld, int kt, bool next, bool next2) {
     wait_b(0, std::integral_constant<int, kYoungerStep1>{});
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
       mfma(0, m);
       __builtin_amdgcn_sched_barrier(0);
-      if (m % TN == TN / 2 - 1 && m / TN < TN) read_b(1, m / TN, b_stage(u), 1);   // one per row group
+      if (m % BSTEP0 == BSTEP0 / 2 - 1 && m / BSTEP0 < TN) read_b(1, m / BSTEP0, b_cur, 1);   // one per row group (or TM MFMAs)
       if (m % TN == TN - 1) read_a(m / TN, a_cur, 1);
-      if constexpr (R3) {
+      if constexpr (RF) {
+        if (m % LEV == LEV - 1 && m / LEV < LF0 && next2) load_at(m / LEV, a_ld, kt + 2);
+      } else if constexpr (R3) {
         if (m % LEV == LEV - 1 && m / LEV < NJA && next2) load_a(m / LEV, a_ld, kt + 2);
       } else {
         if (L1 + m / LEV < L && m % LEV == LEV - 1 && next) load(L1 + m / LEV, u ^ 1, kt + 1);
@@ -903,7 +923,8 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
   // Second K step: two row groups, the barriers, then behind the MFMAs the first-step fragments of slab kt + 1
   // (weight stage u ^ 1, token stage at a_nxt) and loads of slab kt + 2 into the stage the release barrier freed:
   // its first L1 loads (two-stage form) or its weight panel (ring form).
-  auto step1 = [&](int u, int a_nxt, int kt, bool next, bool next2) {
+  // (Ring of whole stages: the rest of slab kt + 2, into the stage at a_ld, which slab kt - 1 left two barriers ago.)
+  auto step1 = [&](int u, int b_nxt, int a_nxt, int a_ld, int kt, bool next, bool next2) {
     wait_b(1, std::integral_constant<int, kYoungerStep0>{});
     __builtin_amdgcn_sched_barrier(0);
     // Behind the barrier: the first-step fragments of slab kt + 1.  Token fragments of the row groups that ran
@@ -911,13 +932,13 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
     // MFMAs before its first use), token fragments of the other groups as their last MFMA issues.
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-      if (m == RPOS) {
+      if (!RF && m == RPOS) {
         dma_wait_barrier<63>();  // every wave's reads of stage u have returned: the stage is free for slab kt + 2
         __builtin_amdgcn_sched_barrier(0);
       }
       if (m == BAR) {
         // slab kt + 1 has landed; the loads of slab kt + 2 issued since stay in flight
-        if (next2) dma_wait_barrier<(R3 ? NJA : 0) + NPRE>();
+        if (next2) dma_wait_barrier<RF ? LF0 + LF1 : (R3 ? NJA : 0) + NPRE>();
         else dma_wait_barrier<0>();
         if constexpr (KM) {
           if (next && !next2 && kb.last_rows < kBK) clear_tail(b_stage(u ^ 1));  // slab kt + 1 is the last: never in the steady loop
@@ -929,10 +950,12 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
       if (next) {
         if (m >= BAR && m < BAR + 2 * G0 && (m - BAR) % 2 == 0) read_a((m - BAR) / 2, a_nxt, 0);
         if (m >= BAR + 2 * G0 && (m - BAR - 2 * G0) % BSTEP == 0 && (m - BAR - 2 * G0) / BSTEP < TN)
-          read_b(0, (m - BAR - 2 * G0) / BSTEP, b_stage(u ^ 1), 0);
+          read_b(0, (m - BAR - 2 * G0) / BSTEP, b_nxt, 0);
         if (m / TN >= G0 && m % TN == TN - 1) read_a(m / TN, a_nxt, 0);
       }
-      if (m >= RPOS && (m - RPOS) % LEV == LEV - 1 && (m - RPOS) / LEV < L1 && next2) {
+      if constexpr (RF) {
+        if (m % LEV == LEV - 1 && LF0 + m / LEV < L && next2) load_at(LF0 + m / LEV, a_ld, kt + 2);
+      } else if (m >= RPOS && (m - RPOS) % LEV == LEV - 1 && (m - RPOS) / LEV < L1 && next2) {
         if constexpr (R3) load_b((m - RPOS) / LEV, b_stage(u), kt + 2);
         else load((m - RPOS) / LEV, u, kt + 2);
       }
@@ -949,7 +972,11 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
 #pragma unroll
   for (int l = NJB; l < L; ++l) load(l, 0, 0, pad);
   if (nk > 1) {
-    if constexpr (R3) {  // token panel first, as the steady schedule issues them
+    if constexpr (RF) {
+#pragma unroll
+      for (int l = 0; l < L; ++l) load(l, 1, 1);
+      dma_wait_barrier<L>();
+    } else if constexpr (R3) {  // token panel first, as the steady schedule issues them
 #pragma unroll
       for (int l = 0; l < NJA; ++l) load_a(l, a_stage(1), 1);
 #pragma unroll
@@ -965,7 +992,7 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
   }
   if (pad > 0) {  // uniform over the launch's workgroups of this K range
     clear_head<Cfg>(tl, pad, lds + a_stage(0), lds + b_stage(0));
-    dma_wait_barrier<R3 ? L : L1>();
+    dma_wait_barrier<R3 || RF ? L : L1>();
   }
   if constexpr (KM) {
     if (nk == 1 && kb.last_rows < kBK) clear_tail(b_stage(0));
@@ -976,13 +1003,13 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
   for (int i = 0; i < TM; ++i) read_a(i, a_stage(0), 0);
 
   int k0 = 0;
-  if constexpr (R3) {
-    // token stages of slabs k0, k0 + 1, k0 + 2 (byte offsets), rotated once per slab
+  if constexpr (R3 || RF) {
+    // token stages (RF: whole stages) of slabs k0, k0 + 1, k0 + 2 (byte offsets), rotated once per slab
     int s0 = a_stage(0), s1 = a_stage(1), s2 = a_stage(2);
     // slab kt with its weight panel in stage u
     auto slab = [&](int u, int kt, bool next, bool next2) {
-      step0(u, s0, s2, kt, next, next2);
-      step1(u, s1, kt, next, next2);
+      step0(u, RF ? s0 + A_BYTES : b_stage(u), s0, s2, kt, next, next2);
+      step1(u, RF ? s1 + A_BYTES : b_stage(u ^ 1), s1, s2, kt, next, next2);
       const int t = s0;
       s0 = s1;
       s1 = s2;
@@ -998,8 +1025,8 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
     }
   } else {
     auto slab = [&](int u, int kt, bool next, bool next2) {
-      step0(u, a_stage(u), 0, kt, next, next2);
-      step1(u, a_stage(u ^ 1), kt, next, next2);
+      step0(u, b_stage(u), a_stage(u), 0, kt, next, next2);
+      step1(u, b_stage(u ^ 1), a_stage(u ^ 1), 0, kt, next, next2);
     };
     for (; k0 + 3 < nk; k0 += 2) {  // every guard inside is true: no branches
       slab(0, k0, true, true);
@@ -1462,58 +1489,13 @@ __device__ __forceinline__ void routed_partial_store(float* base, int64_t ld, co
   }
 }
 
-// Routed GEMM: rows in routed order, group-pure tiles.
-//   GATHER_A : A row of routed position p is perm[p] (else p)
-//   SCATTER_C: C row of routed position p is perm[p] (else p)
-//   DUAL     : C = silu(A B0^T) * (A B1^T)   (SwiGLU epilogue in fp32 registers)
-// `bid`: the workgroup's index among those of this GEMM (the launch's block index, or its offset inside a
-// launch that runs several GEMMs side by side); `lds`: Cfg::LDS_BYTES, 1 KB aligned.
+// One tile of a routed GEMM (tc), or one of `splits` K ranges of it.
 template <class Cfg>
-__device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds, const int bid) {
+__device__ __forceinline__ void routed_tile(const GemmArgs& g, uint8_t* lds, const TileCoord& tc, const int split, const int splits,
+                                            const int tail_slot) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN;
   constexpr int TM = Cfg::TM, TN = Cfg::TN;
-
-  // ---- tile schedule (all from device-side counts; no host sync) ----
-  const int SBM = g.sched_bm > 0 ? g.sched_bm : BM;
-  const int SBN = g.sched_bn > 0 ? g.sched_bn : Cfg::BN_OUT;
-  const int n_vis = g.counts[0];
-  const int total = routed_tile_count(n_vis, g.M, g.N, SBM, SBN);
-  int L, sub_m = 0, sub_n = 0, split = 0, splits = 1, tail_slot = 0;
-  if (g.tail_mode == 0) {
-    if (g.splits > 1) splits = routed_splits(n_vis, g.M, BM, g.splits, g.splits_more);
-    L = xcd_tile_slot(total * splits, bid);
-    if (splits > 1 && L >= 0) {  // range-major: neighbours in the order share panels, not a K range
-      split = L / total;
-      L -= split * total;
-    }
-  } else {
-    // (tail_mode 1 with a split tail behind it leaves every remainder to the tail)
-    const int full = g.tail_mode == 3 || g.P_tail != nullptr ? total / kCusPerChip * kCusPerChip : whole_round_tiles(total);
-    if (g.tail_mode == 1) {
-      L = xcd_tile_slot(full, bid);
-    } else if (g.tail_mode == 2) {
-      const int qn = SBN / Cfg::BN_OUT, q = (SBM / BM) * qn;  // own tiles per macro tile
-      if (bid >= (total - full) * q) return;
-      L = full + bid / q;
-      sub_m = (bid % q) / qn;
-      sub_n = (bid % q) % qn;
-    } else {
-      const int n_tail = total - full;
-      splits = tail_split_factor(n_tail, cdiv(g.K, kBK));
-      tail_slot = bid;
-      if (tail_slot >= n_tail * splits) return;
-      split = tail_slot / n_tail;
-      L = full + tail_slot % n_tail;
-    }
-  }
-  if (L < 0) return;
-  const TileCoord tc = routed_tile_coord(L, n_vis, g.M, g.N, SBM, SBN, g.group_m > 0 ? g.group_m : Cfg::GROUP_M);
-  const int grp = tc.grp;
-  const int row0 = tc.row0 + sub_m * BM;  // routed position
-  const int row_end = tc.row_end;
-  const int n0 = tc.n0 + sub_n * Cfg::BN_OUT;
-  if (row0 >= row_end || n0 >= g.N) return;  // a sub-tile past the edge of a partial macro tile
-
+  const int grp = tc.grp, row0 = tc.row0, row_end = tc.row_end, n0 = tc.n0;  // row0: routed position
   typename Cfg::Acc acc[TM][TN];
   if constexpr (Cfg::DIRECT) {
     constexpr int NJA = TileLanes<Cfg>::NJA, NJB = TileLanes<Cfg>::NJB;
@@ -1612,6 +1594,58 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
     routed_epilogue<Cfg>(g, acc, row0, row_end, n0, tl, lds);
   }
 }
+
+// Routed GEMM: rows in routed order, group-pure tiles.
+//   GATHER_A : A row of routed position p is perm[p] (else p)
+//   SCATTER_C: C row of routed position p is perm[p] (else p)
+//   DUAL     : C = silu(A B0^T) * (A B1^T)   (SwiGLU epilogue in fp32 registers)
+// `bid`: the workgroup's index among those of this GEMM (the launch's block index, or its offset inside a
+// launch that runs several GEMMs side by side); `lds`: Cfg::LDS_BYTES, 1 KB aligned.
+template <class Cfg>
+__device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds, const int bid) {
+  constexpr int BM = Cfg::BM;
+
+  // ---- tile schedule (all from device-side counts; no host sync) ----
+  const int SBM = g.sched_bm > 0 ? g.sched_bm : BM;
+  const int SBN = g.sched_bn > 0 ? g.sched_bn : Cfg::BN_OUT;
+  const int n_vis = g.counts[0];
+  const int total = routed_tile_count(n_vis, g.M, g.N, SBM, SBN);
+  int L, sub_m = 0, sub_n = 0, split = 0, splits = 1, tail_slot = 0;
+  if (g.tail_mode == 0) {
+    if (g.splits > 1) splits = routed_splits(n_vis, g.M, BM, g.splits, g.splits_more);
+    L = xcd_tile_slot(total * splits, bid);
+    if (splits > 1 && L >= 0) {  // range-major: neighbours in the order share panels, not a K range
+      split = L / total;
+      L -= split * total;
+    }
+  } else {
+    // (tail_mode 1 with a split tail behind it leaves every remainder to the tail)
+    const int full = g.tail_mode == 3 || g.P_tail != nullptr ? total / kCusPerChip * kCusPerChip : whole_round_tiles(total);
+    if (g.tail_mode == 1) {
+      L = xcd_tile_slot(full, bid);
+    } else if (g.tail_mode == 2) {
+      const int qn = SBN / Cfg::BN_OUT, q = (SBM / BM) * qn;  // own tiles per macro tile
+      if (bid >= (total - full) * q) return;
+      L = full + bid / q;
+      sub_m = (bid % q) / qn;
+      sub_n = (bid % q) % qn;
+    } else {
+      const int n_tail = total - full;
+      splits = tail_split_factor(n_tail, cdiv(g.K, kBK));
+      tail_slot = bid;
+      if (tail_slot >= n_tail * splits) return;
+      split = tail_slot / n_tail;
+      L = full + tail_slot % n_tail;
+    }
+  }
+  if (L < 0) return;
+  TileCoord tc = routed_tile_coord(L, n_vis, g.M, g.N, SBM, SBN, g.group_m > 0 ? g.group_m : Cfg::GROUP_M);
+  tc.row0 += sub_m * BM;
+  tc.n0 += sub_n * Cfg::BN_OUT;
+  if (tc.row0 >= tc.row_end || tc.n0 >= g.N) return;  // a sub-tile past the edge of a partial macro tile
+  routed_tile<Cfg>(g, lds, tc, split, splits, tail_slot);
+}
+
 
 template <class Cfg>
 __global__ __launch_bounds__(Cfg::NT) void routed_gemm_kernel(const GemmArgs g) {
@@ -1787,6 +1821,24 @@ __global__ __launch_bounds__(CfgDx::NT) void fused_bwd_kernel(const GemmArgs gx,
   else routed_gemm_body<CfgDx>(gx, lds, (int)blockIdx.x - dw_blocks);
 }
 
+// Tiles of two heights in one launch (mixed_rows): every XCD takes an eighth of the tall tiles' order, then an eighth of the
+// short ones'.
+template <class Tall, class Short>
+__global__ __launch_bounds__(Tall::NT) void routed_mixed_kernel(const GemmArgs g) {
+  static_assert(Tall::NT == Short::NT && Tall::BN_OUT == Short::BN_OUT && Tall::BM == kTallRows && Short::BM == kShortRows, "two heights");
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[Tall::LDS_BYTES > Short::LDS_BYTES ? Tall::LDS_BYTES : Short::LDS_BYTES];
+  bool is_tall;
+  TileCoord tc = mixed_tile_coord((int)blockIdx.x, g.counts[0], g.M, g.N, Tall::BN_OUT, &is_tall);
+  if (tc.grp < 0) return;
+  // (the compiler takes them for values of a lane and would load the weights' addresses through the vector memory path)
+  tc.grp = __builtin_amdgcn_readfirstlane(tc.grp);
+  tc.row0 = __builtin_amdgcn_readfirstlane(tc.row0);
+  tc.row_end = __builtin_amdgcn_readfirstlane(tc.row_end);
+  tc.n0 = __builtin_amdgcn_readfirstlane(tc.n0);
+  if (is_tall) routed_tile<Tall>(g, lds, tc, 0, 1, 0);
+  else routed_tile<Short>(g, lds, tc, 0, 1, 0);
+}
+
 // Upper bound on the number of workgroups the kernel needs, rounded so that every XCD gets the
 // same number of slots.  The kernel derives the real tile count from counts[] on the device.
 template <class Cfg>
@@ -1811,6 +1863,15 @@ inline hipError_t launch_routed_gemm(const GemmArgs& g, hipStream_t stream) {
   if (g.k_rows != 0 && (g.k_rows < 0 || g.k_switch != round_up64(g.k_rows, kBK) || g.K != 2 * g.k_switch)) return hipErrorInvalidValue;
   const int grid = routed_gemm_grid<Cfg>(g.M, g.N, g.splits, g.splits_more);
   hipLaunchKernelGGL(routed_gemm_kernel<Cfg>, dim3(grid), dim3(Cfg::NT), 0, stream, g);
+  return hipGetLastError();
+}
+
+template <class Tall, class Short>
+inline hipError_t launch_routed_mixed(const GemmArgs& g, hipStream_t stream) {
+  if (g.M <= 0 || g.N <= 0) return hipSuccess;
+  if (g.splits > 1 || g.splits_more > 1 || g.tail_mode != 0 || g.P_tail != nullptr || g.k_switch != 0 || !direct_slabs_ok(g.K))
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL((routed_mixed_kernel<Tall, Short>), dim3(mixed_blocks(g.M, g.N, Tall::BN_OUT)), dim3(Tall::NT), 0, stream, g);
   return hipGetLastError();
 }
 

@@ -71,6 +71,109 @@ __host__ __device__ inline TileCoord routed_tile_coord(int L, int n_vis, int M, 
   return t;
 }
 
+// Tiles of two heights in one launch, 256 rows ("tall") and 160 ("short", 11/16 of a tall one's time), chosen on the device from
+// the modalities' rows: all tall, or per modality the numbers of either that cost the least - whichever the chip is done with
+// earlier.  Tall tiles past the last whole round run as two short ones where those and the other short ones are one round.
+// The SwiGLU GEMM over 1353 drawn shapes of 0.5 - 30 rounds that the time model gives to 256x256 tiles, caches not flushed, against
+// those tiles with their remainder as 128x128 ones in a second launch (which takes 5 us where it is empty): 4.9 % less time in the
+// geometric mean (8.5 % below a round, 5.8 % up to two, 4.1 % up to four, 2.3 % up to eight), 79 % of them faster and 1 % by more
+// than 3 % slower (0.90).  M = 300 (150 + 150), K = 4096, 14336 columns: 122.7 -> 111.3 us, the MaskedFFN call 212 -> 184; M = 499,
+// K = 5696, 16192 columns 278 -> 200.
+constexpr int kTallRows = 256, kShortRows = 160, kTallCost = 256, kShortCost = 176;
+// A column's weight panel from memory, by the whole chip: 512 bytes per element of the contraction at 6.2 TB/s against the tall
+// tile's 1.056 us per 64 of them.  Tiles of both heights of one modality read it twice (they run at different times).
+constexpr int kColumnCost64 = 85;  // in 64ths
+struct MixedRows {
+  int tall, shrt;
+};
+// The cheapest: whole tall tiles, and the rest as one short tile, as two with the last tall one, or as a tall one.  (Three and
+// more short tiles are never cheaper than tall ones that hold as many rows.)
+__host__ __device__ inline MixedRows mixed_rows(int rows) {
+  static_assert(2 * kShortCost < 2 * kTallCost && kShortCost < kTallCost && 3 * kShortCost > 2 * kTallCost, "costs");
+  const int whole = rows / kTallRows, rest = rows % kTallRows;
+  if (rest == 0) return {whole, 0};
+  if (whole > 0 && rest <= 2 * kShortRows - kTallRows) return {whole - 1, 2};
+  return rest <= kShortRows ? MixedRows{whole, 1} : MixedRows{whole + 1, 0};
+}
+__host__ __device__ inline bool mixed_splits_rest(int tall, int shrt) {
+  const int rest = tall % kCusPerChip;
+  return rest > 0 && 2 * rest + shrt <= kCusPerChip;
+}
+// When the last CU is done: tall tiles first, a CU that is free takes the next tile.
+__host__ __device__ inline int mixed_time(int tall, int shrt) {
+  static_assert(kTallCost == kCusPerChip, "a shift less");
+  const int rest = tall % kCusPerChip, done = tall - rest;
+  if (mixed_splits_rest(tall, shrt)) return done + kShortCost;
+  if (rest == 0) return done + cdiv(shrt, kCusPerChip) * kShortCost;
+  if (shrt <= kCusPerChip - rest) return done + kTallCost;
+  return done + (rest * kTallCost + shrt * kShortCost) / kCusPerChip + kShortCost / 2;  // (the last tiles of a CU end anywhere in half a tile)
+}
+// The same with `reads` modalities' weights read from memory: of the shorter of the two times, 11/16 is not hidden (as fitted for
+// the time model: kDualCost.hidden).
+__host__ __device__ inline int mixed_time(const MixedRows& v, const MixedRows& x, int tiles_n) {
+  const int reads = (v.tall > 0) + (v.shrt > 0) + (x.tall > 0) + (x.shrt > 0);
+  const int tiles = mixed_time((v.tall + x.tall) * tiles_n, (v.shrt + x.shrt) * tiles_n), bytes = reads * tiles_n * kColumnCost64 / 64;
+  return tiles > bytes ? tiles + bytes * 11 / 16 : bytes + tiles * 11 / 16;
+}
+// The tiles of either modality for n_vis and M - n_vis rows.
+__host__ __device__ inline void mixed_choice(int n_vis, int M, int tiles_n, MixedRows* v, MixedRows* x) {
+  *v = mixed_rows(n_vis);
+  *x = mixed_rows(M - n_vis);
+  const MixedRows all_v{cdiv(n_vis, kTallRows), 0}, all_x{cdiv(M - n_vis, kTallRows), 0};
+  if (mixed_time(all_v, all_x, tiles_n) <= mixed_time(*v, *x, tiles_n)) {
+    *v = all_v;
+    *x = all_x;
+  }
+}
+// Workgroups of a launch, for any split of M rows.
+inline int mixed_blocks(int M, int N, int bn) {
+  const int64_t tiles = (int64_t)(cdiv(M, kTallRows) + 1) * cdiv(N, bn) + kCusPerChip / 2;  // with the second halves of split tiles
+  return kXcds * (int)(cdiv64(tiles, kXcds) + 1);
+}
+constexpr int kMixedGroup = 8;
+// Tile of workgroup `bid`; grp < 0: a surplus workgroup.  Every XCD takes an eighth of the tall tiles' order, then an eighth of the
+// short ones'; an order walks the M-tiles of one height and modality column by column, so that the tiles of a column share the
+// weight panel.
+__host__ __device__ inline TileCoord mixed_tile_coord(int bid, int n_vis, int M, int N, int bn, bool* is_tall) {
+  TileCoord t{-1, 0, 0, 0};
+  const int tiles_n = cdiv(N, bn);
+  MixedRows v, x;
+  mixed_choice(n_vis, M, tiles_n, &v, &x);
+  const int tall = (v.tall + x.tall) * tiles_n, shrt = (v.shrt + x.shrt) * tiles_n;
+  const int whole = mixed_splits_rest(tall, shrt) ? tall / kCusPerChip * kCusPerChip : tall;  // tall tiles that run as such
+  const int halves = 2 * (tall - whole);
+  const int per_tall = cdiv(whole, kXcds), per_short = cdiv(halves + shrt, kXcds);
+  int slot = bid / kXcds;
+  *is_tall = slot < per_tall;
+  if (!*is_tall) slot -= per_tall;
+  const int per = *is_tall ? per_tall : per_short;
+  int L = (bid % kXcds) * per + slot;
+  if (slot >= per || L >= (*is_tall ? whole : halves + shrt)) return t;
+  const bool half = !*is_tall && L < halves;
+  const int second = half ? L & 1 : 0;
+  if (half) L = whole + L / 2;
+  else if (!*is_tall) L -= halves;
+  const bool of_tall = *is_tall || half;
+  const int own_v = of_tall ? v.tall : v.shrt, own_x = of_tall ? x.tall : x.shrt;  // M-tiles of this height by modality
+  const int grp = L < own_v * tiles_n ? 0 : 1;
+  if (grp == 1) L -= own_v * tiles_n;
+  const int own = grp == 0 ? own_v : own_x;
+  int first = 0, gsz = own;  // super-group of M-tiles, dealt evenly (routed_tile_coord)
+  if (own > kMixedGroup) {
+    const int groups = cdiv(own, kMixedGroup), s = ((L / tiles_n + 1) * groups - 1) / own;
+    first = s * own / groups;
+    gsz = (s + 1) * own / groups - first;
+    L -= first * tiles_n;
+  }
+  const int begin = grp == 0 ? 0 : n_vis, end = grp == 0 ? n_vis : M;
+  t.row0 = begin + (of_tall ? 0 : (grp == 0 ? v.tall : x.tall) * kTallRows) + (first + L % gsz) * (of_tall ? kTallRows : kShortRows);
+  t.row_end = half && t.row0 + kTallRows < end ? t.row0 + kTallRows : end;
+  t.row0 += second * kShortRows;
+  t.n0 = (L / gsz) * bn;
+  if (t.row0 < t.row_end) t.grp = grp;
+  return t;
+}
+
 // Weight-gradient GEMMs: [groups][splits][tiles_r x tiles_c].  Workgroup b runs on XCD b % 8, and every XCD takes an eighth of
 // EACH group's order, the group with more rows first: the two groups' tiles cost what the groups have rows, and a group
 // without any only stores zeros.  One order over both groups dealt an absent modality's zeros to four XCDs and all of the products

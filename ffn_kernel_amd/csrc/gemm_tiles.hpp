@@ -67,6 +67,7 @@ struct DualTiles {
   using T2 = RoutedGemmCfg<128, 128, 2, 2, true, true, false, DIRECT, kGroupM>;
   using T3 = RoutedGemmCfg<64, 128, 2, 2, true, true, false, DIRECT, kGroupM>;
   using T4 = RoutedGemmCfg<128, 128, 2, 2, true, true, false, DIRECT, kGroupM, false, DIRECT ? 4 : 2>;
+  using Short = RoutedGemmCfg<160, 256, 2, 2, true, true, false, true, kGroupM, false, 3>;  // beside T1, see mixed_rows
   using T6 = std::conditional_t<DIRECT, RoutedGemmCfg<128, 256, 2, 2, true, true, false, true, kGroupM, false, 3>, T2>;
   using T7 = std::conditional_t<DIRECT, RoutedGemmCfg<64, 128, 2, 2, true, true, false, true, kGroupM, false, 3>, T3>;
 };

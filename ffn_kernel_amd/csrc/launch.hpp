@@ -19,7 +19,8 @@ enum TileId : int {
   // 5 names a form of the weight-gradient GEMM in its plans (kTileGatherDw), not a tile
   TILE_128x256_R3 = 6,  // 128 rows x 256 weight rows (SwiGLU: 128 gate + 128 up), 4 waves, ring of three LDS stages
   TILE_64x128_R3 = 7,   // 64 rows x 128 weight rows (SwiGLU: 64 gate + 64 up), 4 waves, ring of three LDS stages, two workgroups per CU
-  TILE_COUNT = 8
+  TILE_COUNT = 8,       // ids below can be forced; the next follows from TILE_256x256_W4 in the SwiGLU GEMM
+  TILE_MIXED_W4 = 8     // 256x256 and 160x256 tiles in one launch, 4 waves
 };
 
 // The two 256x256 tiles: past one round of the chip they run whole rounds first and the remainder apart.

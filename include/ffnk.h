@@ -68,7 +68,8 @@ enum {
  * its A100-tuned JSON tables: ffn_kernel/utils.py:3-5, ffn_kernel/bf16_*_fwd.json). */
 typedef struct ffnk_tile_config_t {
   int32_t path;        /* FFNK_PATH_*                                              */
-  int32_t block_m;     /* token rows per workgroup tile                            */
+  int32_t block_m;     /* token rows per workgroup tile (SwiGLU GEMM, 256 on four
+                          waves: beside tiles of 160, up to eight rounds of tiles)  */
   int32_t block_n;     /* output columns per workgroup tile                        */
   int32_t block_k;     /* contraction elements per LDS stage / per streamed chunk  */
   int32_t waves_m;     /* wavefront grid inside the workgroup                      */

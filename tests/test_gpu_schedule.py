@@ -171,3 +171,24 @@ def test_backward_ragged_intermediate(dev, forced, tile, splits, h):
         W[i] = behind[:h]
     forced(tile, splits)
     assert_ffn_backward(x, W, mask, g, f"h {h} tile {tile}")
+
+
+# The SwiGLU GEMM on tiles of two heights in one launch: rows of a modality that fill a short tile, that one row more does not,
+# that are two short tiles, a tall one and the rest; one modality; several super-groups.  Contractions of one slab, of fewer than
+# the short tile's stages, ragged ones; columns of whole rounds, just past one (the rest as halves) and a ragged last tile.
+@pytest.mark.parametrize("nv,nt,h", [(1, 511, 32768), (160, 352, 32768), (161, 256, 33000), (262, 157, 32776), (576, 835, 11528),
+                                     (0, 700, 24576), (2060, 100, 7432), (256, 256, 32896)])
+@pytest.mark.parametrize("d", [64, 128, 200, 328])
+def test_tiles_of_two_heights(dev, nv, nt, h, d):
+    note(f"tiles of two heights: nv={nv} nt={nt} h={h} d={d}")
+    cfg = _lib.tile_config(_lib.OP_FFN_UP, nv + nt, d, h)
+    assert (cfg["block_m"], cfg["waves_m"] * cfg["waves_n"]) == (256, 4)  # the plan that the mixed launch follows from
+    x, W, mask, _ = ffn_case(dev, nv, nt, d, h, seed=h + d)
+    W = [w * 0.5 for w in W]
+    out, pre = masked_ffn_forward(x, *[w.T for w in W], mask, save_pre=True)
+    assert_close(out, select_ffn(x, W, mask).cpu(), "out")
+    assert torch.equal(out, masked_ffn_forward(x, *[w.T for w in W], mask))
+    order = torch.cat([mask.nonzero(), (~mask).nonzero()]).flatten()
+    xs, m = x[order].double(), mask[order][:, None]
+    for half, (v, t) in enumerate(((W[0], W[3]), (W[2], W[5]))):
+        assert_close(pre[:, half * h:(half + 1) * h], torch.where(m, xs @ v.double().T, xs @ t.double().T).cpu(), f"pre {half}")

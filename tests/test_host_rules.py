@@ -175,3 +175,26 @@ def test_weight_gradient_order(rules, tiles_r, tiles_c, splits, n_vis, M):
     for groups in per_xcd.values():
         assert groups.count(0) == groups.count(1) <= share
         assert groups == sorted(groups, key=lambda g: g != larger)
+
+
+# Rows of a modality at the edges of what tall and short tiles hold, either modality absent; columns that make less than a round
+# of tiles, just past one (the rest as halves), several.
+@pytest.mark.parametrize("n_vis", [0, 1, 159, 160, 161, 256, 257, 320, 321, 416, 576, 577, 672, 835, 1500, 2060, 4700])
+@pytest.mark.parametrize("n_text", [0, 160, 262, 480, 1025])
+def test_tiles_of_two_heights_cover_every_row(rules, n_vis, n_text):
+    """Every row of either modality in one tile of every column, no tile astride the modalities."""
+    M, bn = n_vis + n_text, 128
+    t = (ctypes.c_int * 4)()
+    for tiles_n in (5, 43, 90, 129, 258) if M else ():
+        covered = {}
+        for b in range(rules.hc_mixed_blocks(M, tiles_n * bn - 120, bn)):
+            rules.hc_mixed_tile(b, n_vis, M, tiles_n * bn - 120, bn, t)
+            grp, row0, end, n0 = t
+            if grp == -1:
+                continue
+            assert grp == (0 if row0 < n_vis else 1) and row0 < end <= (n_vis if grp == 0 else M)
+            covered.setdefault(n0, []).append((row0, end))
+        assert sorted(covered) == list(range(0, tiles_n * bn, bn))
+        for tiles in covered.values():
+            tiles.sort()
+            assert tiles[0][0] == 0 and tiles[-1][1] == M and all(a[1] == b[0] for a, b in zip(tiles, tiles[1:]))
