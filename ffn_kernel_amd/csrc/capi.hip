@@ -1167,7 +1167,8 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
     FFNK_HIP(launch_gather_gemm(routed_tile(M, h, false), up_direct, a, stream), "t3 GEMM");
   }
 
-  // ---- dh = gather(g) @ A2^T: contraction over d needs the down weights as [h, d] rows ----
+  // ---- dh = gather(g) @ A2^T, and on its tiles T13 <- (dt1 | dt3), DH <- the SwiGLU intermediate: contraction over d needs the
+  // down weights as [h, d] rows ----
   const uint16_t* w2t[2] = {W2, U2};
   int64_t ld2 = down_stride_k;
   if (w2_kmajor) {
@@ -1181,15 +1182,12 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
   }
   a.A = g; a.lda = g_stride_m; a.B0[0] = w2t[0]; a.B0[1] = w2t[1]; a.ldb = ld2;
   a.C = DH; a.ldc = h;
+  a.pre = pre ? pre : T13; a.ld_pre = pre ? pre_stride_m : ld13; a.half_pre = (int)(pre ? h : half);
+  a.T13 = T13; a.ld13 = ld13; a.half = (int)half;
   const bool dh_direct = w2_kmajor || direct_ok(d, M, g_stride_m, ld2);
   const int dh_tile = bwd_tile(M, h, d, dh_direct);
   if (w2_kmajor) FFNK_HIP(launch_gather_gemm_kmajor(dh_tile, a, stream), "dh GEMM");
   else FFNK_HIP(launch_gather_gemm(dh_tile, dh_direct, a, stream), "dh GEMM");
-
-  // ---- elementwise: T13 <- (dt1 | dt3), DH <- the SwiGLU intermediate ----
-  FFNK_HIP(launch_swiglu_bwd(pre ? pre : T13, pre ? pre_stride_m : ld13, (int)(pre ? h : half), T13, ld13, (int)half, DH, h, (int)M, (int)h,
-                             stream),
-           "SwiGLU backward pass");
 
   // ---- dx = (dt1 | dt3) @ (A1^T | A3^T)^T: one GEMM over the concatenated contraction ----
   // In place over the K-major up-projection weights, or over one [d, 2h] copy per modality.

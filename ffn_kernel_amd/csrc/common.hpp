@@ -42,6 +42,29 @@ __device__ __forceinline__ float swiglu(float g, float u) {
   return g * s * u;
 }
 
+// SwiGLU backward on eight bf16 values: o1 = dh * t3 * silu'(t1), o3 = dh * silu(t1), oh = silu(t1) * t3.
+// silu'(t) = s + t s (1 - s), s = sigmoid(t), in fp32 (the derivative term sketched in the reference's README.md:159-172 is not this one).
+__device__ __forceinline__ void swiglu_bwd(const uint4& t1, const uint4& t3, const uint4& dh, uint4* o1, uint4* o3, uint4* oh) {
+  auto word = [](const uint4& v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; };
+  auto set = [](uint4* v, int i, uint32_t w) { (i == 0 ? v->x : i == 1 ? v->y : i == 2 ? v->z : v->w) = w; };
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float r1[2], r3[2], rh[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      auto value = [&](const uint4& v) { return __builtin_bit_cast(float, e == 0 ? word(v, i) << 16 : word(v, i) & 0xffff0000u); };
+      const float a = value(t1), b = value(t3), d = value(dh);
+      const float s = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(a * -1.44269504088896341f)), silu = a * s;  // as swiglu()
+      r1[e] = d * b * (s + silu * (1.0f - s));
+      r3[e] = d * silu;
+      rh[e] = silu * b;
+    }
+    set(o1, i, pack2bf(r1[0], r1[1]));
+    set(o3, i, pack2bf(r3[0], r3[1]));
+    set(oh, i, pack2bf(rh[0], rh[1]));
+  }
+}
+
 // p[0] + p[stride] + ... + p[(n - 1) * stride], in that order.  The loads of up to four terms are in flight together: one
 // after the other, a reduce pass over few workgroups is n memory round trips long.  Over 13000 drawn calls with partials a call
 // gains 0.2 - 0.4 us with two or three K ranges, 0.5 - 0.7 with four to seven and 1.4 with eight and more (MaskedLinear at

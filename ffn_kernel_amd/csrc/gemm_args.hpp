@@ -25,6 +25,18 @@ struct GemmArgs {
   // backward need not recompute them.  NULL: not stored.
   uint16_t* C_pre = nullptr;
   int64_t ldc_pre = 0;
+  // Gather kernels only (GATHER_A, rows of C in routed order), SwiGLU backward instead of the plain result: always over K-major weights, by
+  // choice over row-major ones.  With
+  // dh = A B0^T, t1 = pre[row, n], t3 = pre[row, half_pre + n] (rows in routed order):
+  //   T13[row, n] = dh * t3 * silu'(t1),  T13[row, half + n] = dh * silu(t1),  C[row, n] = silu(t1) * t3   for n < N
+  //   T13[row, n] = T13[row, half + n] = 0                                                                 for N <= n < half
+  // pre may be T13 with the same halves and row stride.  half <= N rounded up to 64, whole 16-byte chunks everywhere.
+  const uint16_t* pre = nullptr;
+  int64_t ld_pre = 0;
+  int half_pre = 0;
+  uint16_t* T13 = nullptr;
+  int64_t ld13 = 0;
+  int half = 0;
   const int32_t* perm;   // routed position -> token row
   const int32_t* counts; // counts[0] = visual rows (device memory)
   int M, N, K;           // N = output columns
@@ -52,6 +64,12 @@ struct GemmArgs {
   // runs as smaller tiles over all of K (tail_mode 2).
   float* P_tail = nullptr;
 };
+
+inline bool swiglu_bwd_args_ok(const GemmArgs& g) {
+  const uintptr_t at = reinterpret_cast<uintptr_t>(g.pre) | reinterpret_cast<uintptr_t>(g.T13) | reinterpret_cast<uintptr_t>(g.C);
+  return g.pre != nullptr && g.T13 != nullptr && at % 16 == 0 && (g.ld_pre | g.half_pre | g.ld13 | g.half | g.ldc | g.N) % 8 == 0 && g.half_pre >= g.N &&
+         g.half >= g.N && g.half <= (g.N + 63) / 64 * 64 && g.ld_pre >= g.half_pre + g.N && g.ld13 >= 2 * (int64_t)g.half && g.splits == 1;
+}
 
 // Grouped split-K GEMM used for the weight gradients:
 //   P[grp][split][R, Cc] (fp32) = sum over this split's 64-column slabs of  A[R, k] * B[Cc, k]^T

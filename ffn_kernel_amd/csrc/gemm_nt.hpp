@@ -1354,6 +1354,59 @@ struct WaveRows {
   }
 };
 
+// Epilogue of the feed-forward backward's dh GEMM: the SwiGLU derivative on the tile, dh rounded to bf16 (GemmArgs::T13).  A chunk of
+// eight columns is read from the pre-activations and written by one lane, so that they may be T13 itself.  Bound by its five
+// passes over [M, h] (45 us per round of 256x256 tiles against 7 of plain stores); as a launch of its own the derivative made six
+// and read dh back: forward + backward at M = 4096, d = 4096, h = 14336 3550 -> 3514 us, and up to
+// 1.8 % less over 22 drawn layers that the device bounds, none slower.
+template <class Cfg>
+__device__ __forceinline__ void swiglu_bwd_epilogue(const GemmArgs& g, typename Cfg::Acc (&acc)[Cfg::TM][Cfg::TN], int row0, int row_end,
+                                                    int n0, const TileLanes<Cfg>& tl, uint8_t* lds) {
+  using W = WaveRows<Cfg>;
+  constexpr int BATCH = W::N < 8 ? 2 : 4, BATCHES = W::N / BATCH;
+  static_assert(W::N % (2 * BATCH) == 0, "pairs of batches");
+  const int n = n0 + tl.wn * Cfg::WTN_OUT + W::col(tl.lane), p = row0 + tl.wm * Cfg::WTM + W::row(0, tl.lane);
+  const bool in = n < g.N;
+  uint4 t1[2][BATCH], t3[2][BATCH];
+  auto load = [&](int b, int buf) {
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k) {
+      const int row = min(p + (b * BATCH + k) * W::PER, row_end - 1);  // (past the edges: a row and columns that exist, not stored)
+      const uint16_t* src = g.pre + (int64_t)row * g.ld_pre + min(n, g.N - 8);
+      t1[buf][k] = *reinterpret_cast<const uint4*>(src);
+      t3[buf][k] = *reinterpret_cast<const uint4*>(src + g.half_pre);
+    }
+  };
+  auto step = [&](int b, int buf) {
+    if (b + 1 < BATCHES) load(b + 1, buf ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k) {
+      const int row = p + (b * BATCH + k) * W::PER;
+      uint4 o1, o3, oh;
+      swiglu_bwd(t1[buf][k], t3[buf][k], W::get(lds, tl.wave, tl.lane, b * BATCH + k), &o1, &o3, &oh);
+      if (row >= row_end || n >= g.half) continue;
+      uint16_t* dst = g.T13 + (int64_t)row * g.ld13 + n;
+      if (in) *reinterpret_cast<uint4*>(g.C + (int64_t)row * g.ldc + n) = oh;
+      else o1 = o3 = make_uint4(0, 0, 0, 0);  // (the weight rows there are others')
+      *reinterpret_cast<uint4*>(dst) = o1;
+      *reinterpret_cast<uint4*>(dst + g.half) = o3;
+    }
+  };
+  dma_wait_barrier<0>();  // every wave has read its last fragments
+  W::put(lds, tl.wave, tl.lr, tl.lh, [&](int i, int j, int q4) {
+    const typename Cfg::Acc& t = acc[i][j];
+    return make_uint2(pack2bf(t[4 * q4], t[4 * q4 + 1]), pack2bf(t[4 * q4 + 2], t[4 * q4 + 3]));
+  });
+  __builtin_amdgcn_sched_barrier(0);
+  load(0, 0);
+#pragma unroll 1  // (unrolled, the rows' addresses do not fit beside the four-wave tile's accumulators)
+  for (int b = 0; b < BATCHES; b += 2) {
+    step(b, 0);
+    step(b + 1, 1);
+  }
+}
+
 // Epilogue shared by the routed kernels.  Per accumulator tile a lane holds token row lr and the output
 // columns acc_col(v, lh), i.e. runs of four consecutive columns.
 template <class Cfg>
@@ -1363,6 +1416,12 @@ __device__ __forceinline__ void routed_epilogue(const GemmArgs& g, typename Cfg:
   const int wm = tl.wm, wn = tl.wn;
   const uint32_t lr = tl.lr, lh = tl.lh;
   const bool save = Cfg::DUAL && g.C_pre != nullptr;  // uniform over the launch, like all of these
+  if constexpr (Cfg::GATHER_A && !Cfg::SCATTER_C && !Cfg::DUAL) {
+    if (Cfg::B_KMAJOR || g.T13 != nullptr) {
+      swiglu_bwd_epilogue<Cfg>(g, acc, row0, row_end, n0, tl, lds);
+      return;
+    }
+  }
   // Whole 16-byte chunks of the output's rows: through LDS, any edge a lane's own guard.
   if (g.N % 8 == 0 && g.ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(g.C) & 15) == 0 &&
       (!save || (g.ldc_pre % 8 == 0 && (reinterpret_cast<uintptr_t>(g.C_pre) & 15) == 0))) {
@@ -1860,6 +1919,8 @@ inline hipError_t launch_routed_gemm(const GemmArgs& g, hipStream_t stream) {
                         (g.k_switch > 0 && g.K % kBK != 0) || g.ldb * (kBK * 2) + 2 * (int64_t)g.N >= ((int64_t)1 << 32)))
     return hipErrorInvalidValue;
   if (!Cfg::B_KMAJOR && g.k_switch != 0) return hipErrorInvalidValue;
+  constexpr bool kGather = Cfg::GATHER_A && !Cfg::SCATTER_C && !Cfg::DUAL;
+  if ((g.T13 != nullptr || (kGather && Cfg::B_KMAJOR)) && !(kGather && swiglu_bwd_args_ok(g))) return hipErrorInvalidValue;
   if (g.k_rows != 0 && (g.k_rows < 0 || g.k_switch != round_up64(g.k_rows, kBK) || g.K != 2 * g.k_switch)) return hipErrorInvalidValue;
   const int grid = routed_gemm_grid<Cfg>(g.M, g.N, g.splits, g.splits_more);
   hipLaunchKernelGGL(routed_gemm_kernel<Cfg>, dim3(grid), dim3(Cfg::NT), 0, stream, g);

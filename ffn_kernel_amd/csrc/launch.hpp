@@ -79,14 +79,6 @@ hipError_t launch_gather_transpose2(const uint16_t* src0, int64_t ld0, int cols0
                                     bool routed0 = false, bool routed1 = false);
 // routedN: source N's rows are already in routed order (row p instead of row perm[p]).
 
-// SwiGLU backward, elementwise over routed-order rows (MaskedFFN backward):
-//   t1 = pre[p, j], t3 = pre[p, half_pre + j], dh = DH[p, j]
-//   T13[p, j] <- dh * t3 * silu'(t1),  T13[p, half + j] <- dh * silu(t1),  DH[p, j] <- silu(t1) * t3   for j < h
-//   T13[p, j] <- 0, T13[p, half + j] <- 0                                                              for h <= j < half
-// Row strides ld_pre >= 2 * half_pre, ld13 >= 2 * half, ldh >= h (pre may be T13 with the same halves: in place); all multiples
-// of 8.
-hipError_t launch_swiglu_bwd(const uint16_t* pre, int64_t ld_pre, int half_pre, uint16_t* T13, int64_t ld13, int half, uint16_t* DH,
-                             int64_t ldh, int M, int h, hipStream_t stream);
 // out_g[r * sr + c * sc] = bf16(sum_s P[g][s][r][c]) for g in {0, 1}.
 hipError_t launch_splitk_reduce(const float* P, int splits, int R, int Cc, uint16_t* out0, uint16_t* out1,
                                 int64_t sr, int64_t sc, hipStream_t stream);

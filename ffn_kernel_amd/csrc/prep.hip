@@ -159,54 +159,6 @@ hipError_t launch_gather_transpose2(const uint16_t* src0, int64_t ld0, int cols0
   return hipGetLastError();
 }
 
-// SwiGLU backward in place (see launch.hpp); 8 columns per thread, fp32 maths, bf16 storage.  The
-// derivative is the textbook one, silu'(t) = s + t s (1 - s) with s = sigmoid(t) (the reference's
-// README.md:159-172 sketches this pass; its derivative term there is not this one and is not used).
-__global__ __launch_bounds__(256) void swiglu_bwd_kernel(const uint16_t* pre, int64_t ld_pre, int half_pre, uint16_t* T13,
-                                                         int64_t ld13, int half, uint16_t* __restrict__ DH, int64_t ldh, int M,
-                                                         int h) {
-  const int half8 = half >> 3;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)M * half8) return;
-  const int p = (int)(idx / half8), j = (int)(idx % half8) * 8;
-  const uint16_t* ps1 = pre + (int64_t)p * ld_pre + j;  // may be T13 itself (in place)
-  uint16_t* pt1 = T13 + (int64_t)p * ld13 + j;
-  uint16_t* pt3 = pt1 + half;
-  if (j >= h) {
-    *reinterpret_cast<uint4*>(pt1) = *reinterpret_cast<uint4*>(pt3) = make_uint4(0, 0, 0, 0);
-    return;
-  }
-  uint16_t* pdh = DH + (int64_t)p * ldh + j;
-  uint16_t t1[8], t3[8], dh[8];
-  *reinterpret_cast<uint4*>(t1) = *reinterpret_cast<const uint4*>(ps1);
-  *reinterpret_cast<uint4*>(t3) = *reinterpret_cast<const uint4*>(ps1 + half_pre);
-  *reinterpret_cast<uint4*>(dh) = *reinterpret_cast<const uint4*>(pdh);
-  uint16_t o1[8], o3[8], oh[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float a = bf2f(t1[e]), b = bf2f(t3[e]), g = bf2f(dh[e]);
-    const float s = 1.0f / (1.0f + __expf(-a));
-    const float silu = a * s;
-    o1[e] = f2bf(g * b * (s + silu * (1.0f - s)));
-    o3[e] = f2bf(g * silu);
-    oh[e] = f2bf(silu * b);
-  }
-  *reinterpret_cast<uint4*>(pt1) = *reinterpret_cast<const uint4*>(o1);
-  *reinterpret_cast<uint4*>(pt3) = *reinterpret_cast<const uint4*>(o3);
-  *reinterpret_cast<uint4*>(pdh) = *reinterpret_cast<const uint4*>(oh);
-}
-
-hipError_t launch_swiglu_bwd(const uint16_t* pre, int64_t ld_pre, int half_pre, uint16_t* T13, int64_t ld13, int half, uint16_t* DH,
-                             int64_t ldh, int M, int h, hipStream_t stream) {
-  if (M <= 0 || h <= 0) return hipSuccess;
-  if (h % 8 != 0 || half % 8 != 0 || half_pre % 8 != 0 || ld13 % 8 != 0 || ldh % 8 != 0 || ld_pre % 8 != 0 || half < h || half_pre < h)
-    return hipErrorInvalidValue;
-  const int64_t n = (int64_t)M * (half / 8);
-  hipLaunchKernelGGL(swiglu_bwd_kernel, dim3((unsigned)cdiv64(n, 256)), dim3(256), 0, stream, pre, ld_pre, half_pre, T13, ld13, half, DH,
-                     ldh, M, h);
-  return hipGetLastError();
-}
-
 // out_g[r * sr + c * sc] = bf16(P[g][0][r][c] + P[g][1][r][c] + ...), summed in split order so
 // that the result does not depend on scheduling.  VEC: four consecutive columns per thread (16-byte loads of the
 // partials, one 8-byte store), for outputs whose columns are contiguous (sc == 1) and Cc % 4 == 0.

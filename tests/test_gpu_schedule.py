@@ -192,3 +192,21 @@ def test_tiles_of_two_heights(dev, nv, nt, h, d):
     xs, m = x[order].double(), mask[order][:, None]
     for half, (v, t) in enumerate(((W[0], W[3]), (W[2], W[5]))):
         assert_close(pre[:, half * h:(half + 1) * h], torch.where(m, xs @ v.double().T, xs @ t.double().T).cpu(), f"pre {half}")
+
+
+# The SwiGLU derivative on the dh GEMM's tiles: row and column edges of every tile, halves padded to whole slabs (h = 328, 72) and
+# not, pre-activations kept by a forward (also in rows wider than they are) and recomputed in place; down weights in both layouts.
+@pytest.mark.parametrize("tile", [-1, 0, 1, 2, 3, 4, 6, 7])
+@pytest.mark.parametrize("nv,nt,d,h", [(1, 66, 136, 72), (130, 257, 128, 328), (0, 300, 200, 512)])
+def test_swiglu_backward_in_the_epilogue(dev, forced, tile, nv, nt, d, h):
+    note(f"SwiGLU backward in the epilogue: nv={nv} nt={nt} d={d} h={h} tile={tile}")
+    x, W, mask, g = ffn_case(dev, nv, nt, d, h, seed=d + h)
+    forced(tile)
+    assert_ffn_backward(x, W, mask, g, f"tile {tile}")
+    for views in ([w.T for w in W], [w.T.contiguous() if i % 3 == 1 else w.T for i, w in enumerate(W)]):
+        _, pre = masked_ffn_forward(x, *views, mask, save_pre=True)
+        wide = torch.full((nv + nt, 2 * h + 24), float("nan"), dtype=torch.bfloat16, device=dev)
+        wide[:, :2 * h] = pre
+        kept = masked_ffn_backward(g, x, *views, mask, pre=pre)
+        for other in (masked_ffn_backward(g, x, *views, mask, pre=wide[:, :2 * h]), masked_ffn_backward(g, x, *views, mask)):
+            assert all(torch.equal(a, b) for a, b in zip(kept, other))
