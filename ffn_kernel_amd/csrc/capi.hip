@@ -373,6 +373,22 @@ RoutedPlan ffn_bwd_dx_plan(int64_t M, int64_t d, int64_t contraction, bool dx_di
   if (need) *need = n;
   return dxp;
 }
+// The dx GEMM (plan dxp) in one launch with the weight gradients, uncut: where both run on 256x256 tiles, dx's own rounds would be
+// less than 0.7 full - a split tail or K ranges, and a reduce pass - and its workgroups are done in 3/4 of the time of all work
+// spread over the chip (a tile costs its slabs and about eight more).  Forward + backward, apart -> beside, of 34 drawn layers those
+// inside these lines: 2.2 to 5.0 % less where dx fills half a round or a little more than whole ones (d = 4184, h = 13480, M = 1995
+// 2214 -> 2108 us, d = 4160, h = 9024, M = 1284 1006 -> 967, d = 5760, h = 14336, M = 2589 3462 -> 3359), none slower; M = 4096,
+// d = 4096, h = 14336 3553 -> 3552.  Outside: fuller rounds up to 2.2 % more (d = 4288, h = 14208, M = 7144 6317 -> 6458), 9/10 of
+// the time and more +-0.5 %; below ten slabs per weight-gradient tile those are bound by their stores and slow dx down (d = 6976,
+// h = 23232, M = 471 1817 -> 2066).
+bool ffn_bwd_dx_beside_dw(int64_t M, int64_t d, int64_t h, int64_t contraction, const RoutedPlan& dxp, const TileChoice& dw) {
+  constexpr int64_t kFixed = 8, kDwSlabs = 10;
+  if (!is_big_tile(dxp.tile) || dw.tile != TILE_256x256_W8 || dw.splits != 1 || forced_splits() > 1) return false;
+  const int64_t tiles_n = cdiv64(d, 256), dx_tiles = (cdiv64(M, 256) + 1) * tiles_n, dw_tiles = 2 * kDwBatch * cdiv64(h, 256) * tiles_n;
+  const int64_t slabs = contraction / 64, dw_slabs = cdiv64(M, 128), rounds = cdiv64(dx_tiles, kCus);
+  return dw_slabs >= kDwSlabs && 10 * dx_tiles < 7 * rounds * kCus &&
+         4 * rounds * (slabs + kFixed) * kCus <= 3 * (dx_tiles * (slabs + kFixed) + dw_tiles * (dw_slabs + kFixed));
+}
 // Paths of the MaskedFFN backward for one layout: which weights are read in place and which copied, and whether
 // H, dt1, dt3 are read in place by the weight-gradient GEMMs.  The backward and the lean workspace query both ask
 // here, so that the regions a call touches are the regions its plan holds.
@@ -1214,18 +1230,27 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
   size_t dx_need = 0;
   const RoutedPlan dxp = ffn_bwd_dx_plan(M, d, ld13, dx_direct, 2 * ws_align((size_t)h * d * 2), &dx_need);
   if (dx_need > p.w2t_bytes) return fail(FFNK_E_WORKSPACE, "internal: dx partials %zu > %zu planned", dx_need, p.w2t_bytes);
-  if (dxp.splits > 1) {
-    b.splits = dxp.splits;
-    b.splits_more = dxp.splits_more;
-    b.P = reinterpret_cast<float*>(wsb + p.off_w2t);
-  } else if (dx_need > 0) {
-    b.P_tail = reinterpret_cast<float*>(wsb + p.off_w2t);  // split tail of the last, partial round
+  TileChoice in_place_choice;
+  bool beside_dw = false;
+  if (paths.acts_in_place) {
+    in_place_choice = ffn_bwd_in_place_choice(M, d, h);
+    if (forced_tile() >= 0) in_place_choice.tile = forced_tile();
+    beside_dw = w13_kmajor && ffn_bwd_dx_beside_dw(M, d, h, ld13, dxp, in_place_choice);
   }
-  if (w13_kmajor) FFNK_HIP(launch_down_gemm_kmajor(dxp.tile, b, stream), "dx GEMM");
-  else FFNK_HIP(launch_down_gemm(dxp.tile, dx_direct, b, stream), "dx GEMM");
-  if (dxp.splits > 1)
-    FFNK_HIP(launch_routed_reduce(b.P, dxp.splits, dxp.splits_more, tile_geom(dxp.tile, false).block_m, (int)M, (int)d, rt.counts, rt.perm,
-                                  dx, dx_stride_m, stream), "dx reduce");
+  if (!beside_dw) {
+    if (dxp.splits > 1) {
+      b.splits = dxp.splits;
+      b.splits_more = dxp.splits_more;
+      b.P = reinterpret_cast<float*>(wsb + p.off_w2t);
+    } else if (dx_need > 0) {
+      b.P_tail = reinterpret_cast<float*>(wsb + p.off_w2t);  // split tail of the last, partial round
+    }
+    if (w13_kmajor) FFNK_HIP(launch_down_gemm_kmajor(dxp.tile, b, stream), "dx GEMM");
+    else FFNK_HIP(launch_down_gemm(dxp.tile, dx_direct, b, stream), "dx GEMM");
+    if (dxp.splits > 1)
+      FFNK_HIP(launch_routed_reduce(b.P, dxp.splits, dxp.splits_more, tile_geom(dxp.tile, false).block_m, (int)M, (int)d, rt.counts, rt.perm,
+                                    dx, dx_stride_m, stream), "dx reduce");
+  }
 
   // ---- weight gradients: contraction over the rows of each group.  x and g are gathered into
   // 64-padded transposes; H, dt1 and dt3 (routed order already) are read in place by the K-major
@@ -1237,8 +1262,7 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
   if (in_place) {
     FFNK_HIP(launch_gather_transpose2(g, g_stride_m, (int)d, GT, x, x_stride_m, (int)d, XT, p.ldt, rt.perm, rt.counts, (int)M,
                                       stream, false, false), "g / x transpose");
-    const TileChoice tc = ffn_bwd_in_place_choice(M, d, h);
-    const int tile = forced_tile() >= 0 ? forced_tile() : tc.tile;
+    const TileChoice& tc = in_place_choice;
     // out[r * sr + c * sc]: r runs over h (the in-place operand's columns), c over d
     auto weight_grad = [&](const uint16_t* rows, int64_t ld_rows, const uint16_t* cT, uint16_t* o0, uint16_t* o1, int64_t sr, int64_t sc) {
       SplitKArgs s;
@@ -1252,14 +1276,18 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
     const SplitKArgs dw[kDwBatch] = {weight_grad(DH, h, GT, dW2, dU2, ddown_stride_k, ddown_stride_n),
                                      weight_grad(T13, ld13, XT, dW1, dU1, dup_stride_n, dup_stride_k),
                                      weight_grad(T13 + half, ld13, XT, dW3, dU3, dup_stride_n, dup_stride_k)};
+    if (beside_dw) {
+      FFNK_HIP(launch_dx_dw_batch_kmajor(b, dw, stream), "dx / dW GEMMs");
+      return FFNK_OK;
+    }
     if (tc.splits == 1) {
-      FFNK_HIP(launch_dw_batch_kmajor(tile, dw, stream), "dW GEMMs");
+      FFNK_HIP(launch_dw_batch_kmajor(tc.tile, dw, stream), "dW GEMMs");
       return FFNK_OK;
     }
     for (SplitKArgs s : dw) {
       uint16_t *o0 = s.out[0], *o1 = s.out[1];
       s.out[0] = s.out[1] = nullptr;
-      FFNK_HIP(launch_splitk_gemm_kmajor(tile, s, stream), "dW split-K GEMM");
+      FFNK_HIP(launch_splitk_gemm_kmajor(tc.tile, s, stream), "dW split-K GEMM");
       FFNK_HIP(launch_splitk_reduce(P, tc.splits, (int)h, (int)d, o0, o1, s.out_sr, s.out_sc, stream), "dW reduce");
     }
     return FFNK_OK;

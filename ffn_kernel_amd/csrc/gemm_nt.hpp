@@ -1910,18 +1910,23 @@ inline int routed_gemm_grid(int M, int N, int splits = 1, int splits_more = 1) {
 }
 
 template <class Cfg>
-inline hipError_t launch_routed_gemm(const GemmArgs& g, hipStream_t stream) {
-  if (g.M <= 0 || g.N <= 0) return hipSuccess;
-  if ((g.splits > 1 || g.splits_more > 1) && (Cfg::DUAL || !Cfg::DIRECT || g.tail_mode != 0 || g.P == nullptr)) return hipErrorInvalidValue;
-  if ((g.splits > 1) != (g.splits_more > 1)) return hipErrorInvalidValue;
-  if (Cfg::DIRECT && !direct_slabs_ok(g.K)) return hipErrorInvalidValue;
+inline bool routed_gemm_args_ok(const GemmArgs& g) {
+  if ((g.splits > 1 || g.splits_more > 1) && (Cfg::DUAL || !Cfg::DIRECT || g.tail_mode != 0 || g.P == nullptr)) return false;
+  if ((g.splits > 1) != (g.splits_more > 1)) return false;
+  if (Cfg::DIRECT && !direct_slabs_ok(g.K)) return false;
   if (Cfg::B_KMAJOR && (g.N % 8 != 0 || g.k_switch % kBK != 0 || g.k_switch < 0 || g.k_switch >= g.K ||
                         (g.k_switch > 0 && g.K % kBK != 0) || g.ldb * (kBK * 2) + 2 * (int64_t)g.N >= ((int64_t)1 << 32)))
-    return hipErrorInvalidValue;
-  if (!Cfg::B_KMAJOR && g.k_switch != 0) return hipErrorInvalidValue;
+    return false;
+  if (!Cfg::B_KMAJOR && g.k_switch != 0) return false;
   constexpr bool kGather = Cfg::GATHER_A && !Cfg::SCATTER_C && !Cfg::DUAL;
-  if ((g.T13 != nullptr || (kGather && Cfg::B_KMAJOR)) && !(kGather && swiglu_bwd_args_ok(g))) return hipErrorInvalidValue;
-  if (g.k_rows != 0 && (g.k_rows < 0 || g.k_switch != round_up64(g.k_rows, kBK) || g.K != 2 * g.k_switch)) return hipErrorInvalidValue;
+  if ((g.T13 != nullptr || (kGather && Cfg::B_KMAJOR)) && !(kGather && swiglu_bwd_args_ok(g))) return false;
+  return g.k_rows == 0 || (g.k_rows > 0 && g.k_switch == round_up64(g.k_rows, kBK) && g.K == 2 * g.k_switch);
+}
+
+template <class Cfg>
+inline hipError_t launch_routed_gemm(const GemmArgs& g, hipStream_t stream) {
+  if (g.M <= 0 || g.N <= 0) return hipSuccess;
+  if (!routed_gemm_args_ok<Cfg>(g)) return hipErrorInvalidValue;
   const int grid = routed_gemm_grid<Cfg>(g.M, g.N, g.splits, g.splits_more);
   hipLaunchKernelGGL(routed_gemm_kernel<Cfg>, dim3(grid), dim3(Cfg::NT), 0, stream, g);
   return hipGetLastError();

@@ -16,10 +16,9 @@ struct DwBatch {
 };
 
 template <class AlongR, class AlongC>
-__global__ __launch_bounds__(AlongC::NT) void dw_batch_kernel(const DwBatch b) {
+__device__ __forceinline__ void dw_batch_body(const DwBatch& b, uint8_t* lds, const int block) {
   static_assert(AlongR::LDS_BYTES == AlongC::LDS_BYTES && AlongR::NT == AlongC::NT && kDwBatch == 3, "the same tile");
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[AlongC::LDS_BYTES];
-  const int which = (int)blockIdx.x / b.blocks, bid = (int)blockIdx.x - which * b.blocks;
+  const int which = block / b.blocks, bid = block - which * b.blocks;
   // Selected member by member: an index into the kernel's arguments would put them in scratch memory.
   auto pick = [&](auto first, auto second, auto third) { return which == 0 ? first : which == 1 ? second : third; };
   SplitKArgs s = b.s[0];
@@ -36,33 +35,65 @@ __global__ __launch_bounds__(AlongC::NT) void dw_batch_kernel(const DwBatch b) {
 }
 
 template <class AlongR, class AlongC>
-static hipError_t launch_batch(DwBatch& b, hipStream_t stream) {
-  for (const SplitKArgs& s : b.s)
-    if (s.R % 8 != 0 || s.lda * (kBK * 2) + 2 * (int64_t)s.R >= ((int64_t)1 << 32)) return hipErrorInvalidValue;
-  b.blocks = dw_blocks(cdiv(b.s[0].R, AlongC::BN), cdiv(b.s[0].Cc, AlongC::BM), 1);
+__global__ __launch_bounds__(AlongC::NT) void dw_batch_kernel(const DwBatch b) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[AlongC::LDS_BYTES];
+  dw_batch_body<AlongR, AlongC>(b, lds, (int)blockIdx.x);
+}
+
+// The layer's dx GEMM ahead of them in the same launch: its few, long workgroups start first, the weight gradients' many short ones
+// fill the CUs around them.
+template <class Dx, class AlongR, class AlongC>
+__global__ __launch_bounds__(AlongC::NT) void dx_dw_batch_kernel(const GemmArgs gx, const DwBatch b, const int dx_blocks) {
+  static_assert(Dx::NT == AlongC::NT, "one workgroup size");
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[Dx::LDS_BYTES > AlongC::LDS_BYTES ? Dx::LDS_BYTES : AlongC::LDS_BYTES];
+  if ((int)blockIdx.x < dx_blocks) routed_gemm_body<Dx>(gx, lds, (int)blockIdx.x);
+  else dw_batch_body<AlongR, AlongC>(b, lds, (int)blockIdx.x - dx_blocks);
+}
+
+static bool fill_batch(const SplitKArgs (&g)[kDwBatch], int bm, int bn, DwBatch* b) {
+  b->along_r = 0;
+  for (int i = 0; i < kDwBatch; ++i) {
+    const SplitKArgs& s = g[i];
+    if (s.R <= 0 || s.Cc <= 0 || s.R != g[0].R || s.Cc != g[0].Cc || s.splits != 1 || s.out[0] == nullptr) return false;
+    if (s.R % 8 != 0 || s.lda * (kBK * 2) + 2 * (int64_t)s.R >= ((int64_t)1 << 32)) return false;
+    b->s[i] = s;
+    b->along_r |= (s.out_sr == 1 && s.out_sc != 1) << i;
+  }
+  b->blocks = dw_blocks(cdiv(g[0].R, bn), cdiv(g[0].Cc, bm), 1);
+  return true;
+}
+
+template <class AlongR, class AlongC>
+static hipError_t launch_batch(const SplitKArgs (&g)[kDwBatch], hipStream_t stream) {
+  DwBatch b;
+  if (!fill_batch(g, AlongC::BM, AlongC::BN, &b)) return hipErrorInvalidValue;
   hipLaunchKernelGGL((dw_batch_kernel<AlongR, AlongC>), dim3(kDwBatch * b.blocks), dim3(AlongC::NT), 0, stream, b);
+  return hipGetLastError();
+}
+
+hipError_t launch_dx_dw_batch_kmajor(const GemmArgs& gx, const SplitKArgs (&g)[kDwBatch], hipStream_t stream) {
+  using Dx = KMajorTiles<false, true>::T0;
+  using R = KMajorDwTiles<false>::T0;
+  using C = KMajorDwTiles<true>::T0;
+  DwBatch b;
+  if (gx.M <= 0 || gx.N <= 0 || gx.splits != 1 || gx.tail_mode != 0 || gx.P_tail != nullptr || !routed_gemm_args_ok<Dx>(gx) || !fill_batch(g, C::BM, C::BN, &b))
+    return hipErrorInvalidValue;
+  const int dx_blocks = routed_gemm_grid<Dx>(gx.M, gx.N);  // a multiple of the XCD count
+  hipLaunchKernelGGL((dx_dw_batch_kernel<Dx, R, C>), dim3(dx_blocks + kDwBatch * b.blocks), dim3(C::NT), 0, stream, gx, b, dx_blocks);
   return hipGetLastError();
 }
 
 hipError_t launch_dw_batch_kmajor(int tile, const SplitKArgs (&g)[kDwBatch], hipStream_t stream) {
   using R = KMajorDwTiles<false>;
   using C = KMajorDwTiles<true>;
-  DwBatch b;
-  b.along_r = 0;
-  for (int i = 0; i < kDwBatch; ++i) {
-    if (g[i].R <= 0 || g[i].Cc <= 0 || g[i].R != g[0].R || g[i].Cc != g[0].Cc || g[i].splits != 1 || g[i].out[0] == nullptr)
-      return hipErrorInvalidValue;
-    b.s[i] = g[i];
-    b.along_r |= (g[i].out_sr == 1 && g[i].out_sc != 1) << i;
-  }
   switch (tile) {
-    case TILE_256x256_W8: return launch_batch<R::T0, C::T0>(b, stream);
-    case TILE_256x256_W4: return launch_batch<R::T1, C::T1>(b, stream);
-    case TILE_SMALL_W4: return launch_batch<R::T3, C::T3>(b, stream);
+    case TILE_256x256_W8: return launch_batch<R::T0, C::T0>(g, stream);
+    case TILE_256x256_W4: return launch_batch<R::T1, C::T1>(g, stream);
+    case TILE_SMALL_W4: return launch_batch<R::T3, C::T3>(g, stream);
     case TILE_64x128_R3:
     case TILE_128x256_R3:  // no such weight-gradient tile
     case TILE_128x128_R4:  // no ring here: the group's last slab is cleared in LDS
-    case TILE_128x128_W4: return launch_batch<R::T2, C::T2>(b, stream);
+    case TILE_128x128_W4: return launch_batch<R::T2, C::T2>(g, stream);
     default: return hipErrorInvalidValue;
   }
 }

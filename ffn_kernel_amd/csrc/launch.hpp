@@ -53,6 +53,8 @@ hipError_t launch_splitk_gemm_kmajor(int tile, const SplitKArgs& g, hipStream_t 
 // Three of them, unsplit (results to `out`), of the same extents, in one launch.
 constexpr int kDwBatch = 3;
 hipError_t launch_dw_batch_kmajor(int tile, const SplitKArgs (&g)[kDwBatch], hipStream_t stream);
+// The same on 256x256 tiles with the dx GEMM (as launch_down_gemm_kmajor on the eight-wave 256x256 tile, uncut, no tail) ahead of them.
+hipError_t launch_dx_dw_batch_kmajor(const GemmArgs& gx, const SplitKArgs (&g)[kDwBatch], hipStream_t stream);
 
 // The MaskedLinear backward's dx GEMM (K-major weights, as launch_linear_gemm_kmajor on the 128x128 tile)
 // and its weight-gradient GEMM (as launch_splitk_gemm on the 128x128 tile) in ONE launch: weight-gradient

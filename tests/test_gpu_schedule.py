@@ -210,3 +210,12 @@ def test_swiglu_backward_in_the_epilogue(dev, forced, tile, nv, nt, d, h):
         kept = masked_ffn_backward(g, x, *views, mask, pre=pre)
         for other in (masked_ffn_backward(g, x, *views, mask, pre=wide[:, :2 * h]), masked_ffn_backward(g, x, *views, mask)):
             assert all(torch.equal(a, b) for a, b in zip(kept, other))
+
+
+# dx in one launch with the weight gradients on 256x256 tiles: ragged extents, rows of both modalities, of one, and a single one.
+@pytest.mark.parametrize("nv,nt,d,h", [(1200, 1301, 3080, 1000), (0, 2500, 4096, 1024), (1599, 1, 4104, 1032)])
+def test_dx_beside_the_weight_gradients(dev, forced, nv, nt, d, h):
+    note(f"dx beside dW: nv={nv} nt={nt} d={d} h={h}")
+    case = ffn_case(dev, nv, nt, d, h, seed=d + h)
+    forced(0)
+    assert_ffn_backward(*case, "one launch")
