@@ -198,3 +198,15 @@ def test_tiles_of_two_heights_cover_every_row(rules, n_vis, n_text):
         for tiles in covered.values():
             tiles.sort()
             assert tiles[0][0] == 0 and tiles[-1][1] == M and all(a[1] == b[0] for a, b in zip(tiles, tiles[1:]))
+
+
+def test_the_swiglu_derivative_divides(tmp_path):
+    """The sigmoid of the feed-forward backward is a correctly rounded division, as it was in a pass of its own: one for each of the
+    eight values, none left to the bare reciprocal (v_rcp_f32, one ulp)."""
+    src = tmp_path / "derivative.hip"
+    src.write_text(f'#include "{build.CSRC}/common.hpp"\n'
+                   "__global__ void derivative(const uint4* in, uint4* out) {\n"
+                   "  ffnk::swiglu_bwd(in[0], in[1], in[2], out, out + 1, out + 2);\n}\n")
+    asm = subprocess.run([shutil.which("hipcc") or "/opt/rocm/bin/hipcc", *build.HIPCC_FLAGS, "--cuda-device-only", "-S", str(src), "-o", "-"],
+                         check=True, capture_output=True, text=True).stdout
+    assert [asm.count(i) for i in ("v_rcp_f32", "v_div_fmas_f32", "v_div_fixup_f32")] == [8, 8, 8]
