@@ -55,17 +55,21 @@ def _compile(src: Path) -> Path:
     return obj
 
 
-def _compile_call() -> Path:
-    """csrc/call.cpp -> _call.so, a CPython extension on torch's headers (host code only)."""
+def call_command(src: Path, out: Path) -> list:
+    """g++ on a CPython extension over torch's headers (host code only)."""
     import torch
     from torch.utils.cpp_extension import include_paths, library_paths
 
-    tmp = CALL_PATH.with_suffix(".so.tmp")
     cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{sysconfig.get_paths()['include']}"]
-    cmd += [flag for p in include_paths("cuda") for flag in ("-isystem", p)] + [str(CSRC / "call.cpp"), "-o", str(tmp)]
-    cmd += [f"-L{p}" for p in library_paths()] + ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
+    cmd += [flag for p in include_paths("cuda") for flag in ("-isystem", p)] + [str(src), "-o", str(out)]
+    return cmd + [f"-L{p}" for p in library_paths()] + ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+
+
+def _compile_call() -> Path:
+    """csrc/call.cpp -> _call.so."""
+    tmp = CALL_PATH.with_suffix(".so.tmp")
+    proc = subprocess.run(call_command(CSRC / "call.cpp", tmp), capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"g++ failed on call.cpp:\n{proc.stderr}")
     if proc.stderr.strip():

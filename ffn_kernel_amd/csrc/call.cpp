@@ -100,13 +100,20 @@ struct Call {
   }
 };
 
-// The foreign call without the GIL, as ctypes makes it.
+struct WithoutGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
+// The foreign call without the GIL, as ctypes makes it.  f reads the tensors' addresses, and torch throws where one has none (an
+// output that a dispatch mode made a fake tensor): the error is made a Python one by the caller, which needs the GIL back.
 template <class F>
 bool run(const char* name, F&& f) {
   int rc;
-  Py_BEGIN_ALLOW_THREADS
-  rc = f();
-  Py_END_ALLOW_THREADS
+  {
+    WithoutGil released;
+    rc = f();
+  }
   if (rc == 0) return true;
   PyObject* r = PyObject_CallFunction(check, "is", rc, name);
   Py_XDECREF(r);

@@ -1,9 +1,13 @@
 """_call.so against the Python path behind it: the same results, bit for bit, for every form that it takes, and NotImplemented -
 hence the Python path's own handling - for the others."""
+import ctypes
+import subprocess
+from pathlib import Path
+
 import pytest
 import torch
 
-from ffn_kernel_amd import MaskedFFN, MaskedLinear, ops
+from ffn_kernel_amd import MaskedFFN, MaskedLinear, build, ops
 from helpers import note
 
 
@@ -49,6 +53,12 @@ def test_other_arguments_are_left_to_python():
     assert call.linear_bwd(x, x, w, w, mask, None) is NotImplemented
     assert call.ffn_fwd(x, w, w, w, w, w, w, mask, False, None) is NotImplemented
     assert call.ffn_bwd(x, x, w, w, w, w, w, w, mask, None, None) is NotImplemented
+
+
+def test_an_exception_out_of_a_foreign_call_finds_the_gil_held(tmp_path):
+    so = tmp_path / "call_checks.so"
+    subprocess.run(build.call_command(Path(__file__).with_name("call_checks.cpp"), so), check=True, capture_output=True)
+    assert ctypes.PyDLL(str(so)).cc_gil_held_after_throw() == 1
 
 
 def same(a, b):
@@ -159,3 +169,20 @@ def test_current_stream_and_autograd(dev, both):
         same(a, b)
         assert len(names) == 2
         same(a, both(lambda: on_side(op, weights))[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("unsafe", [True, False])
+@pytest.mark.parametrize("M", [2, 300])
+def test_outputs_without_memory_are_refused(dev, M, unsafe):
+    """Under a mode that makes the call's own tensors fake ones - their address reads as zero, or throws - the call raises, and the
+    next one runs."""
+    import torch._functorch.config as config
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    note(f"native call: fake outputs M={M} unsafe={unsafe}")
+    x, w, mask = rnd(dev, M, 64), rnd(dev, 32, 64).T, torch.rand(M, device=dev) < 0.5
+    before = ops.masked_linear_forward(x, w, w, mask)
+    with config.patch(fake_tensor_allow_unsafe_data_ptr_access=unsafe), FakeTensorMode(allow_non_fake_inputs=True):
+        with pytest.raises((ValueError, RuntimeError)):
+            ops.masked_linear_forward(x, w, w, mask)
+    assert torch.equal(ops.masked_linear_forward(x, w, w, mask), before)
