@@ -506,12 +506,6 @@ bool gather_dw_ok(int64_t M, int64_t K, int64_t N, const void* g, int64_t g_stri
          M * g_stride_m * 2 + 2 * N < k4g && M * x_stride_m * 2 + 2 * K < k4g &&
          ((reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(x)) & 15) == 0;
 }
-// Tile of the dx GEMM in a launch of its own.
-int linear_dx_tile(int64_t M, int64_t K, int64_t N, bool direct) {
-  const int f = forced_tile();  // a forced ring tile of three stages stands for the two-stage tile here, as in the weight-gradient GEMM
-  if (f >= 0) return f == TILE_128x256_R3 ? TILE_128x128_W4 : f == TILE_64x128_R3 ? TILE_SMALL_W4 : f;
-  return bwd_tile(M, K, N, direct);
-}
 // One launch for both GEMMs: the dx GEMM on a 128x128 tile over weights read in place, and the weight gradients on the
 // same tile (the in-place form has no other).
 bool bwd_is_fused(int64_t M, int64_t K, const BwdPlan& p, bool w_kmajor, bool in_place) {
@@ -614,7 +608,7 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
         tile = in_place ? TILE_128x128_W4 : bp.tc.tile; contraction = M;
         splits = bwd_dw_launch_splits(M, K, N, bp, fused);
       } else {
-        tile = fused ? routed_tile(M, K, false, 0, TUNED_NONE) : linear_dx_tile(M, K, N, w_kmajor); contraction = N;
+        tile = fused ? routed_tile(M, K, false, 0, TUNED_NONE) : bwd_tile(M, K, N, w_kmajor); contraction = N;
         in_place = false;
       }
       break;
@@ -1081,7 +1075,7 @@ int ffnk_masked_linear_bwd_routed(const uint16_t* g, int64_t g_stride_m, const u
   const bool gather = p.gather && gather_dw_ok(M, K, N, g, g_stride_m, x, x_stride_m);
   const bool fused = bwd_is_fused(M, K, p, w_kmajor, gather);
   if (!fused) {
-    const int dx_tile = linear_dx_tile(M, K, N, dx_direct);
+    const int dx_tile = bwd_tile(M, K, N, dx_direct);
     if (w_kmajor) FFNK_HIP(launch_linear_gemm_kmajor(dx_tile, a, stream), "dx GEMM");
     else FFNK_HIP(launch_linear_gemm(dx_tile, dx_direct, a, stream), "dx GEMM");
   }

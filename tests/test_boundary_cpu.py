@@ -38,12 +38,12 @@ def test_workspace_bytes():
         _lib.workspace_bytes(_lib.OP_LINEAR_FWD, -1, 1, 1)
 
 
-# Forced tiles are reported as they run: the K-major dx GEMM and the weight-gradient GEMM have no ring tiles of three stages,
-# a staged contraction no ring at all, and the four-wave 256x256 tile exists on the direct path only.
+# Forced tiles are reported as they run: the weight-gradient GEMM has no ring tiles of three stages, a staged contraction no ring
+# at all, and the four-wave 256x256 tile exists on the direct path only.
 @pytest.mark.parametrize("tile,linear,staged,dx,dw", [(1, (256, 256, 3), (256, 256, 2), (256, 256, 3), (256, 256, 3)),
                                                       (4, (128, 128, 4), (128, 128, 2), (128, 128, 4), (128, 128, 4)),
-                                                      (6, (128, 256, 3), (128, 128, 2), (128, 128, 2), (128, 128, 2)),
-                                                      (7, (64, 128, 3), (128, 64, 2), (128, 64, 2), (128, 128, 2))])
+                                                      (6, (128, 256, 3), (128, 128, 2), (128, 256, 3), (128, 128, 2)),
+                                                      (7, (64, 128, 3), (128, 64, 2), (64, 128, 3), (128, 128, 2))])
 def test_tile_config_names_the_tile_that_runs(tile, linear, staged, dx, dw):
     lib = _lib.load()
     lib.ffnk_debug_force_tile(tile)

@@ -42,6 +42,9 @@ def test_linear_fwd_bwd(dev, forced, tile, splits, K, N):
     note(f"ragged linear fwd + bwd K={K} N={N} tile={tile} splits={splits}")
     x, Wv, Wt, mask, g = linear_case(dev, 301, K, N, 0.45, seed=K + N)
     forced(tile, splits)
+    if tile in (6, 7) and N >= 128:  # dx on the ring tiles of three stages themselves
+        cfg = _lib.tile_config(_lib.OP_BWD_DX, 301, K, N)
+        assert (cfg["block_m"], cfg["lds_stages"]) == ((128, 64)[tile - 6], 3)
     y = MaskedLinear.apply(x, Wv.T, Wt.T, mask)
     dx, dv, dt = masked_linear_backward(g, x, Wv.T, Wt.T, mask)
     forced()

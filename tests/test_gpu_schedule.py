@@ -82,15 +82,17 @@ def select_ffn(x, W, mask):
                                               (65, 63, 1024, 520, 3), (200, 130, 1536, 128, 5)])
 def test_ring_tiles(dev, forced, tile, nv, nt, K, N, splits):
     note(f"ring tile {tile}: nv={nv} nt={nt} K={K} N={N} splits={splits}")
-    x, Wv, Wt, mask, _ = make_linear(dev, nv, nt, K, N, seed=K + N)
+    x, Wv, Wt, mask, g = make_linear(dev, nv, nt, K, N, seed=K + N)
     forced(tile, splits)
     y = MaskedLinear.apply(x, Wv.T, Wt.T, mask)
+    dx = masked_linear_backward(g, x, Wv.T, Wt.T, mask)[0]  # over K-major weights, contraction N
     h = 136  # M, d, h beyond the decode kernels' shapes: h is no multiple of 128
     gen = torch.Generator(device=dev).manual_seed(3)
     W = [(torch.randn(*s, generator=gen, device=dev) * 0.05).to(torch.bfloat16) for s in ((h, K), (K, h), (h, K)) * 2]
     out = MaskedFFN.apply(x, *[w.T for w in W], mask)
     forced()
     assert_close(y, torch.where(mask[:, None], x.double() @ Wv.double().T, x.double() @ Wt.double().T).cpu(), "y")
+    assert_close(dx, torch.where(mask[:, None], g.double() @ Wv.double(), g.double() @ Wt.double()).cpu(), "dx")
     assert_close(out, select_ffn(x, W, mask).cpu(), "ffn")
 
 
