@@ -1887,7 +1887,7 @@ __global__ __launch_bounds__(Tall::NT) void routed_mixed_kernel(const GemmArgs g
   static_assert(Tall::NT == Short::NT && Tall::BN_OUT == Short::BN_OUT && Tall::BM == kTallRows && Short::BM == kShortRows, "two heights");
   __shared__ __attribute__((aligned(1024))) uint8_t lds[Tall::LDS_BYTES > Short::LDS_BYTES ? Tall::LDS_BYTES : Short::LDS_BYTES];
   bool is_tall;
-  TileCoord tc = mixed_tile_coord((int)blockIdx.x, g.counts[0], g.M, g.N, Tall::BN_OUT, &is_tall);
+  TileCoord tc = mixed_tile_coord((int)blockIdx.x, g.counts[0], g.M, g.N, Tall::BN_OUT, g.group_m > 0 ? g.group_m : Tall::GROUP_M, &is_tall);
   if (tc.grp < 0) return;
   // (the compiler takes them for values of a lane and would load the weights' addresses through the vector memory path)
   tc.grp = __builtin_amdgcn_readfirstlane(tc.grp);

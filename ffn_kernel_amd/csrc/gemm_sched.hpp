@@ -130,11 +130,10 @@ inline int mixed_blocks(int M, int N, int bn) {
   const int64_t tiles = (int64_t)(cdiv(M, kTallRows) + 1) * cdiv(N, bn) + kCusPerChip / 2;  // with the second halves of split tiles
   return kXcds * (int)(cdiv64(tiles, kXcds) + 1);
 }
-constexpr int kMixedGroup = 8;
 // Tile of workgroup `bid`; grp < 0: a surplus workgroup.  Every XCD takes an eighth of the tall tiles' order, then an eighth of the
-// short ones'; an order walks the M-tiles of one height and modality column by column, so that the tiles of a column share the
-// weight panel.
-__host__ __device__ inline TileCoord mixed_tile_coord(int bid, int n_vis, int M, int N, int bn, bool* is_tall) {
+// short ones'; an order walks the M-tiles of one height and modality in super-groups of `group`, column by column, so that the tiles
+// of a column share the weight panel.
+__host__ __device__ inline TileCoord mixed_tile_coord(int bid, int n_vis, int M, int N, int bn, int group, bool* is_tall) {
   TileCoord t{-1, 0, 0, 0};
   const int tiles_n = cdiv(N, bn);
   MixedRows v, x;
@@ -159,8 +158,8 @@ __host__ __device__ inline TileCoord mixed_tile_coord(int bid, int n_vis, int M,
   if (grp == 1) L -= own_v * tiles_n;
   const int own = grp == 0 ? own_v : own_x;
   int first = 0, gsz = own;  // super-group of M-tiles, dealt evenly (routed_tile_coord)
-  if (own > kMixedGroup) {
-    const int groups = cdiv(own, kMixedGroup), s = ((L / tiles_n + 1) * groups - 1) / own;
+  if (own > group) {
+    const int groups = cdiv(own, group), s = ((L / tiles_n + 1) * groups - 1) / own;
     first = s * own / groups;
     gsz = (s + 1) * own / groups - first;
     L -= first * tiles_n;

@@ -33,9 +33,9 @@ void hc_dw_tile(int bid, int tiles_r, int tiles_c, int splits, int n_vis, int M,
 
 // Workgroups of a launch on tiles of two heights; the tile of workgroup `bid`: {group, first row, end, first column}, group -1: none.
 int hc_mixed_blocks(int M, int N, int bn) { return mixed_blocks(M, N, bn); }
-void hc_mixed_tile(int bid, int n_vis, int M, int N, int bn, int* out) {
+void hc_mixed_tile(int bid, int n_vis, int M, int N, int bn, int group, int* out) {
   bool tall;
-  const TileCoord t = mixed_tile_coord(bid, n_vis, M, N, bn, &tall);
+  const TileCoord t = mixed_tile_coord(bid, n_vis, M, N, bn, group, &tall);
   const int end = t.row0 + (tall ? kTallRows : kShortRows);
   out[0] = t.grp; out[1] = t.row0; out[2] = end < t.row_end ? end : t.row_end; out[3] = t.n0;
 }

@@ -196,6 +196,22 @@ def test_tiles_of_two_heights(dev, nv, nt, h, d):
         assert_close(pre[:, half * h:(half + 1) * h], torch.where(m, xs @ v.double().T, xs @ t.double().T).cpu(), f"pre {half}")
 
 
+# The order of that launch in super-groups of other sizes: the same tiles, the same sums.
+@pytest.mark.parametrize("group", [1, 3, 64])
+def test_tiles_of_two_heights_in_super_groups(dev, group):
+    note(f"tiles of two heights: super-groups of {group}")
+    lib = _lib.load()
+    x, W, mask, _ = ffn_case(dev, 2060, 100, 128, 7432, seed=9)
+    out = masked_ffn_forward(x, *[w.T for w in W], mask)
+    try:
+        lib.ffnk_debug_force_group_m(group)
+        assert _lib.tile_config(_lib.OP_FFN_UP, 2160, 128, 7432)["group_m"] == group
+        other = masked_ffn_forward(x, *[w.T for w in W], mask)
+    finally:
+        lib.ffnk_debug_force_group_m(0)
+    assert torch.equal(out, other)
+
+
 # The SwiGLU derivative on the dh GEMM's tiles: row and column edges of every tile, halves padded to whole slabs (h = 328, 72) and
 # not, pre-activations kept by a forward (also in rows wider than they are) and recomputed in place; down weights in both layouts.
 @pytest.mark.parametrize("tile", [-1, 0, 1, 2, 3, 4, 6, 7])

@@ -188,7 +188,7 @@ def test_tiles_of_two_heights_cover_every_row(rules, n_vis, n_text):
     for tiles_n in (5, 43, 90, 129, 258) if M else ():
         covered = {}
         for b in range(rules.hc_mixed_blocks(M, tiles_n * bn - 120, bn)):
-            rules.hc_mixed_tile(b, n_vis, M, tiles_n * bn - 120, bn, t)
+            rules.hc_mixed_tile(b, n_vis, M, tiles_n * bn - 120, bn, 8, t)
             grp, row0, end, n0 = t
             if grp == -1:
                 continue
@@ -198,6 +198,28 @@ def test_tiles_of_two_heights_cover_every_row(rules, n_vis, n_text):
         for tiles in covered.values():
             tiles.sort()
             assert tiles[0][0] == 0 and tiles[-1][1] == M and all(a[1] == b[0] for a, b in zip(tiles, tiles[1:]))
+
+
+@pytest.mark.parametrize("group", [1, 2, 3, 8, 64])
+@pytest.mark.parametrize("n_vis,M", [(0, 2560), (1285, 4000)])
+def test_tiles_of_two_heights_in_super_groups(rules, group, n_vis, M):
+    """Every tile once whatever the super-group size, and an XCD's whole tall tiles of a modality at most that many to a column."""
+    bn, N, t = 128, 29 * 128, (ctypes.c_int * 4)()
+    tiles, longest, per_xcd = set(), 0, {}
+    for b in range(rules.hc_mixed_blocks(M, N, bn)):
+        rules.hc_mixed_tile(b, n_vis, M, N, bn, group, t)
+        if t[0] >= 0:
+            assert tuple(t) not in tiles
+            tiles.add(tuple(t))
+            if t[2] - t[1] > 160:
+                per_xcd.setdefault(b % 8, []).append((t[0], t[3]))
+    assert sum((end - row0) * min(bn, N - n0) for _, row0, end, n0 in tiles) == M * N
+    for order in per_xcd.values():
+        run = 1
+        for prev, cur in zip(order, order[1:]):
+            run = run + 1 if cur == prev else 1
+            longest = max(longest, run)
+    assert min(group, 4) <= longest <= group
 
 
 def test_the_swiglu_derivative_divides(tmp_path):
