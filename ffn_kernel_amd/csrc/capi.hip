@@ -347,6 +347,13 @@ RoutedPlan ffn_down_plan(int64_t M, int64_t d, int64_t h, size_t ws_limit = kAny
   if (forced_tile() >= 0 || forced_splits() >= 1 || fixed >= ws_limit || plan_partial_bytes(p, M, d, h) <= ws_limit - fixed) return p;
   return model_routed_plan(false, M, d, h, M < 65536 && d % 4 == 0, ws_limit - fixed);
 }
+// The SwiGLU GEMM's plan is the four-wave 256x256 tile, and it has up to eight rounds of the chip: that tile beside 160-row ones in
+// one launch (mixed_rows), also where it is forced, so that what the tuner times is what a plan of it runs.  Past that the two
+// launches of whole rounds and remainder are the faster (M = 32768, d = 4096, h = 14336, 56 rounds: 7834 us against 8002;
+// M = 23225, d = 2624, h = 8512, one modality, 24 rounds: 2241 against 2281).
+bool up_two_heights(int tile, bool direct, int64_t M, int64_t h) {
+  return tile == TILE_256x256_W4 && direct && cdiv64(M, kTallRows) * cdiv64(h, 128) <= 8 * kCus;
+}
 // Tile of an unsplit GEMM of the backward: the time model's, although it was fitted to row-major weights - over 2320 drawn GEMMs
 // on K-major weights (M = 65 ... 16384, up to two rounds of 256x256 tiles and past them) its plans are 1.8 % (MaskedLinear's
 // dx), 2.9 % (dh) and 3.0 % (the feed-forward dx, K split) behind the best of all tiles and split factors in the geometric mean,
@@ -514,6 +521,25 @@ bool bwd_is_fused(int64_t M, int64_t K, const BwdPlan& p, bool w_kmajor, bool in
 int bwd_dw_launch_splits(int64_t M, int64_t K, int64_t N, const BwdPlan& p, bool fused) {
   if (!fused || p.tc.tuned || forced_splits() >= 1) return p.tc.splits;
   return fused_bwd_splits(M, K, N, p.tc.splits);
+}
+
+// The feed-forward backward's dx and (where H, dt1 and dt3 are read in place) weight-gradient GEMMs.
+struct FfnBwdGemms {
+  RoutedPlan dx;
+  size_t dx_need;  // bytes of partials or split tail, if dx has a launch of its own
+  TileChoice dw{};
+  bool beside = false;
+};
+FfnBwdGemms ffn_bwd_gemms(int64_t M, int64_t d, int64_t h, const FfnBwdPaths& paths, bool w13_kmajor) {
+  FfnBwdGemms g;
+  const int64_t contraction = 2 * paths.half;
+  g.dx = ffn_bwd_dx_plan(M, d, contraction, paths.dx_direct, 2 * ws_align((size_t)h * d * 2), &g.dx_need);
+  if (paths.acts_in_place) {
+    g.dw = ffn_bwd_in_place_choice(M, d, h);
+    if (forced_tile() >= 0) g.dw.tile = forced_tile();
+    g.beside = w13_kmajor && ffn_bwd_dx_beside_dw(M, d, h, contraction, g.dx, g.dw);
+  }
+  return g;
 }
 
 }  // namespace
@@ -704,6 +730,18 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
     }
   }
   return FFNK_OK;
+}
+
+int ffnk_debug_ffn_joint(int64_t M, int64_t d, int64_t h) {
+  if (int e = check_extents(M, d, h)) return e;
+  int joint = 0;
+  if (!use_stream_path(M, d, h) && d % 8 == 0 && up_two_heights(routed_tile(M, h, true, d), direct_ok(d, M, d, d), M, h)) joint |= 1;
+  if (M > 0 && d > 0 && h > 0 && d % 8 == 0 && h % 8 == 0) {
+    bool w13_kmajor = false;
+    const FfnBwdPaths paths = ffn_bwd_paths(M, d, h, d, d, 1, h, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, &w13_kmajor);
+    if (ffn_bwd_gemms(M, d, h, paths, w13_kmajor).beside) joint |= 2;
+  }
+  return joint;
 }
 
 int ffnk_masked_linear_fwd(const uint16_t* x, int64_t x_stride_m, const uint16_t* Wv, const uint16_t* Wt,
@@ -911,11 +949,7 @@ int ffn_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, cons
   up.C_pre = pre; up.ldc_pre = pre_stride_m;
   const bool up_direct = direct_ok(d, M, x_stride_m, up_stride_n);
   int up_tile = routed_tile(M, h, true, d);
-  // Where the plan is the four-wave 256x256 tile, up to eight rounds of the chip: beside 160-row ones in one launch (mixed_rows).
-  // Past that the two launches of whole rounds and remainder are the faster (M = 32768, d = 4096, h = 14336, 56 rounds: 7834 us
-  // against 8002; M = 23225, d = 2624, h = 8512, one modality, 24 rounds: 2241 against 2281).  A forced tile is run as it is.
-  if (up_tile == TILE_256x256_W4 && up_direct && forced_tile() < 0 && cdiv64(M, kTallRows) * cdiv64(h, 128) <= 8 * kCus)
-    up_tile = TILE_MIXED_W4;
+  if (up_two_heights(up_tile, up_direct, M, h)) up_tile = TILE_MIXED_W4;
   FFNK_HIP(launch_up_gemm(up_tile, up_direct, up, stream), "up-projection GEMM");
   FFNK_HIP(mark(1), "event record");
   GemmArgs dn;
@@ -1221,17 +1255,11 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
   // Few output tiles over a 2h-long contraction: split K like the forward's down projection.  The
   // fp32 partials live where the W2^T copies were (dead since the dh GEMM), if they fit there.
   const bool dx_direct = paths.dx_direct;
-  size_t dx_need = 0;
-  const RoutedPlan dxp = ffn_bwd_dx_plan(M, d, ld13, dx_direct, 2 * ws_align((size_t)h * d * 2), &dx_need);
+  const FfnBwdGemms gemms = ffn_bwd_gemms(M, d, h, paths, w13_kmajor);
+  const RoutedPlan& dxp = gemms.dx;
+  const size_t dx_need = gemms.dx_need;
   if (dx_need > p.w2t_bytes) return fail(FFNK_E_WORKSPACE, "internal: dx partials %zu > %zu planned", dx_need, p.w2t_bytes);
-  TileChoice in_place_choice;
-  bool beside_dw = false;
-  if (paths.acts_in_place) {
-    in_place_choice = ffn_bwd_in_place_choice(M, d, h);
-    if (forced_tile() >= 0) in_place_choice.tile = forced_tile();
-    beside_dw = w13_kmajor && ffn_bwd_dx_beside_dw(M, d, h, ld13, dxp, in_place_choice);
-  }
-  if (!beside_dw) {
+  if (!gemms.beside) {
     if (dxp.splits > 1) {
       b.splits = dxp.splits;
       b.splits_more = dxp.splits_more;
@@ -1256,7 +1284,7 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
   if (in_place) {
     FFNK_HIP(launch_gather_transpose2(g, g_stride_m, (int)d, GT, x, x_stride_m, (int)d, XT, p.ldt, rt.perm, rt.counts, (int)M,
                                       stream, false, false), "g / x transpose");
-    const TileChoice& tc = in_place_choice;
+    const TileChoice& tc = gemms.dw;
     // out[r * sr + c * sc]: r runs over h (the in-place operand's columns), c over d
     auto weight_grad = [&](const uint16_t* rows, int64_t ld_rows, const uint16_t* cT, uint16_t* o0, uint16_t* o1, int64_t sr, int64_t sc) {
       SplitKArgs s;
@@ -1270,7 +1298,7 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
     const SplitKArgs dw[kDwBatch] = {weight_grad(DH, h, GT, dW2, dU2, ddown_stride_k, ddown_stride_n),
                                      weight_grad(T13, ld13, XT, dW1, dU1, dup_stride_n, dup_stride_k),
                                      weight_grad(T13 + half, ld13, XT, dW3, dU3, dup_stride_n, dup_stride_k)};
-    if (beside_dw) {
+    if (gemms.beside) {
       FFNK_HIP(launch_dx_dw_batch_kmajor(b, dw, stream), "dx / dW GEMMs");
       return FFNK_OK;
     }

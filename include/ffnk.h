@@ -117,7 +117,7 @@ FFNK_API size_t ffnk_workspace_bytes(int op, int64_t M, int64_t K, int64_t N);
 /* Scratch of ffnk_masked_ffn_bwd / ffnk_masked_ffn_bwd_saved for one layout of the weights (element strides as
  * passed to those calls), assuming 16-byte aligned pointers.  ffnk_workspace_bytes(FFNK_OP_FFN_BWD, ...) covers every
  * layout and reserves room for copies of the weights and transposes of the intermediates that the usual layout
- * (nn.Linear.weight.T views, d and h multiples of 64) never touches - 1.6 GB of 2.7 GB at M = 8192, d = 4096,
+ * (nn.Linear.weight.T views) never touches - 1.6 GB of 2.7 GB at M = 8192, d = 4096,
  * h = 14336; this query leaves that out.  A call whose pointers turn out not to be aligned needs the larger size
  * and says so (FFNK_E_WORKSPACE).  No counterpart in the reference, whose MaskedFFN.backward raises
  * (ffn_kernel/ops.py:34-38).  Returns (size_t)-1 for invalid extents. */
@@ -131,8 +131,8 @@ FFNK_API int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile
 /*
  * Tuner-only hooks (python -m ffn_kernel_amd.tune, the counterpart of the reference's find_spec scripts
  * sweeps, and the tests that run every compiled tile).  ffnk_debug_force_tile: every LDS-tiled GEMM
- * launched by this process uses tile id `tile` (0 = 256x256 / 8 waves, 1 = 256x256 / 4 waves,
- * 2 = 128x128 / 4 waves, 3 = small, 4 = 128x128 / 4 waves behind a ring of four LDS stages, 6 = 128x256 and
+ * launched by this process uses tile id `tile` (0 = 256x256 / 8 waves, 1 = 256x256 / 4 waves - in the SwiGLU GEMM
+ * beside 160x256 ones up to eight rounds, as in a plan -, 2 = 128x128 / 4 waves, 3 = small, 4 = 128x128 / 4 waves behind a ring of four LDS stages, 6 = 128x256 and
  * 7 = 64x128 behind a ring of three; GEMMs without a ring run 2 or 3 in their place); -1 returns to the tile table
  * (measured plans first, then the rules); -2 uses the rules only, ignoring the measured plans (what the tuner compares
  * against).  Other values count as -1.
@@ -153,6 +153,10 @@ FFNK_API int ffnk_debug_force_bwd_gather(int on);
  * The counterpart of the GROUP_SIZE_M dimension of the reference's searches (find_spec/bf16_linear_fwd.py:45-53).
  * Returns the previous value. */
 FFNK_API int ffnk_debug_force_group_m(int group_m);
+/* Which launches of a MaskedFFN call (nn.Linear.weight.T views, contiguous and aligned operands, M past the weight-streaming kernels)
+ * hold more than one kind of tile, under the current settings of the hooks above: bit 0 = the SwiGLU GEMM runs 256- and 160-row
+ * tiles in one launch, bit 1 = the backward's dx GEMM runs in one launch with the weight gradients.  Negative: invalid extents. */
+FFNK_API int ffnk_debug_ffn_joint(int64_t M, int64_t d, int64_t h);
 
 /*
  * MaskedLinear forward — replaces _bf16_linear_forward (ffn_kernel/linear.py:418-452):

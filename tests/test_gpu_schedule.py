@@ -108,14 +108,16 @@ def test_split_factor_by_row_tiles(dev, nv, K, N):
 
 
 # The remainder of a launch on 256-row SwiGLU tiles: exactly half a round (256 + 128 tiles), one tile past it (256 + 129: another
-# whole round), and one tile past a round.  d = 64, h = 128 * tiles_n columns.
-@pytest.mark.parametrize("tiles_m,h", [(6, 64 * 128), (55, 7 * 128), (257, 128)])
+# whole round), and one tile past a round; the same past eight rounds, below which the four-wave tile runs beside 160-row ones.
+# d = 64, h = 128 * tiles_n columns.
+@pytest.mark.parametrize("tiles_m,h", [(6, 64 * 128), (55, 7 * 128), (257, 128), (17, 128 * 128), (311, 7 * 128), (683, 3 * 128)])
 def test_whole_rounds_and_remainder(dev, forced, tiles_m, h):
     note(f"remainder of whole rounds: {tiles_m} M-tiles, h={h}")
     x, _, _, mask, _ = make_linear(dev, 256 * 2, 256 * (tiles_m - 2) - 5, 64, 8, seed=tiles_m)
     gen = torch.Generator(device=dev).manual_seed(5)
     W = [(torch.randn(*s, generator=gen, device=dev) * 0.05).to(torch.bfloat16) for s in ((h, 64), (64, h), (h, 64)) * 2]
     forced(1)
+    assert _lib.load().ffnk_debug_ffn_joint(x.shape[0], 64, h) & 1 == (tiles_m * h <= 8 * 256 * 128)
     out = MaskedFFN.apply(x, *[w.T for w in W], mask)
     forced()
     assert_close(out, select_ffn(x, W, mask).cpu(), "ffn")
@@ -184,7 +186,7 @@ def test_backward_ragged_intermediate(dev, forced, tile, splits, h):
 def test_tiles_of_two_heights(dev, nv, nt, h, d):
     note(f"tiles of two heights: nv={nv} nt={nt} h={h} d={d}")
     cfg = _lib.tile_config(_lib.OP_FFN_UP, nv + nt, d, h)
-    assert (cfg["block_m"], cfg["waves_m"] * cfg["waves_n"]) == (256, 4)  # the plan that the mixed launch follows from
+    assert (cfg["block_m"], cfg["waves_m"] * cfg["waves_n"]) == (256, 4) and _lib.load().ffnk_debug_ffn_joint(nv + nt, d, h) & 1
     x, W, mask, _ = ffn_case(dev, nv, nt, d, h, seed=h + d)
     W = [w * 0.5 for w in W]
     out, pre = masked_ffn_forward(x, *[w.T for w in W], mask, save_pre=True)

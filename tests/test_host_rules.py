@@ -222,6 +222,19 @@ def test_tiles_of_two_heights_in_super_groups(rules, group, n_vis, M):
     assert min(group, 4) <= longest <= group
 
 
+# The four-wave 256x256 tile of the SwiGLU GEMM, planned or forced (as the tuner times it): beside 160-row tiles up to eight rounds.
+@pytest.mark.parametrize("tile,M,d,h,joint", [(-1, 300, 4096, 14336, 1), (-1, 32768, 4096, 14336, 0), (1, 300, 136, 264, 1), (0, 300, 4096, 14336, 0),
+                                              (1, 4096, 64, 16384, 1), (1, 4097, 64, 16384, 0), (1, 300, 72, 264, 0)])
+def test_where_tiles_of_two_heights_run(tile, M, d, h, joint):
+    from ffn_kernel_amd import _lib
+    lib = _lib.load()
+    lib.ffnk_debug_force_tile(tile)
+    try:
+        assert lib.ffnk_debug_ffn_joint(M, d, h) & 1 == joint
+    finally:
+        lib.ffnk_debug_force_tile(-1)
+
+
 def test_the_swiglu_derivative_divides(tmp_path):
     """The sigmoid of the feed-forward backward is a correctly rounded division, as it was in a pass of its own: one for each of the
     eight values, none left to the bare reciprocal (v_rcp_f32, one ulp)."""
