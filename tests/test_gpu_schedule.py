@@ -238,4 +238,5 @@ def test_dx_beside_the_weight_gradients(dev, forced, nv, nt, d, h):
     note(f"dx beside dW: nv={nv} nt={nt} d={d} h={h}")
     case = ffn_case(dev, nv, nt, d, h, seed=d + h)
     forced(0)
+    assert _lib.load().ffnk_debug_ffn_joint(nv + nt, d, h) & 2
     assert_ffn_backward(*case, "one launch")

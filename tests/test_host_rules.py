@@ -235,6 +235,25 @@ def test_where_tiles_of_two_heights_run(tile, M, d, h, joint):
         lib.ffnk_debug_force_tile(-1)
 
 
+# The feed-forward backward's dx beside the weight gradients (tile 0 forced: both on 256x256 tiles), either side of each line: ten
+# slabs per weight-gradient tile, 0.7 of dx's rounds filled, 3/4 of the time of all work; not in K ranges, not on other tiles, and
+# the layers that the lines were drawn by.
+@pytest.mark.parametrize("tile,splits,M,d,h,joint", [
+    (0, -1, 1152, 7424, 4096, 0), (0, -1, 1153, 7424, 4096, 2), (0, -1, 2560, 4096, 1024, 2), (0, -1, 2561, 4096, 1024, 0),
+    (0, -1, 2304, 3072, 4096, 0), (0, -1, 2305, 3072, 4096, 2), (0, 2, 2500, 4096, 1024, 0), (2, -1, 2500, 4096, 1024, 0),
+    (-1, -1, 4096, 4096, 14336, 2), (-1, -1, 1995, 4184, 13480, 2), (-1, -1, 7144, 4288, 14208, 0), (-1, -1, 471, 6976, 23232, 0)])
+def test_where_dx_runs_beside_the_weight_gradients(tile, splits, M, d, h, joint):
+    from ffn_kernel_amd import _lib
+    lib = _lib.load()
+    lib.ffnk_debug_force_tile(tile)
+    lib.ffnk_debug_force_splits(splits)
+    try:
+        assert lib.ffnk_debug_ffn_joint(M, d, h) & 2 == joint
+    finally:
+        lib.ffnk_debug_force_tile(-1)
+        lib.ffnk_debug_force_splits(-1)
+
+
 def test_the_swiglu_derivative_divides(tmp_path):
     """The sigmoid of the feed-forward backward is a correctly rounded division, as it was in a pass of its own: one for each of the
     eight values, none left to the bare reciprocal (v_rcp_f32, one ulp)."""
