@@ -390,7 +390,8 @@ def main() -> int:
         achieved = up_flops / (up_avg * 1e-3) / 1e12
         roofline = {"bound": "mfma", "achieved": achieved, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                     "frac": achieved / PEAK_BF16_TFLOPS, "traffic": traffic,
-                    "kernel": "routed_gemm_kernel (up-projection + SwiGLU: whole-round launch + remainder launch)",
+                    "kernel": ("routed_mixed_kernel (up-projection + SwiGLU: 256- and 160-row tiles in one launch)" if _lib.load().ffnk_debug_ffn_joint(M, w.d, w.h) & 1
+                               else "routed_gemm_kernel (up-projection + SwiGLU: whole-round launch + remainder launch)"),
                     "kernel_ms": up_avg,
                     "down_kernel_ms": down_avg,
                     "down_achieved": 2 * M * w.d * w.h / (down_avg * 1e-3) / 1e12}
