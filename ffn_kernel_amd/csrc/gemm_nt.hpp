@@ -1313,7 +1313,7 @@ __device__ __forceinline__ int xcd_tile_slot(int total, int bid) {
 // Against stores from the accumulators: MaskedLinear M = 28536, K = 1536, N = 2624 237 -> 214 us, M = 16798, K = 960, N = 1536
 // 79.7 -> 74.1; forward + backward M = 1560, K = 4928, N = 7168 468 -> 434; MaskedFFN forward + backward d = 4096, h = 14336,
 // M = 4096 3725 -> 3582, d = 3456, h = 11072, M = 90 506 -> 418 (its weight gradients are nothing but stores: 67 -> 43 us each);
-// MaskedFFN forward d = 1024, h = 2048, M = 8192 137.3 -> 134.6, d = 4096, h = 14336, M = 32768 7883 -> 7826.
+// MaskedFFN forward d = 1024, h = 2048, M = 8192 137.3 -> 134.6; M = 32768, d = 4096, h = 14336 the same within the runs' spread.
 // Rows are COLS results; 16-byte chunks are XORed with the row so that the 16 rows of a write and the rows of a read each
 // cover all banks.
 template <class Cfg>
@@ -1358,7 +1358,8 @@ struct WaveRows {
 // eight columns is read from the pre-activations and written by one lane, so that they may be T13 itself.  Bound by its five
 // passes over [M, h] (45 us per round of 256x256 tiles against 7 of plain stores); as a launch of its own the derivative made six
 // and read dh back: forward + backward at M = 4096, d = 4096, h = 14336 3550 -> 3514 us, and up to
-// 1.8 % less over 22 drawn layers that the device bounds, none slower.
+// 1.8 % less over 22 drawn layers that the device bounds, none slower (timed with v_rcp_f32 for swiglu_bwd's division, which
+// takes 8 of these us back).
 template <class Cfg>
 __device__ __forceinline__ void swiglu_bwd_epilogue(const GemmArgs& g, typename Cfg::Acc (&acc)[Cfg::TM][Cfg::TN], int row0, int row_end,
                                                     int n0, const TileLanes<Cfg>& tl, uint8_t* lds) {

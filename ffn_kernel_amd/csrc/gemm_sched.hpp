@@ -76,9 +76,10 @@ __host__ __device__ inline TileCoord routed_tile_coord(int L, int n_vis, int M, 
 // earlier.  Tall tiles past the last whole round run as two short ones where those and the other short ones are one round.
 // The SwiGLU GEMM over 1353 drawn shapes of 0.5 - 30 rounds that the time model gives to 256x256 tiles, caches not flushed, against
 // those tiles with their remainder as 128x128 ones in a second launch (which takes 5 us where it is empty): 4.9 % less time in the
-// geometric mean (8.5 % below a round, 5.8 % up to two, 4.1 % up to four, 2.3 % up to eight), 79 % of them faster and 1 % by more
-// than 3 % slower (0.90).  M = 300 (150 + 150), K = 4096, 14336 columns: 122.7 -> 111.3 us, the MaskedFFN call 212 -> 184; M = 499,
-// K = 5696, 16192 columns 278 -> 200.
+// geometric mean (8.5 % below a round, 5.8 % up to two, 4.1 % up to four, 2.3 % up to eight), 79 % of them faster.  Caches flushed,
+// 3000 others: 3.5 % less, 1.8 % of them more than 3 % slower (the worst 13 %): calls whose rows end just past a whole round, where
+// the mask decides which side wins.  M = 300 (150 + 150), K = 4096, 14336 columns: 122.7 -> 111.3 us, the MaskedFFN call 207 -> 184;
+// M = 499, K = 5696, 16192 columns 278 -> 200.
 constexpr int kTallRows = 256, kShortRows = 160, kTallCost = 256, kShortCost = 176;
 // A column's weight panel from memory, by the whole chip: 512 bytes per element of the contraction at 6.2 TB/s against the tall
 // tile's 1.056 us per 64 of them.  Tiles of both heights of one modality read it twice (they run at different times).

@@ -383,10 +383,10 @@ def masked_ffn_forward(a, w1, w2, w3, u1, u2, u3, mask, save_pre: bool = False, 
 def masked_ffn_backward(grad, a, w1, w2, w3, u1, u2, u3, mask, pre=None, routing: Routing | None = None):
     """(da, dw1, dw2, dw3, du1, du2, du3) of MaskedFFN.  The reference stops at NotImplementedError
     here (ops.py:34-38); the decomposition follows its README sketch (README.md:159-172): routed
-    GEMMs around one elementwise SwiGLU-gradient pass.  Weight gradients keep the strides of the
-    weight views they belong to, as the linear backward's do.  pre: the pre-activations that
-    masked_ffn_forward(..., save_pre=True) returned for the same inputs (read-only); None: they are
-    recomputed."""
+    GEMMs, the SwiGLU derivative in the epilogue of the one that makes dh.  Weight gradients keep the
+    strides of the weight views they belong to, as the linear backward's do.  pre: the pre-activations
+    that masked_ffn_forward(..., save_pre=True) returned for the same inputs (read-only); None: they are
+    recomputed, which may sum in another order than the forward did."""
     grads = _native().ffn_bwd(grad, a, w1, w2, w3, u1, u2, u3, mask, pre, routing)
     if grads is not NotImplemented:
         return grads

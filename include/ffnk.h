@@ -286,7 +286,7 @@ FFNK_API int ffnk_masked_linear_bwd_routed(const uint16_t* g, int64_t g_stride_m
 /*
  * MaskedFFN backward.  The reference declares it but raises NotImplementedError
  * (ffn_kernel/ops.py:34-38); its README (README.md:159-172) sketches the decomposition used
- * here: an elementwise SwiGLU-gradient pass between routed GEMMs.  For row m with
+ * here: routed GEMMs around the SwiGLU derivative (in the dh GEMM's epilogue).  For row m with
  * (A1, A2, A3) = mask[m] ? (W1, W2, W3) : (U1, U2, U3), t1 = x[m] @ A1, t3 = x[m] @ A3:
  *   dh  = g[m] @ A2^T
  *   dt1 = dh * t3 * silu'(t1),  dt3 = dh * silu(t1),  silu'(t) = s + t s (1 - s), s = sigmoid(t)
@@ -298,9 +298,10 @@ FFNK_API int ffnk_masked_linear_bwd_routed(const uint16_t* g, int64_t g_stride_m
  * dW1/dW3/dU1/dU3: logical [d, h] with strides (dup_stride_k, dup_stride_n); dW2/dU2: logical
  * [h, d] with strides (ddown_stride_k, ddown_stride_n).  t1, t3, dh, dt1, dt3 and the
  * intermediate are held in bf16 between the GEMMs (the forward does the same for the
- * intermediate); accumulation is fp32; deterministic, no atomics.  With d and h multiples of 64 and
- * the weight views the reference passes (or a down weight whose d axis is contiguous) every GEMM reads
- * the weights in place; other extents and strides are first copied into the workspace.
+ * intermediate); accumulation is fp32; deterministic, no atomics.  With the weight views the reference
+ * passes (or a down weight whose d axis is contiguous) every GEMM reads the weights in place; other
+ * strides, unaligned weights and extents under 128 that are no multiples of 64 are first copied into the
+ * workspace.
  * Workspace: ffnk_workspace_bytes(FFNK_OP_FFN_BWD, M, d, h).  Layouts outside the above
  * (d or h not a multiple of 8, unaligned rows, up_stride_k != 1) return FFNK_E_STRIDE.
  */
@@ -328,7 +329,8 @@ FFNK_API int ffnk_masked_ffn_bwd(const uint16_t* g, int64_t g_stride_m,
  * ffnk_masked_ffn_fwd_save is ffnk_masked_ffn_fwd and additionally writes pre: [M, 2h] bf16, row
  * stride pre_stride_m (>= 2h, multiple of 8, rows 16-byte aligned), rows in ROUTED order (visual
  * rows first, each group ascending), columns [0, h) = t1 = x A1, [h, 2h) = t3 = x A3, rounded to
- * bf16 from the fp32 accumulators - what the recomputing backward would produce.  Only the LDS-tiled
+ * bf16 from the fp32 accumulators - what the recomputing backward would produce, up to the order of its
+ * fp32 sums (its GEMMs may run on other tiles).  Only the LDS-tiled
  * path can do it: ffnk_masked_ffn_can_save(M, d, h) says whether this shape qualifies (M > 64, d and h
  * multiples of 8); the fast layout of ffnk_masked_ffn_fwd is required on top.  FFNK_E_STRIDE otherwise.
  *
