@@ -53,7 +53,7 @@ _SIGNATURES = {
                                     c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64,  # dW1 dW3 dU1 dU3
                                     c_void_p, c_void_p, c_int64, c_int64,            # dW2 dU2
                                     c_int64, c_int64, c_int64, c_void_p, c_size_t, c_void_p]),
-    # the *_routed variants: the plain signature (+ pre where optional) + const ffnk_routing_t*
+    # the *_routed variants (and the *_routing ones, whose partition the call makes): the plain signature (+ pre where optional) + const ffnk_routing_t*
     "ffnk_masked_linear_fwd_routed": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_void_p,
                                               c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_size_t,
                                               c_void_p, c_void_p]),
@@ -89,6 +89,8 @@ _SIGNATURES = {
                                           c_void_p, c_void_p, c_int64, c_int64,
                                           c_int64, c_int64, c_int64, c_void_p, c_size_t, c_void_p]),
 }
+for _name in ("ffnk_masked_linear_fwd", "ffnk_masked_ffn_fwd"):
+    _SIGNATURES[f"{_name}_routing"] = _SIGNATURES[f"{_name}_routed"]
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
 
@@ -104,6 +106,11 @@ class TileConfig(ctypes.Structure):
 class RoutingStruct(ctypes.Structure):
     """Mirror of ffnk_routing_t: device addresses of perm int32[M] and counts int32[2]."""
     _fields_ = [("perm", c_void_p), ("counts", c_void_p)]
+
+
+class PartitionStruct(ctypes.Structure):
+    """A ffnk_routing_t and whether a launch has been made that fills it (csrc/call.cpp: Partition)."""
+    _fields_ = [("routing", RoutingStruct), ("made", c_int32)]
 
 
 class FfnkError(RuntimeError):

@@ -22,18 +22,47 @@ namespace {
 struct Library {
   decltype(&ffnk_workspace_bytes) workspace_bytes;
   decltype(&ffnk_masked_ffn_can_save) can_save;
-  decltype(&ffnk_masked_linear_fwd_routed) linear_fwd;
+  decltype(&ffnk_route) route;
+  decltype(&ffnk_masked_linear_fwd_routed) linear_fwd, linear_fwd_routing;
   decltype(&ffnk_masked_linear_bwd_routed) linear_bwd;
-  decltype(&ffnk_masked_ffn_fwd_routed) ffn_fwd;
+  decltype(&ffnk_masked_ffn_fwd_routed) ffn_fwd, ffn_fwd_routing;
   decltype(&ffnk_masked_ffn_bwd_routed) ffn_bwd;
 } lib;
-PyObject* routing_address = nullptr;    // (routing or None, mask, M, stream) -> address of a ffnk_routing_t, or 0
+PyObject* routing_address = nullptr;    // (routing or None, mask, M, stream) -> address of a Partition, or 0
 PyObject* ffn_bwd_workspace = nullptr;  // (a, d, h, row stride of the upstream gradient) -> workspace tensor
 PyObject* check = nullptr;              // (return code, function name): raises
 int64_t routed_min_rows = 0;            // below: no partition is shared
 
+// _lib.PartitionStruct: memory for a row partition, and whether a launch that fills it has been made.
+struct Partition {
+  ffnk_routing_t routing;
+  int32_t made;
+};
+const ffnk_routing_t* routing_of(const Partition* p) { return p ? &p->routing : nullptr; }
+
 const uint16_t* in(const at::Tensor& t) { return static_cast<const uint16_t*>(t.const_data_ptr()); }
 uint16_t* out(const at::Tensor& t) { return static_cast<uint16_t*>(t.mutable_data_ptr()); }
+
+struct WithoutGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
+// The foreign call without the GIL, as ctypes makes it.  f reads the tensors' addresses, and torch throws where one has none (an
+// output that a dispatch mode made a fake tensor): the error is made a Python one by the caller, which needs the GIL back.
+template <class F>
+bool run(const char* name, F&& f) {
+  int rc;
+  {
+    WithoutGil released;
+    rc = f();
+  }
+  if (rc == 0) return true;
+  PyObject* r = PyObject_CallFunction(check, "is", rc, name);
+  Py_XDECREF(r);
+  if (r) PyErr_SetString(PyExc_RuntimeError, name);
+  return false;
+}
 
 // The tensors of a call; `ok` goes false at the first one that is not plain.
 struct Call {
@@ -83,14 +112,25 @@ struct Call {
     return at::empty({(int64_t)(bytes > 16 ? bytes : 16)}, like.options().dtype(at::kByte));
   }
   // The partition the call runs with; false with a Python error set.
-  bool routing(PyObject* given, PyObject* mask, const ffnk_routing_t** r) const {
+  bool routing(PyObject* given, PyObject* mask, Partition** r) const {
     *r = nullptr;
     if (given == Py_None && M < routed_min_rows) return true;
     PyObject* address = PyObject_CallFunction(routing_address, "OOLK", given, mask, (long long)M, (unsigned long long)(uintptr_t)stream);
     if (!address) return false;
-    *r = static_cast<const ffnk_routing_t*>(PyLong_AsVoidPtr(address));
+    *r = static_cast<Partition*>(PyLong_AsVoidPtr(address));
     Py_DECREF(address);
     return !PyErr_Occurred();
+  }
+  // A backward whose forward left none.
+  bool fill(Partition* r, const at::Tensor& mask) const {
+    if (!r || r->made) return true;
+    if (!run("ffnk_route", [&] {
+          return lib.route(static_cast<const uint8_t*>(mask.const_data_ptr()), M, const_cast<int32_t*>(r->routing.perm),
+                           const_cast<int32_t*>(r->routing.counts), stream);
+        }))
+      return false;
+    r->made = 1;
+    return true;
   }
 
  private:
@@ -99,27 +139,6 @@ struct Call {
     return nullptr;
   }
 };
-
-struct WithoutGil {
-  PyThreadState* state = PyEval_SaveThread();
-  ~WithoutGil() { PyEval_RestoreThread(state); }
-};
-
-// The foreign call without the GIL, as ctypes makes it.  f reads the tensors' addresses, and torch throws where one has none (an
-// output that a dispatch mode made a fake tensor): the error is made a Python one by the caller, which needs the GIL back.
-template <class F>
-bool run(const char* name, F&& f) {
-  int rc;
-  {
-    WithoutGil released;
-    rc = f();
-  }
-  if (rc == 0) return true;
-  PyObject* r = PyObject_CallFunction(check, "is", rc, name);
-  Py_XDECREF(r);
-  if (r) PyErr_SetString(PyExc_RuntimeError, name);
-  return false;
-}
 
 int64_t size_of(PyObject* o, int64_t dim) {  // -1: no 2-D tensor
   if (!THPVariable_CheckExact(o)) return -1;
@@ -138,14 +157,17 @@ PyObject* linear_fwd(PyObject*, PyObject* const* p, Py_ssize_t n) {
   const size_t bytes = lib.workspace_bytes(FFNK_OP_LINEAR_FWD, c.M, K, N);
   if (bytes == (size_t)-1) Py_RETURN_NOTIMPLEMENTED;
   at::Tensor y = c.empty(*a, c.M, N);
-  const ffnk_routing_t* r;
+  Partition* r;
   if (!c.routing(p[4], p[3], &r)) return nullptr;
   at::Tensor ws = c.workspace(*a, bytes);
+  const bool fills = r && !r->made;
   if (!run("ffnk_masked_linear_fwd", [&] {
-        return lib.linear_fwd(in(*a), Call::ld(*a), in(*b1), in(*b2), 1, K, static_cast<const uint8_t*>(mask->const_data_ptr()), out(y),
-                              N, c.M, K, N, ws.mutable_data_ptr(), (size_t)ws.numel(), c.stream, r);
+        return (fills ? lib.linear_fwd_routing : lib.linear_fwd)(
+            in(*a), Call::ld(*a), in(*b1), in(*b2), 1, K, static_cast<const uint8_t*>(mask->const_data_ptr()), out(y), N, c.M, K, N,
+            ws.mutable_data_ptr(), (size_t)ws.numel(), c.stream, routing_of(r));
       }))
     return nullptr;
+  if (fills) r->made = 1;
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
 }
@@ -161,13 +183,14 @@ PyObject* linear_bwd(PyObject*, PyObject* const* p, Py_ssize_t n) {
   const size_t bytes = lib.workspace_bytes(FFNK_OP_LINEAR_BWD, c.M, K, N);
   if (bytes == (size_t)-1) Py_RETURN_NOTIMPLEMENTED;
   at::Tensor da = c.empty(*a, c.M, K), d1 = c.empty_weight(*b1, K, N), d2 = c.empty_weight(*b2, K, N);
-  const ffnk_routing_t* r;
+  Partition* r;
   if (!c.routing(p[5], p[4], &r)) return nullptr;
   at::Tensor ws = c.workspace(*a, bytes);
+  if (!c.fill(r, *mask)) return nullptr;
   if (!run("ffnk_masked_linear_bwd", [&] {
         return lib.linear_bwd(in(*g), Call::ld(*g), in(*a), Call::ld(*a), in(*b1), in(*b2), 1, K,
                               static_cast<const uint8_t*>(mask->const_data_ptr()), out(da), K, out(d1), out(d2), 1, K, c.M, K, N,
-                              ws.mutable_data_ptr(), (size_t)ws.numel(), c.stream, r);
+                              ws.mutable_data_ptr(), (size_t)ws.numel(), c.stream, routing_of(r));
       }))
     return nullptr;
   return Py_BuildValue("NNN", THPVariable_Wrap(std::move(da)), THPVariable_Wrap(std::move(d1)), THPVariable_Wrap(std::move(d2)));
@@ -190,15 +213,18 @@ PyObject* ffn_fwd(PyObject*, PyObject* const* p, Py_ssize_t n) {
   if (bytes == (size_t)-1) Py_RETURN_NOTIMPLEMENTED;
   at::Tensor y = c.empty(*a, c.M, d), pre;
   if (save && lib.can_save(c.M, d, h)) pre = c.empty(*a, c.M, 2 * h);
-  const ffnk_routing_t* r;
+  Partition* r;
   if (!c.routing(p[9], p[7], &r)) return nullptr;
   at::Tensor ws = c.workspace(*a, bytes);
+  const bool fills = r && !r->made;
   if (!run("ffnk_masked_ffn_fwd", [&] {
-        return lib.ffn_fwd(in(*a), Call::ld(*a), in(*w[0]), in(*w[2]), in(*w[3]), in(*w[5]), 1, d, in(*w[1]), in(*w[4]), 1, h,
-                           static_cast<const uint8_t*>(mask->const_data_ptr()), out(y), d, pre.defined() ? out(pre) : nullptr,
-                           pre.defined() ? 2 * h : 0, c.M, d, h, ws.mutable_data_ptr(), (size_t)ws.numel(), c.stream, r);
+        return (fills ? lib.ffn_fwd_routing : lib.ffn_fwd)(
+            in(*a), Call::ld(*a), in(*w[0]), in(*w[2]), in(*w[3]), in(*w[5]), 1, d, in(*w[1]), in(*w[4]), 1, h,
+            static_cast<const uint8_t*>(mask->const_data_ptr()), out(y), d, pre.defined() ? out(pre) : nullptr,
+            pre.defined() ? 2 * h : 0, c.M, d, h, ws.mutable_data_ptr(), (size_t)ws.numel(), c.stream, routing_of(r));
       }))
     return nullptr;
+  if (fills) r->made = 1;
   if (!save) return THPVariable_Wrap(std::move(y));
   return Py_BuildValue("NN", THPVariable_Wrap(std::move(y)), pre.defined() ? THPVariable_Wrap(std::move(pre)) : Py_NewRef(Py_None));
   END_HANDLE_TH_ERRORS
@@ -227,13 +253,14 @@ PyObject* ffn_bwd(PyObject*, PyObject* const* p, Py_ssize_t n) {
   THPObjectPtr space(PyObject_CallFunction(ffn_bwd_workspace, "OLLL", p[1], (long long)d, (long long)h, (long long)Call::ld(*g)));
   if (!space) return nullptr;
   const at::Tensor& ws = THPVariable_Unpack(space.get());
-  const ffnk_routing_t* r;
+  Partition* r;
   if (!c.routing(p[10], p[8], &r)) return nullptr;
+  if (!c.fill(r, *mask)) return nullptr;
   if (!run("ffnk_masked_ffn_bwd", [&] {
         return lib.ffn_bwd(in(*g), Call::ld(*g), in(*a), Call::ld(*a), in(*w[0]), in(*w[2]), in(*w[3]), in(*w[5]), 1, d, in(*w[1]),
                            in(*w[4]), 1, h, static_cast<const uint8_t*>(mask->const_data_ptr()), pre ? in(*pre) : nullptr,
                            pre ? Call::ld(*pre) : 0, out(da), d, out(dw[0]), out(dw[2]), out(dw[3]), out(dw[5]), 1, d, out(dw[1]),
-                           out(dw[4]), 1, h, c.M, d, h, ws.mutable_data_ptr(), (size_t)ws.numel(), c.stream, r);
+                           out(dw[4]), 1, h, c.M, d, h, ws.mutable_data_ptr(), (size_t)ws.numel(), c.stream, routing_of(r));
       }))
     return nullptr;
   PyObject* grads = PyTuple_New(7);

@@ -97,23 +97,49 @@ int forced_splits() {
 int64_t padded_rows(int64_t M) { return round_up64(M, 64) + 64; }  // >= pad64(nv) + pad64(M - nv)
 
 // The row partition a call works with: the caller's (ffnk_routing_t, made by ffnk_route for the same mask
-// and M) or, without one, the workspace's own region, filled by a route launch at the head of the call.
+// and M) or, without one, the workspace's own region.
 struct Routing {
   const int32_t* perm;
   const int32_t* counts;
+  const uint8_t* mask = nullptr;  // the call's first GEMM makes it (GemmArgs::mask)
 };
-int resolve_routing(const ffnk_routing_t* rt, const RouteWs& r, const uint8_t* mask, int64_t M, hipStream_t stream,
+// `make`: the caller's is still to be made, and left there for the calls behind this one.  `in_gemm`: the call's first GEMM can
+// make a partition; a launch of its own at the head of the call does where it cannot.
+int resolve_routing(const ffnk_routing_t* rt, bool make, const RouteWs& r, const uint8_t* mask, int64_t M, bool in_gemm, hipStream_t stream,
                     Routing* out) {
+  int32_t *perm = r.perm, *counts = r.counts;
   if (rt != nullptr) {
     if (!rt->perm || !rt->counts) return fail(FFNK_E_NULL, "routing: perm or counts is NULL");
-    out->perm = rt->perm;
-    out->counts = rt->counts;
-    return FFNK_OK;
+    perm = const_cast<int32_t*>(rt->perm);
+    counts = const_cast<int32_t*>(rt->counts);
   }
-  FFNK_HIP(launch_route(mask, (int)M, r.perm, r.counts, stream), "route kernel");
-  out->perm = r.perm;
-  out->counts = r.counts;
+  out->perm = perm;
+  out->counts = counts;
+  if (rt != nullptr && !make) return FFNK_OK;
+  if (in_gemm) out->mask = mask;
+  else FFNK_HIP(launch_route(mask, (int)M, perm, counts, stream), "route kernel");
   return FFNK_OK;
+}
+// Paths without a partition of their own leave the caller's all the same.
+int leave_routing(const ffnk_routing_t* rt, bool make, const uint8_t* mask, int64_t M, hipStream_t stream) {
+  Routing unused;
+  return make ? resolve_routing(rt, true, RouteWs{}, mask, M, false, stream, &unused) : FFNK_OK;
+}
+// The first GEMM of a forward makes the partition (GemmArgs::mask): one launch, results by whole 16-byte chunks, up to one and a half
+// rounds of the chip.  Every workgroup then counts the mask, 0.7 us more than it takes to read a partition (64x128 tiles at
+// M = 2048, 1 us for a 256x256 tile at M = 8192), against 3 to 4 us for the launch on the device and as much again on the host:
+// MaskedLinear, masks of both modalities, K = N = 1024, M = 2048 18.0 -> 14.1 us, M = 3001, K = 2056, N = 1544 38.7 -> 36.6,
+// forward + backward at K = N = 1024, M = 8192 108-125 -> 83-117 (runs of one side differ widely); MaskedFFN d = 4096, h = 14336, M = 300 177.8 ->
+// 173.8.  Past that every tile pays: d = 1024, h = 2048, M = 8192 (2.1 rounds) 133.7 -> 135.3, d = 4096, h = 14336, M = 1411 (2.6)
+// 474.7 -> 475.3.
+bool gemm_routes(int tile, bool direct, bool dual, int splits, int64_t M, int64_t N, const uint8_t* mask, const uint16_t* C, int64_t ldc) {
+  if (!direct || M > kScanMaxRows || !aligned16(mask) || !aligned16(C) || N % 8 != 0 || ldc % 8 != 0) return false;
+  const TileGeom t = tile_geom(tile == TILE_MIXED_W4 ? TILE_256x256_W4 : tile, dual);
+  const int64_t tiles = (cdiv64(M, t.block_m) + 1) * cdiv64(N, t.block_n_out) * splits;
+  if (is_big_tile(tile) && splits == 1 && tiles > kCus) return false;  // (a second launch for the remainder: dispatch_tile_with_tail)
+  if (tile == TILE_256x256_W4 && !dual) return false;                  // (RoutedGemmCfg::SELF_ROUTED)
+  const int per_cu = tile == TILE_SMALL_W4 ? 3 : tile == TILE_128x128_W4 || tile == TILE_64x128_R3 ? 2 : 1;
+  return 2 * tiles <= 3 * (int64_t)kCus * per_cu;
 }
 
 struct BwdPlan {
@@ -542,6 +568,82 @@ FfnBwdGemms ffn_bwd_gemms(int64_t M, int64_t d, int64_t h, const FfnBwdPaths& pa
   return g;
 }
 
+int linear_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* Wv, const uint16_t* Wt, int64_t w_stride_k,
+                    int64_t w_stride_n, const uint8_t* mask, uint16_t* y, int64_t y_stride_m, int64_t M, int64_t K, int64_t N, void* ws,
+                    size_t ws_bytes, void* stream_, const ffnk_routing_t* routing, bool make) {
+  hipStream_t stream = (hipStream_t)stream_;
+  if (int e = check_extents(M, K, N)) return e;
+  if (M == 0 || N == 0) return mask || M == 0 ? leave_routing(routing, make, mask, M, stream) : FFNK_OK;
+  if (!x && K > 0) return fail(FFNK_E_NULL, "x is NULL");
+  if ((!Wv || !Wt) && K > 0) return fail(FFNK_E_NULL, "weight pointer is NULL");
+  if (!mask || !y) return fail(FFNK_E_NULL, "mask or y is NULL");
+  if (!aligned2(x) || !aligned2(Wv) || !aligned2(Wt) || !aligned2(y)) return fail(FFNK_E_ALIGN, "bf16 pointer not 2-byte aligned");
+  if (y_stride_m < N) return fail(FFNK_E_STRIDE, "y_stride_m=%lld < N=%lld", (long long)y_stride_m, (long long)N);
+
+  const bool fast = K > 0 && K % 8 == 0 && x_stride_m % 8 == 0 && x_stride_m >= K && aligned16(x) &&
+                    w_stride_k == 1 && w_stride_n % 8 == 0 && w_stride_n >= K && aligned16(Wv) && aligned16(Wt);
+  if (!fast) {
+    GenericLinearArgs a;
+    a.x = x; a.sxm = x_stride_m; a.sxk = 1;
+    a.W[0] = Wv; a.W[1] = Wt; a.swk = w_stride_k; a.swn = w_stride_n;
+    a.mask = mask; a.y = y; a.sym = y_stride_m; a.syn = 1;
+    a.M = (int)M; a.K = (int)K; a.N = (int)N;
+    FFNK_HIP(launch_generic_linear(a, stream), "generic linear kernel");
+    return leave_routing(routing, make, mask, M, stream);
+  }
+  const size_t need = ffnk_workspace_bytes(FFNK_OP_LINEAR_FWD, M, K, N);
+  if (ws_bytes < need || !ws) return fail(FFNK_E_WORKSPACE, "workspace %zu < %zu bytes", ws_bytes, need);
+  if (!aligned16(ws)) return fail(FFNK_E_ALIGN, "workspace not 16-byte aligned");
+  const RouteWs r = carve_route(static_cast<uint8_t*>(ws), M);
+  const bool far_rows = M * x_stride_m >= ((int64_t)1 << 30);  // past the LDS-transposed streams' 32-bit offsets
+  const int kind = linear_stream_kind(M, K, N);
+  if (kind && !(kind == 2 && far_rows && !stream_tile_down_ok((int)M, (int)N, (int)K))) {
+    // Decode sizes: the weight-streaming kernels of the FFN's down projection, fed token rows in
+    // token order; they route from the mask themselves.
+    if (kind == 2 && far_rows)
+      return fail(FFNK_E_STRIDE, "x_stride_m=%lld: the decode kernels address the token rows with 32-bit offsets",
+                  (long long)x_stride_m);
+    const int splits = linear_stream_splits(M, K, N);
+    StreamArgs a;
+    a.X = x; a.ldx = x_stride_m; a.gather_x = 1; a.mask = mask; a.M = (int)M;
+    a.W0[0] = Wv; a.W0[1] = Wt; a.W1[0] = a.W1[1] = nullptr; a.ldw = w_stride_n;
+    a.Nrows = (int)N; a.K = (int)K; a.splits = splits; a.H = nullptr; a.ldh = 0;
+    a.P = splits > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + r.bytes) : nullptr;
+    a.out = y; a.ldo = y_stride_m;
+    FFNK_HIP(kind == 1 ? launch_stream_dot_down(a, stream) : launch_stream_tile_down(a, stream), "streaming linear");
+    if (splits > 1)
+      FFNK_HIP(launch_stream_reduce(a.P, splits, (int)M, (int)N, mask, y, y_stride_m, stream), "streaming reduce");
+    return leave_routing(routing, make, mask, M, stream);
+  }
+  const bool direct = direct_ok(K, M, x_stride_m, w_stride_n);
+  RoutedPlan plan = linear_plan(M, K, N);
+  if (!direct) {
+    plan.splits = plan.splits_more = 1;
+    plan.tile = routed_tile(M, N, false, K);
+  }
+  Routing rt;
+  const bool in_gemm = gemm_routes(plan.tile, direct, false, max_splits(plan), M, N, mask, y, y_stride_m);
+  if (int e = resolve_routing(routing, make, r, mask, M, in_gemm, stream, &rt)) return e;
+  GemmArgs g;
+  g.A = x; g.lda = x_stride_m;
+  g.B0[0] = Wv; g.B0[1] = Wt; g.B1[0] = g.B1[1] = nullptr; g.ldb = w_stride_n;
+  g.C = y; g.ldc = y_stride_m;
+  g.perm = rt.perm; g.counts = rt.counts; g.mask = rt.mask;
+  g.M = (int)M; g.N = (int)N; g.K = (int)K; g.group_m = plan_group_m(TUNED_PLAIN, M, K, N);
+  if (plan.splits > 1) {
+    g.splits = plan.splits;
+    g.splits_more = plan.splits_more;
+    g.P = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + r.bytes);
+  } else if (direct && is_big_tile(plan.tile)) {
+    g.P_tail = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + r.bytes);
+  }
+  FFNK_HIP(launch_linear_gemm(plan.tile, direct, g, stream), "linear GEMM");
+  if (plan.splits > 1)
+    FFNK_HIP(launch_routed_reduce(g.P, plan.splits, plan.splits_more, tile_geom(plan.tile, false).block_m, (int)M, (int)N, rt.counts,
+                                  rt.perm, y, y_stride_m, stream), "linear reduce");
+  return FFNK_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -756,76 +858,15 @@ int ffnk_masked_linear_fwd_routed(const uint16_t* x, int64_t x_stride_m, const u
                                   int64_t w_stride_k, int64_t w_stride_n, const uint8_t* mask, uint16_t* y,
                                   int64_t y_stride_m, int64_t M, int64_t K, int64_t N, void* ws, size_t ws_bytes,
                                   void* stream_, const ffnk_routing_t* routing) {
-  hipStream_t stream = (hipStream_t)stream_;
-  if (int e = check_extents(M, K, N)) return e;
-  if (M == 0 || N == 0) return FFNK_OK;
-  if (!x && K > 0) return fail(FFNK_E_NULL, "x is NULL");
-  if ((!Wv || !Wt) && K > 0) return fail(FFNK_E_NULL, "weight pointer is NULL");
-  if (!mask || !y) return fail(FFNK_E_NULL, "mask or y is NULL");
-  if (!aligned2(x) || !aligned2(Wv) || !aligned2(Wt) || !aligned2(y)) return fail(FFNK_E_ALIGN, "bf16 pointer not 2-byte aligned");
-  if (y_stride_m < N) return fail(FFNK_E_STRIDE, "y_stride_m=%lld < N=%lld", (long long)y_stride_m, (long long)N);
+  return linear_fwd_impl(x, x_stride_m, Wv, Wt, w_stride_k, w_stride_n, mask, y, y_stride_m, M, K, N, ws, ws_bytes, stream_, routing, false);
+}
 
-  const bool fast = K > 0 && K % 8 == 0 && x_stride_m % 8 == 0 && x_stride_m >= K && aligned16(x) &&
-                    w_stride_k == 1 && w_stride_n % 8 == 0 && w_stride_n >= K && aligned16(Wv) && aligned16(Wt);
-  if (!fast) {
-    GenericLinearArgs a;
-    a.x = x; a.sxm = x_stride_m; a.sxk = 1;
-    a.W[0] = Wv; a.W[1] = Wt; a.swk = w_stride_k; a.swn = w_stride_n;
-    a.mask = mask; a.y = y; a.sym = y_stride_m; a.syn = 1;
-    a.M = (int)M; a.K = (int)K; a.N = (int)N;
-    FFNK_HIP(launch_generic_linear(a, stream), "generic linear kernel");
-    return FFNK_OK;
-  }
-  const size_t need = ffnk_workspace_bytes(FFNK_OP_LINEAR_FWD, M, K, N);
-  if (ws_bytes < need || !ws) return fail(FFNK_E_WORKSPACE, "workspace %zu < %zu bytes", ws_bytes, need);
-  if (!aligned16(ws)) return fail(FFNK_E_ALIGN, "workspace not 16-byte aligned");
-  const RouteWs r = carve_route(static_cast<uint8_t*>(ws), M);
-  const bool far_rows = M * x_stride_m >= ((int64_t)1 << 30);  // past the LDS-transposed streams' 32-bit offsets
-  const int kind = linear_stream_kind(M, K, N);
-  if (kind && !(kind == 2 && far_rows && !stream_tile_down_ok((int)M, (int)N, (int)K))) {
-    // Decode sizes: the weight-streaming kernels of the FFN's down projection, fed token rows in
-    // token order; they route from the mask themselves.
-    if (kind == 2 && far_rows)
-      return fail(FFNK_E_STRIDE, "x_stride_m=%lld: the decode kernels address the token rows with 32-bit offsets",
-                  (long long)x_stride_m);
-    const int splits = linear_stream_splits(M, K, N);
-    StreamArgs a;
-    a.X = x; a.ldx = x_stride_m; a.gather_x = 1; a.mask = mask; a.M = (int)M;
-    a.W0[0] = Wv; a.W0[1] = Wt; a.W1[0] = a.W1[1] = nullptr; a.ldw = w_stride_n;
-    a.Nrows = (int)N; a.K = (int)K; a.splits = splits; a.H = nullptr; a.ldh = 0;
-    a.P = splits > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + r.bytes) : nullptr;
-    a.out = y; a.ldo = y_stride_m;
-    FFNK_HIP(kind == 1 ? launch_stream_dot_down(a, stream) : launch_stream_tile_down(a, stream), "streaming linear");
-    if (splits > 1)
-      FFNK_HIP(launch_stream_reduce(a.P, splits, (int)M, (int)N, mask, y, y_stride_m, stream), "streaming reduce");
-    return FFNK_OK;
-  }
-  Routing rt;
-  if (int e = resolve_routing(routing, r, mask, M, stream, &rt)) return e;
-  GemmArgs g;
-  g.A = x; g.lda = x_stride_m;
-  g.B0[0] = Wv; g.B0[1] = Wt; g.B1[0] = g.B1[1] = nullptr; g.ldb = w_stride_n;
-  g.C = y; g.ldc = y_stride_m;
-  g.perm = rt.perm; g.counts = rt.counts;
-  g.M = (int)M; g.N = (int)N; g.K = (int)K; g.group_m = plan_group_m(TUNED_PLAIN, M, K, N);
-  const bool direct = direct_ok(K, M, x_stride_m, w_stride_n);
-  RoutedPlan plan = linear_plan(M, K, N);
-  if (!direct) {
-    plan.splits = plan.splits_more = 1;
-    plan.tile = routed_tile(M, N, false, K);
-  }
-  if (plan.splits > 1) {
-    g.splits = plan.splits;
-    g.splits_more = plan.splits_more;
-    g.P = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + r.bytes);
-  } else if (direct && is_big_tile(plan.tile)) {
-    g.P_tail = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + r.bytes);
-  }
-  FFNK_HIP(launch_linear_gemm(plan.tile, direct, g, stream), "linear GEMM");
-  if (plan.splits > 1)
-    FFNK_HIP(launch_routed_reduce(g.P, plan.splits, plan.splits_more, tile_geom(plan.tile, false).block_m, (int)M, (int)N, rt.counts,
-                                  rt.perm, y, y_stride_m, stream), "linear reduce");
-  return FFNK_OK;
+int ffnk_masked_linear_fwd_routing(const uint16_t* x, int64_t x_stride_m, const uint16_t* Wv, const uint16_t* Wt,
+                                   int64_t w_stride_k, int64_t w_stride_n, const uint8_t* mask, uint16_t* y,
+                                   int64_t y_stride_m, int64_t M, int64_t K, int64_t N, void* ws, size_t ws_bytes,
+                                   void* stream_, const ffnk_routing_t* made) {
+  if (!made) return fail(FFNK_E_NULL, "made is NULL");
+  return linear_fwd_impl(x, x_stride_m, Wv, Wt, w_stride_k, w_stride_n, mask, y, y_stride_m, M, K, N, ws, ws_bytes, stream_, made, true);
 }
 
 int ffnk_masked_ffn_fwd(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, const uint16_t* W3,
@@ -847,14 +888,14 @@ int ffn_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, cons
                  const uint16_t* U3, int64_t up_stride_k, int64_t up_stride_n, const uint16_t* W2, const uint16_t* U2,
                  int64_t down_stride_k, int64_t down_stride_n, const uint8_t* mask, uint16_t* out, int64_t out_stride_m,
                  uint16_t* pre, int64_t pre_stride_m, int64_t M, int64_t d, int64_t h, void* ws, size_t ws_bytes,
-                 void* stream_, void* const* events, const ffnk_routing_t* routing = nullptr, size_t ws_limit = kAnyRoom) {
+                 void* stream_, void* const* events, const ffnk_routing_t* routing = nullptr, size_t ws_limit = kAnyRoom, bool make = false) {
   hipStream_t stream = (hipStream_t)stream_;
   auto mark = [&](int i) -> hipError_t {
     if (events && events[i]) return hipEventRecord((hipEvent_t)events[i], stream);
     return hipSuccess;
   };
   if (int e = check_extents(M, d, h)) return e;
-  if (M == 0 || d == 0) return FFNK_OK;
+  if (M == 0 || d == 0) return mask || M == 0 ? leave_routing(routing, make, mask, M, stream) : FFNK_OK;
   if (!x || !mask || !out) return fail(FFNK_E_NULL, "x, mask or out is NULL");
   if (h > 0 && (!W1 || !W3 || !U1 || !U3 || !W2 || !U2)) return fail(FFNK_E_NULL, "weight pointer is NULL");
   if (!aligned2(x) || !aligned2(out) || !aligned2(W1) || !aligned2(W3) || !aligned2(U1) || !aligned2(U3) ||
@@ -902,7 +943,7 @@ int ffn_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, cons
     a.M = (int)M; a.K = (int)h; a.N = (int)d;
     FFNK_HIP(launch_generic_linear(a, stream), "generic down kernel");
     FFNK_HIP(mark(2), "event record");
-    return FFNK_OK;
+    return leave_routing(routing, make, mask, M, stream);
   }
 
   const bool far_rows = M * x_stride_m >= ((int64_t)1 << 30);  // past the LDS-transposed streams' 32-bit offsets
@@ -934,22 +975,23 @@ int ffn_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, cons
     if (splits > 1)
       FFNK_HIP(launch_stream_reduce(P, splits, (int)M, (int)d, mask, out, out_stride_m, stream), "streaming reduce");
     FFNK_HIP(mark(2), "event record");
-    return FFNK_OK;
+    return leave_routing(routing, make, mask, M, stream);
   }
 
+  const bool up_direct = direct_ok(d, M, x_stride_m, up_stride_n);
+  int up_tile = routed_tile(M, h, true, d);
+  if (up_two_heights(up_tile, up_direct, M, h)) up_tile = TILE_MIXED_W4;
   Routing rt;
-  if (int e = resolve_routing(routing, r, mask, M, stream, &rt)) return e;
+  const bool in_gemm = gemm_routes(up_tile, up_direct, true, 1, M, h, mask, H, ldh);
+  if (int e = resolve_routing(routing, make, r, mask, M, in_gemm, stream, &rt)) return e;
   FFNK_HIP(mark(0), "event record");
   GemmArgs up;
   up.A = x; up.lda = x_stride_m;
   up.B0[0] = W1; up.B0[1] = U1; up.B1[0] = W3; up.B1[1] = U3; up.ldb = up_stride_n;
   up.C = H; up.ldc = ldh;
-  up.perm = rt.perm; up.counts = rt.counts;
+  up.perm = rt.perm; up.counts = rt.counts; up.mask = rt.mask;
   up.M = (int)M; up.N = (int)h; up.K = (int)d; up.group_m = plan_group_m(TUNED_DUAL, M, d, h);
   up.C_pre = pre; up.ldc_pre = pre_stride_m;
-  const bool up_direct = direct_ok(d, M, x_stride_m, up_stride_n);
-  int up_tile = routed_tile(M, h, true, d);
-  if (up_two_heights(up_tile, up_direct, M, h)) up_tile = TILE_MIXED_W4;
   FFNK_HIP(launch_up_gemm(up_tile, up_direct, up, stream), "up-projection GEMM");
   FFNK_HIP(mark(1), "event record");
   GemmArgs dn;
@@ -1021,6 +1063,17 @@ int ffnk_masked_ffn_fwd_routed(const uint16_t* x, int64_t x_stride_m, const uint
                       out, out_stride_m, pre, pre_stride_m, M, d, h, ws, ws_bytes, stream_, nullptr, routing);
 }
 
+int ffnk_masked_ffn_fwd_routing(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, const uint16_t* W3,
+                               const uint16_t* U1, const uint16_t* U3, int64_t up_stride_k, int64_t up_stride_n,
+                               const uint16_t* W2, const uint16_t* U2, int64_t down_stride_k, int64_t down_stride_n,
+                               const uint8_t* mask, uint16_t* out, int64_t out_stride_m, uint16_t* pre,
+                               int64_t pre_stride_m, int64_t M, int64_t d, int64_t h, void* ws, size_t ws_bytes,
+                               void* stream_, const ffnk_routing_t* made) {
+  if (!made) return fail(FFNK_E_NULL, "made is NULL");
+  return ffn_fwd_impl(x, x_stride_m, W1, W3, U1, U3, up_stride_k, up_stride_n, W2, U2, down_stride_k, down_stride_n, mask,
+                      out, out_stride_m, pre, pre_stride_m, M, d, h, ws, ws_bytes, stream_, nullptr, made, kAnyRoom, true);
+}
+
 int ffnk_masked_ffn_can_save(int64_t M, int64_t d, int64_t h) {
   return (M > 0 && d > 0 && h > 0 && d % 8 == 0 && h % 8 == 0 && !use_stream_path(M, d, h)) ? 1 : 0;
 }
@@ -1080,7 +1133,7 @@ int ffnk_masked_linear_bwd_routed(const uint16_t* g, int64_t g_stride_m, const u
   uint8_t* wsb = static_cast<uint8_t*>(ws);
   const RouteWs r = carve_route(wsb, M);
   Routing rt;
-  if (int e = resolve_routing(routing, r, mask, M, stream, &rt)) return e;
+  if (int e = resolve_routing(routing, false, r, mask, M, false, stream, &rt)) return e;
 
   // ---- dx = gather(g) @ W_g^T, contraction over N: needs the weights as [K, N] rows, N contiguous ----
   const uint16_t* wt[2] = {Wv, Wt};
@@ -1195,7 +1248,7 @@ int ffn_bwd_impl(const uint16_t* g, int64_t g_stride_m, const uint16_t* x, int64
   uint16_t* T13 = reinterpret_cast<uint16_t*>(wsb + p.off_t13);
   uint16_t* DH = reinterpret_cast<uint16_t*>(wsb + p.off_dh);
   Routing rt;
-  if (int e = resolve_routing(routing, r, mask, M, stream, &rt)) return e;
+  if (int e = resolve_routing(routing, false, r, mask, M, false, stream, &rt)) return e;
 
   // ---- pre-activations, routed order: T13[:, 0:h] = x A1, T13[:, half:half + h] = x A3 ----
   GemmArgs a;

@@ -4,6 +4,8 @@
 
 namespace ffnk {
 
+constexpr int kScanMaxRows = 8192;  // rows that a workgroup counts by itself (RowScan)
+
 struct GemmArgs {
   const uint16_t* A;     // [*, K] rows, K contiguous
   int64_t lda;
@@ -40,6 +42,9 @@ struct GemmArgs {
   const int32_t* perm;   // routed position -> token row
   const int32_t* counts; // counts[0] = visual rows (device memory)
   int M, N, K;           // N = output columns
+  // Forward GEMMs with gathered rows, in one launch: the partition is not there yet.  Every workgroup makes it from the mask
+  // (16-byte aligned, M <= kScanMaxRows) and the launch leaves it in perm and counts for the ones behind it.
+  const uint8_t* mask = nullptr;
   // Tile schedule.  The order of macro tiles is computed on a grid of sched_bm x sched_bn output
   // tiles (0 = the kernel's own tile).  tail_mode 0: the launch covers every tile.  1: only the tiles
   // that fill whole rounds of the chip (the first floor(tiles / 256) * 256 of the order).  2: only the

@@ -20,6 +20,7 @@
 #include "common.hpp"
 #include "gemm_args.hpp"
 #include "gemm_sched.hpp"
+#include "route_rows.hpp"
 
 namespace ffnk {
 
@@ -114,6 +115,9 @@ struct RoutedGemmCfg {
   // weight panel's (acc_col).  Same products in the same order.  Weight-gradient kernels, see splitk_store.
   static constexpr bool SWAP = SWAP_;
   static constexpr int NWAVES = WAVES_M * WAVES_N;
+  // Can make the row partition itself (GemmArgs::mask).  Not the single-weight four-wave 256x256 tile, which has no registers left
+  // and is for long contractions past a round of the chip.
+  static constexpr bool SELF_ROUTED = GATHER_A_ && DIRECT_ && !B_KMAJOR_ && (DUAL_ || (SCATTER_C_ && !(BM_ == 256 && NWAVES == 4)));
   static constexpr int NT = NWAVES * kWave;
   static constexpr int BN_OUT = DUAL ? BN / 2 : BN;        // output columns per tile
   static constexpr int WTM = BM / WAVES_M;                 // rows per wave
@@ -1325,6 +1329,7 @@ struct WaveRows {
   static constexpr int N = ROWS / PER;                              // loads and stores per lane
   static constexpr int RP = 16 / CH;                                // rows that cover the banks once
   static constexpr int BYTES = ROWS * COLS * 2;                     // of LDS per wave
+  static constexpr int ROW_REGS = cdiv(ROWS, kWave);                // output rows held by a lane
   static_assert(CH == 4 || CH == 8 || CH == 16, "rows of 32, 64 or 128 results");
   static_assert(Cfg::NWAVES * BYTES <= Cfg::LDS_BYTES, "the K loop's stages hold the tile's results");
 
@@ -1412,7 +1417,8 @@ __device__ __forceinline__ void swiglu_bwd_epilogue(const GemmArgs& g, typename 
 // columns acc_col(v, lh), i.e. runs of four consecutive columns.
 template <class Cfg>
 __device__ __forceinline__ void routed_epilogue(const GemmArgs& g, typename Cfg::Acc (&acc)[Cfg::TM][Cfg::TN], int row0,
-                                                int row_end, int n0, const TileLanes<Cfg>& tl, uint8_t* lds) {
+                                                int row_end, int n0, const TileLanes<Cfg>& tl, uint8_t* lds,
+                                                const int (&self_rows)[WaveRows<Cfg>::ROW_REGS]) {
   constexpr int TM = Cfg::TM, TN_OUT = Cfg::TN_OUT, MT = Cfg::MT, RUNS = Cfg::ACC_N / 4;
   const int wm = tl.wm, wn = tl.wn;
   const uint32_t lr = tl.lr, lh = tl.lh;
@@ -1429,11 +1435,12 @@ __device__ __forceinline__ void routed_epilogue(const GemmArgs& g, typename Cfg:
     using W = WaveRows<Cfg>;
     const int n = n0 + wn * Cfg::WTN_OUT + W::col(tl.lane), p0 = row0 + wm * Cfg::WTM;
     // Output rows of the wave's tile, one per lane; a store's lanes fetch theirs from the lane that holds it.
-    int rows[cdiv(W::ROWS, kWave)];
+    int rows[W::ROW_REGS];
 #pragma unroll
-    for (int q = 0; q < cdiv(W::ROWS, kWave); ++q) {
+    for (int q = 0; q < W::ROW_REGS; ++q) {
       const int p = p0 + q * kWave + tl.lane;
-      rows[q] = p < row_end && q * kWave + tl.lane < W::ROWS ? (Cfg::SCATTER_C ? g.perm[p] : p) : -1;
+      if (Cfg::SELF_ROUTED && Cfg::SCATTER_C && g.mask != nullptr) rows[q] = self_rows[q];
+      else rows[q] = p < row_end && q * kWave + tl.lane < W::ROWS ? (Cfg::SCATTER_C ? g.perm[p] : p) : -1;
     }
     dma_wait_barrier<0>();  // every wave has read its last fragments
     auto out = [&](uint16_t* base, int64_t ld) {
@@ -1552,7 +1559,7 @@ __device__ __forceinline__ void routed_partial_store(float* base, int64_t ld, co
 // One tile of a routed GEMM (tc), or one of `splits` K ranges of it.
 template <class Cfg>
 __device__ __forceinline__ void routed_tile(const GemmArgs& g, uint8_t* lds, const TileCoord& tc, const int split, const int splits,
-                                            const int tail_slot) {
+                                            const int tail_slot, const RowScan<Cfg::NT>& scan) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN;
   constexpr int TM = Cfg::TM, TN = Cfg::TN;
   const int grp = tc.grp, row0 = tc.row0, row_end = tc.row_end, n0 = tc.n0;  // row0: routed position
@@ -1582,10 +1589,32 @@ __device__ __forceinline__ void routed_tile(const GemmArgs& g, uint8_t* lds, con
     for (int j = 0; j < NJA; ++j) {
       int p = row0 + rl.load_row(j);
       p = min(p, row_end - 1);  // rows past the group end repeat the last row; never stored
-      src[j] = Cfg::GATHER_A ? g.perm[p] : p - row0;
+      src[j] = !Cfg::GATHER_A ? p - row0 : Cfg::SELF_ROUTED && g.mask != nullptr ? 0 : g.perm[p];
       baseA[j] = a0;
     }
+    int self_rows[WaveRows<Cfg>::ROW_REGS];  // GemmArgs::mask: what the epilogue would read from perm
     auto offsets_a = [&]() {
+      if constexpr (Cfg::SELF_ROUTED) {
+        if (g.mask != nullptr) {
+          // The rows go through the token panel's first stage, which no load has been issued for yet.
+          using Scan = RowScan<Cfg::NT>;
+          const int n = min(row_end - row0, BM);
+          scan.place(grp, row0, row0 + n, lds);
+          dma_wait_barrier<63>();
+#pragma unroll
+          for (int j = 0; j < NJA; ++j) src[j] = Scan::row(lds, min(rl.load_row(j), n - 1));
+#pragma unroll
+          for (int q = 0; q < WaveRows<Cfg>::ROW_REGS; ++q) {
+            const int r = q * kWave + rl.lane, p = rl.wm * Cfg::WTM + r;
+            self_rows[q] = Cfg::SCATTER_C && p < n && r < WaveRows<Cfg>::ROWS ? Scan::row(lds, min(p, n - 1)) : -1;
+          }
+          if (n0 == 0 && split == 0) {  // one workgroup per row leaves the partition to the launches behind this one
+            int32_t* perm = const_cast<int32_t*>(g.perm);
+            for (int p = (int)threadIdx.x; p < n; p += Cfg::NT) perm[row0 + p] = Scan::row(lds, p);
+          }
+          dma_wait_barrier<63>();
+        }
+      }
 #pragma unroll
       for (int j = 0; j < NJA; ++j) offA[j] = (uint32_t)(((int64_t)src[j] * g.lda + rl.c_log * 8) * 2);
     };
@@ -1628,7 +1657,7 @@ __device__ __forceinline__ void routed_tile(const GemmArgs& g, uint8_t* lds, con
       else
         routed_partial_store<Cfg>(g.P + (int64_t)split * g.M * g.N, g.N, g, acc, row0, row_end, n0, rl.wm, rl.wn, rl.lr, rl.lh);
     } else {
-      routed_epilogue<Cfg>(g, acc, row0, row_end, n0, rl, lds);
+      routed_epilogue<Cfg>(g, acc, row0, row_end, n0, rl, lds, self_rows);
     }
   } else {
     constexpr int NJA = TileLanes<Cfg>::NJA, NJB = TileLanes<Cfg>::NJB;
@@ -1651,8 +1680,26 @@ __device__ __forceinline__ void routed_tile(const GemmArgs& g, uint8_t* lds, con
       pb[j] = (up ? g.B1[grp] : g.B0[grp]) + (int64_t)n * g.ldb + tl.c_log * 8;
     }
     gemm_mainloop_staged<Cfg>(tl, pa, pb, g.K, lds, acc);
-    routed_epilogue<Cfg>(g, acc, row0, row_end, n0, tl, lds);
+    int no_rows[WaveRows<Cfg>::ROW_REGS];
+    routed_epilogue<Cfg>(g, acc, row0, row_end, n0, tl, lds, no_rows);
   }
+}
+
+// Visual rows: from the partition, or counted here (GemmArgs::mask).  `bid`: the workgroup's index in the GEMM.
+template <class Cfg>
+__device__ __forceinline__ int visual_rows(const GemmArgs& g, uint8_t* lds, const int bid, RowScan<Cfg::NT>& scan) {
+  if constexpr (Cfg::SELF_ROUTED) {
+    if (g.mask != nullptr) {
+      scan.scan(g.mask, g.M, lds);
+      if (bid == 0 && threadIdx.x == 0) {
+        int32_t* counts = const_cast<int32_t*>(g.counts);
+        counts[0] = scan.n_vis;
+        counts[1] = g.M - scan.n_vis;
+      }
+      return scan.n_vis;
+    }
+  }
+  return g.counts[0];
 }
 
 // Routed GEMM: rows in routed order, group-pure tiles.
@@ -1668,7 +1715,8 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
   // ---- tile schedule (all from device-side counts; no host sync) ----
   const int SBM = g.sched_bm > 0 ? g.sched_bm : BM;
   const int SBN = g.sched_bn > 0 ? g.sched_bn : Cfg::BN_OUT;
-  const int n_vis = g.counts[0];
+  RowScan<Cfg::NT> scan;
+  const int n_vis = visual_rows<Cfg>(g, lds, bid, scan);
   const int total = routed_tile_count(n_vis, g.M, g.N, SBM, SBN);
   int L, sub_m = 0, sub_n = 0, split = 0, splits = 1, tail_slot = 0;
   if (g.tail_mode == 0) {
@@ -1703,7 +1751,7 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
   tc.row0 += sub_m * BM;
   tc.n0 += sub_n * Cfg::BN_OUT;
   if (tc.row0 >= tc.row_end || tc.n0 >= g.N) return;  // a sub-tile past the edge of a partial macro tile
-  routed_tile<Cfg>(g, lds, tc, split, splits, tail_slot);
+  routed_tile<Cfg>(g, lds, tc, split, splits, tail_slot, scan);
 }
 
 
@@ -1888,15 +1936,17 @@ __global__ __launch_bounds__(Tall::NT) void routed_mixed_kernel(const GemmArgs g
   static_assert(Tall::NT == Short::NT && Tall::BN_OUT == Short::BN_OUT && Tall::BM == kTallRows && Short::BM == kShortRows, "two heights");
   __shared__ __attribute__((aligned(1024))) uint8_t lds[Tall::LDS_BYTES > Short::LDS_BYTES ? Tall::LDS_BYTES : Short::LDS_BYTES];
   bool is_tall;
-  TileCoord tc = mixed_tile_coord((int)blockIdx.x, g.counts[0], g.M, g.N, Tall::BN_OUT, g.group_m > 0 ? g.group_m : Tall::GROUP_M, &is_tall);
+  RowScan<Tall::NT> scan;
+  const int n_vis = visual_rows<Tall>(g, lds, (int)blockIdx.x, scan);
+  TileCoord tc = mixed_tile_coord((int)blockIdx.x, n_vis, g.M, g.N, Tall::BN_OUT, g.group_m > 0 ? g.group_m : Tall::GROUP_M, &is_tall);
   if (tc.grp < 0) return;
   // (the compiler takes them for values of a lane and would load the weights' addresses through the vector memory path)
   tc.grp = __builtin_amdgcn_readfirstlane(tc.grp);
   tc.row0 = __builtin_amdgcn_readfirstlane(tc.row0);
   tc.row_end = __builtin_amdgcn_readfirstlane(tc.row_end);
   tc.n0 = __builtin_amdgcn_readfirstlane(tc.n0);
-  if (is_tall) routed_tile<Tall>(g, lds, tc, 0, 1, 0);
-  else routed_tile<Short>(g, lds, tc, 0, 1, 0);
+  if (is_tall) routed_tile<Tall>(g, lds, tc, 0, 1, 0, scan);
+  else routed_tile<Short>(g, lds, tc, 0, 1, 0, scan);
 }
 
 // Upper bound on the number of workgroups the kernel needs, rounded so that every XCD gets the
@@ -1911,7 +1961,14 @@ inline int routed_gemm_grid(int M, int N, int splits = 1, int splits_more = 1) {
 }
 
 template <class Cfg>
+inline bool self_routed_args_ok(const GemmArgs& g) {
+  return g.mask == nullptr || (Cfg::SELF_ROUTED && g.M <= kScanMaxRows && reinterpret_cast<uintptr_t>(g.mask) % 16 == 0 && g.tail_mode == 0 &&
+                               g.N % 8 == 0 && g.ldc % 8 == 0 && reinterpret_cast<uintptr_t>(g.C) % 16 == 0);
+}
+
+template <class Cfg>
 inline bool routed_gemm_args_ok(const GemmArgs& g) {
+  if (!self_routed_args_ok<Cfg>(g)) return false;
   if ((g.splits > 1 || g.splits_more > 1) && (Cfg::DUAL || !Cfg::DIRECT || g.tail_mode != 0 || g.P == nullptr)) return false;
   if ((g.splits > 1) != (g.splits_more > 1)) return false;
   if (Cfg::DIRECT && !direct_slabs_ok(g.K)) return false;
@@ -1936,7 +1993,8 @@ inline hipError_t launch_routed_gemm(const GemmArgs& g, hipStream_t stream) {
 template <class Tall, class Short>
 inline hipError_t launch_routed_mixed(const GemmArgs& g, hipStream_t stream) {
   if (g.M <= 0 || g.N <= 0) return hipSuccess;
-  if (g.splits > 1 || g.splits_more > 1 || g.tail_mode != 0 || g.P_tail != nullptr || g.k_switch != 0 || !direct_slabs_ok(g.K))
+  if (g.splits > 1 || g.splits_more > 1 || g.tail_mode != 0 || g.P_tail != nullptr || g.k_switch != 0 || !direct_slabs_ok(g.K) ||
+      !self_routed_args_ok<Tall>(g))
     return hipErrorInvalidValue;
   hipLaunchKernelGGL((routed_mixed_kernel<Tall, Short>), dim3(mixed_blocks(g.M, g.N, Tall::BN_OUT)), dim3(Tall::NT), 0, stream, g);
   return hipGetLastError();

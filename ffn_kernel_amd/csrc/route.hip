@@ -10,6 +10,7 @@
 // linear in M: kRouteMaxBlocks * M bytes.
 #include "common.hpp"
 #include "launch.hpp"
+#include "route_rows.hpp"
 
 namespace ffnk {
 
@@ -17,19 +18,6 @@ constexpr int kRouteThreads = 256;
 constexpr int kRouteRowsPerThread = 4;
 constexpr int kRouteChunk = kRouteThreads * kRouteRowsPerThread;  // 1024 rows per pass of a block: the launch is latency-bound, short chains per thread
 constexpr int kRouteMaxBlocks = 256;                              // one per CU; past 256 K rows a block places several chunks in turn
-
-// 16-bit mask of the non-zero bytes of a 16-byte vector (bit j = byte j).
-__device__ __forceinline__ uint32_t nonzero_bytes16(uint4 v) {
-  uint32_t w[4] = {v.x, v.y, v.z, v.w};
-  uint32_t bits = 0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    uint32_t t = (w[i] | ((w[i] & 0x7f7f7f7fu) + 0x7f7f7f7fu)) & 0x80808080u;  // bit 7 of each non-zero byte
-    uint32_t nib = (((t >> 7) * 0x01020408u) >> 24) & 0xFu;                     // gather to 4 bits
-    bits |= nib << (4 * i);
-  }
-  return bits;
-}
 
 // Bits [lo, hi) of a 16-bit field, lo/hi clamped to [0, 16].
 __device__ __forceinline__ uint32_t range_bits16(int64_t lo, int64_t hi) {

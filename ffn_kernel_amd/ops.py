@@ -116,13 +116,20 @@ class Routing:
     mask inside every tile of every launch (linear.py:120-149, ffn.py:61-105)."""
     __slots__ = ("perm", "counts", "M", "_struct", "address")
 
-    def __init__(self, perm: torch.Tensor, counts: torch.Tensor):
+    def __init__(self, perm: torch.Tensor, counts: torch.Tensor, made: bool = True):
         self.perm, self.counts, self.M = perm, counts, perm.shape[0]
-        self._struct = _lib.RoutingStruct(perm.data_ptr(), counts.data_ptr())
+        self._struct = _lib.PartitionStruct(_lib.RoutingStruct(perm.data_ptr(), counts.data_ptr()), int(made))
         self.address = ctypes.addressof(self._struct)
 
     def ref(self):
-        return ctypes.byref(self._struct)
+        return ctypes.byref(self._struct.routing)
+
+    def make(self, mask: torch.Tensor, stream: int) -> "Routing":
+        """Fill it from `mask` on `stream`, unless that has been done."""
+        if not self._struct.made:
+            _lib.check(_lib.load().ffnk_route(mask.data_ptr(), self.M, self.perm.data_ptr(), self.counts.data_ptr(), stream), "ffnk_route")
+            self._struct.made = 1
+        return self
 
 
 def route(mask: torch.Tensor) -> Routing:
@@ -132,11 +139,11 @@ def route(mask: torch.Tensor) -> Routing:
     M, dev = mask.shape[0], mask.device
     mask = mask if mask.stride(0) == 1 or M <= 1 else mask.contiguous()
     buf = torch.empty(M + 2, dtype=torch.int32, device=dev)
-    routing = Routing(buf[:M], buf[M:])
+    routing = Routing(buf[:M], buf[M:], made=False)
+    if _route_cache.in_call:  # a call that is under way makes it
+        return routing
     with _on_device(dev):
-        rc = _lib.load().ffnk_route(mask.data_ptr(), M, routing.perm.data_ptr(), routing.counts.data_ptr(), _stream_ptr(dev))
-    _lib.check(rc, "ffnk_route")
-    return routing
+        return routing.make(mask, _stream_ptr(dev))
 
 
 class _RouteCache(threading.local):
@@ -145,6 +152,7 @@ class _RouteCache(threading.local):
     key = None
     mask = None     # keeps the mask's memory alive, so that its address cannot be handed to another tensor
     routing = None
+    in_call = False  # route() leaves the partition to the call that asks for it
     last = None     # the partition the last forward on this thread ran with (read back by the autograd functions)
 
 
@@ -170,6 +178,15 @@ def shared_routing(mask: torch.Tensor, M: int, stream: int | None = None):
     partitioned again - and the stream.  Returns None where no partition is shared: decode sizes, the cache
     switched off, tensors without a version counter, a stream under graph capture (a captured graph must not
     point at memory this cache may drop later)."""
+    routing = _shared_routing(mask, M, stream)
+    if routing is not None:
+        with _on_device(mask.device):
+            routing.make(mask, _stream_ptr(mask.device) if stream is None else stream)
+    return routing
+
+
+def _shared_routing(mask: torch.Tensor, M: int, stream: int | None = None):
+    """shared_routing, or the room for one that the caller has to fill: a forward fills it on its way."""
     if M < _ROUTED_MIN_ROWS or not _route_cache.enabled:
         return None
     try:
@@ -181,24 +198,34 @@ def shared_routing(mask: torch.Tensor, M: int, stream: int | None = None):
     key = (mask.data_ptr(), M, version, _stream_ptr(mask.device) if stream is None else stream)
     if _route_cache.key == key:
         return _route_cache.routing
-    routing = route(mask)
+    _route_cache.in_call = True
+    try:
+        routing = route(mask)
+    finally:
+        _route_cache.in_call = False
     _route_cache.key, _route_cache.mask, _route_cache.routing = key, mask, routing
     return routing
 
 
-def _routing_arg(routing, mask: torch.Tensor, M: int, stream: int):
-    """(Routing or None, its ffnk_routing_t* or None) for a call: the caller's, else the shared one."""
+def _routing_of_call(routing, mask: torch.Tensor, M: int, stream: int):
+    """The Routing that a call runs with, or None: the caller's, else the shared one, which may have to be filled."""
     if routing is None:
-        routing = shared_routing(mask, M, stream)
+        routing = _shared_routing(mask, M, stream)
     elif routing.M != M or routing.perm.device != mask.device:
         raise ValueError(f"routing is for {routing.M} rows on {routing.perm.device}, the call has {M} on {mask.device}")
     _route_cache.last = routing
-    return routing, (routing.ref() if routing is not None else None)
+    return routing
+
+
+def _routing_arg(routing, mask: torch.Tensor, M: int, stream: int):
+    """(Routing or None, its ffnk_routing_t* or None) for a call, filled."""
+    routing = _routing_of_call(routing, mask, M, stream)
+    return routing, (routing.make(mask, stream).ref() if routing is not None else None)
 
 
 def _routing_address(routing, mask: torch.Tensor, M: int, stream: int) -> int:
-    """_routing_arg for _call.so: the partition is kept by _route_cache.last while the call runs."""
-    routing, _ = _routing_arg(routing, mask, M, stream)
+    """_routing_of_call for _call.so: the address of its PartitionStruct, kept by _route_cache.last while the call runs."""
+    routing = _routing_of_call(routing, mask, M, stream)
     return 0 if routing is None else routing.address
 
 
@@ -227,8 +254,9 @@ def _native():
     global _native_call
     if _native_call is None:
         module, lib = _lib.load_call(), _lib.load()
-        names = ("ffnk_workspace_bytes", "ffnk_masked_ffn_can_save", "ffnk_masked_linear_fwd_routed",
-                 "ffnk_masked_linear_bwd_routed", "ffnk_masked_ffn_fwd_routed", "ffnk_masked_ffn_bwd_routed")
+        names = ("ffnk_workspace_bytes", "ffnk_masked_ffn_can_save", "ffnk_route", "ffnk_masked_linear_fwd_routed",
+                 "ffnk_masked_linear_fwd_routing", "ffnk_masked_linear_bwd_routed", "ffnk_masked_ffn_fwd_routed",
+                 "ffnk_masked_ffn_fwd_routing", "ffnk_masked_ffn_bwd_routed")
         module.bind(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names), _routing_address,
                     _ffn_bwd_workspace, _lib.check, _ROUTED_MIN_ROWS)
         _native_call = module

@@ -185,6 +185,17 @@ FFNK_API int ffnk_masked_linear_fwd_routed(const uint16_t* x, int64_t x_stride_m
                                   int64_t M, int64_t K, int64_t N,
                                   void* ws, size_t ws_bytes, void* stream, const ffnk_routing_t* routing);
 
+/* ffnk_masked_linear_fwd that leaves its row partition in `made` (perm int32[M], counts int32[2], device memory) for the calls
+ * behind it, as ffnk_route would write it: the first of the operations that share one.  Up to 8192 rows the GEMM makes it itself,
+ * a launch less than ffnk_route and ffnk_masked_linear_fwd_routed. */
+FFNK_API int ffnk_masked_linear_fwd_routing(const uint16_t* x, int64_t x_stride_m,
+                                  const uint16_t* Wv, const uint16_t* Wt,
+                                  int64_t w_stride_k, int64_t w_stride_n,
+                                  const uint8_t* mask,
+                                  uint16_t* y, int64_t y_stride_m,
+                                  int64_t M, int64_t K, int64_t N,
+                                  void* ws, size_t ws_bytes, void* stream, const ffnk_routing_t* made);
+
 /*
  * MaskedFFN forward — replaces _bf16_ffn_forward followed by _bf16_linear_forward
  * (ffn_kernel/ops.py:30-32, ffn_kernel/ffn.py:527-560):
@@ -370,7 +381,7 @@ FFNK_API int ffnk_masked_ffn_bwd_saved(const uint16_t* g, int64_t g_stride_m,
 
 /*
  * The MaskedFFN forward and backward with the row partition handed in (see ffnk_routing_t; routing == NULL:
- * a route launch at the head of the call, as in the plain entry points).  `pre` is optional in both:
+ * the call makes its own, as in the plain entry points).  `pre` is optional in both:
  * forward: NULL = ffnk_masked_ffn_fwd, else ffnk_masked_ffn_fwd_save; backward: NULL = ffnk_masked_ffn_bwd
  * (recompute), else ffnk_masked_ffn_bwd_saved.  Replaces the per-tile mask tests of ffn_kernel/ffn.py:61-105
  * and ffn_kernel/linear.py:120-149.
@@ -386,6 +397,19 @@ FFNK_API int ffnk_masked_ffn_fwd_routed(const uint16_t* x, int64_t x_stride_m,
                                uint16_t* pre, int64_t pre_stride_m,
                                int64_t M, int64_t d, int64_t h,
                                void* ws, size_t ws_bytes, void* stream, const ffnk_routing_t* routing);
+
+/* The MaskedFFN forward that leaves its row partition in `made` (ffnk_masked_linear_fwd_routing). */
+FFNK_API int ffnk_masked_ffn_fwd_routing(const uint16_t* x, int64_t x_stride_m,
+                               const uint16_t* W1, const uint16_t* W3,
+                               const uint16_t* U1, const uint16_t* U3,
+                               int64_t up_stride_k, int64_t up_stride_n,
+                               const uint16_t* W2, const uint16_t* U2,
+                               int64_t down_stride_k, int64_t down_stride_n,
+                               const uint8_t* mask,
+                               uint16_t* out, int64_t out_stride_m,
+                               uint16_t* pre, int64_t pre_stride_m,
+                               int64_t M, int64_t d, int64_t h,
+                               void* ws, size_t ws_bytes, void* stream, const ffnk_routing_t* made);
 
 FFNK_API int ffnk_masked_ffn_bwd_routed(const uint16_t* g, int64_t g_stride_m,
                                const uint16_t* x, int64_t x_stride_m,
