@@ -127,7 +127,7 @@ struct RoutedGemmCfg {
   // power limit and the narrower accumulator traffic is worth 5 % there); the others with 32x32x16.  K-major
   // weight panels included: MaskedFFN forward + backward at d = 4096, h = 14336 runs 4.5 % (M = 4096) to 7 %
   // (M = 32768) faster than with the backward's 256-row GEMMs on the two-stage 32x32x16 loop.
-  static constexpr bool MFMA16 = DIRECT_ && (BM_ == 256 || BM_ == 160);
+  static constexpr bool MFMA16 = DIRECT_ && (BM_ == 256 || BM_ == 160 || (BM_ == 192 && BN_ == 256));
   // Cache policy of the token panel's global->LDS loads.  The down projection's token rows (the routed intermediate,
   // read in place) pass each XCD once: a round of tiles reads a line and no later round does.  Loaded with the
   // non-temporal hint they do not push the weight panels out of L2 (cfg4 down projection 2.91 -> 2.85 ms, M = 16384
@@ -148,7 +148,7 @@ struct RoutedGemmCfg {
   static constexpr int STAGES = STAGES_;
   // The 256-row direct tiles take STAGES == 3 to mean: token panel in a ring of three stages, weight panel in two
   // (gemm_mainloop_fixed16) - exactly the 160 KB of LDS a CU has.
-  static constexpr bool A_RING3 = MFMA16 && STAGES_ == 3 && BM_ == 256;
+  static constexpr bool A_RING3 = MFMA16 && STAGES_ == 3 && BM_ >= 192;
   static constexpr bool RING = STAGES_ > 2 && !MFMA16;
   // The 160-row tile fits whole stages three times (gemm_mainloop_fixed16).
   static constexpr bool RING3 = MFMA16 && BM_ == 160;
@@ -730,7 +730,7 @@ __device__ __forceinline__ void gemm_mainloop_fixed16(const TileLanes<Cfg>& tl,
   static_assert(!RF || (L - LF0) * LEV <= NM, "ring schedule does not fit this wave tile");
   constexpr int NPRE = (BAR - RPOS) / LEV;  // ... of them ahead of the data barrier (a load follows the last MFMA of its group of LEV)
   static_assert(RPOS >= 0 && RPOS < BAR && NPRE <= L1, "release barrier ahead of the data barrier");
-  static_assert(TM >= 3 && (RF || TM >= TN) && L1 >= 1 && L1 <= L && (L - L1) * LEV <= NM, "schedule does not fit this wave tile");
+  static_assert(TM >= 3 && (!KM || TM >= TN) && L1 >= 1 && L1 <= L && (L - L1) * LEV <= NM, "schedule does not fit this wave tile");
   static_assert(!RF || !KM, "ring of whole stages: row-major weights");
   constexpr int BSTEP0 = TM >= TN ? TN : TM;  // first step: MFMAs from one weight-fragment read to the next
   static_assert(!R3 || (NJA * LEV <= NM && RPOS + NJB * LEV <= NM), "ring schedule does not fit this wave tile");
@@ -1949,6 +1949,28 @@ __global__ __launch_bounds__(Tall::NT) void routed_mixed_kernel(const GemmArgs g
   else routed_tile<Short>(g, lds, tc, 0, 1, 0, scan);
 }
 
+// 192-row tiles among 128-row ones (stretch_rows).
+template <class Tall, class Base, int SLOTS>
+__global__ __launch_bounds__(Base::NT) void routed_stretch_kernel(const GemmArgs g) {
+  static_assert(Tall::NT == Base::NT && Tall::BN_OUT == Base::BN_OUT && Tall::BM == kStretchRows && Base::BM == kStretchBase, "two heights");
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[Tall::LDS_BYTES > Base::LDS_BYTES ? Tall::LDS_BYTES : Base::LDS_BYTES];
+  static_assert(sizeof(lds) * (SLOTS / kCusPerChip) <= 160 * 1024, "workgroups per CU");
+  RowScan<Base::NT> scan;
+  const int n_vis = visual_rows<Base>(g, lds, (int)blockIdx.x, scan);
+  const int tiles_n = cdiv(g.N, Base::BN_OUT);
+  const Stretch s = stretch_rows(n_vis, g.M, tiles_n, SLOTS);
+  const int L = xcd_tile_slot((s.tiles_v + s.tiles_x) * tiles_n, (int)blockIdx.x);
+  if (L < 0) return;
+  bool is_tall;
+  TileCoord tc = stretch_tile_coord(L, s, n_vis, g.M, tiles_n, Base::BN_OUT, g.group_m > 0 ? g.group_m : Base::GROUP_M, &is_tall);
+  tc.grp = __builtin_amdgcn_readfirstlane(tc.grp);  // (see routed_mixed_kernel)
+  tc.row0 = __builtin_amdgcn_readfirstlane(tc.row0);
+  tc.row_end = __builtin_amdgcn_readfirstlane(tc.row_end);
+  tc.n0 = __builtin_amdgcn_readfirstlane(tc.n0);
+  if (is_tall) routed_tile<Tall>(g, lds, tc, 0, 1, 0, scan);
+  else routed_tile<Base>(g, lds, tc, 0, 1, 0, scan);
+}
+
 // Upper bound on the number of workgroups the kernel needs, rounded so that every XCD gets the
 // same number of slots.  The kernel derives the real tile count from counts[] on the device.
 template <class Cfg>
@@ -1987,6 +2009,14 @@ inline hipError_t launch_routed_gemm(const GemmArgs& g, hipStream_t stream) {
   if (!routed_gemm_args_ok<Cfg>(g)) return hipErrorInvalidValue;
   const int grid = routed_gemm_grid<Cfg>(g.M, g.N, g.splits, g.splits_more);
   hipLaunchKernelGGL(routed_gemm_kernel<Cfg>, dim3(grid), dim3(Cfg::NT), 0, stream, g);
+  return hipGetLastError();
+}
+
+template <class Tall, class Base, int SLOTS>
+inline hipError_t launch_routed_stretch(const GemmArgs& g, hipStream_t stream) {
+  if (g.M <= 0 || g.N <= 0) return hipSuccess;
+  if (!routed_gemm_args_ok<Base>(g) || g.splits > 1 || g.tail_mode != 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((routed_stretch_kernel<Tall, Base, SLOTS>), dim3(routed_gemm_grid<Base>(g.M, g.N)), dim3(Base::NT), 0, stream, g);
   return hipGetLastError();
 }
 

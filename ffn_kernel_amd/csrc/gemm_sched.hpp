@@ -40,10 +40,10 @@ __host__ __device__ inline int routed_splits(int n_vis, int M, int bm, int split
 // d = 4096, h = 14336: forward at M = 1411 (three M-tiles of each modality) 507.5 -> 501.7 us, the backward's dx GEMM at
 // M = 4096 (eight of each; before, all sixteen were one super-group and 41 % of its L2 requests missed, now 33 %) 775 -> 706 us;
 // forward at M = 902, d = 7296 and at M = 4381, d = 1728: 1.0-1.5 % faster.  Dealt evenly at any size, M = 32768 lost 1.5 %.
-__host__ __device__ inline TileCoord routed_tile_coord(int L, int n_vis, int M, int N, int bm, int bn, int group_m) {
-  const int tiles_v = cdiv(n_vis, bm);
-  const int tiles_m = tiles_v + cdiv(M - n_vis, bm);
-  const int tiles_n = cdiv(N, bn);
+struct OrderPos {
+  int tile_m, tile_n;
+};
+__host__ __device__ inline OrderPos order_pos(int L, int tiles_v, int tiles_m, int tiles_n, int group_m) {
   int first_m, gsz;
   if (tiles_m > kEvenGroups * group_m) {
     first_m = L / (group_m * tiles_n) * group_m;
@@ -61,13 +61,63 @@ __host__ __device__ inline TileCoord routed_tile_coord(int L, int n_vis, int M, 
     }
   }
   L -= first_m * tiles_n;
-  const int tile_m = first_m + L % gsz;
-  const int tile_n = L / gsz;
+  return {first_m + L % gsz, L / gsz};
+}
+__host__ __device__ inline TileCoord routed_tile_coord(int L, int n_vis, int M, int N, int bm, int bn, int group_m) {
+  const int tiles_v = cdiv(n_vis, bm);
+  const OrderPos at = order_pos(L, tiles_v, tiles_v + cdiv(M - n_vis, bm), cdiv(N, bn), group_m);
   TileCoord t;
-  t.grp = tile_m < tiles_v ? 0 : 1;
-  t.row0 = t.grp == 0 ? tile_m * bm : n_vis + (tile_m - tiles_v) * bm;
+  t.grp = at.tile_m < tiles_v ? 0 : 1;
+  t.row0 = t.grp == 0 ? at.tile_m * bm : n_vis + (at.tile_m - tiles_v) * bm;
   t.row_end = t.grp == 0 ? n_vis : M;
-  t.n0 = tile_n * bn;
+  t.n0 = at.tile_n * bn;
+  return t;
+}
+
+// 192-row tiles among 128-row ones where the 128-row tiles end just past a whole round of the chip's `slots` - as those of two
+// modalities do whenever the rows of both together fill whole rounds: one M-tile goes, and the rows of one or two others of its
+// modality are 192 high.  A launch of 65 x 8 tiles on 512 places ran its last 8 workgroups by themselves, 13 of 31 us at K = 1024
+// and 20 of 51 at K = 2048.  Rows of both modalities mixed, weights not in a cache, 128x128 tiles: MaskedLinear M = 8192, K = N = 1024
+// 32.4 -> 23.2 us, M = 16384, K = N = 512 20.8 -> 15.0; 128x256 tiles: M = 8192, N = 1024, K = 2048 55 -> 43, K = 4096 95 -> 73,
+// M = 2048, K = N = 4096 97 -> 76, M = 4096, K = 6144, N = 2048 142 -> 103; MaskedFFN d = 1024, h = 2048, M = 8192 134.7 -> 126.1.
+// A mask that leaves whole rounds of 128-row tiles (one modality alone) runs 0 to 4 % slower than on the kernel of those alone.
+constexpr int kStretchRows = 192, kStretchBase = 128;
+struct Stretch {
+  int tiles_v, tiles_x;  // M-tiles by modality
+  int tall_v, tall_x;    // ... the first of them 192 rows high
+};
+// One M-tile less of tiles_m fits the whole rounds, and what is past them is no more than an eighth of a round (past that the
+// 256-row tiles are the faster ones).
+__host__ __device__ inline bool stretch_fits(int64_t tiles_m, int64_t tiles_n, int slots) {
+  const int64_t tiles = tiles_m * tiles_n, rest = tiles % slots;
+  return rest > 0 && rest < tiles && rest <= tiles_n && rest <= slots / 8;
+}
+// ... for some split of M rows, which has cdiv(M, kStretchBase) M-tiles or one more.
+inline bool may_stretch(int64_t M, int64_t tiles_n, int slots) {
+  const int64_t tiles_m = cdiv64(M, kStretchBase);
+  return stretch_fits(tiles_m, tiles_n, slots) || stretch_fits(tiles_m + 1, tiles_n, slots);
+}
+__host__ __device__ inline Stretch stretch_rows(int n_vis, int M, int tiles_n, int slots) {
+  Stretch s{cdiv(n_vis, kStretchBase), cdiv(M - n_vis, kStretchBase), 0, 0};
+  if (!stretch_fits(s.tiles_v + s.tiles_x, tiles_n, slots)) return s;
+  // (a modality of one M-tile keeps it: its rows have nowhere to go)
+  const int last_v = s.tiles_v > 1 ? n_vis - (s.tiles_v - 1) * kStretchBase : 2 * kStretchBase;
+  const int last_x = s.tiles_x > 1 ? M - n_vis - (s.tiles_x - 1) * kStretchBase : 2 * kStretchBase;
+  const bool v = last_v <= last_x;
+  const int tall = cdiv(v ? last_v : last_x, kStretchRows - kStretchBase), left = (v ? s.tiles_v : s.tiles_x) - 1;
+  if (tall > left || tall > 2) return s;
+  if (v) return {left, s.tiles_x, tall, 0};
+  return {s.tiles_v, left, 0, tall};
+}
+__host__ __device__ inline TileCoord stretch_tile_coord(int L, const Stretch& s, int n_vis, int M, int tiles_n, int bn, int group_m, bool* is_tall) {
+  const OrderPos at = order_pos(L, s.tiles_v, s.tiles_v + s.tiles_x, tiles_n, group_m);
+  TileCoord t;
+  t.grp = at.tile_m < s.tiles_v ? 0 : 1;
+  const int m = t.grp == 0 ? at.tile_m : at.tile_m - s.tiles_v, tall = t.grp == 0 ? s.tall_v : s.tall_x;
+  *is_tall = m < tall;
+  t.row0 = (t.grp == 0 ? 0 : n_vis) + m * kStretchBase + (m < tall ? m : tall) * (kStretchRows - kStretchBase);
+  t.row_end = t.grp == 0 ? n_vis : M;
+  t.n0 = at.tile_n * bn;
   return t;
 }
 

@@ -129,6 +129,11 @@ constexpr TileCost kPlainCosts[] = {
     {TILE_128x256_R3, 1, 6.127, 0.679, 5.596, 1.317, {0.694, 1.0}, {0.825, 1.0}},
     {TILE_64x128_R3, 2, 2.924, 0.519, 5.577, 1.38, {0.404, 0.589, 0.868, 1.0}, {0.425, 0.499, 0.808, 1.0}}};
 
+// Part of a round that a single-weight launch of 128-row tiles takes for what is just past its whole rounds, with 192-row tiles
+// among them (stretch_rows).  Measured 0.05 - 0.27 (128x128) and 0.04 - 0.26 (128x256) at K = 512 ... 8192.
+constexpr double kStretchPart128 = 0.17, kStretchPart256 = 0.21;
+inline double stretch_part(int tile) { return tile == TILE_128x128_W4 ? kStretchPart128 : tile == TILE_128x256_R3 ? kStretchPart256 : 0.0; }
+
 // Part of a round that `rest` workgroups take on per_cu slots of every CU.
 inline double round_part(const double* knots, int64_t rest) {
   const int n = (int)cdiv64(rest, kCus);
@@ -137,7 +142,7 @@ inline double round_part(const double* knots, int64_t rest) {
 }
 
 inline double routed_tile_time(const TileCost& c, bool dual, int64_t tiles_m, int modalities, int64_t M, int64_t n_out, int64_t K,
-                               int splits) {
+                               int splits, bool stretch = true) {
   const GemmCost& g = dual ? kDualCost : kPlainCost;
   const TileGeom t = tile_geom(c.tile, dual);
   const int64_t slabs = cdiv64(K, 64), slots = (int64_t)kCus * c.per_cu;
@@ -147,7 +152,9 @@ inline double routed_tile_time(const TileCost& c, bool dual, int64_t tiles_m, in
   const double round = c.base + per_slab * (double)cdiv64(slabs, splits);
   double time = (double)full * round;
   if (rest > 0) {
-    if (!is_big_tile(c.tile) || splits > 1 || full == 0 || (dual && rest > slots / 2)) {  // whole_round_tiles
+    if (stretch && !dual && splits == 1 && stretch_part(c.tile) > 0.0 && stretch_fits(tiles_m, cdiv64(n_out, t.block_n_out), (int)slots)) {
+      time += round * stretch_part(c.tile);
+    } else if (!is_big_tile(c.tile) || splits > 1 || full == 0 || (dual && rest > slots / 2)) {  // whole_round_tiles
       time += round * round_part(full > 0 ? c.again : c.first, rest);
     } else if (dual) {  // four 128-row tiles for each of the remainder
       const TileCost& s = kDualCosts[1];
@@ -174,16 +181,16 @@ inline bool routed_split_ok(int64_t K, int s) {
 // where that starts another round the times differ by up to a half.  One more it is at (M / block_m rounded up) *
 // ((M - 1) mod block_m) of the M - 1 ways to split M; masks that set every row by itself split M about evenly.  The score is
 // the product of three times: over all splits (weight 1), at an even split (weight 2), of one modality alone (weight 2).
-inline double plan_score(const TileCost& c, bool dual, int64_t M, int64_t n_out, int64_t K, int splits, int splits_more) {
+inline double plan_score(const TileCost& c, bool dual, int64_t M, int64_t n_out, int64_t K, int splits, int splits_more, bool stretch = true) {
   const int64_t bm = tile_geom(c.tile, dual).block_m, less = cdiv64(M, bm);
   const double p = M > 1 ? (double)(less * ((M - 1) % bm)) / (double)(M - 1) : 0.0;
   int64_t dev = 0;  // a third of sqrt(M): how far such a mask is off an even split
   while ((dev + 1) * (dev + 1) * 9 <= M) ++dev;
   const int64_t visual = (M + 1) / 2 + dev < M ? (M + 1) / 2 + dev : M;
   const bool even_more = cdiv64(visual, bm) + cdiv64(M - visual, bm) > less;
-  const double t = routed_tile_time(c, dual, less, 2, M, n_out, K, splits);
-  const double more = routed_tile_time(c, dual, less + 1, 2, M, n_out, K, splits_more);
-  const double one = routed_tile_time(c, dual, less, 1, M, n_out, K, splits);
+  const double t = routed_tile_time(c, dual, less, 2, M, n_out, K, splits, stretch);
+  const double more = routed_tile_time(c, dual, less + 1, 2, M, n_out, K, splits_more, stretch);
+  const double one = routed_tile_time(c, dual, less, 1, M, n_out, K, splits, stretch);
   const double even = even_more ? more : t;
   return ((1.0 - p) * t + p * more) * even * even * one * one;
 }
@@ -231,7 +238,7 @@ inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_
   auto fits = [&](const RoutedPlan& q) { return dual || plan_partial_bytes(q, M, n_out, K) <= room; };
   auto consider = [&](const TileCost& c, int s, int s_more) {
     if (!fits({c.tile, s, s_more})) return;
-    const double t = plan_score(c, dual, M, n_out, K, s, s_more);
+    const double t = plan_score(c, dual, M, n_out, K, s, s_more, false);
     if (best < 0.0 || t < best) {
       best = t;
       p = {c.tile, s, s_more};
@@ -254,10 +261,34 @@ inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_
       }
       if (s > 1) consider(c, s, s_more);
     }
-    if (c.tile == rule.tile && (rule.splits == 1 || split) && fits(rule)) keep = plan_score(c, dual, M, n_out, K, rule.splits, rule.splits_more);
+    if (c.tile == rule.tile && (rule.splits == 1 || split) && fits(rule)) keep = plan_score(c, dual, M, n_out, K, rule.splits, rule.splits_more, false);
   }
   constexpr double m = kModelMargin * kModelMargin * kModelMargin * kModelMargin * kModelMargin;  // a score is five times long
-  return keep > 0.0 && keep < best * m ? rule : p;
+  if (keep > 0.0 && keep < best * m) p = rule;
+  if (dual) return p;
+  // 128-row tiles with 192-row ones among them where those save a round of the two modalities' tiles and one modality alone does not
+  // take longer for it (its tiles may fill whole rounds of 256-row ones).
+  const RoutedPlan without = p;
+  auto cost = [&](int tile) -> const TileCost& {
+    int i = 0;
+    while (costs[i].tile != tile) ++i;
+    return costs[i];
+  };
+  auto one = [&](const RoutedPlan& q) {
+    return routed_tile_time(cost(q.tile), false, cdiv64(M, tile_geom(q.tile, false).block_m), 1, M, n_out, K, q.splits);
+  };
+  best = plan_score(cost(p.tile), false, M, n_out, K, p.splits, p.splits_more) / m;
+  for (int i = 0; i < n_costs; ++i) {
+    const TileCost& c = costs[i];
+    const RoutedPlan q{c.tile, 1, 1};
+    if (stretch_part(c.tile) == 0.0 || !may_stretch(M, cdiv64(n_out, tile_geom(c.tile, false).block_n_out), kCus * c.per_cu)) continue;
+    const double t = plan_score(c, false, M, n_out, K, 1, 1);
+    if (t < best && one(q) <= kModelMargin * one(without)) {
+      best = t;
+      p = q;
+    }
+  }
+  return p;
 }
 
 // The model is a pure function of the extents and takes 5 us of host time (single-weight GEMMs); every thread keeps the last

@@ -240,3 +240,37 @@ def test_dx_beside_the_weight_gradients(dev, forced, nv, nt, d, h):
     forced(0)
     assert _lib.load().ffnk_debug_ffn_joint(nv + nt, d, h) & 2
     assert_ffn_backward(*case, "one launch")
+
+
+# 192-row tiles among 128-row ones (csrc/gemm_sched.hpp: stretch_rows): a round of the chip and one M-tile more, the last M-tile of
+# the stretched modality at one row, at the edges of what one and two taller tiles hold, whole, and in either modality; contraction
+# of a few slabs, whole and ragged.
+@pytest.mark.parametrize("tile,N", [(2, 8192), (6, 8192)])
+@pytest.mark.parametrize("K", [192, 328])
+@pytest.mark.parametrize("nv,nt", [(513, 511), (576, 448), (577, 447), (448, 576), (447, 577), (639, 385), (1000, 24), (0, 1025), (1025, 0)])
+def test_stretched_tiles(dev, forced, tile, N, K, nv, nt):
+    note(f"192-row tiles among 128-row ones: tile={tile} K={K} {nv} visual, {nt} text rows")
+    x, Wv, Wt, mask, _ = make_linear(dev, nv, nt, K, N, seed=nv + K)
+    forced(tile=tile, splits=1)
+    y = MaskedLinear.apply(x, Wv.T, Wt.T, mask)
+    forced()
+    ref = torch.where(mask[:, None], x.double() @ Wv.double().T, x.double() @ Wt.double().T)
+    assert_close(y, ref.cpu(), "y")
+
+
+@pytest.mark.parametrize("tile", [2, 6])
+def test_stretched_down_projection(dev, forced, tile):
+    nv, nt, d, h = 540, 484, 8192, 192
+    note(f"192-row tiles in the down projection: tile={tile}")
+    x, _, _, mask, _ = make_linear(dev, nv, nt, d, 8, seed=5)
+    gen = torch.Generator(device=dev).manual_seed(6)
+    w = [(torch.randn(*s, generator=gen, device=dev) * 0.02).bfloat16() for s in [(h, d), (d, h), (h, d)] * 2]
+    forced(tile=tile, splits=1)
+    y = MaskedFFN.apply(x, *(v.T for v in w), mask)
+    forced()
+
+    def half(w1, w2, w3):
+        g, u = x.double() @ w1.double().T, x.double() @ w3.double().T
+        return (torch.nn.functional.silu(g) * u).bfloat16().double() @ w2.double().T
+
+    assert_close(y, torch.where(mask[:, None], half(*w[:3]), half(*w[3:])).cpu(), "y")

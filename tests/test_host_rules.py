@@ -264,3 +264,30 @@ def test_the_swiglu_derivative_divides(tmp_path):
     asm = subprocess.run([shutil.which("hipcc") or "/opt/rocm/bin/hipcc", *build.HIPCC_FLAGS, "--cuda-device-only", "-S", str(src), "-o", "-"],
                          check=True, capture_output=True, text=True).stdout
     assert [asm.count(i) for i in ("v_rcp_f32", "v_div_fmas_f32", "v_div_fixup_f32")] == [8, 8, 8]
+
+
+# 128-row tiles with 192-row ones among them: every result in one tile, no more tiles than 128-row ones, whole rounds where one
+# M-tile less makes them, and no stretch that the host's launch does not allow for.
+@pytest.mark.parametrize("tiles_n,slots,tiles_m", [(8, 512, 64), (8, 256, 32), (32, 256, 8), (64, 512, 8), (20, 256, 12), (3, 512, 170), (128, 256, 4), (256, 256, 1)])
+def test_stretched_tiles_cover_the_output(rules, tiles_n, slots, tiles_m):
+    t = (ctypes.c_int * 4)()
+    stretched = 0
+    for M in (tiles_m * 128, tiles_m * 128 - 1, tiles_m * 128 + 1, tiles_m * 128 + 60, tiles_m * 128 + 65, tiles_m * 128 - 127):
+        splits = {0, 1, M, M - 1, M // 2, 64, 65, 127, 128, 129, 192, 193, M - 64, M - 192} | {M // 2 + i for i in (-70, -64, 1, 60, 63, 64, 65, 127)}
+        for n_vis in sorted(v for v in splits if 0 <= v <= M):
+            plain = (-(-n_vis // 128) + -(-(M - n_vis) // 128)) * tiles_n
+            count = rules.hc_stretch_tiles(n_vis, M, tiles_n, slots)
+            assert count in (plain, plain - tiles_n)
+            if count < plain:
+                stretched += 1
+                assert rules.hc_may_stretch(M, tiles_n, slots) and plain // slots > (count - 1) // slots
+            rows = {}
+            for L in range(count):
+                rules.hc_stretch_tile(L, n_vis, M, tiles_n, slots, 128, 4, t)
+                assert 0 <= t[1] < t[2] <= (n_vis if t[0] == 0 else M) and (t[0] == 0 or t[1] >= n_vis)
+                rows.setdefault(t[3], []).append((t[1], t[2]))
+            assert sorted(rows) == [n * 128 for n in range(tiles_n)]
+            for spans in rows.values():
+                spans.sort()
+                assert spans[0][0] == 0 and spans[-1][1] == M and all(a[1] == b[0] for a, b in zip(spans, spans[1:]))
+    assert stretched > 0 or slots // tiles_n < 2 or tiles_n > slots // 8
