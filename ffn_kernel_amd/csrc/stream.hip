@@ -189,7 +189,7 @@ __global__ __launch_bounds__(NWV * kWave, OCC) void stream_kernel(const StreamAr
   // the groups was measured 1.5x slower when one modality is absent: its empty workgroups still take
   // their turn in the round-robin placement over CUs, so the real ones pile up on half of the CUs.)
   const int per_grp = row_blocks * a.splits;
-  t.grp = blockIdx.x / per_grp;
+  t.grp = first_group(n_vis) ^ (int)(blockIdx.x / per_grp);
   const int rem = blockIdx.x % per_grp;
   t.split = rem / row_blocks;
   t.p0 = t.grp == 0 ? 0 : n_vis;            // first routed position of the group

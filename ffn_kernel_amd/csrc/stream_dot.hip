@@ -197,7 +197,7 @@ __device__ __forceinline__ int route8(const uint8_t* mask, int M, int* s_perm, i
   return *s_nvis;
 }
 
-// grid.x = 2 * row_blocks (visual workgroups first), blockDim.x = 64 * (K / (512 * C)); rpb weight
+// grid.x = 2 * row_blocks (M == 1: row_blocks; first_group), blockDim.x = 64 * (K / (512 * C)); rpb weight
 // rows per workgroup.  Dynamic LDS: [waves][rpb * MATS][T_MAX] floats.
 template <int T_MAX, bool DUAL, int C, int DEPTH, int NWV_MAX, bool RAGGED>
 __global__ __launch_bounds__(NWV_MAX * kWave) void stream_dot_kernel(const StreamArgs a, const int rpb) {
@@ -205,9 +205,9 @@ __global__ __launch_bounds__(NWV_MAX * kWave) void stream_dot_kernel(const Strea
   __shared__ int s_perm[kDotMaxM];
   __shared__ int s_nvis;
   const int n_vis = route8(a.mask, a.M, s_perm, &s_nvis);
-  const int row_blocks = gridDim.x >> 1;
+  const int row_blocks = a.M == 1 ? gridDim.x : gridDim.x >> 1;
   DotTile t;
-  t.grp = blockIdx.x / row_blocks;
+  t.grp = first_group(n_vis) ^ (int)(blockIdx.x / row_blocks);
   t.p0 = t.grp == 0 ? 0 : n_vis;
   t.mg = t.grp == 0 ? n_vis : a.M - n_vis;
   if (t.mg == 0) return;  // modality absent: its weights are never read
@@ -275,13 +275,14 @@ static void launch_dot_c(const StreamArgs& a, hipStream_t stream) {
   const int waves = stream_dot_waves(a.K);
   const int rpb = stream_dot_rows_per_block(a.Nrows, DUAL, a.K);
   const int row_blocks = cdiv(a.Nrows, rpb);
+  const int blocks = a.M == 1 ? row_blocks : 2 * row_blocks;  // (one row: the device knows which modality is meant)
   const size_t lds = (size_t)waves * rpb * (DUAL ? 2 : 1) * T_MAX * sizeof(float);
   if (waves <= 4)
-    hipLaunchKernelGGL((stream_dot_kernel<T_MAX, DUAL, C, 8, 4, RAGGED>), dim3(2 * row_blocks), dim3(waves * kWave), lds, stream, a, rpb);
+    hipLaunchKernelGGL((stream_dot_kernel<T_MAX, DUAL, C, 8, 4, RAGGED>), dim3(blocks), dim3(waves * kWave), lds, stream, a, rpb);
   else if (waves <= 8)
-    hipLaunchKernelGGL((stream_dot_kernel<T_MAX, DUAL, C, 8, 8, RAGGED>), dim3(2 * row_blocks), dim3(waves * kWave), lds, stream, a, rpb);
+    hipLaunchKernelGGL((stream_dot_kernel<T_MAX, DUAL, C, 8, 8, RAGGED>), dim3(blocks), dim3(waves * kWave), lds, stream, a, rpb);
   else
-    hipLaunchKernelGGL((stream_dot_kernel<T_MAX, DUAL, C, 4, 16, RAGGED>), dim3(2 * row_blocks), dim3(waves * kWave), lds, stream, a, rpb);
+    hipLaunchKernelGGL((stream_dot_kernel<T_MAX, DUAL, C, 4, 16, RAGGED>), dim3(blocks), dim3(waves * kWave), lds, stream, a, rpb);
 }
 
 template <bool DUAL>

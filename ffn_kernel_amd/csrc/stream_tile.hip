@@ -371,7 +371,7 @@ __device__ __forceinline__ int route64(const uint8_t* mask, int M, int* s_perm, 
   return *s_nvis;
 }
 
-// grid.x = 2 groups x splits x row blocks (visual workgroups first); 256 threads.
+// grid.x = 2 groups x splits x row blocks (first_group).
 template <int NTM_MAX, bool DUAL, int kTWaves, int kTD, bool XDMA, int FORM>
 __global__ __launch_bounds__(kTWaves * kWave, 2) void stream_tile_kernel(const StreamArgs a) {
   constexpr bool RAGGED = FORM != FORM_WHOLE;
@@ -386,7 +386,7 @@ __global__ __launch_bounds__(kTWaves * kWave, 2) void stream_tile_kernel(const S
   const int row_blocks = RAGGED ? cdiv(a.Nrows, ROWS) : a.Nrows / ROWS;
   const int per_grp = row_blocks * a.splits;
   TileJob t;
-  t.grp = blockIdx.x / per_grp;
+  t.grp = first_group(n_vis) ^ (int)(blockIdx.x / per_grp);
   const int rem = blockIdx.x % per_grp;
   t.split = rem / row_blocks;
   t.p0 = t.grp == 0 ? 0 : n_vis;
