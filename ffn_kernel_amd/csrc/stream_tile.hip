@@ -40,13 +40,24 @@ constexpr int kTK = 128;    // K elements per chunk (16 pieces of 16 bytes per r
 // dma: the token-row slab is filled by direct global -> LDS loads (no staging registers, which is
 // what lets the 3- and 4-m-tile shapes run two-wavefront workgroups) instead of through registers.
 struct TileShapeEntry { int waves, depth, dma; };
-// One table per projection.  Four wavefronts per up-projection workgroup for three and four m-tiles (half the
-// slab traffic per weight byte, 80 KB of LDS, one round of workgroups instead of 1.75 with both modalities at
-// M = 64) measured 1-2 % slower than two at M = 48 and 64 and the same at M = 32; the tables stay equal.
 constexpr TileShapeEntry kTileShapesUp[4] = {{2, 4, 0}, {2, 3, 0}, {2, 3, 1}, {2, 3, 1}};
 constexpr TileShapeEntry kTileShapesDown[4] = {{2, 4, 0}, {2, 3, 0}, {2, 3, 1}, {2, 3, 1}};
 constexpr const TileShapeEntry& tile_shape(int ntm_max, bool dual) { return dual ? kTileShapesUp[ntm_max - 1] : kTileShapesDown[ntm_max - 1]; }
 constexpr int kTMaxM = 64;
+// The up projection at three and four m-tiles with four wavefronts per workgroup: half the slab traffic per weight byte, which
+// above 32 rows is as much as the weights; 80 KB of LDS at four m-tiles, two workgroups per CU as with two wavefronts, and half as
+// many workgroups, so long streams only.  Workgroups of one XCD start at different chunks (spread): with the two-wavefront
+// kernels' start, which has four values per XCD at 32 chunks, a 64-row workgroup at K = 4096 was 4 to 8 % slower instead.
+// Whole call, us, two -> four wavefronts, one modality / both: M = 64, d = 4096, h = 14336 76.3 -> 71.5 / 126 -> 121.5, h = 16384
+// 80.3 -> 77.2 / 137 -> 132, h = 11008 68.7 -> 61.9 / 112 -> 107; d = 5120, h = 13824 103 -> 96.5 / 174 -> 163; d = 8192, h = 22016
+// 232 -> 210 / 356 -> 346; d = 3072, h = 10240 60.2 -> 56.5 / 92.5 -> 91; fewer rows lose with both modalities (d = 4096, h = 8960
+// 95 -> 98, d = 2560 71 -> 76).  M = 36 ... 48, where two wavefronts fit three times: d = 4096, h = 14336 72.0 -> 67.8 / 123 -> 118,
+// d = 6144 117 -> 109 / 187 -> 181, but h = 22016, d = 8192 190 -> 204 and h = 10240, d = 3072 76 -> 82 (both).
+constexpr int kWideWaves = 4, kWideRows = 16 * kWideWaves;
+bool stream_tile_wide(int M, int Nrows, int K) {
+  if (M <= 32 || M > kTMaxM || K % kTK != 0 || Nrows % kWideRows != 0) return false;
+  return M > 48 ? Nrows >= 10240 : Nrows >= 12288 && Nrows <= 16384;
+}
 
 // FORM_WHOLE: K whole chunks, Nrows whole row blocks.  The other two (RAGGED) take any multiples of 8: the last chunk
 // overlaps the one before it; the last row block starts at Nrows - ROWS, streams rows of the block before it a second
@@ -122,7 +133,8 @@ __device__ __forceinline__ void tile_rows(const StreamArgs& a, const TileJob& t,
   // are a power-of-two number of bytes apart, so workgroups sitting at the same K offset would all
   // pull from the same few HBM channels.
   const int nc = t.nc;
-  const int rot = (int)((blockIdx.x * 11u) % (unsigned)nc);
+  const unsigned spread = kTWaves == kWideWaves ? (blockIdx.x >> 3) * 11u + (blockIdx.x & 7u) * (unsigned)nc / 8u : blockIdx.x * 11u;
+  const int rot = (int)(spread % (unsigned)nc);
   // RAGGED: a last chunk that would pass the end of the rows starts earlier, overlapping the chunk before it; what the two
   // share (overlap(c) pieces of 8 elements) is cleared in both operands' fragments, so that no product is counted twice
   // and a non-finite value meets no zero it would not meet elsewhere.
@@ -449,7 +461,7 @@ int stream_tile_down_splits(int M, int d, int h) {
 }
 
 template <int NTM_MAX, bool DUAL>
-static void launch_tile_n(const StreamArgs& a, hipStream_t stream) {
+static void launch_tile_narrow(const StreamArgs& a, hipStream_t stream) {
   constexpr int W = tile_shape(NTM_MAX, DUAL).waves, D = tile_shape(NTM_MAX, DUAL).depth;
   constexpr bool X = tile_shape(NTM_MAX, DUAL).dma != 0;
   constexpr int ROWS = (DUAL ? 16 : 32) * W;
@@ -460,6 +472,22 @@ static void launch_tile_n(const StreamArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL((stream_tile_kernel<NTM_MAX, DUAL, W, D, X, FORM_RAGGED>), dim3(blocks), dim3(W * kWave), 0, stream, a);
   else
     hipLaunchKernelGGL((stream_tile_kernel<NTM_MAX, DUAL, W, D, X, FORM_SPLIT_LINES>), dim3(blocks), dim3(W * kWave), 0, stream, a);
+}
+
+template <int NTM_MAX>
+static void launch_tile_wide(const StreamArgs& a, hipStream_t stream) {
+  constexpr int D = tile_shape(NTM_MAX, true).depth;
+  constexpr bool X = tile_shape(NTM_MAX, true).dma != 0;
+  hipLaunchKernelGGL((stream_tile_kernel<NTM_MAX, true, kWideWaves, D, X, FORM_WHOLE>), dim3(2 * (a.Nrows / kWideRows)),
+                     dim3(kWideWaves * kWave), 0, stream, a);
+}
+
+template <int NTM_MAX, bool DUAL>
+static void launch_tile_n(const StreamArgs& a, hipStream_t stream) {
+  if constexpr (DUAL && NTM_MAX >= 3) {
+    if (stream_tile_wide(a.M, a.Nrows, a.K)) return launch_tile_wide<NTM_MAX>(a, stream);
+  }
+  launch_tile_narrow<NTM_MAX, DUAL>(a, stream);
 }
 
 template <bool DUAL>

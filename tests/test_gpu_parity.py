@@ -349,6 +349,24 @@ def test_ffn_decode_long_ranges(dev, kind):
         assert torch.equal(out2, out)
 
 
+# The up projection on workgroups of four wavefronts (stream_tile.hip: stream_tile_wide): the fewest and most rows of three and four
+# m-tiles, the shortest contraction, at the lines and past them (h = 10176, 16448: two wavefronts).
+@pytest.mark.parametrize("M,h", [(33, 12288), (48, 16384), (48, 16448), (49, 10240), (64, 10240), (64, 10176), (64, 17408)])
+@pytest.mark.parametrize("kind", ["visual", "text", "bernoulli"])
+def test_ffn_decode_four_wavefronts(dev, M, h, kind):
+    d = 1024
+    note(f"ffn decode wide M={M} h={h} kind={kind}")
+    w = wl.cfg5_ffn_decode(M, kind, seed=M + h, d=d, h=h)
+    out = MaskedFFN.apply(*w.to(dev).op_args())
+    torch.cuda.synchronize()
+    assert_close(out, om.ffn_select(w.x, w.W, w.mask, torch.float64, round_intermediate=True), f"wide {M} {h} {kind}")
+    if kind != "bernoulli":
+        W = dict(w.W)
+        for k in (("u1", "u2", "u3") if kind == "visual" else ("w1", "w2", "w3")):
+            W[k] = torch.full_like(W[k], float("nan"))
+        assert torch.equal(MaskedFFN.apply(*wl.FFNWorkload("p", w.x, W, w.mask).to(dev).op_args()), out)
+
+
 def test_ffn_decode_matches_tiled_path_rows(dev):
     """The same rows run as a decode call and inside a larger (tiled-path) call agree to bf16 accuracy."""
     note("ffn decode vs tiled")
