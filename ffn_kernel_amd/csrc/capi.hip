@@ -71,7 +71,7 @@ RouteWs carve_route(uint8_t* ws, int64_t M) {
 }
 
 // Tuner overrides, see ffnk_debug_force_tile / ffnk_debug_force_splits.
-std::atomic<int> g_force_tile{-1};    // 0..4, 6, 7: that tile; -1: table, then rules; -2: rules only
+std::atomic<int> g_force_tile{-1};    // 0..4, 6, 7, 16, 17: that tile; -1: table, then rules; -2: rules only
 std::atomic<int> g_force_splits{-1};  // >= 1: that split-K factor where a GEMM can be split
 std::atomic<int> g_force_group_m{0};      // >= 1: M-tiles per super-group in the tile order of every routed GEMM
 std::atomic<int> g_force_bwd_gather{-1};  // MaskedLinear backward: 1 = weight gradients from g and x in place, 0 = from transposes, -1 = plan
@@ -79,9 +79,15 @@ std::atomic<int> g_force_bwd_gather{-1};  // MaskedLinear backward: 1 = weight g
 // Pseudo tile id of a measured weight-gradient plan: g and x read where they lie (gemm_dw_gather.hpp) on the 128x128 tile.
 constexpr int kTileGatherDw = 5;
 
-int forced_tile() {
+bool can_force(int tile) { return (tile >= 0 && tile < TILE_COUNT && tile != kTileGatherDw) || forward_only(tile); }
+int forced_forward_tile() {
   const int t = g_force_tile.load(std::memory_order_relaxed);
-  return (t >= 0 && t < TILE_COUNT && t != kTileGatherDw) ? t : -1;
+  return can_force(t) ? t : -1;
+}
+// ... in every GEMM but the forward's single-weight ones, which alone have the 192- and 160-row tiles.
+int forced_tile() {
+  const int t = forced_forward_tile();
+  return forward_only(t) ? TILE_128x256_R3 : t;
 }
 bool use_tuned() { return g_force_tile.load(std::memory_order_relaxed) != -2; }
 // GemmArgs::group_m of a routed GEMM: the forced value, else the measured plan's, else 0 (the tile's own).
@@ -351,7 +357,7 @@ int down_splits(int64_t M, int64_t d, int64_t h) {
 // `op`: whose measured plans apply (TunedOp).
 RoutedPlan down_plan(int64_t M, int64_t d, int64_t h, int op = TUNED_DOWN) {
   RoutedPlan p;
-  if (const int f = forced_tile(); f >= 0) {
+  if (const int f = op == TUNED_NONE ? forced_tile() : forced_forward_tile(); f >= 0) {
     p.tile = f;
     p.splits = p.splits_more = pick_routed_splits(M, d, h, p.tile);
   } else {
@@ -385,7 +391,7 @@ bool up_two_heights(int tile, bool direct, int64_t M, int64_t h) {
 // dx), 2.9 % (dh) and 3.0 % (the feed-forward dx, K split) behind the best of all tiles and split factors in the geometric mean,
 // the rules by tile count, which these GEMMs ran on before, 32, 23 and 17 %.
 int bwd_tile(int64_t M, int64_t n_out, int64_t K, bool direct) {
-  if (forced_tile() < 0 && direct && model_applies(false, M, n_out, K)) return model_routed_plan(false, M, n_out, K, false).tile;
+  if (forced_tile() < 0 && direct && model_applies(false, M, n_out, K)) return model_routed_plan(false, M, n_out, K, false, kAnyRoom, false).tile;
   return routed_tile(M, n_out, false, 0, TUNED_NONE);
 }
 // dx GEMM of the MaskedFFN backward: few output tiles over a contraction of 2h (or 2 * half), so K is split like the forward's
@@ -395,7 +401,7 @@ RoutedPlan ffn_bwd_dx_plan(int64_t M, int64_t d, int64_t contraction, bool dx_di
   // another loop).
   RoutedPlan dxp = down_plan(M, d, contraction, TUNED_NONE);
   if (forced_tile() < 0 && forced_splits() < 1 && dx_direct && model_applies(false, M, d, contraction))
-    dxp = model_routed_plan(false, M, d, contraction, M < 65536, room);
+    dxp = model_routed_plan(false, M, d, contraction, M < 65536, room, false);
   if (!dx_direct || (size_t)max_splits(dxp) * M * d * 4 > room) {
     dxp.splits = dxp.splits_more = 1;
     dxp.tile = routed_tile(M, d, false, 0, TUNED_NONE);
@@ -651,7 +657,7 @@ extern "C" {
 int ffnk_version(void) { return FFNK_VERSION; }
 
 int ffnk_debug_force_tile(int tile) {
-  return g_force_tile.exchange(((tile >= 0 && tile < TILE_COUNT && tile != kTileGatherDw) || tile == -2) ? tile : -1);
+  return g_force_tile.exchange(can_force(tile) || tile == -2 ? tile : -1);
 }
 
 int ffnk_debug_force_group_m(int group_m) { return g_force_group_m.exchange(group_m >= 1 && group_m <= 64 ? group_m : 0); }
@@ -748,7 +754,7 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
   // Kernels without the two ring tiles of three stages run the two-stage tiles in their place.
   const bool kmajor_dx = op == FFNK_OP_LINEAR_BWD || op == FFNK_OP_BWD_DX;
   if (!direct || op == FFNK_OP_BWD_DW) {
-    if (tile == TILE_128x256_R3) tile = TILE_128x128_W4;
+    if (tile == TILE_128x256_R3 || forward_only(tile)) tile = TILE_128x128_W4;
     if (tile == TILE_64x128_R3) tile = op == FFNK_OP_BWD_DW ? TILE_128x128_W4 : TILE_SMALL_W4;
   }
   if (!direct && tile == TILE_256x256_W4) tile = TILE_256x256_W8;  // the four-wave tile runs on the direct path only
@@ -775,7 +781,7 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
   out->direct_lds = (direct || in_place) ? 1 : 0;
   out->in_place = in_place ? 1 : 0;
   // 4: ring of four stages (128x128); 3: token panel in three stages, weight panel in two (single-weight 256x256 tiles)
-  out->lds_stages = !(direct || in_place) ? 2 : tile == TILE_128x128_R4 ? 4 : (tile == TILE_128x256_R3 || tile == TILE_64x128_R3) ? 3 : (is_big_tile(tile) && !dual) ? 3 : 2;
+  out->lds_stages = !(direct || in_place) ? 2 : tile == TILE_128x128_R4 ? 4 : (tile == TILE_128x256_R3 || tile == TILE_64x128_R3 || forward_only(tile)) ? 3 : (is_big_tile(tile) && !dual) ? 3 : 2;
   if (op == FFNK_OP_FFN_DOWN && !stream) out->split_k = max_splits(ffn_down_plan(M, K, N));
   if (op == FFNK_OP_LINEAR_FWD && linear_stream_kind(M, K, N)) {
     out->path = FFNK_PATH_STREAM;

@@ -127,7 +127,7 @@ struct RoutedGemmCfg {
   // power limit and the narrower accumulator traffic is worth 5 % there); the others with 32x32x16.  K-major
   // weight panels included: MaskedFFN forward + backward at d = 4096, h = 14336 runs 4.5 % (M = 4096) to 7 %
   // (M = 32768) faster than with the backward's 256-row GEMMs on the two-stage 32x32x16 loop.
-  static constexpr bool MFMA16 = DIRECT_ && (BM_ == 256 || BM_ == 160 || (BM_ == 192 && BN_ == 256));
+  static constexpr bool MFMA16 = DIRECT_ && (BM_ == 256 || BM_ == 160 || ((BM_ == 192 || BM_ == 224) && BN_ == 256));
   // Cache policy of the token panel's global->LDS loads.  The down projection's token rows (the routed intermediate,
   // read in place) pass each XCD once: a round of tiles reads a line and no later round does.  Loaded with the
   // non-temporal hint they do not push the weight panels out of L2 (cfg4 down projection 2.91 -> 2.85 ms, M = 16384
@@ -1949,26 +1949,31 @@ __global__ __launch_bounds__(Tall::NT) void routed_mixed_kernel(const GemmArgs g
   else routed_tile<Short>(g, lds, tc, 0, 1, 0, scan);
 }
 
-// 192-row tiles among 128-row ones (stretch_rows).
+// Taller tiles among the others (stretch_rows).
 template <class Tall, class Base, int SLOTS>
 __global__ __launch_bounds__(Base::NT) void routed_stretch_kernel(const GemmArgs g) {
-  static_assert(Tall::NT == Base::NT && Tall::BN_OUT == Base::BN_OUT && Tall::BM == kStretchRows && Base::BM == kStretchBase, "two heights");
+  static_assert(Tall::NT == Base::NT && Tall::BN_OUT == Base::BN_OUT && Tall::BM > Base::BM, "two heights");
+  constexpr StretchShape shape{Base::BM, Tall::BM, SLOTS};
   __shared__ __attribute__((aligned(1024))) uint8_t lds[Tall::LDS_BYTES > Base::LDS_BYTES ? Tall::LDS_BYTES : Base::LDS_BYTES];
   static_assert(sizeof(lds) * (SLOTS / kCusPerChip) <= 160 * 1024, "workgroups per CU");
   RowScan<Base::NT> scan;
   const int n_vis = visual_rows<Base>(g, lds, (int)blockIdx.x, scan);
   const int tiles_n = cdiv(g.N, Base::BN_OUT);
-  const Stretch s = stretch_rows(n_vis, g.M, tiles_n, SLOTS);
-  const int L = xcd_tile_slot((s.tiles_v + s.tiles_x) * tiles_n, (int)blockIdx.x);
+  const int splits = g.splits > 1 ? routed_splits(n_vis, g.M, Base::BM, g.splits, g.splits_more) : 1;
+  const Stretch s = stretch_rows(n_vis, g.M, tiles_n * splits, shape);
+  const int total = (s.tiles_v + s.tiles_x) * tiles_n;
+  int L = xcd_tile_slot(total * splits, (int)blockIdx.x);
   if (L < 0) return;
+  const int split = splits > 1 ? L / total : 0;  // range-major, as in routed_gemm_body
+  L -= split * total;
   bool is_tall;
-  TileCoord tc = stretch_tile_coord(L, s, n_vis, g.M, tiles_n, Base::BN_OUT, g.group_m > 0 ? g.group_m : Base::GROUP_M, &is_tall);
+  TileCoord tc = stretch_tile_coord(L, s, n_vis, g.M, tiles_n, Base::BN_OUT, g.group_m > 0 ? g.group_m : Base::GROUP_M, shape, &is_tall);
   tc.grp = __builtin_amdgcn_readfirstlane(tc.grp);  // (see routed_mixed_kernel)
   tc.row0 = __builtin_amdgcn_readfirstlane(tc.row0);
   tc.row_end = __builtin_amdgcn_readfirstlane(tc.row_end);
   tc.n0 = __builtin_amdgcn_readfirstlane(tc.n0);
-  if (is_tall) routed_tile<Tall>(g, lds, tc, 0, 1, 0, scan);
-  else routed_tile<Base>(g, lds, tc, 0, 1, 0, scan);
+  if (is_tall) routed_tile<Tall>(g, lds, tc, split, splits, 0, scan);
+  else routed_tile<Base>(g, lds, tc, split, splits, 0, scan);
 }
 
 // Upper bound on the number of workgroups the kernel needs, rounded so that every XCD gets the
@@ -2015,8 +2020,8 @@ inline hipError_t launch_routed_gemm(const GemmArgs& g, hipStream_t stream) {
 template <class Tall, class Base, int SLOTS>
 inline hipError_t launch_routed_stretch(const GemmArgs& g, hipStream_t stream) {
   if (g.M <= 0 || g.N <= 0) return hipSuccess;
-  if (!routed_gemm_args_ok<Base>(g) || g.splits > 1 || g.tail_mode != 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((routed_stretch_kernel<Tall, Base, SLOTS>), dim3(routed_gemm_grid<Base>(g.M, g.N)), dim3(Base::NT), 0, stream, g);
+  if (!routed_gemm_args_ok<Base>(g) || g.tail_mode != 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((routed_stretch_kernel<Tall, Base, SLOTS>), dim3(routed_gemm_grid<Base>(g.M, g.N, g.splits, g.splits_more)), dim3(Base::NT), 0, stream, g);
   return hipGetLastError();
 }
 

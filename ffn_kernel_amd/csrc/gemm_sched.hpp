@@ -74,17 +74,20 @@ __host__ __device__ inline TileCoord routed_tile_coord(int L, int n_vis, int M, 
   return t;
 }
 
-// 192-row tiles among 128-row ones where the 128-row tiles end just past a whole round of the chip's `slots` - as those of two
-// modalities do whenever the rows of both together fill whole rounds: one M-tile goes, and the rows of one or two others of its
-// modality are 192 high.  A launch of 65 x 8 tiles on 512 places ran its last 8 workgroups by themselves, 13 of 31 us at K = 1024
+// Taller tiles among the others of a launch (192 rows among 128 or 160, 224 among 192) where those end just past a whole round of
+// the chip - as the tiles of two modalities do whenever the rows of both together fill whole rounds: one M-tile goes, and its rows
+// are spread over taller ones of its modality.  A launch of 65 x 8 tiles on 512 places ran its last 8 workgroups by themselves, 13 of 31 us at K = 1024
 // and 20 of 51 at K = 2048.  Rows of both modalities mixed, weights not in a cache, 128x128 tiles: MaskedLinear M = 8192, K = N = 1024
 // 32.4 -> 23.2 us, M = 16384, K = N = 512 20.8 -> 15.0; 128x256 tiles: M = 8192, N = 1024, K = 2048 55 -> 43, K = 4096 95 -> 73,
 // M = 2048, K = N = 4096 97 -> 76, M = 4096, K = 6144, N = 2048 142 -> 103; MaskedFFN d = 1024, h = 2048, M = 8192 134.7 -> 126.1.
 // A mask that leaves whole rounds of 128-row tiles (one modality alone) runs 0 to 4 % slower than on the kernel of those alone.
-constexpr int kStretchRows = 192, kStretchBase = 128;
+struct StretchShape {
+  int base, tall;  // rows of a tile
+  int slots;       // workgroups that the chip runs at once
+};
 struct Stretch {
   int tiles_v, tiles_x;  // M-tiles by modality
-  int tall_v, tall_x;    // ... the first of them 192 rows high
+  int tall_v, tall_x;    // ... the first of them taller
 };
 // One M-tile less of tiles_m fits the whole rounds, and what is past them is no more than an eighth of a round (past that the
 // 256-row tiles are the faster ones).
@@ -92,30 +95,31 @@ __host__ __device__ inline bool stretch_fits(int64_t tiles_m, int64_t tiles_n, i
   const int64_t tiles = tiles_m * tiles_n, rest = tiles % slots;
   return rest > 0 && rest < tiles && rest <= tiles_n && rest <= slots / 8;
 }
-// ... for some split of M rows, which has cdiv(M, kStretchBase) M-tiles or one more.
-inline bool may_stretch(int64_t M, int64_t tiles_n, int slots) {
-  const int64_t tiles_m = cdiv64(M, kStretchBase);
-  return stretch_fits(tiles_m, tiles_n, slots) || stretch_fits(tiles_m + 1, tiles_n, slots);
+// ... for some split of M rows, which has cdiv(M, base) M-tiles or one more (with their own split-K factors).
+inline bool may_stretch(int64_t M, int64_t tiles_n, const StretchShape& shape, int splits = 1, int splits_more = 1) {
+  const int64_t tiles_m = cdiv64(M, shape.base);
+  return stretch_fits(tiles_m, tiles_n * splits, shape.slots) || stretch_fits(tiles_m + 1, tiles_n * splits_more, shape.slots);
 }
-__host__ __device__ inline Stretch stretch_rows(int n_vis, int M, int tiles_n, int slots) {
-  Stretch s{cdiv(n_vis, kStretchBase), cdiv(M - n_vis, kStretchBase), 0, 0};
-  if (!stretch_fits(s.tiles_v + s.tiles_x, tiles_n, slots)) return s;
-  // (a modality of one M-tile keeps it: its rows have nowhere to go)
-  const int last_v = s.tiles_v > 1 ? n_vis - (s.tiles_v - 1) * kStretchBase : 2 * kStretchBase;
-  const int last_x = s.tiles_x > 1 ? M - n_vis - (s.tiles_x - 1) * kStretchBase : 2 * kStretchBase;
-  const bool v = last_v <= last_x;
-  const int tall = cdiv(v ? last_v : last_x, kStretchRows - kStretchBase), left = (v ? s.tiles_v : s.tiles_x) - 1;
-  if (tall > left || tall > 2) return s;
-  if (v) return {left, s.tiles_x, tall, 0};
-  return {s.tiles_v, left, 0, tall};
+// tiles_n: workgroups per M-tile (column tiles times K ranges).
+__host__ __device__ inline Stretch stretch_rows(int n_vis, int M, int tiles_n, const StretchShape& shape) {
+  const Stretch s{cdiv(n_vis, shape.base), cdiv(M - n_vis, shape.base), 0, 0};
+  if (!stretch_fits(s.tiles_v + s.tiles_x, tiles_n, shape.slots)) return s;
+  // The last M-tile of the modality that takes the fewer taller ones for it.
+  const int more = shape.tall - shape.base, left_v = s.tiles_v - 1, left_x = s.tiles_x - 1;
+  const int tall_v = cdiv(n_vis - left_v * shape.base, more), tall_x = cdiv(M - n_vis - left_x * shape.base, more);
+  const bool can_v = tall_v <= left_v, can_x = tall_x <= left_x;
+  if (can_v && (!can_x || tall_v <= tall_x)) return {left_v, s.tiles_x, tall_v, 0};
+  if (can_x) return {s.tiles_v, left_x, 0, tall_x};
+  return s;
 }
-__host__ __device__ inline TileCoord stretch_tile_coord(int L, const Stretch& s, int n_vis, int M, int tiles_n, int bn, int group_m, bool* is_tall) {
+__host__ __device__ inline TileCoord stretch_tile_coord(int L, const Stretch& s, int n_vis, int M, int tiles_n, int bn, int group_m,
+                                                        const StretchShape& shape, bool* is_tall) {
   const OrderPos at = order_pos(L, s.tiles_v, s.tiles_v + s.tiles_x, tiles_n, group_m);
   TileCoord t;
   t.grp = at.tile_m < s.tiles_v ? 0 : 1;
   const int m = t.grp == 0 ? at.tile_m : at.tile_m - s.tiles_v, tall = t.grp == 0 ? s.tall_v : s.tall_x;
   *is_tall = m < tall;
-  t.row0 = (t.grp == 0 ? 0 : n_vis) + m * kStretchBase + (m < tall ? m : tall) * (kStretchRows - kStretchBase);
+  t.row0 = (t.grp == 0 ? 0 : n_vis) + m * shape.base + (m < tall ? m : tall) * (shape.tall - shape.base);
   t.row_end = t.grp == 0 ? n_vis : M;
   t.n0 = at.tile_n * bn;
   return t;

@@ -21,9 +21,14 @@ struct PlainTiles {
   using T0 = RoutedGemmCfg<256, 256, 2, 4, false, GATHER, SCATTER, DIRECT, kGroupMPlain, false, DIRECT ? kBigStagesPlain : 2>;
   using T1 = RoutedGemmCfg<256, 256, 2, 2, false, GATHER, SCATTER, DIRECT, kGroupMPlain, false, DIRECT ? kBigStagesPlain : 2>;
   using T2 = RoutedGemmCfg<128, 128, 2, 2, false, GATHER, SCATTER, DIRECT, kGroupMPlain>;
-  // among T2 and T6, see stretch_rows
-  using T2Tall = RoutedGemmCfg<192, 128, 2, 2, false, GATHER, SCATTER, DIRECT, kGroupMPlain>;
-  using T6Tall = std::conditional_t<DIRECT, RoutedGemmCfg<192, 256, 2, 2, false, GATHER, SCATTER, true, kGroupMPlain, false, 3>, T2Tall>;
+  using T2Tall = RoutedGemmCfg<192, 128, 2, 2, false, GATHER, SCATTER, DIRECT, kGroupMPlain>;  // among T2, see stretch_rows
+  // The heights between 128 and 256 rows fill the chip at many mid-size M where those two leave a quarter of it (us, before -> now):
+  // M = 1411, K = 14336, N = 4096 185 -> 140 (192 rows, two K ranges: 256 workgroups; before 192 of 128x256, 178 us of K loop), M = 700,
+  // K = N = 8192 113 -> 97, M = 7130, K = 7296, N = 1088 182 -> 105, M = 1848, K = 2560, N = 4352 72 -> 50.  A slab takes 0.94 us on 192 rows
+  // and 0.78 on 160 against 1.2 - 1.3 on 256 and 0.7 - 0.8 on 128.  T8 also among T6 and T9, T8Tall among T8.
+  using T8 = std::conditional_t<DIRECT, RoutedGemmCfg<192, 256, 2, 2, false, GATHER, SCATTER, true, kGroupMPlain, false, 3>, T2Tall>;
+  using T9 = std::conditional_t<DIRECT, RoutedGemmCfg<160, 256, 2, 2, false, GATHER, SCATTER, true, kGroupMPlain, false, 3>, T2Tall>;
+  using T8Tall = std::conditional_t<DIRECT, RoutedGemmCfg<224, 256, 2, 2, false, GATHER, SCATTER, true, kGroupMPlain, false, 3>, T2Tall>;
   using T3 = RoutedGemmCfg<128, 64, 2, 2, false, GATHER, SCATTER, DIRECT, kGroupMPlain>;
   // 128x128 behind a ring of four LDS stages (direct path; otherwise the two-stage tile)
   using T4 = RoutedGemmCfg<128, 128, 2, 2, false, GATHER, SCATTER, DIRECT, kGroupMPlain, false, DIRECT ? 4 : 2>;
@@ -75,7 +80,7 @@ struct DualTiles {
   using T7 = std::conditional_t<DIRECT, RoutedGemmCfg<64, 128, 2, 2, true, true, false, true, kGroupM, false, 3>, T3>;
 };
 
-// A launch on 128-row tiles, with 192-row ones among them where that may save a round.  (The 128x128 tile's own kernel is up to 4 %
+// A launch on Base tiles, with Tall ones among them where that may save a round.  (The 128x128 tile's own kernel is up to 4 %
 // faster than the same tile beside the taller one, so the launch is that of both only where it has to be.)
 template <class Tiles, class = void>
 struct CanStretch : std::false_type {};
@@ -84,7 +89,7 @@ struct CanStretch<Tiles, std::void_t<typename Tiles::T2Tall>> : std::bool_consta
 
 template <class Base, class Tall, int SLOTS>
 inline hipError_t launch_or_stretch(const GemmArgs& g, hipStream_t stream) {
-  if (g.splits == 1 && g.tail_mode == 0 && may_stretch(g.M, cdiv(g.N, Base::BN_OUT), SLOTS))
+  if (g.tail_mode == 0 && may_stretch(g.M, cdiv(g.N, Base::BN_OUT), {Base::BM, Tall::BM, SLOTS}, g.splits, g.splits_more))
     return launch_routed_stretch<Tall, Base, SLOTS>(g, stream);
   return launch_routed_gemm<Base>(g, stream);
 }
@@ -105,9 +110,15 @@ inline hipError_t dispatch_tile(int tile, const GemmArgs& g, hipStream_t stream)
     case TILE_SMALL_W4: return launch_routed_gemm<typename Tiles::T3>(g, stream);
     case TILE_128x128_R4: return launch_routed_gemm<typename Tiles::T4>(g, stream);
     case TILE_128x256_R3:
-      if constexpr (CanStretch<Tiles>::value) return launch_or_stretch<typename Tiles::T6, typename Tiles::T6Tall, kCusPerChip>(g, stream);
+      if constexpr (CanStretch<Tiles>::value) return launch_or_stretch<typename Tiles::T6, typename Tiles::T8, kCusPerChip>(g, stream);
       else return launch_routed_gemm<typename Tiles::T6>(g, stream);
     case TILE_64x128_R3: return launch_routed_gemm<typename Tiles::T7>(g, stream);
+    case TILE_192x256_W4:
+      if constexpr (CanStretch<Tiles>::value) return launch_or_stretch<typename Tiles::T8, typename Tiles::T8Tall, kCusPerChip>(g, stream);
+      else return launch_routed_gemm<typename Tiles::T6>(g, stream);
+    case TILE_160x256_W4:
+      if constexpr (CanStretch<Tiles>::value) return launch_or_stretch<typename Tiles::T9, typename Tiles::T8, kCusPerChip>(g, stream);
+      else return launch_routed_gemm<typename Tiles::T6>(g, stream);
     default: return hipErrorInvalidValue;
   }
 }

@@ -20,6 +20,8 @@ TileGeom tile_geom(int tile, bool dual) {
     case TILE_128x128_R4: return {128, dual ? 64 : 128, 2, 2};
     case TILE_128x256_R3: return {128, dual ? 128 : 256, 2, 2};
     case TILE_64x128_R3: return {64, dual ? 64 : 128, 2, 2};
+    case TILE_192x256_W4: return dual ? TileGeom{128, 128, 2, 2} : TileGeom{192, 256, 2, 2};
+    case TILE_160x256_W4: return dual ? TileGeom{128, 128, 2, 2} : TileGeom{160, 256, 2, 2};
     default: return dual ? TileGeom{64, 64, 2, 2} : TileGeom{128, 64, 2, 2};
   }
 }

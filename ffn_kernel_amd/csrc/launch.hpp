@@ -19,12 +19,17 @@ enum TileId : int {
   // 5 names a form of the weight-gradient GEMM in its plans (kTileGatherDw), not a tile
   TILE_128x256_R3 = 6,  // 128 rows x 256 weight rows (SwiGLU: 128 gate + 128 up), 4 waves, ring of three LDS stages
   TILE_64x128_R3 = 7,   // 64 rows x 128 weight rows (SwiGLU: 64 gate + 64 up), 4 waves, ring of three LDS stages, two workgroups per CU
-  TILE_COUNT = 8,       // ids below can be forced; the next follows from TILE_256x256_W4 in the SwiGLU GEMM
-  TILE_MIXED_W4 = 8     // 256x256 and 160x256 tiles in one launch, 4 waves
+  TILE_COUNT = 8,       // ids below can be forced
+  TILE_MIXED_W4 = 8,    // 256x256 and 160x256 tiles in one launch, 4 waves: follows from TILE_256x256_W4 in the SwiGLU GEMM
+  // 192 and 160 rows x 256 weight rows, 4 waves: the forward's single-weight GEMMs only (can be forced; others run TILE_128x256_R3)
+  TILE_192x256_W4 = 16,
+  TILE_160x256_W4 = 17
 };
 
 // The two 256x256 tiles: past one round of the chip they run whole rounds first and the remainder apart.
 inline bool is_big_tile(int tile) { return tile == TILE_256x256_W8 || tile == TILE_256x256_W4; }
+
+inline bool forward_only(int tile) { return tile == TILE_192x256_W4 || tile == TILE_160x256_W4; }
 
 // Geometry of a tile id, as reported through ffnk_tile_config().
 struct TileGeom {

@@ -127,12 +127,27 @@ constexpr TileCost kPlainCosts[] = {
     {TILE_SMALL_W4, 3, 1.882, 0.891, 5.278, 1.235, {0.327, 0.581, 0.598, 0.682, 0.939, 1.0}, {0.339, 0.404, 0.517, 0.642, 0.899, 1.0}},
     {TILE_128x128_R4, 1, 3.892, 0.417, 6.008, 1.352, {0.642, 1.0}, {0.826, 1.0}},
     {TILE_128x256_R3, 1, 6.127, 0.679, 5.596, 1.317, {0.694, 1.0}, {0.825, 1.0}},
-    {TILE_64x128_R3, 2, 2.924, 0.519, 5.577, 1.38, {0.404, 0.589, 0.868, 1.0}, {0.425, 0.499, 0.808, 1.0}}};
+    {TILE_64x128_R3, 2, 2.924, 0.519, 5.577, 1.38, {0.404, 0.589, 0.868, 1.0}, {0.425, 0.499, 0.808, 1.0}},
+    // (forward GEMMs only; 6700 measurements at 400 shapes of their own, 7.5 and 8 % rms, GemmCost as it is)
+    {TILE_192x256_W4, 1, 5.102, 0.879, 6.529, 1.258, {0.845, 1.0}, {0.929, 1.0}},
+    {TILE_160x256_W4, 1, 4.303, 0.784, 6.305, 1.307, {0.814, 1.0}, {0.852, 1.0}}};
 
-// Part of a round that a single-weight launch of 128-row tiles takes for what is just past its whole rounds, with 192-row tiles
-// among them (stretch_rows).  Measured 0.05 - 0.27 (128x128) and 0.04 - 0.26 (128x256) at K = 512 ... 8192.
-constexpr double kStretchPart128 = 0.17, kStretchPart256 = 0.21;
-inline double stretch_part(int tile) { return tile == TILE_128x128_W4 ? kStretchPart128 : tile == TILE_128x256_R3 ? kStretchPart256 : 0.0; }
+// Single-weight tiles that may have taller ones among them (stretch_rows), and the part of a round that what is just past the whole
+// rounds then takes.  Measured 0.05 - 0.27 (128x128) and 0.04 - 0.26 (128x256) at K = 512 ... 8192; for the other two it is what the taller
+// tile has more rows.
+struct StretchCost {
+  StretchShape shape;
+  double part;
+};
+inline StretchCost stretch_cost(int tile) {
+  switch (tile) {
+    case TILE_128x128_W4: return {{128, 192, 2 * kCus}, 0.17};
+    case TILE_128x256_R3: return {{128, 192, kCus}, 0.21};
+    case TILE_160x256_W4: return {{160, 192, kCus}, 0.17};
+    case TILE_192x256_W4: return {{192, 224, kCus}, 0.17};
+    default: return {{0, 0, 0}, 0.0};
+  }
+}
 
 // Part of a round that `rest` workgroups take on per_cu slots of every CU.
 inline double round_part(const double* knots, int64_t rest) {
@@ -152,8 +167,9 @@ inline double routed_tile_time(const TileCost& c, bool dual, int64_t tiles_m, in
   const double round = c.base + per_slab * (double)cdiv64(slabs, splits);
   double time = (double)full * round;
   if (rest > 0) {
-    if (stretch && !dual && splits == 1 && stretch_part(c.tile) > 0.0 && stretch_fits(tiles_m, cdiv64(n_out, t.block_n_out), (int)slots)) {
-      time += round * stretch_part(c.tile);
+    const StretchCost sc = stretch && !dual ? stretch_cost(c.tile) : StretchCost{};
+    if (sc.part > 0.0 && stretch_fits(tiles_m, cdiv64(n_out, t.block_n_out) * splits, sc.shape.slots)) {
+      time += round * sc.part;
     } else if (!is_big_tile(c.tile) || splits > 1 || full == 0 || (dual && rest > slots / 2)) {  // whole_round_tiles
       time += round * round_part(full > 0 ? c.again : c.first, rest);
     } else if (dual) {  // four 128-row tiles for each of the remainder
@@ -221,14 +237,21 @@ inline size_t plan_partial_bytes(const RoutedPlan& p, int64_t M, int64_t n_out, 
              ? ws_align((size_t)kTailSlots * 256 * 256 * 4) : 0;
 }
 
-// The plan with the smallest score among all tiles and split factors.  `split`: N % 4 == 0 and the reduce pass takes M; `room`:
+// The plan with the smallest score among all tiles and split factors.  `forward`: a GEMM over row-major weights that scatters its
+// rows (CanStretch), which has the 192- and 160-row tiles too.  `split`: N % 4 == 0 and the reduce pass takes M; `room`:
 // bytes that the caller has for partials.  The rules' plan stays unless the model sees a gain of kModelMargin, near which its
 // choice is as often the slower one (MaskedFFN d = 1024, h = 2048, M = 8192, runs of both modalities: 133 us with the model's
 // 256x256 tiles under the down projection, 129 with the rules' 128x128): without it 6.0 % of the SwiGLU and 2.1 % of the
 // single-weight shapes ran more than 3 % slower than on the rules' plan, with it 5.1 % and 1.7 %.
 constexpr double kModelMargin = 1.03;
+// A plan on 192- or 160-row tiles replaces another, up to two rounds of the chip, where the model sees it 7 % ahead over the splits
+// of the rows, no slower with one modality and nowhere kModelMargin behind (the model puts 256- and 128-row tiles 2 - 6 % above
+// what they take, those two 1 %).  3138 timed calls of drawn single-weight GEMMs with such a plan (three masks each): 1.12 times as
+// fast as on the plan it replaced in the geometric mean, 2 % of them more than 3 % slower, 0.2 % more than 8 %.  Between two and three
+// rounds 1.03, with 23 % more than 3 % slower; by the score alone 12 % more than 3 % slower, and 4 % more than 8 %.
+constexpr double kForwardGain = 0.93;
 constexpr size_t kAnyRoom = ~(size_t)0;
-inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split, size_t room = kAnyRoom) {
+inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split, size_t room = kAnyRoom, bool forward = true) {
   constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16};
   const TileCost* costs = dual ? kDualCosts : kPlainCosts;
   const int n_costs = dual ? (int)(sizeof(kDualCosts) / sizeof(TileCost)) : (int)(sizeof(kPlainCosts) / sizeof(TileCost));
@@ -244,72 +267,100 @@ inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_
       p = {c.tile, s, s_more};
     }
   };
+  // The best factors of a tile for each M-tile count; either both are split or neither is (1: none fits).
+  auto best_split = [&](const TileCost& c) {
+    const int64_t less = cdiv64(M, tile_geom(c.tile, false).block_m);
+    int s = 0, s_more = 0;
+    double t_less = 0.0, t_more = 0.0;
+    for (const int k : kSplits) {
+      if (k == 1 || !routed_split_ok(K, k) || !fits({c.tile, k, k})) continue;
+      const bool stretch = forward_only(c.tile);
+      const double a = routed_tile_time(c, false, less, 2, M, n_out, K, k, stretch) * routed_tile_time(c, false, less, 1, M, n_out, K, k, stretch);
+      const double b = routed_tile_time(c, false, less + 1, 2, M, n_out, K, k, stretch);
+      if (s == 0 || a < t_less) { t_less = a; s = k; }
+      if (s_more == 0 || b < t_more) { t_more = b; s_more = k; }
+    }
+    return RoutedPlan{c.tile, s > 1 ? s : 1, s > 1 ? s_more : 1};
+  };
   for (int i = 0; i < n_costs; ++i) {
     const TileCost& c = costs[i];
+    if (forward_only(c.tile)) continue;
     consider(c, 1, 1);
     if (!dual && split && c.tile != TILE_256x256_W4) {
-      // the best factor for each M-tile count; either both are split or neither is
-      const int64_t less = cdiv64(M, tile_geom(c.tile, false).block_m);
-      int s = 0, s_more = 0;
-      double t_less = 0.0, t_more = 0.0;
-      for (const int k : kSplits) {
-        if (k == 1 || !routed_split_ok(K, k) || !fits({c.tile, k, k})) continue;
-        const double a = routed_tile_time(c, false, less, 2, M, n_out, K, k) * routed_tile_time(c, false, less, 1, M, n_out, K, k);
-        const double b = routed_tile_time(c, false, less + 1, 2, M, n_out, K, k);
-        if (s == 0 || a < t_less) { t_less = a; s = k; }
-        if (s_more == 0 || b < t_more) { t_more = b; s_more = k; }
-      }
-      if (s > 1) consider(c, s, s_more);
+      const RoutedPlan q = best_split(c);
+      if (q.splits > 1) consider(c, q.splits, q.splits_more);
     }
     if (c.tile == rule.tile && (rule.splits == 1 || split) && fits(rule)) keep = plan_score(c, dual, M, n_out, K, rule.splits, rule.splits_more, false);
   }
   constexpr double m = kModelMargin * kModelMargin * kModelMargin * kModelMargin * kModelMargin;  // a score is five times long
   if (keep > 0.0 && keep < best * m) p = rule;
-  if (dual) return p;
-  // 128-row tiles with 192-row ones among them where those save a round of the two modalities' tiles and one modality alone does not
-  // take longer for it (its tiles may fill whole rounds of 256-row ones).
-  const RoutedPlan without = p;
+  if (dual || !forward) return p;
+  // The heights between 128 and 256 rows, where they lead at nearly every split of the rows (kForwardGain).
   auto cost = [&](int tile) -> const TileCost& {
     int i = 0;
     while (costs[i].tile != tile) ++i;
     return costs[i];
   };
-  auto one = [&](const RoutedPlan& q) {
-    return routed_tile_time(cost(q.tile), false, cdiv64(M, tile_geom(q.tile, false).block_m), 1, M, n_out, K, q.splits);
-  };
-  best = plan_score(cost(p.tile), false, M, n_out, K, p.splits, p.splits_more) / m;
+  RoutedPlan between = p;
+  best = -1.0;
   for (int i = 0; i < n_costs; ++i) {
     const TileCost& c = costs[i];
-    const RoutedPlan q{c.tile, 1, 1};
-    if (stretch_part(c.tile) == 0.0 || !may_stretch(M, cdiv64(n_out, tile_geom(c.tile, false).block_n_out), kCus * c.per_cu)) continue;
-    const double t = plan_score(c, false, M, n_out, K, 1, 1);
-    if (t < best && one(q) <= kModelMargin * one(without)) {
-      best = t;
-      p = q;
+    if (!forward_only(c.tile)) continue;
+    const TileGeom geom = tile_geom(c.tile, false);
+    for (const RoutedPlan q : {RoutedPlan{c.tile, 1, 1}, split ? best_split(c) : RoutedPlan{c.tile, 1, 1}}) {
+      if (cdiv64(M, geom.block_m) * cdiv64(n_out, geom.block_n_out) * q.splits > 2 * kCus) continue;
+      const double t = plan_score(c, false, M, n_out, K, q.splits, q.splits_more);
+      if (fits(q) && (best < 0.0 || t < best)) {
+        best = t;
+        between = q;
+      }
     }
   }
-  return p;
+  if (best < 0.0) return p;
+  auto time_at = [&](const RoutedPlan& q, int64_t n_vis) {
+    const int64_t bm = tile_geom(q.tile, false).block_m, tiles_m = cdiv64(n_vis, bm) + cdiv64(M - n_vis, bm);
+    const int splits = routed_splits((int)n_vis, (int)M, (int)bm, q.splits, q.splits_more);
+    const StretchCost sc = stretch_cost(q.tile);
+    bool stretch = sc.part > 0.0;
+    if (stretch) {
+      const Stretch s = stretch_rows((int)n_vis, (int)M, (int)cdiv64(n_out, tile_geom(q.tile, false).block_n_out) * splits, sc.shape);
+      stretch = s.tall_v + s.tall_x > 0;
+    }
+    return routed_tile_time(cost(q.tile), false, tiles_m, n_vis < M ? 2 : 1, M, n_out, K, splits, stretch);
+  };
+  constexpr int kSplitsOfRows = 16;
+  double product = 1.0, worst = 0.0;
+  for (int i = 1; i <= kSplitsOfRows; ++i) {  // one modality, and splits from one end to the other that share no remainder
+    const int64_t at = i == kSplitsOfRows ? M : M * i / kSplitsOfRows + i * 37 % 61, n_vis = at < 1 ? 1 : at < M ? at : i == kSplitsOfRows ? M : M - 1;
+    const double r = time_at(between, n_vis) / time_at(p, n_vis);
+    product *= r;
+    worst = r > worst ? r : worst;
+    if (i == kSplitsOfRows && r > 1.0) return p;
+  }
+  double gain = 1.0;
+  for (int i = 0; i < kSplitsOfRows; ++i) gain *= kForwardGain;
+  return worst < kModelMargin && product < gain ? between : p;
 }
 
 // The model is a pure function of the extents and takes 5 us of host time (single-weight GEMMs); every thread keeps the last
 // plans.  Extents are mostly multiples of 32 and more: the slot comes from the top of a product, where all their bits arrive.
-inline unsigned model_plan_slot(bool dual, int64_t M, int64_t n_out, int64_t K, bool split, size_t room) {
+inline unsigned model_plan_slot(bool dual, int64_t M, int64_t n_out, int64_t K, bool split, size_t room, bool forward = true) {
   constexpr uint64_t kMul = 0x9E3779B97F4A7C15ull;
   uint64_t x = (uint64_t)M;
-  for (const uint64_t v : {(uint64_t)n_out, (uint64_t)K, (uint64_t)room * 4 + (dual ? 2 : 0) + (split ? 1 : 0)}) x = (x ^ (x >> 29)) * kMul + v;
+  for (const uint64_t v : {(uint64_t)n_out, (uint64_t)K, (uint64_t)room * 8 + (forward ? 0 : 4) + (dual ? 2 : 0) + (split ? 1 : 0)}) x = (x ^ (x >> 29)) * kMul + v;
   return (unsigned)((x ^ (x >> 32)) * kMul >> 59);
 }
-inline RoutedPlan model_routed_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split, size_t room = kAnyRoom) {
+inline RoutedPlan model_routed_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split, size_t room = kAnyRoom, bool forward = true) {
   struct Entry {
     int64_t M = -1, n_out, K;
-    bool dual, split;
+    bool dual, split, forward;
     size_t room;
     RoutedPlan plan;
   };
   static thread_local Entry memo[32];
-  Entry& e = memo[model_plan_slot(dual, M, n_out, K, split, room)];
-  if (e.M != M || e.n_out != n_out || e.K != K || e.dual != dual || e.split != split || e.room != room)
-    e = Entry{M, n_out, K, dual, split, room, compute_model_plan(dual, M, n_out, K, split, room)};
+  Entry& e = memo[model_plan_slot(dual, M, n_out, K, split, room, forward)];
+  if (e.M != M || e.n_out != n_out || e.K != K || e.dual != dual || e.split != split || e.forward != forward || e.room != room)
+    e = Entry{M, n_out, K, dual, split, forward, room, compute_model_plan(dual, M, n_out, K, split, room, forward)};
   return e.plan;
 }
 

@@ -44,6 +44,7 @@ from . import _lib
 from .ops import masked_linear_backward, masked_linear_forward
 
 TILES = {0: "256x256/8w", 1: "256x256/4w", 2: "128x128/4w", 3: "small/4w", 4: "128x128/ring4", 6: "128x256/ring3", 7: "64x128/ring3"}
+FORWARD_TILES = {16: "192x256/4w", 17: "160x256/4w"}  # of plans that the library's model makes; not searched
 GROUP_MS = (2, 4, 8, 16)   # M-tiles per super-group tried in the second stage
 GM_MIN_ROWS = 4096         # ... for buckets that reach this many rows
 TILE_IN_PLACE = 5  # weight-gradient plans only (kTileGatherDw in csrc/capi.hip): g and x read where they lie
@@ -196,7 +197,8 @@ def _tile_id(cfg, dual):
     cols = cfg["block_n"] * (2 if dual else 1)
     if cfg["block_m"] == 256:
         return 0 if cfg["waves_m"] * cfg["waves_n"] == 8 else 1
-    return {(128, 128, 4): 4, (128, 256, 3): 6, (64, 128, 3): 7, (128, 128, 2): 2}.get((cfg["block_m"], cols, cfg["lds_stages"]), 3)
+    return {(128, 128, 4): 4, (128, 256, 3): 6, (64, 128, 3): 7, (128, 128, 2): 2,
+            (192, 256, 3): 16, (160, 256, 3): 17}.get((cfg["block_m"], cols, cfg["lds_stages"]), 3)
 
 
 def _gm_stage(measure, ref, own, margin):
@@ -285,6 +287,8 @@ def tune_ffn(d, h, bucket, trials, dev, ev, margin):
 
         def stage(plan, which):
             def measure(g):
+                if plan[0] in FORWARD_TILES:
+                    return None
                 ts = []
                 for x, mask in scen:
                     with _Forced(plan[0], plan[1], g):
@@ -353,6 +357,8 @@ def tune_linear_fwd(K, N, bucket, trials, dev, margin):
         plan = best if best is not None else (_tile_id(base_cfg, False), base_cfg["split_k"])
 
         def measure(g):
+            if plan[0] in FORWARD_TILES:
+                return None
             ts = []
             for x, mask in scen:
                 with _Forced(plan[0], plan[1], g):

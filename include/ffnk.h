@@ -133,7 +133,8 @@ FFNK_API int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile
  * sweeps, and the tests that run every compiled tile).  ffnk_debug_force_tile: every LDS-tiled GEMM
  * launched by this process uses tile id `tile` (0 = 256x256 / 8 waves, 1 = 256x256 / 4 waves - in the SwiGLU GEMM
  * beside 160x256 ones up to eight rounds, as in a plan -, 2 = 128x128 / 4 waves, 3 = small, 4 = 128x128 / 4 waves behind a ring of four LDS stages, 6 = 128x256 and
- * 7 = 64x128 behind a ring of three; GEMMs without a ring run 2 or 3 in their place); -1 returns to the tile table
+ * 7 = 64x128 behind a ring of three, 16 = 192x256 and 17 = 160x256 in the forward's single-weight GEMMs (6 in the others);
+ * GEMMs without a ring run 2 or 3 in their place); -1 returns to the tile table
  * (measured plans first, then the rules); -2 uses the rules only, ignoring the measured plans (what the tuner compares
  * against).  Other values count as -1.
  * ffnk_debug_force_splits: every GEMM that can cut its contraction (single-weight routed GEMMs with

@@ -40,17 +40,18 @@ void hc_mixed_tile(int bid, int n_vis, int M, int N, int bn, int group, int* out
   out[0] = t.grp; out[1] = t.row0; out[2] = end < t.row_end ? end : t.row_end; out[3] = t.n0;
 }
 
-// Tiles of a launch on 128-row tiles with 192-row ones among them: how many; tile L: {group, first row, end, first column}.
-int hc_may_stretch(int M, int tiles_n, int slots) { return may_stretch(M, tiles_n, slots) ? 1 : 0; }
-int hc_stretch_tiles(int n_vis, int M, int tiles_n, int slots) {
-  const Stretch s = stretch_rows(n_vis, M, tiles_n, slots);
+// Tiles of a launch with taller tiles among the others: how many; tile L: {group, first row, end, first column}.
+int hc_may_stretch(int M, int tiles_n, int base, int tall, int slots) { return may_stretch(M, tiles_n, {base, tall, slots}) ? 1 : 0; }
+int hc_stretch_tiles(int n_vis, int M, int tiles_n, int base, int tall, int slots) {
+  const Stretch s = stretch_rows(n_vis, M, tiles_n, {base, tall, slots});
   return (s.tiles_v + s.tiles_x) * tiles_n;
 }
-void hc_stretch_tile(int L, int n_vis, int M, int tiles_n, int slots, int bn, int group, int* out) {
-  const Stretch s = stretch_rows(n_vis, M, tiles_n, slots);
-  bool tall;
-  const TileCoord t = stretch_tile_coord(L, s, n_vis, M, tiles_n, bn, group, &tall);
-  const int end = t.row0 + (tall ? kStretchRows : kStretchBase);
+void hc_stretch_tile(int L, int n_vis, int M, int tiles_n, int base, int tall, int slots, int bn, int group, int* out) {
+  const StretchShape shape{base, tall, slots};
+  const Stretch s = stretch_rows(n_vis, M, tiles_n, shape);
+  bool is_tall;
+  const TileCoord t = stretch_tile_coord(L, s, n_vis, M, tiles_n, bn, group, shape, &is_tall);
+  const int end = t.row0 + (is_tall ? tall : base);
   out[0] = t.grp; out[1] = t.row0; out[2] = end < t.row_end ? end : t.row_end; out[3] = t.n0;
 }
 

@@ -258,7 +258,36 @@ def test_stretched_tiles(dev, forced, tile, N, K, nv, nt):
     assert_close(y, ref.cpu(), "y")
 
 
-@pytest.mark.parametrize("tile", [2, 6])
+# The same on 160-row tiles (192-row ones among them) and 192-row tiles (224), unsplit and cut into two K ranges, where the last M-tile
+# takes one to six taller ones, and where a modality has too few M-tiles for that.
+@pytest.mark.parametrize("tile,base", [(16, 192), (17, 160)])
+@pytest.mark.parametrize("N,splits,K", [(8192, 1, 328), (4096, 2, 712)])
+@pytest.mark.parametrize("more", [0, 1, 32, 33, 100, 150, 300])
+def test_stretched_tiles_between(dev, forced, tile, base, N, splits, K, more):
+    nv = 4 * base + more
+    nt = 8 * base - nv
+    note(f"tiles between 128 and 256 rows: tile={tile} K={K} splits={splits} {nv} visual, {nt} text rows")
+    x, Wv, Wt, mask, _ = make_linear(dev, nv, nt, K, N, seed=nv + K)
+    forced(tile=tile, splits=splits)
+    y = MaskedLinear.apply(x, Wv.T, Wt.T, mask)
+    forced()
+    ref = torch.where(mask[:, None], x.double() @ Wv.double().T, x.double() @ Wt.double().T)
+    assert_close(y, ref.cpu(), "y")
+
+
+@pytest.mark.parametrize("tile", [16, 17])
+@pytest.mark.parametrize("nv,nt", [(1, 0), (0, 159), (161, 192), (193, 1), (400, 225)])
+def test_tiles_between_at_few_rows(dev, forced, tile, nv, nt):
+    note(f"tiles between 128 and 256 rows: tile={tile} {nv} visual, {nt} text rows")
+    x, Wv, Wt, mask, _ = make_linear(dev, nv + 64, nt, 192, 264, seed=nv)
+    forced(tile=tile, splits=1)
+    y = MaskedLinear.apply(x, Wv.T, Wt.T, mask)
+    forced()
+    ref = torch.where(mask[:, None], x.double() @ Wv.double().T, x.double() @ Wt.double().T)
+    assert_close(y, ref.cpu(), "y")
+
+
+@pytest.mark.parametrize("tile", [2, 6, 16, 17])
 def test_stretched_down_projection(dev, forced, tile):
     nv, nt, d, h = 540, 484, 8192, 192
     note(f"192-row tiles in the down projection: tile={tile}")

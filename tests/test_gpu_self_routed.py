@@ -74,7 +74,7 @@ def _linear(x, W, mask, N):
     return call
 
 
-@pytest.mark.parametrize("tile", [-1, 0, 2, 3, 4, 6, 7])
+@pytest.mark.parametrize("tile", [-1, 0, 2, 3, 4, 6, 7, 16, 17])
 @pytest.mark.parametrize("M", [65, 129, 257, 700, 2047, 2049, 4097, 8191, 8192, 8193])
 def test_linear_forward_makes_the_partition(dev, M, tile):
     K, N = 192, 256

@@ -266,28 +266,30 @@ def test_the_swiglu_derivative_divides(tmp_path):
     assert [asm.count(i) for i in ("v_rcp_f32", "v_div_fmas_f32", "v_div_fixup_f32")] == [8, 8, 8]
 
 
-# 128-row tiles with 192-row ones among them: every result in one tile, no more tiles than 128-row ones, whole rounds where one
+# Taller tiles among the others of a launch: every result in one tile, no more tiles than without, whole rounds where one
 # M-tile less makes them, and no stretch that the host's launch does not allow for.
+@pytest.mark.parametrize("base,tall", [(128, 192), (160, 192), (192, 224)])
 @pytest.mark.parametrize("tiles_n,slots,tiles_m", [(8, 512, 64), (8, 256, 32), (32, 256, 8), (64, 512, 8), (20, 256, 12), (3, 512, 170), (128, 256, 4), (256, 256, 1)])
-def test_stretched_tiles_cover_the_output(rules, tiles_n, slots, tiles_m):
+def test_stretched_tiles_cover_the_output(rules, base, tall, tiles_n, slots, tiles_m):
     t = (ctypes.c_int * 4)()
-    stretched = 0
-    for M in (tiles_m * 128, tiles_m * 128 - 1, tiles_m * 128 + 1, tiles_m * 128 + 60, tiles_m * 128 + 65, tiles_m * 128 - 127):
-        splits = {0, 1, M, M - 1, M // 2, 64, 65, 127, 128, 129, 192, 193, M - 64, M - 192} | {M // 2 + i for i in (-70, -64, 1, 60, 63, 64, 65, 127)}
+    stretched, whole = 0, tiles_m * base
+    for M in (whole, whole - 1, whole + 1, whole + 60, whole + 65, whole - base + 1):
+        splits = {0, 1, M, M - 1, M // 2, 64, 65, base - 1, base, base + 1, tall, tall + 1, M - 64, M - tall}
+        splits |= {M // 2 + i for i in (-70, -64, 1, 31, 32, 33, 60, 63, 64, 65, base - 1)}
         for n_vis in sorted(v for v in splits if 0 <= v <= M):
-            plain = (-(-n_vis // 128) + -(-(M - n_vis) // 128)) * tiles_n
-            count = rules.hc_stretch_tiles(n_vis, M, tiles_n, slots)
+            plain = (-(-n_vis // base) + -(-(M - n_vis) // base)) * tiles_n
+            count = rules.hc_stretch_tiles(n_vis, M, tiles_n, base, tall, slots)
             assert count in (plain, plain - tiles_n)
             if count < plain:
                 stretched += 1
-                assert rules.hc_may_stretch(M, tiles_n, slots) and plain // slots > (count - 1) // slots
+                assert rules.hc_may_stretch(M, tiles_n, base, tall, slots) and plain // slots > (count - 1) // slots
             rows = {}
             for L in range(count):
-                rules.hc_stretch_tile(L, n_vis, M, tiles_n, slots, 128, 4, t)
+                rules.hc_stretch_tile(L, n_vis, M, tiles_n, base, tall, slots, 128, 4, t)
                 assert 0 <= t[1] < t[2] <= (n_vis if t[0] == 0 else M) and (t[0] == 0 or t[1] >= n_vis)
                 rows.setdefault(t[3], []).append((t[1], t[2]))
             assert sorted(rows) == [n * 128 for n in range(tiles_n)]
             for spans in rows.values():
                 spans.sort()
                 assert spans[0][0] == 0 and spans[-1][1] == M and all(a[1] == b[0] for a, b in zip(spans, spans[1:]))
-    assert stretched > 0 or slots // tiles_n < 2 or tiles_n > slots // 8
+    assert stretched > 0 or tiles_n > slots // 8
