@@ -1931,14 +1931,15 @@ __global__ __launch_bounds__(CfgDx::NT) void fused_bwd_kernel(const GemmArgs gx,
 
 // Tiles of two heights in one launch (mixed_rows): every XCD takes an eighth of the tall tiles' order, then an eighth of the
 // short ones'.
-template <class Tall, class Short>
+template <class Tall, class Short, class Quarter>
 __global__ __launch_bounds__(Tall::NT) void routed_mixed_kernel(const GemmArgs g) {
   static_assert(Tall::NT == Short::NT && Tall::BN_OUT == Short::BN_OUT && Tall::BM == kTallRows && Short::BM == kShortRows, "two heights");
+  static_assert(Tall::NT == Quarter::NT && Tall::BN_OUT == Quarter::BN_OUT && Quarter::BM == kQuarterRows && Quarter::LDS_BYTES <= Short::LDS_BYTES, "pieces");
   __shared__ __attribute__((aligned(1024))) uint8_t lds[Tall::LDS_BYTES > Short::LDS_BYTES ? Tall::LDS_BYTES : Short::LDS_BYTES];
-  bool is_tall;
+  bool is_tall, is_quarter = false;
   RowScan<Tall::NT> scan;
   const int n_vis = visual_rows<Tall>(g, lds, (int)blockIdx.x, scan);
-  TileCoord tc = mixed_tile_coord((int)blockIdx.x, n_vis, g.M, g.N, Tall::BN_OUT, g.group_m > 0 ? g.group_m : Tall::GROUP_M, &is_tall);
+  TileCoord tc = mixed_tile_coord((int)blockIdx.x, n_vis, g.M, g.N, Tall::BN_OUT, g.group_m > 0 ? g.group_m : Tall::GROUP_M, &is_tall, &is_quarter);
   if (tc.grp < 0) return;
   // (the compiler takes them for values of a lane and would load the weights' addresses through the vector memory path)
   tc.grp = __builtin_amdgcn_readfirstlane(tc.grp);
@@ -1946,6 +1947,7 @@ __global__ __launch_bounds__(Tall::NT) void routed_mixed_kernel(const GemmArgs g
   tc.row_end = __builtin_amdgcn_readfirstlane(tc.row_end);
   tc.n0 = __builtin_amdgcn_readfirstlane(tc.n0);
   if (is_tall) routed_tile<Tall>(g, lds, tc, 0, 1, 0, scan);
+  else if (is_quarter) routed_tile<Quarter>(g, lds, tc, 0, 1, 0, scan);
   else routed_tile<Short>(g, lds, tc, 0, 1, 0, scan);
 }
 
@@ -2025,13 +2027,13 @@ inline hipError_t launch_routed_stretch(const GemmArgs& g, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <class Tall, class Short>
+template <class Tall, class Short, class Quarter>
 inline hipError_t launch_routed_mixed(const GemmArgs& g, hipStream_t stream) {
   if (g.M <= 0 || g.N <= 0) return hipSuccess;
   if (g.splits > 1 || g.splits_more > 1 || g.tail_mode != 0 || g.P_tail != nullptr || g.k_switch != 0 || !direct_slabs_ok(g.K) ||
       !self_routed_args_ok<Tall>(g))
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL((routed_mixed_kernel<Tall, Short>), dim3(mixed_blocks(g.M, g.N, Tall::BN_OUT)), dim3(Tall::NT), 0, stream, g);
+  hipLaunchKernelGGL((routed_mixed_kernel<Tall, Short, Quarter>), dim3(mixed_blocks(g.M, g.N, Tall::BN_OUT)), dim3(Tall::NT), 0, stream, g);
   return hipGetLastError();
 }
 

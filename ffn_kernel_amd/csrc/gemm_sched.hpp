@@ -134,7 +134,7 @@ __host__ __device__ inline TileCoord stretch_tile_coord(int L, const Stretch& s,
 // 3000 others: 3.5 % less, 1.8 % of them more than 3 % slower (the worst 13 %): calls whose rows end just past a whole round, where
 // the mask decides which side wins.  M = 300 (150 + 150), K = 4096, 14336 columns: 122.7 -> 111.3 us, the MaskedFFN call 207 -> 184;
 // M = 499, K = 5696, 16192 columns 278 -> 200.
-constexpr int kTallRows = 256, kShortRows = 160, kTallCost = 256, kShortCost = 176;
+constexpr int kTallRows = 256, kShortRows = 160, kQuarterRows = 64, kTallCost = 256, kShortCost = 176;
 // A column's weight panel from memory, by the whole chip: 512 bytes per element of the contraction at 6.2 TB/s against the tall
 // tile's 1.056 us per 64 of them.  Tiles of both heights of one modality read it twice (they run at different times).
 constexpr int kColumnCost64 = 85;  // in 64ths
@@ -150,15 +150,25 @@ __host__ __device__ inline MixedRows mixed_rows(int rows) {
   if (whole > 0 && rest <= 2 * kShortRows - kTallRows) return {whole - 1, 2};
   return rest <= kShortRows ? MixedRows{whole, 1} : MixedRows{whole + 1, 0};
 }
-__host__ __device__ inline bool mixed_splits_rest(int tall, int shrt) {
+// Into how many pieces the tall tiles past the last whole round are cut: two short ones each where those and the other short ones are
+// one round, four of kQuarterRows behind whole rounds where those are one.  A round of such pieces, which share every column's weight
+// panel, ends in 0.4 (64 of them) to 0.6 (256) of a tall one's time against 0.7 for two short ones each.  The SwiGLU GEMM of
+// MaskedFFN with up to 60 tiles past whole rounds, halves -> quarters: d = 1024, h = 2048, M = 8192 (16 past two rounds) 80.2 -> 75.2 us,
+// d = 2048, h = 4672, M = 3679 (43) 132.5 -> 124.1, d = 1536, h = 3264, M = 2931 (56) 67.7 -> 62.9, d = 4096, h = 14336, M = 1100 (48)
+// 247 -> 238; calls 2 to 5 % less, others the same.
+constexpr int kQuarterCost = 96, kQuarterRest = 21;  // of a round of pieces, and what each cut tile adds to it in 16ths
+__host__ __device__ inline int mixed_pieces(int tall, int shrt) {
   const int rest = tall % kCusPerChip;
-  return rest > 0 && 2 * rest + shrt <= kCusPerChip;
+  if (rest == 0) return 1;
+  if (shrt == 0 && tall > rest && 4 * rest <= kCusPerChip) return 4;
+  return 2 * rest + shrt <= kCusPerChip ? 2 : 1;
 }
 // When the last CU is done: tall tiles first, a CU that is free takes the next tile.
 __host__ __device__ inline int mixed_time(int tall, int shrt) {
   static_assert(kTallCost == kCusPerChip, "a shift less");
-  const int rest = tall % kCusPerChip, done = tall - rest;
-  if (mixed_splits_rest(tall, shrt)) return done + kShortCost;
+  const int rest = tall % kCusPerChip, done = tall - rest, pieces = mixed_pieces(tall, shrt);
+  if (pieces == 4) return done + kQuarterCost + rest * kQuarterRest / 16;
+  if (pieces == 2) return done + kShortCost;
   if (rest == 0) return done + cdiv(shrt, kCusPerChip) * kShortCost;
   if (shrt <= kCusPerChip - rest) return done + kTallCost;
   return done + (rest * kTallCost + shrt * kShortCost) / kCusPerChip + kShortCost / 2;  // (the last tiles of a CU end anywhere in half a tile)
@@ -182,32 +192,35 @@ __host__ __device__ inline void mixed_choice(int n_vis, int M, int tiles_n, Mixe
 }
 // Workgroups of a launch, for any split of M rows.
 inline int mixed_blocks(int M, int N, int bn) {
-  const int64_t tiles = (int64_t)(cdiv(M, kTallRows) + 1) * cdiv(N, bn) + kCusPerChip / 2;  // with the second halves of split tiles
+  const int64_t tiles = (int64_t)(cdiv(M, kTallRows) + 1) * cdiv(N, bn) + kCusPerChip * 3 / 4;  // with the other pieces of cut tiles
   return kXcds * (int)(cdiv64(tiles, kXcds) + 1);
 }
 // Tile of workgroup `bid`; grp < 0: a surplus workgroup.  Every XCD takes an eighth of the tall tiles' order, then an eighth of the
 // short ones'; an order walks the M-tiles of one height and modality in super-groups of `group`, column by column, so that the tiles
 // of a column share the weight panel.
-__host__ __device__ inline TileCoord mixed_tile_coord(int bid, int n_vis, int M, int N, int bn, int group, bool* is_tall) {
+__host__ __device__ inline TileCoord mixed_tile_coord(int bid, int n_vis, int M, int N, int bn, int group, bool* is_tall, bool* is_quarter = nullptr) {
   TileCoord t{-1, 0, 0, 0};
   const int tiles_n = cdiv(N, bn);
   MixedRows v, x;
   mixed_choice(n_vis, M, tiles_n, &v, &x);
   const int tall = (v.tall + x.tall) * tiles_n, shrt = (v.shrt + x.shrt) * tiles_n;
-  const int whole = mixed_splits_rest(tall, shrt) ? tall / kCusPerChip * kCusPerChip : tall;  // tall tiles that run as such
-  const int halves = 2 * (tall - whole);
-  const int per_tall = cdiv(whole, kXcds), per_short = cdiv(halves + shrt, kXcds);
+  const int cut = mixed_pieces(tall, shrt);
+  const int whole = cut > 1 ? tall / kCusPerChip * kCusPerChip : tall;  // tall tiles that run as such
+  const int pieces = cut * (tall - whole);
+  const int per_tall = cdiv(whole, kXcds), per_short = cdiv(pieces + shrt, kXcds);
   int slot = bid / kXcds;
   *is_tall = slot < per_tall;
   if (!*is_tall) slot -= per_tall;
   const int per = *is_tall ? per_tall : per_short;
   int L = (bid % kXcds) * per + slot;
-  if (slot >= per || L >= (*is_tall ? whole : halves + shrt)) return t;
-  const bool half = !*is_tall && L < halves;
-  const int second = half ? L & 1 : 0;
-  if (half) L = whole + L / 2;
-  else if (!*is_tall) L -= halves;
-  const bool of_tall = *is_tall || half;
+  if (slot >= per || L >= (*is_tall ? whole : pieces + shrt)) return t;
+  const bool piece = !*is_tall && L < pieces;
+  const int part = piece ? L & (cut - 1) : 0;
+  if (piece) L = whole + (cut == 4 ? L / 4 : L / 2);
+  else if (!*is_tall) L -= pieces;
+  const bool quarter = piece && cut == 4;
+  if (is_quarter != nullptr) *is_quarter = quarter;
+  const bool of_tall = *is_tall || piece;
   const int own_v = of_tall ? v.tall : v.shrt, own_x = of_tall ? x.tall : x.shrt;  // M-tiles of this height by modality
   const int grp = L < own_v * tiles_n ? 0 : 1;
   if (grp == 1) L -= own_v * tiles_n;
@@ -221,8 +234,9 @@ __host__ __device__ inline TileCoord mixed_tile_coord(int bid, int n_vis, int M,
   }
   const int begin = grp == 0 ? 0 : n_vis, end = grp == 0 ? n_vis : M;
   t.row0 = begin + (of_tall ? 0 : (grp == 0 ? v.tall : x.tall) * kTallRows) + (first + L % gsz) * (of_tall ? kTallRows : kShortRows);
-  t.row_end = half && t.row0 + kTallRows < end ? t.row0 + kTallRows : end;
-  t.row0 += second * kShortRows;
+  t.row_end = piece && t.row0 + kTallRows < end ? t.row0 + kTallRows : end;
+  t.row0 += part * (quarter ? kQuarterRows : kShortRows);
+  if (quarter && t.row0 + kQuarterRows < t.row_end) t.row_end = t.row0 + kQuarterRows;
   t.n0 = (L / gsz) * bn;
   if (t.row0 < t.row_end) t.grp = grp;
   return t;

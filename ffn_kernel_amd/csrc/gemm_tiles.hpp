@@ -76,6 +76,7 @@ struct DualTiles {
   using T3 = RoutedGemmCfg<64, 128, 2, 2, true, true, false, DIRECT, kGroupM>;
   using T4 = RoutedGemmCfg<128, 128, 2, 2, true, true, false, DIRECT, kGroupM, false, DIRECT ? 4 : 2>;
   using Short = RoutedGemmCfg<160, 256, 2, 2, true, true, false, true, kGroupM, false, 3>;  // beside T1, see mixed_rows
+  using Quarter = RoutedGemmCfg<64, 256, 2, 2, true, true, false, true, kGroupM, false, 3>;  // pieces of T1 past whole rounds, see mixed_pieces
   using T6 = std::conditional_t<DIRECT, RoutedGemmCfg<128, 256, 2, 2, true, true, false, true, kGroupM, false, 3>, T2>;
   using T7 = std::conditional_t<DIRECT, RoutedGemmCfg<64, 128, 2, 2, true, true, false, true, kGroupM, false, 3>, T3>;
 };

@@ -6,7 +6,7 @@ namespace ffnk {
 hipError_t launch_up_gemm(int tile, bool direct, const GemmArgs& g, hipStream_t stream) {
   if (tile == TILE_MIXED_W4) {
     if (!direct) return hipErrorInvalidValue;
-    return launch_routed_mixed<DualTiles<true>::T1, DualTiles<true>::Short>(g, stream);
+    return launch_routed_mixed<DualTiles<true>::T1, DualTiles<true>::Short, DualTiles<true>::Quarter>(g, stream);
   }
   return direct ? dispatch_tile_with_tail<DualTiles<true>>(tile, g, stream)
                 : dispatch_tile<DualTiles<false>>(tile, g, stream);

@@ -303,3 +303,28 @@ def test_stretched_down_projection(dev, forced, tile):
         return (torch.nn.functional.silu(g) * u).bfloat16().double() @ w2.double().T
 
     assert_close(y, torch.where(mask[:, None], half(*w[:3]), half(*w[3:])).cpu(), "y")
+
+
+# 256-row tiles of the SwiGLU GEMM past a whole round, cut into 64-row pieces (mixed_pieces): a few tiles and a quarter of a round, a
+# last column tile that is half full, modalities that end at the edges of a piece, pre-activations kept or not.
+@pytest.mark.parametrize("nv,nt,h", [(1500, 0, 5440), (760, 740, 5504), (0, 1473, 5504), (1281, 200, 5504), (1217, 0, 8192), (513, 705, 8128)])
+@pytest.mark.parametrize("save", [False, True])
+def test_swiglu_tiles_in_quarters(dev, forced, nv, nt, h, save):
+    d = 128
+    note(f"SwiGLU tiles in quarters: {nv} visual, {nt} text rows, h={h} save={save}")
+    x, _, _, mask, _ = make_linear(dev, nv, nt, d, 8, seed=nv + h)
+    gen = torch.Generator(device=dev).manual_seed(h)
+    w = [(torch.randn(*s, generator=gen, device=dev) * 0.05).bfloat16() for s in [(h, d), (d, h), (h, d)] * 2]
+    forced(tile=1)
+    y = masked_ffn_forward(x, *(v.T for v in w), mask, save_pre=save)
+    forced()
+
+    def half(w1, w2, w3):
+        g, u = x.double() @ w1.double().T, x.double() @ w3.double().T
+        return (torch.nn.functional.silu(g) * u).bfloat16().double() @ w2.double().T
+
+    assert_close(y[0] if save else y, torch.where(mask[:, None], half(*w[:3]), half(*w[3:])).cpu(), "y")
+    if save:
+        order = torch.cat([mask.nonzero()[:, 0], (~mask).nonzero()[:, 0]])
+        pre = torch.where(mask[:, None], x.double() @ torch.cat([w[0], w[2]]).double().T, x.double() @ torch.cat([w[3], w[5]]).double().T)
+        assert_close(y[1], pre[order].cpu(), "pre")
