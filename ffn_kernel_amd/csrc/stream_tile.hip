@@ -71,6 +71,7 @@ enum { FORM_WHOLE, FORM_RAGGED, FORM_SPLIT_LINES };
 struct TileJob {
   int grp, split, p0, mg, n0, c0, nc;  // n0: first weight row of the workgroup; c0 / nc: chunk range
   int n_store;                         // first weight row whose outputs the workgroup stores (n0 where Nrows is whole row blocks)
+  unsigned at;                         // number of the workgroup where both modalities are there, visual ones first
 };
 
 // xs: [2][NTM * 16 token rows][16 pieces] 16-byte slots; wst: this wavefront's [2 tiles][16 rows][16 pieces].
@@ -131,9 +132,10 @@ __device__ __forceinline__ void tile_rows(const StreamArgs& a, const TileJob& t,
 
   // Workgroups walk their chunk range from different starting chunks (wrapping around): weight rows
   // are a power-of-two number of bytes apart, so workgroups sitting at the same K offset would all
-  // pull from the same few HBM channels.
+  // pull from the same few HBM channels.  Never from where the workgroup lies in the launch, which depends on the modalities that
+  // are there (first_group): a row's sums are the same beside rows of the other modality and without them.
   const int nc = t.nc;
-  const unsigned spread = kTWaves == kWideWaves ? (blockIdx.x >> 3) * 11u + (blockIdx.x & 7u) * (unsigned)nc / 8u : blockIdx.x * 11u;
+  const unsigned spread = kTWaves == kWideWaves ? (t.at >> 3) * 11u + (t.at & 7u) * (unsigned)nc / 8u : t.at * 11u;
   const int rot = (int)(spread % (unsigned)nc);
   // RAGGED: a last chunk that would pass the end of the rows starts earlier, overlapping the chunk before it; what the two
   // share (overlap(c) pieces of 8 elements) is cleared in both operands' fragments, so that no product is counted twice
@@ -404,6 +406,7 @@ __global__ __launch_bounds__(kTWaves * kWave, 2) void stream_tile_kernel(const S
   t.p0 = t.grp == 0 ? 0 : n_vis;
   t.mg = t.grp == 0 ? n_vis : a.M - n_vis;
   if (t.mg == 0) return;  // modality absent: its weights are never read (uniform over the workgroup)
+  t.at = (unsigned)(t.grp * per_grp + rem);
   t.n_store = (rem % row_blocks) * ROWS;
   t.n0 = RAGGED ? min(t.n_store, a.Nrows - ROWS) : t.n_store;
   const int n_chunks = RAGGED ? cdiv(a.K, kTK) : a.K / kTK;

@@ -367,6 +367,21 @@ def test_ffn_decode_four_wavefronts(dev, M, h, kind):
         assert torch.equal(MaskedFFN.apply(*wl.FFNWorkload("p", w.x, W, w.mask).to(dev).op_args()), out)
 
 
+# A row's result depends on that row, its modality's weights and the path alone, bit for bit: beside rows of the other modality and
+# without them, over two, three and four m-tiles; whole and ragged extents, one K range and several.
+@pytest.mark.parametrize("d,h", [(1024, 2048), (1152, 1408), (1096, 1416), (1024, 8192)])
+@pytest.mark.parametrize("nt,nv", [(20, 12), (17, 30), (33, 31), (40, 24)])
+def test_ffn_decode_rows_beside_the_other_modality(dev, nt, nv, d, h):
+    note(f"ffn decode, {nt} text rows alone and beside {nv} visual ones, d={d} h={h}")
+    mask = torch.zeros(nt + nv, dtype=torch.bool)
+    mask[torch.randperm(nt + nv, generator=torch.Generator().manual_seed(nt))[:nv]] = True
+    w = wl.make_ffn("rows", nt + nv, d, h, mask, seed=nt + h, w_std=0.05).to(dev)
+    both = MaskedFFN.apply(*w.op_args())
+    for rows in (~w.mask, w.mask):
+        alone = MaskedFFN.apply(*wl.FFNWorkload("a", w.x[rows], w.W, w.mask[rows]).op_args())
+        assert torch.equal(alone, both[rows])
+
+
 def test_ffn_decode_matches_tiled_path_rows(dev):
     """The same rows run as a decode call and inside a larger (tiled-path) call agree to bf16 accuracy."""
     note("ffn decode vs tiled")
