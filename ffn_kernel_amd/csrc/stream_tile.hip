@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "gemm_sched.hpp"
 #include "launch.hpp"
 
 namespace ffnk {
@@ -46,14 +47,26 @@ constexpr const TileShapeEntry& tile_shape(int ntm_max, bool dual) { return dual
 constexpr int kTMaxM = 64;
 // The up projection at three and four m-tiles with four wavefronts per workgroup: half the slab traffic per weight byte, which
 // above 32 rows is as much as the weights; 80 KB of LDS at four m-tiles, two workgroups per CU as with two wavefronts, and half as
-// many workgroups, so long streams only.  Workgroups of one XCD start at different chunks (spread): with the two-wavefront
-// kernels' start, which has four values per XCD at 32 chunks, a 64-row workgroup at K = 4096 was 4 to 8 % slower instead.
+// many workgroups, so long streams only.
 // Whole call, us, two -> four wavefronts, one modality / both: M = 64, d = 4096, h = 14336 76.3 -> 71.5 / 126 -> 121.5, h = 16384
 // 80.3 -> 77.2 / 137 -> 132, h = 11008 68.7 -> 61.9 / 112 -> 107; d = 5120, h = 13824 103 -> 96.5 / 174 -> 163; d = 8192, h = 22016
 // 232 -> 210 / 356 -> 346; d = 3072, h = 10240 60.2 -> 56.5 / 92.5 -> 91; fewer rows lose with both modalities (d = 4096, h = 8960
 // 95 -> 98, d = 2560 71 -> 76).  M = 36 ... 48, where two wavefronts fit three times: d = 4096, h = 14336 72.0 -> 67.8 / 123 -> 118,
 // d = 6144 117 -> 109 / 187 -> 181, but h = 22016, d = 8192 190 -> 204 and h = 10240, d = 3072 76 -> 82 (both).
 constexpr int kWideWaves = 4, kWideRows = 16 * kWideWaves;
+// The row blocks of a workgroup of four wavefronts: two blocks of a workgroup of two that start at the same chunk (rot), a multiple of
+// nc row blocks apart, so that every sum has the order that it has there.  Of the whole groups of nc blocks the first half goes with
+// the second; the blocks behind them go with those nc ahead, or alone.  (d = 8192, h = 22016, M = 64: 219 us with every pair nc blocks
+// apart, the same channels for both; 211 so.  Pairs of neighbours with a start of their own: 211 as well, d = 4096, h = 14336 70.5
+// against 70.8, one modality, 119.6 against 122.3, both.)  Every XCD takes neighbours, which start at different chunks: where the
+// workgroups of an XCD had four starts at 32 chunks, K = 4096 took 4 to 8 % longer.
+struct WideJobs {
+  int paired, jobs;  // row blocks of the first half; workgroups
+};
+__host__ __device__ constexpr WideJobs wide_jobs(int row_blocks, int nc) {
+  const int paired = row_blocks / (2 * nc) * nc, rest = row_blocks - 2 * paired;
+  return {paired, paired + (rest < nc ? rest : nc)};
+}
 bool stream_tile_wide(int M, int Nrows, int K) {
   if (M <= 32 || M > kTMaxM || K % kTK != 0 || Nrows % kWideRows != 0) return false;
   return M > 48 ? Nrows >= 10240 : Nrows >= 12288 && Nrows <= 16384;
@@ -72,13 +85,15 @@ struct TileJob {
   int grp, split, p0, mg, n0, c0, nc;  // n0: first weight row of the workgroup; c0 / nc: chunk range
   int n_store;                         // first weight row whose outputs the workgroup stores (n0 where Nrows is whole row blocks)
   unsigned at;                         // number of the workgroup where both modalities are there, visual ones first
+  int ahead;                           // four wavefronts: weight rows from the first row block to the second, 0: there is no second
 };
 
 // xs: [2][NTM * 16 token rows][16 pieces] 16-byte slots; wst: this wavefront's [2 tiles][16 rows][16 pieces].
 template <int NTM, bool DUAL, int kTWaves, int kTD, bool XDMA, int FORM>
 __device__ __forceinline__ void tile_rows(const StreamArgs& a, const TileJob& t, const int* s_perm, u32x4_t* xs,
                                           u32x4_t* wst) {
-  constexpr bool RAGGED = FORM != FORM_WHOLE;
+  constexpr bool RAGGED = FORM != FORM_WHOLE, WIDE = kTWaves == kWideWaves;
+  static_assert(!WIDE || (DUAL && !RAGGED && XDMA), "four wavefronts: whole up projections");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 15, lq = lane >> 4;
   const int64_t kbase = (int64_t)t.c0 * kTK;
@@ -86,7 +101,11 @@ __device__ __forceinline__ void tile_rows(const StreamArgs& a, const TileJob& t,
   // weight tiles of this wavefront
   int rbase[2];
   const uint16_t* wp[2];
-  if (DUAL) {
+  if (WIDE) {
+    rbase[0] = rbase[1] = t.n0 + (wave & 1) * 16 + (wave >> 1) * t.ahead;
+    wp[0] = a.W0[t.grp];
+    wp[1] = a.W1[t.grp];
+  } else if (DUAL) {
     rbase[0] = rbase[1] = t.n0 + wave * 16;
     wp[0] = a.W0[t.grp];
     wp[1] = a.W1[t.grp];
@@ -135,8 +154,7 @@ __device__ __forceinline__ void tile_rows(const StreamArgs& a, const TileJob& t,
   // pull from the same few HBM channels.  Never from where the workgroup lies in the launch, which depends on the modalities that
   // are there (first_group): a row's sums are the same beside rows of the other modality and without them.
   const int nc = t.nc;
-  const unsigned spread = kTWaves == kWideWaves ? (t.at >> 3) * 11u + (t.at & 7u) * (unsigned)nc / 8u : t.at * 11u;
-  const int rot = (int)(spread % (unsigned)nc);
+  const int rot = (int)(t.at * 11u % (unsigned)nc);
   // RAGGED: a last chunk that would pass the end of the rows starts earlier, overlapping the chunk before it; what the two
   // share (overlap(c) pieces of 8 elements) is cleared in both operands' fragments, so that no product is counted twice
   // and a non-finite value meets no zero it would not meet elsewhere.
@@ -332,6 +350,7 @@ __device__ __forceinline__ void tile_rows(const StreamArgs& a, const TileJob& t,
     }
   }
 
+  if (WIDE && t.ahead == 0 && wave >= 2) return;  // (the first two wavefronts' rows again)
   // acc[w][m][v]: weight row rbase[w] + 4 * lq + v, token row m * 16 + lrow of the group.
 #pragma unroll
   for (int m = 0; m < NTM; ++m) {
@@ -385,7 +404,7 @@ __device__ __forceinline__ int route64(const uint8_t* mask, int M, int* s_perm, 
   return *s_nvis;
 }
 
-// grid.x = 2 groups x splits x row blocks (first_group).
+// grid.x = 2 groups x splits x row blocks (first_group); four wavefronts: 2 groups x wide_jobs, rounded up to whole XCDs.
 template <int NTM_MAX, bool DUAL, int kTWaves, int kTD, bool XDMA, int FORM>
 __global__ __launch_bounds__(kTWaves * kWave, 2) void stream_tile_kernel(const StreamArgs a) {
   constexpr bool RAGGED = FORM != FORM_WHOLE;
@@ -396,12 +415,28 @@ __global__ __launch_bounds__(kTWaves * kWave, 2) void stream_tile_kernel(const S
   int* s_perm = reinterpret_cast<int*>(wst_all);
   int* s_nvis_p = s_perm + kTMaxM;
   const int n_vis = route64(a.mask, a.M, s_perm, s_nvis_p);
-  constexpr int ROWS = DUAL ? 16 * kTWaves : 32 * kTWaves;
+  constexpr bool WIDE = kTWaves == kWideWaves;
+  constexpr int ROWS = (DUAL ? 16 : 32) * (WIDE ? 2 : kTWaves);
   const int row_blocks = RAGGED ? cdiv(a.Nrows, ROWS) : a.Nrows / ROWS;
   const int per_grp = row_blocks * a.splits;
   TileJob t;
-  t.grp = first_group(n_vis) ^ (int)(blockIdx.x / per_grp);
-  const int rem = blockIdx.x % per_grp;
+  int rem;
+  if (WIDE) {
+    // Every XCD takes an eighth of the jobs.
+    const int nc = a.K / kTK;
+    const WideJobs w = wide_jobs(row_blocks, nc);
+    const int per_xcd = cdiv(w.jobs, kXcds);
+    t.grp = first_group(n_vis) ^ (int)(blockIdx.x / (per_xcd * kXcds));
+    const int slot = blockIdx.x % (per_xcd * kXcds), job = slot % kXcds * per_xcd + slot / kXcds;
+    if (job >= w.jobs) return;  // (uniform over the workgroup)
+    rem = job < w.paired ? job : job + w.paired;
+    const int ahead = job < w.paired ? w.paired : nc;
+    t.ahead = rem + ahead < row_blocks ? ahead * ROWS : 0;
+  } else {
+    t.grp = first_group(n_vis) ^ (int)(blockIdx.x / per_grp);
+    rem = blockIdx.x % per_grp;
+    t.ahead = 0;
+  }
   t.split = rem / row_blocks;
   t.p0 = t.grp == 0 ? 0 : n_vis;
   t.mg = t.grp == 0 ? n_vis : a.M - n_vis;
@@ -481,7 +516,8 @@ template <int NTM_MAX>
 static void launch_tile_wide(const StreamArgs& a, hipStream_t stream) {
   constexpr int D = tile_shape(NTM_MAX, true).depth;
   constexpr bool X = tile_shape(NTM_MAX, true).dma != 0;
-  hipLaunchKernelGGL((stream_tile_kernel<NTM_MAX, true, kWideWaves, D, X, FORM_WHOLE>), dim3(2 * (a.Nrows / kWideRows)),
+  const int blocks = 2 * kXcds * cdiv(wide_jobs(a.Nrows / (kWideRows / 2), a.K / kTK).jobs, kXcds);
+  hipLaunchKernelGGL((stream_tile_kernel<NTM_MAX, true, kWideWaves, D, X, FORM_WHOLE>), dim3(blocks),
                      dim3(kWideWaves * kWave), 0, stream, a);
 }
 

@@ -382,6 +382,23 @@ def test_ffn_decode_rows_beside_the_other_modality(dev, nt, nv, d, h):
         assert torch.equal(alone, both[rows])
 
 
+# Four wavefronts (two row blocks each, alone where the last ones have no partner) sum as two do, bit for bit: rows of up to 32 alone
+# run on two.
+@pytest.mark.parametrize("d", [1024, 1408])
+@pytest.mark.parametrize("M,h", [(64, 10240), (49, 10304), (64, 10560), (48, 12288), (33, 12544)])
+def test_ffn_decode_four_wavefronts_sum_as_two(dev, M, h, d):
+    note(f"ffn decode, {M} rows on four wavefronts and in parts on two, d={d} h={h}")
+    gen = torch.Generator(device=dev).manual_seed(M + h + d)
+    rnd = lambda r, c, std: (torch.randn(r, c, generator=gen, device=dev) * std).to(torch.bfloat16)
+    W = {k: rnd(d, h, 0.05) if k[1] == "2" else rnd(h, d, 0.05) for k in ("w1", "w2", "w3", "u1", "u2", "u3")}
+    w = wl.FFNWorkload("w", rnd(M, d, 1.0), W, torch.arange(M, device=dev) % 2 == 0)
+    for mask in (w.mask, torch.ones_like(w.mask), torch.zeros_like(w.mask)):
+        whole = MaskedFFN.apply(*wl.FFNWorkload("w", w.x, W, mask).op_args())
+        for rows in torch.arange(M, device=dev).split((M + 2) // 3):
+            part = MaskedFFN.apply(*wl.FFNWorkload("p", w.x[rows], W, mask[rows]).op_args())
+            assert torch.equal(part, whole[rows])
+
+
 def test_ffn_decode_matches_tiled_path_rows(dev):
     """The same rows run as a decode call and inside a larger (tiled-path) call agree to bf16 accuracy."""
     note("ffn decode vs tiled")
