@@ -47,12 +47,7 @@ constexpr const TileShapeEntry& tile_shape(int ntm_max, bool dual) { return dual
 constexpr int kTMaxM = 64;
 // The up projection at three and four m-tiles with four wavefronts per workgroup: half the slab traffic per weight byte, which
 // above 32 rows is as much as the weights; 80 KB of LDS at four m-tiles, two workgroups per CU as with two wavefronts, and half as
-// many workgroups, so long streams only.
-// Whole call, us, two -> four wavefronts, one modality / both: M = 64, d = 4096, h = 14336 76.3 -> 71.5 / 126 -> 121.5, h = 16384
-// 80.3 -> 77.2 / 137 -> 132, h = 11008 68.7 -> 61.9 / 112 -> 107; d = 5120, h = 13824 103 -> 96.5 / 174 -> 163; d = 8192, h = 22016
-// 232 -> 210 / 356 -> 346; d = 3072, h = 10240 60.2 -> 56.5 / 92.5 -> 91; fewer rows lose with both modalities (d = 4096, h = 8960
-// 95 -> 98, d = 2560 71 -> 76).  M = 36 ... 48, where two wavefronts fit three times: d = 4096, h = 14336 72.0 -> 67.8 / 123 -> 118,
-// d = 6144 117 -> 109 / 187 -> 181, but h = 22016, d = 8192 190 -> 204 and h = 10240, d = 3072 76 -> 82 (both).
+// many workgroups.
 constexpr int kWideWaves = 4, kWideRows = 16 * kWideWaves;
 // The row blocks of a workgroup of four wavefronts: two blocks of a workgroup of two that start at the same chunk (rot), a multiple of
 // nc row blocks apart, so that every sum has the order that it has there.  Of the whole groups of nc blocks the first half goes with
@@ -67,9 +62,20 @@ __host__ __device__ constexpr WideJobs wide_jobs(int row_blocks, int nc) {
   const int paired = row_blocks / (2 * nc) * nc, rest = row_blocks - 2 * paired;
   return {paired, paired + (rest < nc ? rest : nc)};
 }
+// Where the two-wavefront kernel's workgroups (`blocks` of each modality) are past what the chip holds at once or just short of it,
+// and the others' (`jobs`) well spread: above 48 rows, where two workgroups of either kernel fit a CU, from 320 blocks to a workgroup
+// per CU, and from a tenth past two per CU to one and a half of the others; up to 48, where three of the two-wavefront kernel's do,
+// where both modalities are past those and one is less than a workgroup per CU.  Two against four wavefronts, whole call, 119 layers
+// with d = 1024 ... 8192 and h = 2 ... 3.5 d, at two row counts, one modality and both: inside the lines 1.3 to 11 % faster with one
+// modality and 0 to 6 % with both (us, M = 64, d = 4096, h = 14336 75.8 -> 72.2; M = 55 ... 61, d = 4096, h = 11008 8 / 4 %, d = 6144,
+// h = 20608 8 / 4 %), none slower.  Outside them, one modality / both: blocks 136 ... 256 14 % slower / 4 % faster; 512 ... 556 5 to
+// 20 % slower / 2 % slower to 5 % faster; above 48 rows past 384 jobs 8 % faster / 7 % slower; up to 48 rows at 274 ... 384 blocks 8 %
+// faster / 8 % slower, past 255 jobs 5 to 20 % slower / 2 % faster to 12 % slower.
 bool stream_tile_wide(int M, int Nrows, int K) {
   if (M <= 32 || M > kTMaxM || K % kTK != 0 || Nrows % kWideRows != 0) return false;
-  return M > 48 ? Nrows >= 10240 : Nrows >= 12288 && Nrows <= 16384;
+  const int blocks = Nrows / (kWideRows / 2), jobs = wide_jobs(blocks, K / kTK).jobs;
+  if (M <= 48) return blocks > 384 && jobs < 256;
+  return (blocks >= 320 && jobs <= 256) || (blocks >= 560 && jobs <= 384);
 }
 
 // FORM_WHOLE: K whole chunks, Nrows whole row blocks.  The other two (RAGGED) take any multiples of 8: the last chunk
