@@ -797,6 +797,7 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
     } else {
       out->block_m = 16 * (int)cdiv64(M, 16);
       out->block_n = stream_tile_rows_per_block((int)M, false);
+      out->waves_n = stream_tile_waves((int)M, (int)N, (int)K, false);
       out->block_k = 128;
       out->lds_stages = stream_tile_depth((int)M, false);
       out->direct_lds = stream_tile_direct((int)M, false);
@@ -821,8 +822,8 @@ int ffnk_tile_config(int op, int64_t M, int64_t K, int64_t N, ffnk_tile_config_t
     const int kind = up ? kinds.up : kinds.down;
     if (kind == STREAM_TILE) {
       // LDS-transposed streams: block_n weight rows (of each matrix) x 128-element chunks, three in flight
-      // (a workgroup of four wavefronts takes two such blocks: stream_tile_wide)
       out->block_n = stream_tile_rows_per_block((int)M, up);
+      out->waves_n = stream_tile_waves((int)M, (int)(up ? N : K), (int)(up ? K : N), up);
       out->block_k = 128;
       out->lds_stages = stream_tile_depth((int)M, up);
       out->direct_lds = stream_tile_direct((int)M, up);

@@ -132,7 +132,7 @@ bool stream_tile_down_ok(int M, int Nrows, int K);  // single-weight projection 
 bool stream_tile_any_ok(int M, int d, int h);           // extents any multiples of 8
 bool stream_tile_down_any_ok(int M, int Nrows, int K);
 int stream_tile_rows_per_block(int M, bool dual);
-bool stream_tile_wide(int M, int Nrows, int K);  // an up projection on workgroups of four wavefronts, 64 rows each
+int stream_tile_waves(int M, int Nrows, int K, bool dual);  // wavefronts of a workgroup: four take two row blocks
 int stream_tile_depth(int M, bool dual);
 int stream_tile_direct(int M, bool dual);  // 1: the token-row slab is filled by direct global->LDS loads
 int stream_tile_down_splits(int M, int d, int h);

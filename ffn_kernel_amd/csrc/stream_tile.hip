@@ -71,7 +71,7 @@ __host__ __device__ constexpr WideJobs wide_jobs(int row_blocks, int nc) {
 // h = 20608 8 / 4 %), none slower.  Outside them, one modality / both: blocks 136 ... 256 14 % slower / 4 % faster; 512 ... 556 5 to
 // 20 % slower / 2 % slower to 5 % faster; above 48 rows past 384 jobs 8 % faster / 7 % slower; up to 48 rows at 274 ... 384 blocks 8 %
 // faster / 8 % slower, past 255 jobs 5 to 20 % slower / 2 % faster to 12 % slower.
-bool stream_tile_wide(int M, int Nrows, int K) {
+static bool stream_tile_wide(int M, int Nrows, int K) {
   if (M <= 32 || M > kTMaxM || K % kTK != 0 || Nrows % kWideRows != 0) return false;
   const int blocks = Nrows / (kWideRows / 2), jobs = wide_jobs(blocks, K / kTK).jobs;
   if (M <= 48) return blocks > 384 && jobs < 256;
@@ -465,6 +465,9 @@ __global__ __launch_bounds__(kTWaves * kWave, 2) void stream_tile_kernel(const S
 static const TileShapeEntry& shape_for(int M, bool dual) { return tile_shape(cdiv(M < 1 ? 1 : M > kTMaxM ? kTMaxM : M, 16), dual); }
 
 int stream_tile_rows_per_block(int M, bool dual) { return (dual ? 16 : 32) * shape_for(M, dual).waves; }
+int stream_tile_waves(int M, int Nrows, int K, bool dual) {
+  return dual && stream_tile_wide(M, Nrows, K) ? kWideWaves : shape_for(M, dual).waves;
+}
 int stream_tile_direct(int M, bool dual) { return shape_for(M, dual).dma; }
 int stream_tile_depth(int M, bool dual) { return shape_for(M, dual).depth; }
 

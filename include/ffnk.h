@@ -69,8 +69,11 @@ enum {
 typedef struct ffnk_tile_config_t {
   int32_t path;        /* FFNK_PATH_*                                              */
   int32_t block_m;     /* token rows per workgroup tile (SwiGLU GEMM, 256 on four
-                          waves: beside tiles of 160, up to eight rounds of tiles)  */
-  int32_t block_n;     /* output columns per workgroup tile                        */
+                          waves: beside tiles of 160 and 64, up to eight rounds of
+                          tiles; single-weight forwards, 128 ... 192: the first ones
+                          of a modality 192 or 224 where that spares a last M-tile) */
+  int32_t block_n;     /* output columns per workgroup tile (128-element streams: of
+                          one row block; on four wavefronts a workgroup takes two)  */
   int32_t block_k;     /* contraction elements per LDS stage / per streamed chunk  */
   int32_t waves_m;     /* wavefront grid inside the workgroup                      */
   int32_t waves_n;

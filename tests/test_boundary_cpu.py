@@ -55,6 +55,20 @@ def test_tile_config_names_the_tile_that_runs(tile, linear, staged, dx, dw):
     assert got == [linear, staged, dx, dw]
 
 
+# Decode up projections: two or four wavefronts (two row blocks) by workgroups per CU, either side of each line.  d = 1024 (8 chunks):
+# a workgroup of four takes two row blocks but for the last up to 8; d = 4352 (34).
+@pytest.mark.parametrize("M,d,h,waves", [(32, 4096, 14336, 2), (33, 4096, 14336, 4), (64, 4096, 14336, 4), (48, 1024, 12288, 2),
+                                         (48, 1024, 12416, 4), (48, 1024, 16000, 4), (48, 1024, 16384, 2), (49, 1024, 10112, 2),
+                                         (49, 1024, 10240, 4), (64, 1024, 16384, 4), (64, 1024, 16512, 2), (64, 1024, 17792, 2),
+                                         (64, 1024, 17920, 4), (64, 1024, 24576, 4), (64, 1024, 24704, 2), (64, 4352, 15616, 4),
+                                         (64, 4352, 15872, 2)])
+def test_decode_wavefronts_are_reported(M, d, h, waves):
+    up = _lib.tile_config(_lib.OP_FFN_UP, M, d, h)
+    assert up["path"] == _lib.PATH_STREAM and (up["waves_m"], up["waves_n"], up["block_n"]) == (1, waves, 32)
+    down = _lib.tile_config(_lib.OP_FFN_DOWN, M, d, h)
+    assert (down["waves_n"], down["block_n"]) == (2, 64)
+
+
 # The tuner pins the plan it reads back from ffnk_tile_config: every tile of both kinds of GEMM must come back as itself.
 @pytest.mark.parametrize("K", [4096, 4104])
 @pytest.mark.parametrize("op,dual", [(_lib.OP_LINEAR_FWD, False), (_lib.OP_FFN_DOWN, False), (_lib.OP_FFN_UP, True)])
