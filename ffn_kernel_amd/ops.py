@@ -170,12 +170,12 @@ def set_route_cache(enabled: bool) -> bool:
 
 
 def shared_routing(mask: torch.Tensor, M: int, stream: int | None = None):
-    """The row partition for `mask` (contiguous, on a GPU), made once and shared by the calls that follow with
+    """The row partition for `mask` (M rows, on a GPU), made once and shared by the calls that follow with
     the same mask: the operations of a transformer layer all route by one mask, and each would otherwise
     launch its own partition kernel ahead of its GEMM.  The one-entry cache is keyed on the address of the
     mask's first element (the entry keeps the tensor, so the memory cannot be handed to another one), the row
     count, the version counter - every in-place write through torch bumps it, so a mask changed in place is
-    partitioned again - and the stream.  Returns None where no partition is shared: decode sizes, the cache
+    partitioned again - and the stream.  A strided mask gets a partition of its own each time.  Returns None where no partition is shared: decode sizes, the cache
     switched off, tensors without a version counter, a stream under graph capture (a captured graph must not
     point at memory this cache may drop later)."""
     routing = _shared_routing(mask, M, stream)
@@ -195,6 +195,8 @@ def _shared_routing(mask: torch.Tensor, M: int, stream: int | None = None):
         return None
     if torch.cuda.is_current_stream_capturing():
         return None
+    if mask.dim() != 1 or mask.shape[0] != M or (mask.stride(0) != 1 and M > 1):
+        return route(mask)  # (what a call of M rows at this address must not be given)
     key = (mask.data_ptr(), M, version, _stream_ptr(mask.device) if stream is None else stream)
     if _route_cache.key == key:
         return _route_cache.routing

@@ -1252,6 +1252,19 @@ def test_a_mask_changed_in_place_is_partitioned_again(dev, monkeypatch):
     assert len(calls) == 5
 
 
+def test_shared_routing_of_a_strided_mask(dev):
+    """A strided mask, and one of more rows than asked for, are partitioned as route() does, and leave nothing that a contiguous mask
+    at the same address would be given."""
+    note("shared routing: strided masks")
+    from ffn_kernel_amd import ops
+    M = 300
+    m = torch.rand(2 * M, generator=torch.Generator().manual_seed(3)).to(dev) < 0.4
+    for mask in (m[::2], m[:M], m, m[:M]):
+        got, want = ops.shared_routing(mask, M), ops.route(mask.contiguous())
+        assert got.M == want.M and torch.equal(got.perm, want.perm) and torch.equal(got.counts, want.counts)
+    assert ops.shared_routing(m[:M], M) is ops.shared_routing(m[:M], M)
+
+
 def test_routed_entry_points_reject_half_a_partition(dev):
     note("ffnk_masked_linear_fwd_routed with perm but no counts")
     lib = _lib.load()
