@@ -132,18 +132,24 @@ class Routing:
         return self
 
 
-def route(mask: torch.Tensor) -> Routing:
-    """Partition the rows by mask on the mask's device and current stream (ffnk_route)."""
+def _room(M: int, dev: torch.device) -> Routing:
+    """Memory for a partition that is still to be made."""
+    buf = torch.empty(M + 2, dtype=torch.int32, device=dev)
+    return Routing(buf[:M], buf[M:], made=False)
+
+
+def _require_route_mask(mask) -> None:
     if not isinstance(mask, torch.Tensor) or mask.dtype != torch.bool or mask.dim() != 1 or not mask.is_cuda:
         raise ValueError("route: mask must be a 1-D torch.bool tensor on a GPU")
+
+
+def route(mask: torch.Tensor) -> Routing:
+    """Partition the rows by mask on the mask's device and current stream (ffnk_route)."""
+    _require_route_mask(mask)
     M, dev = mask.shape[0], mask.device
     mask = mask if mask.stride(0) == 1 or M <= 1 else mask.contiguous()
-    buf = torch.empty(M + 2, dtype=torch.int32, device=dev)
-    routing = Routing(buf[:M], buf[M:], made=False)
-    if _route_cache.in_call:  # a call that is under way makes it
-        return routing
     with _on_device(dev):
-        return routing.make(mask, _stream_ptr(dev))
+        return _room(M, dev).make(mask, _stream_ptr(dev))
 
 
 class _RouteCache(threading.local):
@@ -152,7 +158,6 @@ class _RouteCache(threading.local):
     key = None
     mask = None     # keeps the mask's memory alive, so that its address cannot be handed to another tensor
     routing = None
-    in_call = False  # route() leaves the partition to the call that asks for it
     last = None     # the partition the last forward on this thread ran with (read back by the autograd functions)
 
 
@@ -175,18 +180,19 @@ def shared_routing(mask: torch.Tensor, M: int, stream: int | None = None):
     launch its own partition kernel ahead of its GEMM.  The one-entry cache is keyed on the address of the
     mask's first element (the entry keeps the tensor, so the memory cannot be handed to another one), the row
     count, the version counter - every in-place write through torch bumps it, so a mask changed in place is
-    partitioned again - and the stream.  A strided mask gets a partition of its own each time.  Returns None where no partition is shared: decode sizes, the cache
-    switched off, tensors without a version counter, a stream under graph capture (a captured graph must not
-    point at memory this cache may drop later)."""
-    routing = _shared_routing(mask, M, stream)
+    partitioned again - and the stream.  A strided mask gets a partition of its own each time.  Returns None
+    where no partition is shared: decode sizes, the cache switched off, tensors without a version counter, a
+    stream under graph capture (a captured graph must not point at memory this cache may drop later)."""
+    routing = _shared_routing(mask, M, stream, dense=False)
     if routing is not None:
         with _on_device(mask.device):
             routing.make(mask, _stream_ptr(mask.device) if stream is None else stream)
     return routing
 
 
-def _shared_routing(mask: torch.Tensor, M: int, stream: int | None = None):
-    """shared_routing, or the room for one that the caller has to fill: a forward fills it on its way."""
+def _shared_routing(mask: torch.Tensor, M: int, stream: int | None = None, dense: bool = True):
+    """shared_routing, or the room for one that the caller has to fill: a forward fills it on its way.  dense: the mask is known to be
+    M consecutive bytes, as every call's is."""
     if M < _ROUTED_MIN_ROWS or not _route_cache.enabled:
         return None
     try:
@@ -195,16 +201,13 @@ def _shared_routing(mask: torch.Tensor, M: int, stream: int | None = None):
         return None
     if torch.cuda.is_current_stream_capturing():
         return None
-    if mask.dim() != 1 or mask.shape[0] != M or (mask.stride(0) != 1 and M > 1):
+    if not dense and (mask.dim() != 1 or mask.shape[0] != M or mask.stride(0) != 1):
         return route(mask)  # (what a call of M rows at this address must not be given)
     key = (mask.data_ptr(), M, version, _stream_ptr(mask.device) if stream is None else stream)
     if _route_cache.key == key:
         return _route_cache.routing
-    _route_cache.in_call = True
-    try:
-        routing = route(mask)
-    finally:
-        _route_cache.in_call = False
+    _require_route_mask(mask)
+    routing = _room(M, mask.device)
     _route_cache.key, _route_cache.mask, _route_cache.routing = key, mask, routing
     return routing
 

@@ -1167,13 +1167,18 @@ def test_ffn_bwd_lean_workspace_is_enough_and_changes_nothing(dev, M, d, h, layo
 
 
 # ------------------------------------------------------------------ one row partition shared by several calls
-def _count_route_launches(monkeypatch):
-    """Count the partitions made from Python (ops.route) while the block runs."""
+def _note_partitions(monkeypatch):
+    """The partitions that calls get memory for from here on."""
     from ffn_kernel_amd import ops
-    calls = []
-    real = ops.route
-    monkeypatch.setattr(ops, "route", lambda mask: (calls.append(mask.shape[0]), real(mask))[1])
-    return calls
+    rooms = []
+    real = ops._room
+
+    def room(M, dev):
+        rooms.append(real(M, dev))
+        return rooms[-1]
+
+    monkeypatch.setattr(ops, "_room", room)
+    return rooms
 
 
 def test_routing_is_shared_between_the_calls_of_a_layer_and_with_the_backward(dev, monkeypatch):
@@ -1204,11 +1209,21 @@ def test_routing_is_shared_between_the_calls_of_a_layer_and_with_the_backward(de
         ops.set_route_cache(old)
     ops.set_route_cache(False)
     ops.set_route_cache(True)  # start from an empty cache
-    calls = _count_route_launches(monkeypatch)
+    rooms = _note_partitions(monkeypatch)
     got = layer()
-    assert calls == [M], f"one partition for the whole layer, got {calls}"
+    assert [r.M for r in rooms] == [M] and rooms[0]._struct.made == 1, "one partition for the whole layer"
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+    # ... which every call reads and none makes again: with another mask's rows in it, the results are that mask's
+    other = ops.route(~mask)
+    rooms[0].perm.copy_(other.perm)
+    rooms[0].counts.copy_(other.counts)
+    got = layer()
+    assert len(rooms) == 2 and torch.equal(rooms[0].perm, other.perm) and torch.equal(rooms[0].counts, other.counts)
+    mask.logical_not_()
+    for a, b in zip(got, layer()):
+        assert torch.equal(a, b)
+    mask.logical_not_()
     # an explicit partition works the same and bypasses the cache
     r = ops.route(mask)
     assert torch.equal(ops.masked_linear_forward(lw.x, lw.Wv.T, lw.Wt.T, mask, routing=r), want[0])
@@ -1232,7 +1247,7 @@ def test_a_mask_changed_in_place_is_partitioned_again(dev, monkeypatch):
 
     ops.set_route_cache(False)
     ops.set_route_cache(True)
-    calls = _count_route_launches(monkeypatch)
+    calls = _note_partitions(monkeypatch)
     assert_close(MaskedLinear.apply(w.x, w.Wv.T, w.Wt.T, mask), ref(mask), "first mask")
     MaskedLinear.apply(w.x, w.Wv.T, w.Wt.T, mask)
     assert len(calls) == 1
