@@ -131,6 +131,11 @@ int leave_routing(const ffnk_routing_t* rt, bool make, const uint8_t* mask, int6
   Routing unused;
   return make ? resolve_routing(rt, true, RouteWs{}, mask, M, false, stream, &unused) : FFNK_OK;
 }
+// A call that leaves the partition does so whatever its other extents are.
+int check_made(const ffnk_routing_t* made, const uint8_t* mask, int64_t M) {
+  if (!made || !made->perm || !made->counts) return fail(FFNK_E_NULL, "made, its perm or its counts is NULL");
+  return !mask && M > 0 ? fail(FFNK_E_NULL, "mask is NULL") : FFNK_OK;
+}
 // The first GEMM of a forward makes the partition (GemmArgs::mask): one launch, results by whole 16-byte chunks, up to one and a half
 // rounds of the chip.  Every workgroup then counts the mask, 0.7 us more than it takes to read a partition (64x128 tiles at
 // M = 2048, 1 us for a 256x256 tile at M = 8192), against 3 to 4 us for the launch on the device and as much again on the host:
@@ -579,7 +584,7 @@ int linear_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* Wv, c
                     size_t ws_bytes, void* stream_, const ffnk_routing_t* routing, bool make) {
   hipStream_t stream = (hipStream_t)stream_;
   if (int e = check_extents(M, K, N)) return e;
-  if (M == 0 || N == 0) return mask || M == 0 ? leave_routing(routing, make, mask, M, stream) : FFNK_OK;
+  if (M == 0 || N == 0) return leave_routing(routing, make, mask, M, stream);
   if (!x && K > 0) return fail(FFNK_E_NULL, "x is NULL");
   if ((!Wv || !Wt) && K > 0) return fail(FFNK_E_NULL, "weight pointer is NULL");
   if (!mask || !y) return fail(FFNK_E_NULL, "mask or y is NULL");
@@ -873,7 +878,7 @@ int ffnk_masked_linear_fwd_routing(const uint16_t* x, int64_t x_stride_m, const 
                                    int64_t w_stride_k, int64_t w_stride_n, const uint8_t* mask, uint16_t* y,
                                    int64_t y_stride_m, int64_t M, int64_t K, int64_t N, void* ws, size_t ws_bytes,
                                    void* stream_, const ffnk_routing_t* made) {
-  if (!made) return fail(FFNK_E_NULL, "made is NULL");
+  if (int e = check_made(made, mask, M)) return e;
   return linear_fwd_impl(x, x_stride_m, Wv, Wt, w_stride_k, w_stride_n, mask, y, y_stride_m, M, K, N, ws, ws_bytes, stream_, made, true);
 }
 
@@ -903,7 +908,7 @@ int ffn_fwd_impl(const uint16_t* x, int64_t x_stride_m, const uint16_t* W1, cons
     return hipSuccess;
   };
   if (int e = check_extents(M, d, h)) return e;
-  if (M == 0 || d == 0) return mask || M == 0 ? leave_routing(routing, make, mask, M, stream) : FFNK_OK;
+  if (M == 0 || d == 0) return leave_routing(routing, make, mask, M, stream);
   if (!x || !mask || !out) return fail(FFNK_E_NULL, "x, mask or out is NULL");
   if (h > 0 && (!W1 || !W3 || !U1 || !U3 || !W2 || !U2)) return fail(FFNK_E_NULL, "weight pointer is NULL");
   if (!aligned2(x) || !aligned2(out) || !aligned2(W1) || !aligned2(W3) || !aligned2(U1) || !aligned2(U3) ||
@@ -1077,7 +1082,7 @@ int ffnk_masked_ffn_fwd_routing(const uint16_t* x, int64_t x_stride_m, const uin
                                const uint8_t* mask, uint16_t* out, int64_t out_stride_m, uint16_t* pre,
                                int64_t pre_stride_m, int64_t M, int64_t d, int64_t h, void* ws, size_t ws_bytes,
                                void* stream_, const ffnk_routing_t* made) {
-  if (!made) return fail(FFNK_E_NULL, "made is NULL");
+  if (int e = check_made(made, mask, M)) return e;
   return ffn_fwd_impl(x, x_stride_m, W1, W3, U1, U3, up_stride_k, up_stride_n, W2, U2, down_stride_k, down_stride_n, mask,
                       out, out_stride_m, pre, pre_stride_m, M, d, h, ws, ws_bytes, stream_, nullptr, made, kAnyRoom, true);
 }

@@ -237,6 +237,22 @@ def test_ffn_save_entries_reject_bad_arguments_without_a_gpu():
     assert bwd() == -5
 
 
+def test_entries_that_leave_a_partition_refuse_what_they_cannot_fill():
+    lib = _lib.load()
+    one = ctypes.c_void_p(16)
+    whole, half = _lib.RoutingStruct(16, 16), _lib.RoutingStruct(16, None)
+    def linear(mask, made, N=64):
+        return lib.ffnk_masked_linear_fwd_routing(one, 64, one, one, 1, 64, mask, one, N, 128, 64, N, None, 0, None, made)
+    def ffn(mask, made, d=64):
+        return lib.ffnk_masked_ffn_fwd_routing(one, d, one, one, one, one, 1, d, one, one, 1, 64, mask, one, d, None, 0,
+                                               128, d, 64, None, 0, None, made)
+    for call in (linear, ffn):
+        assert call(one, None) == -1
+        for extent in (64, 0):
+            assert call(None, ctypes.byref(whole), extent) == -1
+            assert call(one, ctypes.byref(half), extent) == -1
+
+
 def test_ops_validate_inputs():
     x = torch.zeros(4, 8, dtype=torch.bfloat16)
     w = torch.zeros(8, 8, dtype=torch.bfloat16)
