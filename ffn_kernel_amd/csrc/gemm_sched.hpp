@@ -152,10 +152,11 @@ __host__ __device__ inline MixedRows mixed_rows(int rows) {
 }
 // Into how many pieces the tall tiles past the last whole round are cut: two short ones each where those and the other short ones are
 // one round, four of kQuarterRows behind whole rounds where those are one.  A round of such pieces, which share every column's weight
-// panel, ends in 0.4 (64 of them) to 0.6 (256) of a tall one's time against 0.7 for two short ones each.  The SwiGLU GEMM of
-// MaskedFFN with up to 60 tiles past whole rounds, halves -> quarters: d = 1024, h = 2048, M = 8192 (16 past two rounds) 80.2 -> 75.2 us,
+// panel, ends in 0.4 (64 of them) to 0.6 (256) of a tall one's time against 0.7 for two short ones each; the estimate puts it up to a
+// tenth higher, at the halves' where it would pass them.  The SwiGLU GEMM of MaskedFFN with up to 60 tiles past whole rounds, halves ->
+// quarters: d = 1024, h = 2048, M = 8192 (16 past two rounds) 80.2 -> 75.2 us,
 // d = 2048, h = 4672, M = 3679 (43) 132.5 -> 124.1, d = 1536, h = 3264, M = 2931 (56) 67.7 -> 62.9, d = 4096, h = 14336, M = 1100 (48)
-// 247 -> 238; calls 2 to 5 % less, others the same.
+// 247 -> 238; calls 2 to 5 % less, others the same; with 62 to 64 of them (d = 4096, h = 8192, M = 1280, one modality 224.6 -> 218.8) 3 to 4 %.
 constexpr int kQuarterCost = 96, kQuarterRest = 21;  // of a round of pieces, and what each cut tile adds to it in 16ths
 __host__ __device__ inline int mixed_pieces(int tall, int shrt) {
   const int rest = tall % kCusPerChip;
@@ -167,7 +168,8 @@ __host__ __device__ inline int mixed_pieces(int tall, int shrt) {
 __host__ __device__ inline int mixed_time(int tall, int shrt) {
   static_assert(kTallCost == kCusPerChip, "a shift less");
   const int rest = tall % kCusPerChip, done = tall - rest, pieces = mixed_pieces(tall, shrt);
-  if (pieces == 4) return done + kQuarterCost + rest * kQuarterRest / 16;
+  const int quarters = kQuarterCost + rest * kQuarterRest / 16;
+  if (pieces == 4) return done + (quarters < kShortCost ? quarters : kShortCost);
   if (pieces == 2) return done + kShortCost;
   if (rest == 0) return done + cdiv(shrt, kCusPerChip) * kShortCost;
   if (shrt <= kCusPerChip - rest) return done + kTallCost;

@@ -40,6 +40,8 @@ void hc_mixed_tile(int bid, int n_vis, int M, int N, int bn, int group, int* out
   out[0] = t.grp; out[1] = t.row0; out[2] = end < t.row_end ? end : t.row_end; out[3] = t.n0;
 }
 
+int hc_mixed_time(int tall, int shrt) { return mixed_time(tall, shrt); }
+
 // Tiles of a launch with taller tiles among the others: how many; tile L: {group, first row, end, first column}.
 int hc_may_stretch(int M, int tiles_n, int base, int tall, int slots) { return may_stretch(M, tiles_n, {base, tall, slots}) ? 1 : 0; }
 int hc_stretch_tiles(int n_vis, int M, int tiles_n, int base, int tall, int slots) {

@@ -266,6 +266,12 @@ def test_the_swiglu_derivative_divides(tmp_path):
     assert [asm.count(i) for i in ("v_rcp_f32", "v_div_fmas_f32", "v_div_fixup_f32")] == [8, 8, 8]
 
 
+# The estimate agrees with the schedule: what is cut into four is nowhere put above two short pieces each (176 of a tall tile's 256).
+def test_quarters_are_not_priced_above_halves(rules):
+    times = [rules.hc_mixed_time(256 + rest, 0) for rest in range(1, 65)]
+    assert times == sorted(times) and times[-1] <= 256 + 176 == rules.hc_mixed_time(256 + 65, 0)
+
+
 # Taller tiles among the others of a launch: every result in one tile, no more tiles than without, whole rounds where one
 # M-tile less makes them, and no stretch that the host's launch does not allow for.
 @pytest.mark.parametrize("base,tall", [(128, 192), (160, 192), (192, 224)])
