@@ -89,6 +89,24 @@ def test_linear_forward_makes_the_partition(dev, M, tile):
         _lib.load().ffnk_debug_force_tile(old)
 
 
+# Launches with taller tiles among the others (csrc/gemm_sched.hpp: stretch_rows): a round of the chip and one M-tile more, the last
+# M-tile of either modality spread over one taller tile, several and as many as there are, and of a modality with too few.
+@pytest.mark.parametrize("tile,base,N,splits,K", [(2, 128, 8192, 1, 192), (6, 128, 8192, 1, 192), (6, 128, 4096, 2, 712),
+                                                  (16, 192, 8192, 1, 192), (17, 160, 8192, 1, 192), (17, 160, 4096, 2, 712)])
+def test_stretched_forward_makes_the_partition(dev, tile, base, N, splits, K):
+    M = 8 * base
+    x, W = _randn((M, K), 1, dev), [_randn((N, K), 2, dev), _randn((N, K), 3, dev)]
+    old = _lib.load().ffnk_debug_force_tile(tile), _lib.load().ffnk_debug_force_splits(splits)
+    try:
+        for n_vis in (1, base, base + 1, 4 * base - 100, 4 * base - 1, 4 * base, 4 * base + 1, 4 * base + 33, 4 * base + 100, M - base - 1, M - 1, M):
+            note(f"self-routed linear with taller tiles, tile={tile} splits={splits} {n_vis} of {M} visual")
+            mask = (torch.randperm(M, generator=torch.Generator().manual_seed(n_vis)) < n_vis).to(dev)
+            _check_same(str(n_vis), _linear(x, W, mask, N), mask, dev)
+    finally:
+        _lib.load().ffnk_debug_force_tile(old[0])
+        _lib.load().ffnk_debug_force_splits(old[1])
+
+
 def test_split_contraction_and_unaligned_mask(dev):
     M, K, N = 333, 4096, 256
     x, W = _randn((M, K), 1, dev), [_randn((N, K), 2, dev), _randn((N, K), 3, dev)]
