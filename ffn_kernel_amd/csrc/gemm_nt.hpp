@@ -115,7 +115,7 @@ struct RoutedGemmCfg {
   // weight panel's (acc_col).  Same products in the same order.  Weight-gradient kernels, see splitk_store.
   static constexpr bool SWAP = SWAP_;
   static constexpr int NWAVES = WAVES_M * WAVES_N;
-  // Can make the row partition itself (GemmArgs::mask).  Not the single-weight four-wave 256x256 tile, which has no registers left
+  // Has kernels that make the row partition themselves (GemmArgs::mask), SELF below.  Not the single-weight four-wave 256x256 tile, which has no registers left
   // and is for long contractions past a round of the chip.
   static constexpr bool SELF_ROUTED = GATHER_A_ && DIRECT_ && !B_KMAJOR_ && (DUAL_ || (SCATTER_C_ && !(BM_ == 256 && NWAVES == 4)));
   static constexpr int NT = NWAVES * kWave;
@@ -1415,7 +1415,7 @@ __device__ __forceinline__ void swiglu_bwd_epilogue(const GemmArgs& g, typename 
 
 // Epilogue shared by the routed kernels.  Per accumulator tile a lane holds token row lr and the output
 // columns acc_col(v, lh), i.e. runs of four consecutive columns.
-template <class Cfg>
+template <class Cfg, bool SELF = false>
 __device__ __forceinline__ void routed_epilogue(const GemmArgs& g, typename Cfg::Acc (&acc)[Cfg::TM][Cfg::TN], int row0,
                                                 int row_end, int n0, const TileLanes<Cfg>& tl, uint8_t* lds,
                                                 const int (&self_rows)[WaveRows<Cfg>::ROW_REGS]) {
@@ -1439,7 +1439,7 @@ __device__ __forceinline__ void routed_epilogue(const GemmArgs& g, typename Cfg:
 #pragma unroll
     for (int q = 0; q < W::ROW_REGS; ++q) {
       const int p = p0 + q * kWave + tl.lane;
-      if (Cfg::SELF_ROUTED && Cfg::SCATTER_C && g.mask != nullptr) rows[q] = self_rows[q];
+      if (SELF && Cfg::SCATTER_C) rows[q] = self_rows[q];
       else rows[q] = p < row_end && q * kWave + tl.lane < W::ROWS ? (Cfg::SCATTER_C ? g.perm[p] : p) : -1;
     }
     dma_wait_barrier<0>();  // every wave has read its last fragments
@@ -1556,8 +1556,8 @@ __device__ __forceinline__ void routed_partial_store(float* base, int64_t ld, co
   }
 }
 
-// One tile of a routed GEMM (tc), or one of `splits` K ranges of it.
-template <class Cfg>
+// One tile of a routed GEMM (tc), or one of `splits` K ranges of it.  SELF: its rows come from `scan` (GemmArgs::mask).
+template <class Cfg, bool SELF>
 __device__ __forceinline__ void routed_tile(const GemmArgs& g, uint8_t* lds, const TileCoord& tc, const int split, const int splits,
                                             const int tail_slot, const RowScan<Cfg::NT>& scan) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN;
@@ -1589,31 +1589,29 @@ __device__ __forceinline__ void routed_tile(const GemmArgs& g, uint8_t* lds, con
     for (int j = 0; j < NJA; ++j) {
       int p = row0 + rl.load_row(j);
       p = min(p, row_end - 1);  // rows past the group end repeat the last row; never stored
-      src[j] = !Cfg::GATHER_A ? p - row0 : Cfg::SELF_ROUTED && g.mask != nullptr ? 0 : g.perm[p];
+      src[j] = !Cfg::GATHER_A ? p - row0 : SELF ? 0 : g.perm[p];
       baseA[j] = a0;
     }
-    int self_rows[WaveRows<Cfg>::ROW_REGS];  // GemmArgs::mask: what the epilogue would read from perm
+    int self_rows[WaveRows<Cfg>::ROW_REGS];  // SELF: what the epilogue would read from perm
     auto offsets_a = [&]() {
-      if constexpr (Cfg::SELF_ROUTED) {
-        if (g.mask != nullptr) {
-          // The rows go through the token panel's first stage, which no load has been issued for yet.
-          using Scan = RowScan<Cfg::NT>;
-          const int n = min(row_end - row0, BM);
-          scan.place(grp, row0, row0 + n, lds);
-          dma_wait_barrier<63>();
+      if constexpr (SELF) {
+        // The rows go through the token panel's first stage, which no load has been issued for yet.
+        using Scan = RowScan<Cfg::NT>;
+        const int n = min(row_end - row0, BM);
+        scan.place(grp, row0, row0 + n, lds);
+        dma_wait_barrier<63>();
 #pragma unroll
-          for (int j = 0; j < NJA; ++j) src[j] = Scan::row(lds, min(rl.load_row(j), n - 1));
+        for (int j = 0; j < NJA; ++j) src[j] = Scan::row(lds, min(rl.load_row(j), n - 1));
 #pragma unroll
-          for (int q = 0; q < WaveRows<Cfg>::ROW_REGS; ++q) {
-            const int r = q * kWave + rl.lane, p = rl.wm * Cfg::WTM + r;
-            self_rows[q] = Cfg::SCATTER_C && p < n && r < WaveRows<Cfg>::ROWS ? Scan::row(lds, min(p, n - 1)) : -1;
-          }
-          if (n0 == 0 && split == 0) {  // one workgroup per row leaves the partition to the launches behind this one
-            int32_t* perm = const_cast<int32_t*>(g.perm);
-            for (int p = (int)threadIdx.x; p < n; p += Cfg::NT) perm[row0 + p] = Scan::row(lds, p);
-          }
-          dma_wait_barrier<63>();
+        for (int q = 0; q < WaveRows<Cfg>::ROW_REGS; ++q) {
+          const int r = q * kWave + rl.lane, p = rl.wm * Cfg::WTM + r;
+          self_rows[q] = Cfg::SCATTER_C && p < n && r < WaveRows<Cfg>::ROWS ? Scan::row(lds, min(p, n - 1)) : -1;
         }
+        if (n0 == 0 && split == 0) {  // one workgroup per row leaves the partition to the launches behind this one
+          int32_t* perm = const_cast<int32_t*>(g.perm);
+          for (int p = (int)threadIdx.x; p < n; p += Cfg::NT) perm[row0 + p] = Scan::row(lds, p);
+        }
+        dma_wait_barrier<63>();
       }
 #pragma unroll
       for (int j = 0; j < NJA; ++j) offA[j] = (uint32_t)(((int64_t)src[j] * g.lda + rl.c_log * 8) * 2);
@@ -1657,7 +1655,7 @@ __device__ __forceinline__ void routed_tile(const GemmArgs& g, uint8_t* lds, con
       else
         routed_partial_store<Cfg>(g.P + (int64_t)split * g.M * g.N, g.N, g, acc, row0, row_end, n0, rl.wm, rl.wn, rl.lr, rl.lh);
     } else {
-      routed_epilogue<Cfg>(g, acc, row0, row_end, n0, rl, lds, self_rows);
+      routed_epilogue<Cfg, SELF>(g, acc, row0, row_end, n0, rl, lds, self_rows);
     }
   } else {
     constexpr int NJA = TileLanes<Cfg>::NJA, NJB = TileLanes<Cfg>::NJB;
@@ -1685,21 +1683,20 @@ __device__ __forceinline__ void routed_tile(const GemmArgs& g, uint8_t* lds, con
   }
 }
 
-// Visual rows: from the partition, or counted here (GemmArgs::mask).  `bid`: the workgroup's index in the GEMM.
-template <class Cfg>
+// Visual rows: from the partition, or counted here (SELF).  `bid`: the workgroup's index in the GEMM.
+template <class Cfg, bool SELF>
 __device__ __forceinline__ int visual_rows(const GemmArgs& g, uint8_t* lds, const int bid, RowScan<Cfg::NT>& scan) {
-  if constexpr (Cfg::SELF_ROUTED) {
-    if (g.mask != nullptr) {
-      scan.scan(g.mask, g.M, lds);
-      if (bid == 0 && threadIdx.x == 0) {
-        int32_t* counts = const_cast<int32_t*>(g.counts);
-        counts[0] = scan.n_vis;
-        counts[1] = g.M - scan.n_vis;
-      }
-      return scan.n_vis;
+  if constexpr (SELF) {
+    scan.scan(g.mask, g.M, lds);
+    if (bid == 0 && threadIdx.x == 0) {
+      int32_t* counts = const_cast<int32_t*>(g.counts);
+      counts[0] = scan.n_vis;
+      counts[1] = g.M - scan.n_vis;
     }
+    return scan.n_vis;
+  } else {
+    return g.counts[0];
   }
-  return g.counts[0];
 }
 
 // Routed GEMM: rows in routed order, group-pure tiles.
@@ -1708,7 +1705,7 @@ __device__ __forceinline__ int visual_rows(const GemmArgs& g, uint8_t* lds, cons
 //   DUAL     : C = silu(A B0^T) * (A B1^T)   (SwiGLU epilogue in fp32 registers)
 // `bid`: the workgroup's index among those of this GEMM (the launch's block index, or its offset inside a
 // launch that runs several GEMMs side by side); `lds`: Cfg::LDS_BYTES, 1 KB aligned.
-template <class Cfg>
+template <class Cfg, bool SELF = false>
 __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds, const int bid) {
   constexpr int BM = Cfg::BM;
 
@@ -1716,7 +1713,7 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
   const int SBM = g.sched_bm > 0 ? g.sched_bm : BM;
   const int SBN = g.sched_bn > 0 ? g.sched_bn : Cfg::BN_OUT;
   RowScan<Cfg::NT> scan;
-  const int n_vis = visual_rows<Cfg>(g, lds, bid, scan);
+  const int n_vis = visual_rows<Cfg, SELF>(g, lds, bid, scan);
   const int total = routed_tile_count(n_vis, g.M, g.N, SBM, SBN);
   int L, sub_m = 0, sub_n = 0, split = 0, splits = 1, tail_slot = 0;
   if (g.tail_mode == 0) {
@@ -1751,14 +1748,16 @@ __device__ __forceinline__ void routed_gemm_body(const GemmArgs& g, uint8_t* lds
   tc.row0 += sub_m * BM;
   tc.n0 += sub_n * Cfg::BN_OUT;
   if (tc.row0 >= tc.row_end || tc.n0 >= g.N) return;  // a sub-tile past the edge of a partial macro tile
-  routed_tile<Cfg>(g, lds, tc, split, splits, tail_slot, scan);
+  routed_tile<Cfg, SELF>(g, lds, tc, split, splits, tail_slot, scan);
 }
 
 
-template <class Cfg>
+// SELF is a kernel of its own: with both in one, chosen by g.mask, launches that read a partition paid for the other's code (the SwiGLU
+// GEMM of MaskedFFN d = 1024, h = 2048, M = 32768 260.7 us, without 256.5; d = 512, h = 1536, M = 16384 78.0, 76.2).
+template <class Cfg, bool SELF>
 __global__ __launch_bounds__(Cfg::NT) void routed_gemm_kernel(const GemmArgs g) {
   __shared__ __attribute__((aligned(1024))) uint8_t lds[Cfg::LDS_BYTES];
-  routed_gemm_body<Cfg>(g, lds, (int)blockIdx.x);
+  routed_gemm_body<Cfg, SELF>(g, lds, (int)blockIdx.x);
 }
 
 // Store a weight-gradient tile: bf16 with the caller's strides when the contraction was not split, fp32 partials
@@ -1931,14 +1930,14 @@ __global__ __launch_bounds__(CfgDx::NT) void fused_bwd_kernel(const GemmArgs gx,
 
 // Tiles of two heights in one launch (mixed_rows): every XCD takes an eighth of the tall tiles' order, then an eighth of the
 // short ones'.
-template <class Tall, class Short, class Quarter>
+template <class Tall, class Short, class Quarter, bool SELF>
 __global__ __launch_bounds__(Tall::NT) void routed_mixed_kernel(const GemmArgs g) {
   static_assert(Tall::NT == Short::NT && Tall::BN_OUT == Short::BN_OUT && Tall::BM == kTallRows && Short::BM == kShortRows, "two heights");
   static_assert(Tall::NT == Quarter::NT && Tall::BN_OUT == Quarter::BN_OUT && Quarter::BM == kQuarterRows && Quarter::LDS_BYTES <= Short::LDS_BYTES, "pieces");
   __shared__ __attribute__((aligned(1024))) uint8_t lds[Tall::LDS_BYTES > Short::LDS_BYTES ? Tall::LDS_BYTES : Short::LDS_BYTES];
   bool is_tall, is_quarter = false;
   RowScan<Tall::NT> scan;
-  const int n_vis = visual_rows<Tall>(g, lds, (int)blockIdx.x, scan);
+  const int n_vis = visual_rows<Tall, SELF>(g, lds, (int)blockIdx.x, scan);
   TileCoord tc = mixed_tile_coord((int)blockIdx.x, n_vis, g.M, g.N, Tall::BN_OUT, g.group_m > 0 ? g.group_m : Tall::GROUP_M, &is_tall, &is_quarter);
   if (tc.grp < 0) return;
   // (the compiler takes them for values of a lane and would load the weights' addresses through the vector memory path)
@@ -1946,20 +1945,20 @@ __global__ __launch_bounds__(Tall::NT) void routed_mixed_kernel(const GemmArgs g
   tc.row0 = __builtin_amdgcn_readfirstlane(tc.row0);
   tc.row_end = __builtin_amdgcn_readfirstlane(tc.row_end);
   tc.n0 = __builtin_amdgcn_readfirstlane(tc.n0);
-  if (is_tall) routed_tile<Tall>(g, lds, tc, 0, 1, 0, scan);
-  else if (is_quarter) routed_tile<Quarter>(g, lds, tc, 0, 1, 0, scan);
-  else routed_tile<Short>(g, lds, tc, 0, 1, 0, scan);
+  if (is_tall) routed_tile<Tall, SELF>(g, lds, tc, 0, 1, 0, scan);
+  else if (is_quarter) routed_tile<Quarter, SELF>(g, lds, tc, 0, 1, 0, scan);
+  else routed_tile<Short, SELF>(g, lds, tc, 0, 1, 0, scan);
 }
 
 // Taller tiles among the others (stretch_rows).
-template <class Tall, class Base, int SLOTS>
+template <class Tall, class Base, int SLOTS, bool SELF>
 __global__ __launch_bounds__(Base::NT) void routed_stretch_kernel(const GemmArgs g) {
   static_assert(Tall::NT == Base::NT && Tall::BN_OUT == Base::BN_OUT && Tall::BM > Base::BM, "two heights");
   constexpr StretchShape shape{Base::BM, Tall::BM, SLOTS};
   __shared__ __attribute__((aligned(1024))) uint8_t lds[Tall::LDS_BYTES > Base::LDS_BYTES ? Tall::LDS_BYTES : Base::LDS_BYTES];
   static_assert(sizeof(lds) * (SLOTS / kCusPerChip) <= 160 * 1024, "workgroups per CU");
   RowScan<Base::NT> scan;
-  const int n_vis = visual_rows<Base>(g, lds, (int)blockIdx.x, scan);
+  const int n_vis = visual_rows<Base, SELF>(g, lds, (int)blockIdx.x, scan);
   const int tiles_n = cdiv(g.N, Base::BN_OUT);
   const int splits = g.splits > 1 ? routed_splits(n_vis, g.M, Base::BM, g.splits, g.splits_more) : 1;
   const Stretch s = stretch_rows(n_vis, g.M, tiles_n * splits, shape);
@@ -1974,8 +1973,8 @@ __global__ __launch_bounds__(Base::NT) void routed_stretch_kernel(const GemmArgs
   tc.row0 = __builtin_amdgcn_readfirstlane(tc.row0);
   tc.row_end = __builtin_amdgcn_readfirstlane(tc.row_end);
   tc.n0 = __builtin_amdgcn_readfirstlane(tc.n0);
-  if (is_tall) routed_tile<Tall>(g, lds, tc, split, splits, 0, scan);
-  else routed_tile<Base>(g, lds, tc, split, splits, 0, scan);
+  if (is_tall) routed_tile<Tall, SELF>(g, lds, tc, split, splits, 0, scan);
+  else routed_tile<Base, SELF>(g, lds, tc, split, splits, 0, scan);
 }
 
 // Upper bound on the number of workgroups the kernel needs, rounded so that every XCD gets the
@@ -2015,7 +2014,13 @@ inline hipError_t launch_routed_gemm(const GemmArgs& g, hipStream_t stream) {
   if (g.M <= 0 || g.N <= 0) return hipSuccess;
   if (!routed_gemm_args_ok<Cfg>(g)) return hipErrorInvalidValue;
   const int grid = routed_gemm_grid<Cfg>(g.M, g.N, g.splits, g.splits_more);
-  hipLaunchKernelGGL(routed_gemm_kernel<Cfg>, dim3(grid), dim3(Cfg::NT), 0, stream, g);
+  if constexpr (Cfg::SELF_ROUTED) {
+    if (g.mask != nullptr) {
+      hipLaunchKernelGGL((routed_gemm_kernel<Cfg, true>), dim3(grid), dim3(Cfg::NT), 0, stream, g);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((routed_gemm_kernel<Cfg, false>), dim3(grid), dim3(Cfg::NT), 0, stream, g);
   return hipGetLastError();
 }
 
@@ -2023,7 +2028,14 @@ template <class Tall, class Base, int SLOTS>
 inline hipError_t launch_routed_stretch(const GemmArgs& g, hipStream_t stream) {
   if (g.M <= 0 || g.N <= 0) return hipSuccess;
   if (!routed_gemm_args_ok<Base>(g) || g.tail_mode != 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((routed_stretch_kernel<Tall, Base, SLOTS>), dim3(routed_gemm_grid<Base>(g.M, g.N, g.splits, g.splits_more)), dim3(Base::NT), 0, stream, g);
+  const dim3 grid(routed_gemm_grid<Base>(g.M, g.N, g.splits, g.splits_more));
+  if constexpr (Base::SELF_ROUTED) {
+    if (g.mask != nullptr) {
+      hipLaunchKernelGGL((routed_stretch_kernel<Tall, Base, SLOTS, true>), grid, dim3(Base::NT), 0, stream, g);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((routed_stretch_kernel<Tall, Base, SLOTS, false>), grid, dim3(Base::NT), 0, stream, g);
   return hipGetLastError();
 }
 
@@ -2033,7 +2045,9 @@ inline hipError_t launch_routed_mixed(const GemmArgs& g, hipStream_t stream) {
   if (g.splits > 1 || g.splits_more > 1 || g.tail_mode != 0 || g.P_tail != nullptr || g.k_switch != 0 || !direct_slabs_ok(g.K) ||
       !self_routed_args_ok<Tall>(g))
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL((routed_mixed_kernel<Tall, Short, Quarter>), dim3(mixed_blocks(g.M, g.N, Tall::BN_OUT)), dim3(Tall::NT), 0, stream, g);
+  const dim3 grid(mixed_blocks(g.M, g.N, Tall::BN_OUT));
+  if (g.mask != nullptr) hipLaunchKernelGGL((routed_mixed_kernel<Tall, Short, Quarter, true>), grid, dim3(Tall::NT), 0, stream, g);
+  else hipLaunchKernelGGL((routed_mixed_kernel<Tall, Short, Quarter, false>), grid, dim3(Tall::NT), 0, stream, g);
   return hipGetLastError();
 }
 

@@ -148,7 +148,7 @@ inline hipError_t dispatch_big_tile_with_tail(const GemmArgs& g, hipStream_t str
     // Split tail: the remaining tiles on the big tile, each cut into K ranges (at most kTailSlots
     // (tile, range) pairs), then the reduce pass.
     a.tail_mode = 3;
-    hipLaunchKernelGGL(routed_gemm_kernel<Big>, dim3(kTailSlots), dim3(Big::NT), 0, stream, a);
+    hipLaunchKernelGGL((routed_gemm_kernel<Big, false>), dim3(kTailSlots), dim3(Big::NT), 0, stream, a);
     if (hipError_t e = hipGetLastError()) return e;
     return launch_routed_tail_reduce(g.P_tail, g.M, g.N, g.K, g.counts, g.perm, Big::BM, Big::BN_OUT, g.group_m > 0 ? g.group_m : Big::GROUP_M, g.C,
                                      g.ldc, stream);
@@ -157,7 +157,7 @@ inline hipError_t dispatch_big_tile_with_tail(const GemmArgs& g, hipStream_t str
   a.sched_bm = Big::BM;
   a.sched_bn = Big::BN_OUT;
   constexpr int q = (Big::BM / Small::BM) * (Big::BN_OUT / Small::BN_OUT);
-  hipLaunchKernelGGL(routed_gemm_kernel<Small>, dim3(kCusPerChip / 2 * q), dim3(Small::NT), 0, stream, a);
+  hipLaunchKernelGGL((routed_gemm_kernel<Small, false>), dim3(kCusPerChip / 2 * q), dim3(Small::NT), 0, stream, a);
   return hipGetLastError();
 }
 
