@@ -152,25 +152,22 @@ __host__ __device__ inline MixedRows mixed_rows(int rows) {
 }
 // Into how many pieces the tall tiles past the last whole round are cut: two short ones each where those and the other short ones are
 // one round, four of kQuarterRows behind whole rounds where those are one.  A round of such pieces, which share every column's weight
-// panel, ends in 0.4 (64 of them) to 0.6 (256) of a tall one's time against 0.7 for two short ones each; the estimate puts it up to a
-// tenth higher, at the halves' where it would pass them.  The SwiGLU GEMM of MaskedFFN with up to 60 tiles past whole rounds, halves ->
-// quarters: d = 1024, h = 2048, M = 8192 (16 past two rounds) 80.2 -> 75.2 us,
-// d = 2048, h = 4672, M = 3679 (43) 132.5 -> 124.1, d = 1536, h = 3264, M = 2931 (56) 67.7 -> 62.9, d = 4096, h = 14336, M = 1100 (48)
-// 247 -> 238; calls 2 to 5 % less, others the same; with 62 to 64 of them (d = 4096, h = 8192, M = 1280, one modality 224.6 -> 218.8) 3 to 4 %.
-constexpr int kQuarterCost = 96, kQuarterRest = 21;  // of a round of pieces, and what each cut tile adds to it in 16ths
+// panel, ends in 0.4 (64 of them) to 0.6 (256) of a tall one's time against 0.7 for two short ones each: MaskedFFN with 1 to 64 tiles past
+// whole rounds, whole call, halves -> quarters: d = 1024, h = 2368, M = 6959 (20) 112.6 -> 107.6 us, d = 2048, h = 4480, M = 3818 (13)
+// 196.6 -> 188.7, d = 1536, h = 3456, M = 2383 (14) 100.5 -> 96.4, d = 4096, h = 8192, M = 1280 (64) 224.6 -> 218.8.
 __host__ __device__ inline int mixed_pieces(int tall, int shrt) {
   const int rest = tall % kCusPerChip;
   if (rest == 0) return 1;
   if (shrt == 0 && tall > rest && 4 * rest <= kCusPerChip) return 4;
   return 2 * rest + shrt <= kCusPerChip ? 2 : 1;
 }
-// When the last CU is done: tall tiles first, a CU that is free takes the next tile.
+// When the last CU is done: tall tiles first, a CU that is free takes the next tile.  Quarters at the price of halves: at their own,
+// tiles of one height were taken where two heights are the faster (d = 3072, h = 8256, M = 1872, spans 301 us against 283; of 240 calls of
+// 60 layers 24 then ran more than 1 % slower than without quarters, the worst 7 %, and 10 so, the worst 2 %; as many gained).
 __host__ __device__ inline int mixed_time(int tall, int shrt) {
   static_assert(kTallCost == kCusPerChip, "a shift less");
-  const int rest = tall % kCusPerChip, done = tall - rest, pieces = mixed_pieces(tall, shrt);
-  const int quarters = kQuarterCost + rest * kQuarterRest / 16;
-  if (pieces == 4) return done + (quarters < kShortCost ? quarters : kShortCost);
-  if (pieces == 2) return done + kShortCost;
+  const int rest = tall % kCusPerChip, done = tall - rest;
+  if (mixed_pieces(tall, shrt) > 1) return done + kShortCost;
   if (rest == 0) return done + cdiv(shrt, kCusPerChip) * kShortCost;
   if (shrt <= kCusPerChip - rest) return done + kTallCost;
   return done + (rest * kTallCost + shrt * kShortCost) / kCusPerChip + kShortCost / 2;  // (the last tiles of a CU end anywhere in half a tile)

@@ -41,6 +41,11 @@ void hc_mixed_tile(int bid, int n_vis, int M, int N, int bn, int group, int* out
 }
 
 int hc_mixed_time(int tall, int shrt) { return mixed_time(tall, shrt); }
+void hc_mixed_choice(int n_vis, int M, int tiles_n, int* out) {
+  MixedRows v, x;
+  mixed_choice(n_vis, M, tiles_n, &v, &x);
+  out[0] = v.tall; out[1] = v.shrt; out[2] = x.tall; out[3] = x.shrt;
+}
 
 // Tiles of a launch with taller tiles among the others: how many; tile L: {group, first row, end, first column}.
 int hc_may_stretch(int M, int tiles_n, int base, int tall, int slots) { return may_stretch(M, tiles_n, {base, tall, slots}) ? 1 : 0; }

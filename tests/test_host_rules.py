@@ -266,10 +266,17 @@ def test_the_swiglu_derivative_divides(tmp_path):
     assert [asm.count(i) for i in ("v_rcp_f32", "v_div_fmas_f32", "v_div_fixup_f32")] == [8, 8, 8]
 
 
-# The estimate agrees with the schedule: what is cut into four is nowhere put above two short pieces each (176 of a tall tile's 256).
-def test_quarters_are_not_priced_above_halves(rules):
-    times = [rules.hc_mixed_time(256 + rest, 0) for rest in range(1, 65)]
-    assert times == sorted(times) and times[-1] <= 256 + 176 == rules.hc_mixed_time(256 + 65, 0)
+# The heights are chosen as if tiles past whole rounds were cut in two wherever they are cut (176 of a tall tile's 256).
+def test_quarters_are_priced_as_halves(rules):
+    assert {rules.hc_mixed_time(256 + rest, 0) for rest in range(1, 129)} == {256 + 176}
+
+
+# The cases that a lower price moved to tiles of one height: two heights again (tall, short M-tiles of either modality).
+@pytest.mark.parametrize("M,n_vis,h,heights", [(1024, 518, 14336, (1, 2, 2, 0)), (4339, 2231, 7296, (9, 0, 7, 2)), (3172, 1610, 7104, (6, 1, 5, 2))])
+def test_two_heights_where_they_are_faster(rules, M, n_vis, h, heights):
+    out = (ctypes.c_int * 4)()
+    rules.hc_mixed_choice(n_vis, M, -(-h // 128), out)
+    assert tuple(out) == heights
 
 
 # Taller tiles among the others of a launch: every result in one tile, no more tiles than without, whole rounds where one
