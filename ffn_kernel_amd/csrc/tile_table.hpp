@@ -222,9 +222,13 @@ inline bool routed_split_ok(int64_t K, int s) {
 // where that starts another round the times differ by up to a half.  One more it is at (M / block_m rounded up) *
 // ((M - 1) mod block_m) of the M - 1 ways to split M; masks that set every row by itself split M about evenly.  The score is
 // the product of three times: over all splits (weight 1), at an even split (weight 2), of one modality alone (weight 2).
-inline bool even_split_has_one_more(int64_t M, int64_t bm) {
-  int64_t dev = 0;  // a third of sqrt(M): how far such a mask is off an even split
+inline int even_deviation(int64_t M) {  // a third of sqrt(M): how far such a mask is off an even split
+  int dev = 0;
   while ((dev + 1) * (dev + 1) * 9 <= M) ++dev;
+  return dev;
+}
+inline bool even_split_has_one_more(int64_t M, int64_t bm) {
+  const int64_t dev = even_deviation(M);
   const int64_t visual = (M + 1) / 2 + dev < M ? (M + 1) / 2 + dev : M;
   return cdiv64(visual, bm) + cdiv64(M - visual, bm) > cdiv64(M, bm);
 }
@@ -277,10 +281,13 @@ inline size_t plan_partial_bytes(const RoutedPlan& p, int64_t M, int64_t n_out, 
 constexpr double kModelMargin = 1.03;
 // A plan on 192- or 160-row tiles replaces another, up to two rounds of the chip, where the model sees it 7 % ahead over the splits
 // of the rows, no slower with one modality and nowhere kModelMargin behind (the model puts 256- and 128-row tiles 2 - 6 % above
-// what they take, those two 1 %).  3138 timed calls of drawn single-weight GEMMs with such a plan (three masks each): 1.12 times as
-// fast as on the plan it replaced in the geometric mean, 2 % of them more than 3 % slower, 0.2 % more than 8 %.  Between two and three
-// rounds 1.03, with 23 % more than 3 % slower; by the score alone 12 % more than 3 % slower, and 4 % more than 8 %.
+// what they take, those two 1 %).  6452 drawn single-weight GEMMs with such a plan, three masks each, timed against the plans without:
+// 1.13 times as fast in the geometric mean with one modality and with both, 1.1 % of the calls more than 3 % slower (4.5 % below 12
+// slabs), 0.02 % more than 10 %.  At 16 splits of the rows instead of kSplitsOfRows, none of them even, 81 more had one: 8 % of their
+// calls more than 3 % slower, the worst by half (K = 3584, N = 6400, M = 1936, even splits: a twelfth M-tile, a second round).  Between
+// two and three rounds 1.03, with 23 % more than 3 % slower; by the score alone 12 % more than 3 % slower, and 4 % more than 8 %.
 constexpr double kForwardGain = 0.93;
+constexpr int kSplitsOfRows = 64;
 constexpr size_t kAnyRoom = ~(size_t)0;
 inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_t K, bool split, size_t room = kAnyRoom, bool forward = true) {
   constexpr int kSplits[] = {2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16}, kMaxCosts = 9;
@@ -360,30 +367,50 @@ inline RoutedPlan compute_model_plan(bool dual, int64_t M, int64_t n_out, int64_
     }
   }
   if (best < 0.0) return p;
-  const TileTimer timers[2] = {TileTimer(cost(p.tile), false, M, n_out, K), TileTimer(cost(between.tile), false, M, n_out, K)};
-  auto time_at = [&](const RoutedPlan& q, const TileTimer& t, int64_t n_vis) {
-    const int64_t bm = t.geom.block_m, tiles_m = cdiv64(n_vis, bm) + cdiv64(M - n_vis, bm);
-    const int splits = routed_splits((int)n_vis, (int)M, (int)bm, q.splits, q.splits_more);
-    bool stretch = t.stretched.part > 0.0;
-    if (stretch) {
-      const Stretch s = stretch_rows((int)n_vis, (int)M, t.tiles_n * splits, t.stretched.shape);
-      stretch = s.tall_v + s.tall_x > 0;
+  // A plan's times by M-tile count and stretch: four numbers, whatever the split of the rows.
+  struct Times {
+    TileTimer t;
+    RoutedPlan q;
+    int less;
+    bool fits[2];
+    double at[2][2];
+    Times(const TileCost& c, const RoutedPlan& plan, int64_t M, int64_t n_out, int64_t K)
+        : t(c, false, M, n_out, K), q(plan), less((int)cdiv64(M, t.geom.block_m)) {
+      for (int more = 0; more < 2; ++more) {
+        const int splits = more ? q.splits_more : q.splits;
+        fits[more] = t.stretched.part > 0.0 && stretch_fits(less + more, (int64_t)t.tiles_n * splits, t.stretched.shape.slots);
+        for (int stretch = 0; stretch <= (fits[more] ? 1 : 0); ++stretch) at[more][stretch] = t.time(less + more, 2, splits, stretch != 0);
+      }
     }
-    return t.time((int)tiles_m, n_vis < M ? 2 : 1, splits, stretch);
+    double time(int n_vis) const {
+      const int bm = t.geom.block_m, M = (int)t.M, more = cdiv(n_vis, bm) + cdiv(M - n_vis, bm) - less;
+      if (!fits[more]) return at[more][0];
+      const Stretch s = stretch_rows(n_vis, M, t.tiles_n * (more ? q.splits_more : q.splits), t.stretched.shape);
+      return at[more][s.tall_v + s.tall_x > 0 ? 1 : 0];
+    }
+    double one_modality() const {
+      const bool stretch = fits[0] && stretch_rows((int)t.M, (int)t.M, t.tiles_n * q.splits, t.stretched.shape).tall_v > 0;
+      return t.time(less, 1, q.splits, stretch);
+    }
   };
-  // One modality, and splits from one end to the other that share no remainder.
-  constexpr int kSplitsOfRows = 16;
-  const double one = time_at(between, timers[1], M) / time_at(p, timers[0], M);
+  const Times a(cost(p.tile), p, M, n_out, K), b(cost(between.tile), between, M, n_out, K);
+  const double one = b.one_modality() / a.one_modality();
   if (one > 1.0) return p;
-  double product = 1.0, gain = 1.0;
+  // About even splits (a mask that sets every row by itself is off by sqrt(M) / 2), where two partial M-tiles are one too many for a
+  // whole round more often than elsewhere ...
+  for (int i = -4; i <= 4; ++i) {
+    const int off = (int)(M / 2) + i * even_deviation(M) / 2, n_vis = off < 1 ? 1 : off < M ? off : (int)M - 1;
+    if (b.time(n_vis) >= kModelMargin * a.time(n_vis)) return p;
+  }
+  // ... and from one end to the other, no two with the same remainder.
+  double product = one, gain = kForwardGain;
   for (int i = 1; i < kSplitsOfRows; ++i) {
     const int64_t at = M * i / kSplitsOfRows + i * 37 % 61, n_vis = at < 1 ? 1 : at < M ? at : M - 1;
-    const double r = time_at(between, timers[1], n_vis) / time_at(p, timers[0], n_vis);
+    const double r = b.time((int)n_vis) / a.time((int)n_vis);
     if (r >= kModelMargin) return p;
     product *= r;
+    gain *= kForwardGain;
   }
-  product *= one;
-  for (int i = 0; i < kSplitsOfRows; ++i) gain *= kForwardGain;
   return product < gain ? between : p;
 }
 

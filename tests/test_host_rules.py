@@ -266,6 +266,14 @@ def test_the_swiglu_derivative_divides(tmp_path):
     assert [asm.count(i) for i in ("v_rcp_f32", "v_div_fmas_f32", "v_div_fixup_f32")] == [8, 8, 8]
 
 
+# 192- and 160-row tiles where one more M-tile, at a few splits of the rows, is a second round: the tiles that were there before.
+@pytest.mark.parametrize("M,K,N", [(1936, 3584, 6400), (2320, 3584, 5376), (2145, 2688, 5504), (396, 5128, 6984)])
+def test_no_second_round_at_some_splits_of_the_rows(rules, M, K, N):
+    out = (ctypes.c_int * 3)()
+    rules.hc_plan(M, N, K, 2 ** 64 - 1, out)
+    assert out[0] not in (16, 17)
+
+
 # The heights are chosen as if tiles past whole rounds were cut in two wherever they are cut (176 of a tall tile's 256).
 def test_quarters_are_priced_as_halves(rules):
     assert {rules.hc_mixed_time(256 + rest, 0) for rest in range(1, 129)} == {256 + 176}
