@@ -119,8 +119,13 @@ def summarize(out: Path, workload: str, traffic_json: Path | None, min_pct: floa
         names = sorted({k for (k, c) in per_kernel if c == "FETCH_SIZE" and pick(k)})
         if names:
             # calls of the workload in the run = dispatches of its most frequent kernel (a row partition shared
-            # between calls is launched once per run and weighs in with that share)
-            n_calls = max(len(per_kernel[(k, "FETCH_SIZE")]) for k in names)
+            # between calls is launched once per run and weighs in with that share); a GEMM that makes the partition
+            # and the same one reading it are one
+            launches = {}
+            for k in names:
+                key = re.sub(r"(routed_\w+_kernel<.*), (true|false)>\(", r"\1>(", k)
+                launches[key] = launches.get(key, 0) + len(per_kernel[(k, "FETCH_SIZE")])
+            n_calls = max(launches.values())
             fetch = sum(sum(per_kernel[(k, "FETCH_SIZE")]) for k in names) / n_calls
             write = sum(sum(per_kernel.get((k, "WRITE_SIZE"), [0.0])) for k in names) / n_calls
             nbytes = (fetch * cal["FETCH_SIZE"] + write * cal["WRITE_SIZE"]) * 1024
@@ -129,7 +134,7 @@ def summarize(out: Path, workload: str, traffic_json: Path | None, min_pct: floa
             lines += [f"  {k[:120]}" for k in names]
             lines.append(f"FETCH_SIZE {fetch:.5g} KiB x {cal['FETCH_SIZE']:.3f} + WRITE_SIZE {write:.5g} KiB x "
                          f"{cal['WRITE_SIZE']:.3f} = {nbytes / 1e6:.1f} MB")
-            dur = sum(avg_ns.get(k, 0.0) for k in names)
+            dur = sum(avg_ns.get(k, 0.0) * len(per_kernel[(k, "FETCH_SIZE")]) for k in names) / n_calls
             if dur > 0:
                 lines.append(f"over the traced {dur / 1e3:.1f} us of these kernels: {nbytes / dur:.0f} GB/s of HBM traffic")
             if traffic_json is not None:
