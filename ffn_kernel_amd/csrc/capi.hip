@@ -139,10 +139,9 @@ int check_made(const ffnk_routing_t* made, const uint8_t* mask, int64_t M) {
 // The first GEMM of a forward makes the partition (GemmArgs::mask): one launch, results by whole 16-byte chunks, up to one and a half
 // rounds of the chip.  Every workgroup then counts the mask, 0.7 us more than it takes to read a partition (64x128 tiles at
 // M = 2048, 1 us for a 256x256 tile at M = 8192), against 3 to 4 us for the launch on the device and as much again on the host:
-// MaskedLinear, masks of both modalities, K = N = 1024, M = 2048 18.0 -> 14.1 us, M = 3001, K = 2056, N = 1544 38.7 -> 36.6,
-// forward + backward at K = N = 1024, M = 8192 108-125 -> 83-117 (runs of one side differ widely); MaskedFFN d = 4096, h = 14336, M = 300 177.8 ->
-// 173.8.  Past that every tile pays: d = 1024, h = 2048, M = 8192 (2.1 rounds) 133.7 -> 135.3, d = 4096, h = 14336, M = 1411 (2.6)
-// 474.7 -> 475.3.
+// MaskedLinear, masks of both modalities, K = N = 1024, M = 2048 17.8 -> 14.0 us, M = 3001, K = 2056, N = 1544 38.8 -> 36.6; forward +
+// backward at K = N = 1024, M = 8192 and MaskedFFN d = 4096, h = 14336, M = 300 level (the runs' spread).  Past that every tile pays:
+// MaskedFFN d = 1024, h = 2048, M = 8192 (2.1 rounds) 133.7 -> 135.3, d = 4096, h = 14336, M = 1411 (2.6) 474.7 -> 475.3.
 bool gemm_routes(int tile, bool direct, bool dual, int splits, int64_t M, int64_t N, const uint8_t* mask, const uint16_t* C, int64_t ldc) {
   if (!direct || M > kScanMaxRows || !aligned16(mask) || !aligned16(C) || N % 8 != 0 || ldc % 8 != 0) return false;
   const TileGeom t = tile_geom(tile == TILE_MIXED_W4 ? TILE_256x256_W4 : tile, dual);

@@ -76,11 +76,11 @@ __host__ __device__ inline TileCoord routed_tile_coord(int L, int n_vis, int M, 
 
 // Taller tiles among the others of a launch (192 rows among 128 or 160, 224 among 192) where those end just past a whole round of
 // the chip - as the tiles of two modalities do whenever the rows of both together fill whole rounds: one M-tile goes, and its rows
-// are spread over taller ones of its modality.  A launch of 65 x 8 tiles on 512 places ran its last 8 workgroups by themselves, 13 of 31 us at K = 1024
-// and 20 of 51 at K = 2048.  Rows of both modalities mixed, weights not in a cache, 128x128 tiles: MaskedLinear M = 8192, K = N = 1024
-// 32.4 -> 23.2 us, M = 16384, K = N = 512 20.8 -> 15.0; 128x256 tiles: M = 8192, N = 1024, K = 2048 55 -> 43, K = 4096 95 -> 73,
-// M = 2048, K = N = 4096 97 -> 76, M = 4096, K = 6144, N = 2048 142 -> 103; MaskedFFN d = 1024, h = 2048, M = 8192 134.7 -> 126.1.
-// A mask that leaves whole rounds of 128-row tiles (one modality alone) runs 0 to 4 % slower than on the kernel of those alone.
+// are spread over taller ones of its modality.  (65 x 8 tiles of 128x128 on 512 places ran the last 8 by themselves, 13 of 31 us at
+// K = 1024, 20 of 51 at K = 2048.)  Rows of both modalities mixed, weights not in a cache, us: 128x128 tiles, M = 16384, K = N = 512
+// 20.9 -> 15.2, M = 32768 33.9 -> 29.8; 128x256 tiles, M = 8192, N = 1024, K = 4096 95.6 -> 74.4, M = 2048, K = N = 4096 98.0 -> 77.7,
+// M = 4096, K = 6144, N = 2048 144.4 -> 105.7.  A mask that leaves whole rounds (one modality alone) runs up to 1 % slower than on the
+// kernel of one height, 128x128 tiles over K = 512 in two rounds 2.5 % (M = 32768 29.3 -> 30.0).
 struct StretchShape {
   int base, tall;  // rows of a tile
   int slots;       // workgroups that the chip runs at once

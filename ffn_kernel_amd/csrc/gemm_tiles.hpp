@@ -23,9 +23,10 @@ struct PlainTiles {
   using T2 = RoutedGemmCfg<128, 128, 2, 2, false, GATHER, SCATTER, DIRECT, kGroupMPlain>;
   using T2Tall = RoutedGemmCfg<192, 128, 2, 2, false, GATHER, SCATTER, DIRECT, kGroupMPlain>;  // among T2, see stretch_rows
   // The heights between 128 and 256 rows fill the chip at many mid-size M where those two leave a quarter of it (us, before -> now):
-  // M = 1411, K = 14336, N = 4096 185 -> 140 (192 rows, two K ranges: 256 workgroups; before 192 of 128x256, 178 us of K loop), M = 700,
-  // K = N = 8192 113 -> 97, M = 7130, K = 7296, N = 1088 182 -> 105, M = 1848, K = 2560, N = 4352 72 -> 50.  A slab takes 0.94 us on 192 rows
-  // and 0.78 on 160 against 1.2 - 1.3 on 256 and 0.7 - 0.8 on 128.  T8 also among T6 and T9, T8Tall among T8.
+  // M = 1411, K = 14336, N = 4096 185 -> 140 (192 rows, two K ranges: 256 workgroups; before 192 of 128x256, 178 us of K loop), M = 7130,
+  // K = 7296, N = 1088 182 -> 105 (160 rows), M = 12288, K = 2048, N = 1024 48.7 -> 44.6 (192), M = 8192, K = 2048, N = 1024, one modality
+  // 40.2 -> 35.6 (160).  A slab takes 0.94 us on 192 rows and 0.78 on 160 against 1.2 - 1.3 on 256 and 0.7 - 0.8 on 128.  T8 also among T6
+  // and T9, T8Tall among T8.
   using T8 = std::conditional_t<DIRECT, RoutedGemmCfg<192, 256, 2, 2, false, GATHER, SCATTER, true, kGroupMPlain, false, 3>, T2Tall>;
   using T9 = std::conditional_t<DIRECT, RoutedGemmCfg<160, 256, 2, 2, false, GATHER, SCATTER, true, kGroupMPlain, false, 3>, T2Tall>;
   using T8Tall = std::conditional_t<DIRECT, RoutedGemmCfg<224, 256, 2, 2, false, GATHER, SCATTER, true, kGroupMPlain, false, 3>, T2Tall>;

@@ -191,7 +191,8 @@ FFNK_API int ffnk_masked_linear_fwd_routed(const uint16_t* x, int64_t x_stride_m
 
 /* ffnk_masked_linear_fwd that leaves its row partition in `made` (perm int32[M], counts int32[2], device memory) for the calls
  * behind it, as ffnk_route would write it: the first of the operations that share one.  Up to 8192 rows the GEMM makes it itself,
- * a launch less than ffnk_route and ffnk_masked_linear_fwd_routed. */
+ * a launch less than ffnk_route and ffnk_masked_linear_fwd_routed.  FFNK_E_NULL without both members or, for M > 0, without a mask,
+ * whatever the other extents are. */
 FFNK_API int ffnk_masked_linear_fwd_routing(const uint16_t* x, int64_t x_stride_m,
                                   const uint16_t* Wv, const uint16_t* Wt,
                                   int64_t w_stride_k, int64_t w_stride_n,
